@@ -30,6 +30,10 @@ struct RopeArgs {
   uint16_t* second;
   int split;
   long long out_stride, second_stride;
+  // the plain float32 modes: elements from one row of the output to the next (0: N)
+  long long row_stride;
+  // split_t operands: what the rows of x and of w were multiplied by, as powers of two
+  const int32_t *x_exp, *w_exp;
 };
 
 // Orders a wave's LDS writes before its own later reads of what other lanes wrote (and the reverse).
@@ -48,6 +52,7 @@ __device__ __forceinline__ void tile_epilogue(floatx16 (&acc)[WM][WN], float* tu
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int li = lane & 31, lk = lane >> 5;
+  const long long stride = rope.row_stride ? rope.row_stride : N;
   if (MODE == kRope) {
     // Tile columns come in groups of 64: 32 dimensions of a head's first half (tile column 2 m of a wave) and
     // their rotation partners, half a head further on (tile column 2 m + 1), so that a lane holds both of a pair.
@@ -183,7 +188,7 @@ __device__ __forceinline__ void tile_epilogue(floatx16 (&acc)[WM][WN], float* tu
           if (col < WN * 32 && nbase + col < N) {
             float v = turn[tr * PITCH + col];
             if (bias && blockIdx.z == 0) v += to_float(bias[nbase + col]);
-            unsafeAtomicAdd(reinterpret_cast<float*>(out) + size_t(tbase + tr) * N + nbase + col, v);
+            unsafeAtomicAdd(reinterpret_cast<float*>(out) + size_t(tbase + tr) * stride + nbase + col, v);
           }
         }
       wave_lds_fence();
@@ -206,8 +211,8 @@ __device__ __forceinline__ void tile_epilogue(floatx16 (&acc)[WM][WN], float* tu
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           v[r] = acc[i][j][4 * rg + r] + ((bias && blockIdx.z == 0 && n + r < N) ? to_float(bias[n + r]) : 0.f);
-        const size_t o = size_t(t) * N + n;
-        const bool whole = n + 4 <= N && (N & 3) == 0;
+        const size_t o = size_t(t) * stride + n;
+        const bool whole = n + 4 <= N && (stride & 3) == 0;
         if (MODE == kStore) {
           uint16_t* dst = reinterpret_cast<uint16_t*>(out) + o;
           if (rope.second) {

@@ -28,6 +28,14 @@ int sp_rmsnorm(void* stream, const float* x, const int32_t* rows, int w_dtype, c
 int sp_gemm(void* stream, int a_dtype, const void* a, int w_dtype, const void* w, int bias_dtype,
             const void* bias, int mode, int out_dtype, void* out, int T, int N, int K);
 
+// float32 products of many tokens as three products of float16 pairs: out[T, N] = or (mode 1) += rows . w[N, K]^T (+ bias), all
+// float32, w split once a call.  rows, by `kind`: 0: a [T, K];  1: act(a[:, :K], a[:, K:]) of a [T, 2 K] (`activation`, `limit` as
+// for sp_gate_up_silu);  2: rmsnorm(a) * norm_w.
+// sp_gemm_f32_split_bytes: the workspace it wants, 0 where it does not take the product.
+int64_t sp_gemm_f32_split_bytes(int T, int N, int K);
+int sp_gemm_f32_split(void* stream, int kind, const float* a, const float* norm_w, float eps, int activation, float limit,
+                      const float* w, int bias_dtype, const void* bias, int mode, float* out, int T, int N, int K, void* workspace, int64_t workspace_bytes);
+
 // Decode-sized products (T <= 64, bfloat16) with neighbouring work folded in.  Activations are x
 // [T, K] bfloat16, or, with residual != null, rmsnorm(residual [T, K] float32) * norm_w computed inside.
 // sp_fused_supported(kind, ...): kind 0..2 = plain modes of sp_gemm, 3 = sp_qkv_rope_cache, 4 = sp_gate_up_silu.

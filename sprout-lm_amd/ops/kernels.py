@@ -578,6 +578,41 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: torch.Tensor
                             _code(out, "gemm output"), out.data_ptr(), T, N, K))
 
 
+def gemm_f32_split_bytes(T: int, N: int, K: int) -> int:
+    """Bytes of workspace `gemm_f32_split` wants for T tokens by N rows of K, or 0 where it does not take the product."""
+    return library().sp_gemm_f32_split_bytes(T, N, K)
+
+
+def gemm_f32_split(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, workspace, bias: torch.Tensor | None = None,
+                   accumulate: bool = False, norm=None, activation: str | None = None, limit: float = 0.0) -> bool:
+    """out = (or, with accumulate, +=) rows @ w.T (+ bias), everything float32, for many tokens; rows = a, or rmsnorm(a) * weight
+    with `norm` = (weight, eps), or act(a[:, :K]) * a[:, K:] with an `activation`.  `workspace`: bytes -> a uint8 tensor.
+    Returns False (and does nothing) where the kernel does not take the product."""
+    T, (N, K) = a.shape[0], w.shape
+    if not (a.dtype == w.dtype == out.dtype == torch.float32) or tuple(out.shape) != (T, N) \
+            or a.shape[1] != (K if activation is None else 2 * K):
+        return False
+    need = gemm_f32_split_bytes(T, N, K)
+    if need == 0 or (a.data_ptr() | w.data_ptr() | out.data_ptr()) & 15:
+        return False
+    if norm is not None and (activation is not None or norm[0].dtype != torch.float32 or norm[0].numel() != K or norm[0].data_ptr() & 15):
+        return False
+    _gpu(a, "gemm input"); _gpu(w, "gemm weight"); _gpu(out, "gemm output")
+    if norm is not None:
+        _gpu(norm[0], "norm weight")
+    if bias is not None:
+        _gpu(bias, "gemm bias")
+        if bias.numel() != N:
+            raise KernelError(f"gemm: bias has {bias.numel()} values for {N} columns")
+    scratch = workspace(need)
+    check(library().sp_gemm_f32_split(
+        _stream(), 2 if norm is not None else 1 if activation is not None else 0, a.data_ptr(), _ptr(norm[0]) if norm else None,
+        float(norm[1]) if norm else 0.0, variant_code(GATE_ACTIVATIONS, activation, "gate activation") if activation else 0,
+        float(limit), w.data_ptr(), _code(bias, "gemm bias") if bias is not None else 0, _ptr(bias), int(accumulate),
+        out.data_ptr(), T, N, K, scratch.data_ptr(), scratch.numel() * scratch.element_size()))
+    return True
+
+
 def rope_cache(qkv: torch.Tensor, positions: torch.Tensor, inv_freq: torch.Tensor, rotary_dim: int, nq: int, nkv: int,
                hd: int, slot_mapping: torch.Tensor | None = None, k_pool: torch.Tensor | None = None,
                v_pool: torch.Tensor | None = None, inv_freq_tail: torch.Tensor | None = None, pairing: str = "halves") -> None:

@@ -20,6 +20,8 @@ def _declare(lib):
         "sp_embed": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_float, c_void],
         "sp_rmsnorm": [c_void, c_void, c_void, c_int, c_void, c_float, c_int, c_void, c_int, c_int],
         "sp_gemm": [c_void, c_int, c_void, c_int, c_void, c_int, c_void, c_int, c_int, c_void, c_int, c_int, c_int],
+        "sp_gemm_f32_split": [c_void, c_int, c_void, c_void, c_float, c_int, c_float, c_void, c_int, c_void, c_int,
+                              c_void, c_int, c_int, c_int, c_void, c_i64],
         "sp_rope_cache": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_int, c_int,
                           c_int, c_int, c_int, c_int, c_int],
         "sp_attention": [c_void, c_int, c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_void,
@@ -109,6 +111,8 @@ def _declare(lib):
         "sp_probe_read": [c_void, c_void, c_i64, c_int, c_void],
         "sp_probe_mfma": [c_void, c_int, c_int, c_void, ctypes.POINTER(ctypes.c_double)],
     }
+    lib.sp_gemm_f32_split_bytes.argtypes = [c_int] * 3
+    lib.sp_gemm_f32_split_bytes.restype = c_i64
     lib.sp_attention_workspace_floats.argtypes = [c_int] * 10
     lib.sp_attention_workspace_floats.restype = c_i64
     lib.sp_rglru_carry_floats.argtypes = [c_int] * 4

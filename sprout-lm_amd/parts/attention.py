@@ -108,7 +108,7 @@ class Attention(Mixer):
         if fold is None or fold.kind != "rms":       # the one prologue the projection kernels have
             return False
         if ctx.act_dtype == torch.float32:
-            return self._fused_f32(ctx, residual, residual, cache, fold)
+            return self._fused_f32(ctx, residual, residual, cache, fold) or self._split_f32(ctx, residual, cache, fold)
         if ctx.act_dtype != torch.bfloat16 or T > 64 or not self._fused(T, cache, True):
             return False
         if not ops.fused_norm_pays(T, self.w_qkv.shape[0], self.hidden):
@@ -146,7 +146,9 @@ class Attention(Mixer):
                          workspace=lambda n: ctx.buffer("attention_partials", (n,), torch.float32),
                          kind=ctx.attention_kind, project=project, scores=self.scores, softcap=self.softcap):
             return
-        ops.gemm(attn, self.w_o, residual, bias=self.b_o, accumulate=True)
+        if not ops.gemm_f32_split(attn, self.w_o, residual, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=self.b_o,
+                                  accumulate=True):
+            ops.gemm(attn, self.w_o, residual, bias=self.b_o, accumulate=True)
 
     def forward(self, ctx, h, residual, cache):
         T = h.shape[0]
@@ -161,6 +163,12 @@ class Attention(Mixer):
             return
         if ctx.act_dtype == torch.float32 and self._fused_f32(ctx, h, residual, cache):
             return
+        qkv, w, b, nkv = self._projections(ctx, T, cache)
+        ops.gemm(h, w, qkv, bias=b)
+        self._rotate_and_attend(ctx, qkv, nkv, residual, cache)
+
+    def _projections(self, ctx, T: int, cache):
+        """Where the projections go, the rows of the matrix and of the bias that the call needs, and its key/value heads."""
         nkv = self.kv_heads if (self.own_kv and cache.writes) else 0
         width = (self.heads + 2 * nkv) * self.head_dim
         qkv = ctx.buffer("qkv", (T, width), ctx.act_dtype)
@@ -168,10 +176,21 @@ class Attention(Mixer):
         if nkv == 0 and self.own_kv:   # a second call of the layer that only reads: q rows only
             w = w[: self.heads * self.head_dim]
             b = None if b is None else b[: self.heads * self.head_dim]
-        ops.gemm(h, w, qkv, bias=b)
+        return qkv, w, b, nkv
+
+    def _split_f32(self, ctx, residual, cache, fold) -> bool:
+        """Many tokens on the float32 path: the norm is folded into the projections' operand."""
+        qkv, w, b, nkv = self._projections(ctx, residual.shape[0], cache)
+        if not ops.gemm_f32_split(residual, w, qkv, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=b,
+                                  norm=(fold.weight, fold.eps)):
+            return False
+        self._rotate_and_attend(ctx, qkv, nkv, residual, cache)
+        return True
+
+    def _rotate_and_attend(self, ctx, qkv, nkv, residual, cache):
         ops.rope_cache(qkv, ctx.positions, self.position.inv_freq, self.position.rotary_dim, self.heads, nkv,
                        self.head_dim, cache.slot_mapping if nkv else None, cache.k if nkv else None,
                        cache.v if nkv else None,
                        inv_freq_tail=getattr(self.position, "inv_freq_tail", None) if qkv.dtype == torch.float32 else None,
                        pairing=self.position.pairing)
-        self._attend(ctx, qkv, width, residual, cache)
+        self._attend(ctx, qkv, qkv.shape[1], residual, cache)

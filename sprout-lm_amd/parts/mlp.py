@@ -58,7 +58,7 @@ class GatedMLP(FeedForward):
             act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
             if not ops.gate_up_silu_f32(self.w_gate_up, residual, act, activation=self.activation, norm_weight=fold.weight,
                                         eps=fold.eps, limit=self.limit):
-                return False
+                return self._split_f32(ctx, residual, fold)
             ops.gemm(act, self.w_down, residual, accumulate=True)
             return True
         if ctx.act_dtype != torch.bfloat16 or T > 64 or not self._fused(T, True):
@@ -69,6 +69,21 @@ class GatedMLP(FeedForward):
         ops.gate_up_silu(self.w_gate_up, act, residual=residual, norm_weight=fold.weight, eps=fold.eps,
                          activation=self.activation, limit=self.limit)
         ops.gemm(act, self.w_down, residual, accumulate=True)
+        return True
+
+    def _split_f32(self, ctx, residual, fold) -> bool:
+        """Many tokens on the float32 path: the norm is folded into the first product's operand, the gate into the second's."""
+        T = residual.shape[0]
+        if min(ops.gemm_f32_split_bytes(T, 2 * self.inner, self.hidden), ops.gemm_f32_split_bytes(T, self.hidden, self.inner)) == 0:
+            return False
+        scratch = lambda n: ctx.buffer("f32_split", (n,), torch.uint8)
+        gu = ctx.buffer("gate_up", (T, 2 * self.inner), ctx.act_dtype)
+        if not ops.gemm_f32_split(residual, self.w_gate_up, gu, scratch, norm=(fold.weight, fold.eps)):
+            return False
+        if not ops.gemm_f32_split(gu, self.w_down, residual, scratch, accumulate=True, activation=self.activation, limit=self.limit):
+            act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
+            ops.silu_mul(gu, act, activation=self.activation, limit=self.limit)
+            ops.gemm(act, self.w_down, residual, accumulate=True)
         return True
 
     def forward(self, ctx, h, residual, row_gate=None, row_gate_column: int = 0):

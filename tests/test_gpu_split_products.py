@@ -1,0 +1,84 @@
+"""float32 products of many tokens as products of float16 pairs, against float64 products of the same numbers."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# What the pairs, the three products and the float32 sums may lose of a sum of K products, against the sum of their
+# magnitudes: each operand is a pair to 2^-23, the product of the lower parts (2^-22) is left out, and 3 K / 16 sums of
+# sixteen products round to 2^-24 of the running sum each (their errors add up in the worst case only: a quarter of that).
+def bound(K):
+    return 3 * 2.0 ** -22 + 3 * K / 16 * 2.0 ** -24 / 4
+
+
+def rows(T, K, seed, span=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(T, K, device=DEV, generator=g)
+    if span:      # rows of very different sizes, and numbers of very different sizes within a row
+        x *= torch.exp2(torch.randint(-span, span + 1, (T, 1), device=DEV, generator=g).float())
+        x *= torch.exp2(torch.randint(-12, 1, (T, K), device=DEV, generator=g).float())
+    return x.contiguous()
+
+
+def scratch(n):
+    return torch.empty(n, dtype=torch.uint8, device=DEV)
+
+
+# one and several tiles of every block shape with remainders, one step and an odd number of steps of K, rows in and beyond a
+# wave's and a block's registers, weights of more than a chunk
+@pytest.mark.parametrize("T,N,K", [(256, 64, 64), (257, 1, 96), (300, 129, 896), (513, 4865, 160), (260, 896, 4864),
+                                   (2048, 1152, 896), (1025, 2432, 2080), (2048, 9728, 96), (256, 70, 8256), (256, 9001, 8192)])
+@pytest.mark.parametrize("kind", ["rows", "norm", "gate"])
+def test_split_products(T, N, K, kind):
+    from sprout_lm_amd import ops
+    span = 40 if kind == "rows" else 0
+    a, w = rows(T, 2 * K if kind == "gate" else K, T + N, span), rows(N, K, K, span)
+    bias = torch.randn(N, device=DEV) if N != 1 else None
+    weight = 1 + 0.1 * torch.randn(K, device=DEV)
+    x = a.double()
+    if kind == "norm":
+        x = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * weight.double()
+    elif kind == "gate":
+        x = torch.nn.functional.silu(x[:, :K]) * x[:, K:]
+    want, size = x @ w.double().t(), x.abs() @ w.double().abs().t()
+    # a norm's scale and a gate are float32 numbers themselves: a few units of their last place, of every product
+    limit = (bound(K) + (0 if kind == "rows" else 2.0 ** -20)) * size + 2.0 ** -22 * (0 if bias is None else bias.double().abs())
+    options = {"norm": {"norm": (weight, 1e-6)}, "gate": {"activation": "silu"}, "rows": {}}[kind]
+    out = torch.full((T, N), float("nan"), device=DEV)
+    assert ops.gemm_f32_split(a, w, out, scratch, bias=bias, **options)
+    ref = want + (0 if bias is None else bias.double())
+    assert ((out.double() - ref).abs() <= limit).all()
+    if kind == "rows":
+        base = torch.randn(T, N, device=DEV)
+        acc = base.clone()
+        assert ops.gemm_f32_split(a, w, acc, scratch, bias=None if bias is None else bias.bfloat16(), accumulate=True)
+        ref = base.double() + want + (0 if bias is None else bias.bfloat16().double())
+        assert ((acc.double() - ref).abs() <= limit + 2.0 ** -23 * (base.double().abs() + want.abs())).all()
+
+
+def test_rows_of_zeros_and_numbers_that_are_not_finite():
+    from sprout_lm_amd import ops
+    a, w = rows(256, 96, 1), rows(70, 96, 2)
+    a[3] = 0
+    a[5, 7], a[9, 0], w[4, 95] = float("inf"), float("nan"), float("-inf")
+    a[11] *= 2.0 ** 120
+    a[12] *= 2.0 ** -120
+    out, plain = torch.empty(256, 70, device=DEV), torch.empty(256, 70, device=DEV)
+    assert ops.gemm_f32_split(a, w, out, scratch)
+    ops.gemm(a, w, plain)
+    assert torch.equal(out.isfinite(), plain.isfinite()) and not out[5].isfinite().any() and not out[9].isfinite().any()
+    good = out.isfinite()
+    assert (out[3][good[3]] == 0).all()
+    size = (a.double().abs() @ w.double().abs().t())[good]
+    assert ((out.double() - a.double() @ w.double().t())[good].abs() <= bound(96) * size).all()
+
+
+def test_what_the_split_product_does_not_take():
+    from sprout_lm_amd import ops
+    out = lambda T, N: torch.empty(T, N, device=DEV)
+    assert not ops.gemm_f32_split(rows(255, 96, 1), rows(8, 96, 2), out(255, 8), scratch)      # few tokens
+    assert not ops.gemm_f32_split(rows(256, 100, 1), rows(8, 100, 2), out(256, 8), scratch)    # K in no whole steps of 32
+    assert not ops.gemm_f32_split(rows(256, 96, 1).bfloat16(), rows(8, 96, 2), out(256, 8), scratch)
+    shifted = torch.empty(256 * 96 + 1, device=DEV)[1:].view(256, 96)                          # operands off 16 bytes
+    assert not ops.gemm_f32_split(shifted, rows(8, 96, 2), out(256, 8), scratch)
