@@ -23,7 +23,8 @@ int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size
 }
 
 size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx) {
-  const size_t splits = attention_prefill_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx);
+  const size_t splits = max(attention_prefill_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx),
+                            attention_rows_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx));
   return splits <= 1 ? 0 : size_t(n_tiles) * 32 * nq * splits * (hd + 2);
 }
 

@@ -1,0 +1,46 @@
+"""Prompt attention with two heads a wave (heads of 64, groups that fill its eight slots) against the general kernel."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def attention(kind, q, k, v, tables, batch, nq, nkv, **options):
+    from sprout_lm_amd import ops
+    out = torch.full_like(q, float("nan"))
+    ops.attention(q, nq * 64, k, v, tables, batch, out, nq, nkv, 64, None, 0.125, kind=kind, **options)
+    return out.double()
+
+
+# (heads, groups, tokens a page, [(context, queries)]): whole walks and 2 to 32 parts of the keys, a part of which lies beyond some
+# rows; groups of 6, 7, 8 and 12 heads (an odd head, a wave without one, two sets); queries in no whole tiles; walks that end
+# in the first and in the last of a stage's steps; more page numbers than LDS holds
+CASES = [(64, 8, 8, [(1024, 1024)]), (48, 8, 32, [(700, 700), (331, 300), (33, 33), (9, 1)]), (24, 2, 64, [(2049, 2049)]),
+         (14, 2, 16, [(4129, 2048)]), (14, 2, 16, [(4224, 2017), (2100, 31)]), (14, 2, 16, [(33001, 250)]),
+         (7, 1, 8, [(16384, 1000), (200, 200)]), (64, 8, 8, [(33000, 2048)]), (56, 8, 16, [(4096, 4096 - 2048), (130, 130)])]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_rows_attention(case):
+    from sprout_lm_amd import ops
+    nq, nkv, page, seqs = CASES[case]
+    g = torch.Generator(device=DEV).manual_seed(case)
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    pages = [-(-c // page) for c, _ in seqs]
+    T, total = sum(n for _, n in seqs), sum(pages) + 3
+    order = torch.randperm(total, device=DEV, generator=g).int()
+    tables = torch.full((len(seqs), max(pages) + 1), -1, dtype=torch.int32, device=DEV)
+    for i, n in enumerate(pages):
+        tables[i, :n] = order[sum(pages[:i]):sum(pages[:i]) + n]
+    k, v = rand(total, nkv, page, 64), rand(total, nkv, 64, page)
+    # keys that stand far out, so that running maxima are moved late in a walk
+    k *= torch.where(torch.rand(total, 1, page, 1, device=DEV, generator=g) < 0.002, 8.0, 1.0)
+    q, k, v = rand(T, nq * 64).bfloat16(), k.bfloat16(), v.bfloat16()
+    batch = ops.AttentionBatch.build([n for _, n in seqs], [c for c, _ in seqs], DEV)
+    got = attention(0, q, k, v, tables, batch, nq, nkv)
+    args = (q, k, v, tables, ops.AttentionBatch.build([n for _, n in seqs], [c for c, _ in seqs], DEV), nq, nkv)
+    want = attention(1, *args)
+    size = attention(1, q, k, v.abs(), *args[3:])
+    # weights rounded to bfloat16 (2^-9 of each, on both sides of the quotient's numerator only) and both results rounded
+    assert ((got - want).abs() <= 2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-6).all()
