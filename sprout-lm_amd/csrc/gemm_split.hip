@@ -146,7 +146,7 @@ int launch_split(hipStream_t s, const SplitSource& src, uint16_t* out, int32_t* 
 // 2,048 by 896 rows of 4,864: 64 x 128 73 us, 64 x 64 82, 128 x 128 108; 256 tokens by 896 rows of 4,864: 64 x 64 41, 64 x 128 66.)
 struct SplitShape { int bm, bn, per_cu; float light_us, full_us; };
 constexpr SplitShape kSplitShapes[] = {{384, 256, 1, 2.5f, 3.8f},   {256, 256, 1, 1.75f, 2.3f}, {256, 128, 1, 1.0f, 1.28f},
-                                       {128, 128, 1, 0.68f, 0.79f}, {64, 128, 2, 0.40f, 0.68f}, {64, 64, 2, 0.23f, 0.5f}};
+                                       {128, 128, 1, 0.68f, 0.79f}, {64, 128, 2, 0.33f, 0.60f}, {64, 64, 2, 0.23f, 0.54f}};
 
 int choose_split_shape(int T, int N, int K) {
   int best = 0;
