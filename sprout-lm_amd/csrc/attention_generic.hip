@@ -268,6 +268,12 @@ int attention_f32_tiles(hipStream_t s, const void* q, int q_stride, const void* 
                         const int32_t* ctx_len, const int32_t* tiles, int n_tiles, void* out, int nq, int nkv, int hd,
                         int page_size, int num_pages, ScoreStage st, float scale);
 
+bool attention_split_takes(int hd, int page_size);
+size_t attention_split_workspace_floats(int n_tiles, int nq, int nkv, int hd, int max_tile_ctx);
+int attention_split(hipStream_t s, const float* q, int q_stride, const float* k_pool, const float* v_pool,
+                    const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
+                    const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int max_tile_ctx, float* out, float* workspace, int nq,
+                    int nkv, int page_size, int num_pages, float scale);
 // Float32 storage goes to the matrix-core kernels of attention_f32.hip where they take the sizes: a step of
 // one-query sequences to the one that shares a sequence's keys out over blocks, any other to the one that walks
 // tiles of 32 queries.
@@ -300,7 +306,8 @@ static bool generic_grouped(bool single, int nq, int nkv) { return single && nkv
 size_t attention_generic_workspace_floats(int dtype, int page_size, int n_tiles, int nq, int nkv, int hd, int max_tile_ctx,
                                           bool single, bool plain) {
   if (f32_one_query(dtype, single, nq, nkv, hd, page_size, plain)) return attention_f32_decode_workspace_floats(n_tiles, nq, hd, max_tile_ctx);
-  if (attention_generic_on_matrix_cores(dtype, nq, nkv, hd, page_size, plain)) return 0;
+  if (attention_generic_on_matrix_cores(dtype, nq, nkv, hd, page_size, plain))
+    return attention_split_takes(hd, page_size) ? attention_split_workspace_floats(n_tiles, nq, nkv, hd, max_tile_ctx) : 0;
   int n_chunks, chunk;
   generic_chunks(n_tiles, generic_grouped(single, nq, nkv) ? nkv : nq, max_tile_ctx, &n_chunks, &chunk);
   return n_chunks > 1 ? size_t(n_tiles) * AQ * nq * n_chunks * (hd + 2) : 0;
@@ -370,9 +377,16 @@ int attention_generic(hipStream_t s, int dtype, const void* q, int q_stride, con
   if (f32_one_query(dtype, single, nq, nkv, hd, page_size, plain))
     return attention_f32_decode(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, ctx_len, tiles, n_tiles,
                                 out, nq, nkv, hd, page_size, num_pages, st, scale, max_tile_ctx, workspace);
-  if (attention_generic_on_matrix_cores(dtype, nq, nkv, hd, page_size, plain))
+  if (attention_generic_on_matrix_cores(dtype, nq, nkv, hd, page_size, plain)) {
+    // scores as they are under a softmax over every earlier key: the kernel of parts
+    if (attention_split_takes(hd, page_size) && st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && !st.sinks && !st.bias && !st.gate &&
+        (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pool) | reinterpret_cast<uintptr_t>(v_pool) |
+         reinterpret_cast<uintptr_t>(out)) % 16 == 0 && q_stride % 4 == 0)
+      return attention_split(s, (const float*)q, q_stride, (const float*)k_pool, (const float*)v_pool, block_tables, max_blocks, q_start,
+                             q_len, ctx_len, tiles, n_tiles, max_tile_ctx, (float*)out, workspace, nq, nkv, page_size, num_pages, scale);
     return attention_f32_tiles(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles,
                                n_tiles, out, nq, nkv, hd, page_size, num_pages, st, scale);
+  }
   if (dtype == kF32)
     return launch_attention_generic<float>(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start,
                                            q_len, ctx_len, tiles, n_tiles, out, nq, nkv, hd, page_size,

@@ -801,10 +801,10 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kerne
 // block as it has lanes for, four splits asked for at a time (one pair a wave, a dimension a lane and a split at a time: 2,048
 // rows of 14 heads of 64 in four splits, 29 MB, 14.4 -> 8.0 us).
 // part_o [tile][row][head][split][HD], part_ml [tile][row][head][split][2] = (maximum in log2 units, sum).
-template <int DT, int NQT, bool SIG>
+template <int DT, int NQT, bool SIG, typename TO = bf16_t>
 __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ q_len, const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, int n_splits,
+    const int32_t* __restrict__ q_len, const int32_t* __restrict__ tiles, TO* __restrict__ out, int n_splits,
     int nq, ScoreStage st, int pairs) {
   constexpr int HD = 16 * DT, ROWS = 16 * NQT, LANES = HD / 4, PER_BLOCK = 256 / LANES;
   const int pair = int(blockIdx.x) * PER_BLOCK + int(threadIdx.x) / LANES, d = 4 * (threadIdx.x % LANES);
@@ -837,9 +837,10 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
     }
   }
   const size_t token = size_t(q_start[seq] + q_off + row);
-  const float inv = row_factor<SIG>(den) * head_gate_of<bf16_t>(st, token, h);
-  *reinterpret_cast<uint2*>(out + token * (size_t(nq) * HD) + h * HD + d) =
-      make_uint2(pack_bf16x2(num[0] * inv, num[1] * inv), pack_bf16x2(num[2] * inv, num[3] * inv));
+  const float inv = row_factor<SIG>(den) * head_gate_of<TO>(st, token, h);
+  TO* dst = out + token * (size_t(nq) * HD) + h * HD + d;
+  if constexpr (sizeof(TO) == 4) *reinterpret_cast<float4*>(dst) = make_float4(num[0] * inv, num[1] * inv, num[2] * inv, num[3] * inv);
+  else *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(num[0] * inv, num[1] * inv), pack_bf16x2(num[2] * inv, num[3] * inv));
 }
 
 // ------------------------------------------------------------------------------------------ decode
@@ -1271,7 +1272,7 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
         constexpr int kPairs = 256 / (HD / 4);
         const int pairs = n_tiles * 16 * NQT * nq;
         attention_prefill_merge_kernel<DT, NQT, SIG><<<(pairs + kPairs - 1) / kPairs, 256, 0, s>>>(
-            part_o, part_ml, q_start, q_len, tiles, (uint16_t*)out, splits, nq, st, pairs);
+            part_o, part_ml, q_start, q_len, tiles, (bf16_t*)out, splits, nq, st, pairs);
       }
     } else {
       attention_prefill_kernel<DT, NQT, SIG><<<dim3(n_tiles, nq), 64, 0, s>>>(

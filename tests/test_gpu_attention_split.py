@@ -1,0 +1,54 @@
+"""float32 prompt attention on numbers in three bfloat16 parts (heads of 64), against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# (heads, groups, tokens a page, [(context, queries)]): one part of the keys and several, some beyond a row's keys; groups of 1 to 8
+# heads (waves without one, two sets); tiles and stages that end early; one-query sequences beside prompts; more page
+# numbers than LDS holds
+CASES = [(4, 4, 4, [(1, 1), (17, 17)]), (2, 1, 16, [(64, 64), (65, 1), (700, 33)]), (14, 2, 16, [(1000, 700), (40, 40), (4000, 1)]),
+         (9, 3, 8, [(513, 513)]), (8, 1, 64, [(129, 129), (2047, 31)]), (5, 1, 32, [(300, 299)]),
+         (2, 1, 4, [(9000, 40)]), (64, 16, 4, [(8700, 520)]), (14, 2, 16, [(2048, 2048)])]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_split_attention(case):
+    from sprout_lm_amd import ops
+    nq, nkv, page, seqs = CASES[case]
+    g = torch.Generator(device=DEV).manual_seed(case)
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    pages = [-(-c // page) for c, _ in seqs]
+    T, total = sum(n for _, n in seqs), sum(pages) + 3
+    order = torch.randperm(total, device=DEV, generator=g).int()
+    tables = torch.full((len(seqs), max(pages) + 1), -1, dtype=torch.int32, device=DEV)
+    k, v, q = rand(total, nkv, page, 64), rand(total, nkv, 64, page), rand(T, nq * 64)
+    k *= torch.where(torch.rand(total, 1, page, 1, device=DEV, generator=g) < 0.01, 8.0, 1.0)      # maxima that move late
+    v *= torch.exp2(torch.randint(-20, 20, (1, nkv, 64, 1), device=DEV, generator=g).float())
+    batch = lambda: ops.AttentionBatch.build([n for _, n in seqs], [c for c, _ in seqs], DEV)
+    for i, n in enumerate(pages):
+        tables[i, :n] = order[sum(pages[:i]):sum(pages[:i]) + n]
+    out = torch.full_like(q, float("nan"))
+    ops.attention(q, nq * 64, k, v, tables, batch(), out, nq, nkv, 64, None, 0.125, kind=0)
+    plain = torch.full_like(q, float("nan"))      # and the kernel on the vector units
+    ops.attention(q, nq * 64, k, v, tables, batch(), plain, nq, nkv, 64, None, 0.125, kind=2)
+    row = 0
+    for i, (ctx, n) in enumerate(seqs):
+        idx = tables[i, :pages[i]].long()
+        keys = k[idx].permute(1, 0, 2, 3).reshape(nkv, -1, 64)[:, :ctx].double()
+        values = v[idx].permute(1, 2, 0, 3).reshape(nkv, 64, -1)[:, :, :ctx].double()
+        hidden = torch.arange(ctx, device=DEV)[None, :] > torch.arange(ctx - n, ctx, device=DEV)[:, None]
+        for h in range(nq):
+            x, kk, vv = q[row:row + n, 64 * h:64 * h + 64].double(), keys[h * nkv // nq], values[h * nkv // nq]
+            s = (x @ kk.t() * 0.125).masked_fill(hidden, float("-inf"))
+            weights = s.softmax(-1)
+            want, size = weights @ vv.t(), weights @ vv.abs().t()
+            # a score: three products of 2^-22 left out or unrepresented, 24 sums of sixteen products each, of the products' magnitudes;
+            # it moves a weight twice (itself and the denominator); exponentials, weights and sums a few units of 2^-23, a chain of
+            # ctx / 64 sums among them
+            reach = (x.abs() @ kk.abs().t() * 0.125).masked_fill(hidden, 0.0).amax(-1, keepdim=True)
+            limit = (2 * (3 * 2.0 ** -22 + 24 * 2.0 ** -24) * reach + 2.0 ** -19 + ctx / 64 * 2.0 ** -24) * size
+            for got in (out, plain):
+                assert ((got[row:row + n, 64 * h:64 * h + 64].double() - want).abs() <= limit).all(), (case, i, h)
+        row += n
