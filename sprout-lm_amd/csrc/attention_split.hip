@@ -7,6 +7,11 @@
 // float32: sixteen numbers an instruction, so with fewer roundings of the sums than the float32 instruction's chain of two.
 // Queries, keys, values and the softmax's weights all pass it like that; scores, statistics and sums are float32.
 //
+// The instruction drops the bits below its sum's last place, so that its sums end a little below the true ones.  In the scores that
+// moves all keys of a query alike, and the softmax drops it.  The sums over the values would carry it to every token alike
+// (2.7e-8 of the results' size at 4,095 keys), where a later average over tokens keeps it and loses the rest of the error: the
+// weights of odd rows have their sign changed, so that half the rows end above.
+//
 // A block of four waves takes 32 queries of four heads of a key/value head, a wave a head; stages of 64 keys are loaded into
 // registers while the one before is used, split there and written to LDS as three planes each (48 KB), key rows and value
 // rows of 128 bytes in the layout of attention_rows.hip, whose tile products these are.  Two blocks run on a CU.  The matrix
@@ -123,6 +128,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
     }
   };
 
+  const uint32_t odd = uint32_t(li & 1) << 31;      // odd rows' sums are held with the other sign (see above)
   uint4 qp[4][3];
   floatx16 o[2];
   float m = kNoKeyYet, l = 0.f;
@@ -192,6 +198,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
         for (int j = 0; j < 8; ++j) {
           e[j] = __builtin_amdgcn_exp2f(fmaf(s[8 * c + j], scale2, -m));
           sum += e[j];
+          e[j] = __uint_as_float(__float_as_uint(e[j]) ^ odd);
         }
         uint4 p[3];
         three_parts8(e, p);
@@ -210,14 +217,14 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
   l += __shfl_xor(l, 32, 64);
   if (!live || li >= nvalid) return;
   float* dst;
-  float factor = 1.f;
+  float factor = li & 1 ? -1.f : 1.f;
   if (n_splits > 1) {
     const size_t slot = ((size_t(tile) * 32 + li) * nq + head) * n_splits + split;
     dst = part_o + slot * HD;
     if (lk == 0) *reinterpret_cast<float2*>(part_ml + 2 * slot) = make_float2(m, l);
   } else {
     dst = out + size_t(qs + q_off + li) * (size_t(nq) * HD) + head * HD;
-    factor = row_factor<false>(l);
+    factor *= row_factor<false>(l);
   }
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)

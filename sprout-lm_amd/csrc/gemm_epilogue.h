@@ -32,7 +32,7 @@ struct RopeArgs {
   long long out_stride, second_stride;
   // the plain float32 modes: elements from one row of the output to the next (0: N)
   long long row_stride;
-  // split_t operands: what the rows of x and of w were multiplied by, as powers of two
+  // split_t operands: what the rows of x and of w were multiplied by, as powers of two (and odd rows by -1)
   const int32_t *x_exp, *w_exp;
 };
 

@@ -276,13 +276,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
   if constexpr (SPLIT) {
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
-      const int ex = rope.x_exp[min(t0 + (wm * WM + i) * 32 + li, T - 1)];
+      const int t = t0 + (wm * WM + i) * 32 + li, ex = rope.x_exp[min(t, T - 1)];
 #pragma unroll
       for (int j = 0; j < WN; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int n = n0 + (wn * WN + j) * 32 + 8 * (r / 4) + 4 * lk + r % 4;
-          acc[i][j][r] = __builtin_amdgcn_ldexpf(acc[i][j][r], -(ex + rope.w_exp[min(n, N - 1)]));
+          const float back = __builtin_amdgcn_ldexpf(acc[i][j][r], -(ex + rope.w_exp[min(n, N - 1)]));
+          acc[i][j][r] = (t ^ n) & 1 ? -back : back;
         }
     }
   }

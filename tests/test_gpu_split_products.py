@@ -82,3 +82,18 @@ def test_what_the_split_product_does_not_take():
     assert not ops.gemm_f32_split(rows(256, 96, 1).bfloat16(), rows(8, 96, 2), out(256, 8), scratch)
     shifted = torch.empty(256 * 96 + 1, device=DEV)[1:].view(256, 96)                          # operands off 16 bytes
     assert not ops.gemm_f32_split(shifted, rows(8, 96, 2), out(256, 8), scratch)
+
+
+@pytest.mark.parametrize("K", [896, 4864])
+def test_the_error_has_no_side(K):
+    """The instruction's sums end below the true ones; odd rows' other sign takes that out of every mean."""
+    from sprout_lm_amd import ops
+    a, w, out = rows(2048, K, 3), rows(896, K, 4), torch.empty(2048, 896, device=DEV)
+    assert ops.gemm_f32_split(a, w, out, scratch)
+    want = a.double() @ w.double().t()
+    error = (out.double() - want) / want.square().mean().sqrt()
+    spread = float(error.square().mean().sqrt())
+    # means of independent errors: 7 deviations over all, over the rows' and over the columns' means together
+    assert abs(float(error.mean())) <= 7 * spread / (2048 * 896) ** 0.5
+    assert float(error.mean(0).square().mean().sqrt()) <= 2 * spread / 2048 ** 0.5
+    assert float(error.mean(1).square().mean().sqrt()) <= 2 * spread / 896 ** 0.5
