@@ -849,7 +849,7 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
 template <int DT, bool POW2, bool SIG>
 __global__ __launch_bounds__(256) void attention_decode_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
-    const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
+    const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks, int mask,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ decode_seqs,
     uint16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int nq,
     int nkv, int kv_stored, int page_size, int num_pages, ScoreStage st, float scale2) {
@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
   __shared__ float s_o[4][16][HD + 1];
   __shared__ float s_m[4][16], s_l[4][16];
   __shared__ int32_t s_table[kDecodeChunk / 4 + 4];      // the chunk's page numbers (pages of 4 tokens or more)
-  const int split = blockIdx.x, g = blockIdx.y, di = blockIdx.z;
+  const int g = blockIdx.y, di = blockIdx.z, split = chunk_of(blockIdx.x, di, mask);
   const int seq = decode_seqs ? decode_seqs[di] : di;   // no list: the batch is one-query sequences only, in order
   const int chunk0 = split * kDecodeChunk;
   // The page numbers of this chunk do not depend on how long the sequence is: they are asked for together with
@@ -1287,12 +1287,12 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
     float* part_ml = workspace ? workspace + size_t(n_decode) * nq * n_splits * HD : nullptr;
     if ((page_size & (page_size - 1)) == 0)
       attention_decode_kernel<DT, true, SIG><<<dim3(n_splits, decode_sets(nq, nkv), n_decode), 256, 0, s>>>(
-          qp, q_stride, kp, vp, block_tables, max_blocks, q_start, ctx_len, decode_seqs, (uint16_t*)out, part_o, part_ml,
-          n_splits, nq, decode_sets(nq, nkv), nkv, page_size, num_pages, st, scale2);
+          qp, q_stride, kp, vp, block_tables, max_blocks, chunk_mask(n_splits), q_start, ctx_len, decode_seqs, (uint16_t*)out,
+          part_o, part_ml, n_splits, nq, decode_sets(nq, nkv), nkv, page_size, num_pages, st, scale2);
     else
       attention_decode_kernel<DT, false, SIG><<<dim3(n_splits, decode_sets(nq, nkv), n_decode), 256, 0, s>>>(
-          qp, q_stride, kp, vp, block_tables, max_blocks, q_start, ctx_len, decode_seqs, (uint16_t*)out, part_o, part_ml,
-          n_splits, nq, decode_sets(nq, nkv), nkv, page_size, num_pages, st, scale2);
+          qp, q_stride, kp, vp, block_tables, max_blocks, chunk_mask(n_splits), q_start, ctx_len, decode_seqs, (uint16_t*)out,
+          part_o, part_ml, n_splits, nq, decode_sets(nq, nkv), nkv, page_size, num_pages, st, scale2);
     if (check_launch("sp_attention (decode)")) return 1;
     if (n_splits > 1) {
       if (n_splits <= 16)

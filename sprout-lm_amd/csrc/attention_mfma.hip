@@ -95,14 +95,14 @@ static int launch_decode_project(hipStream_t s, const void* q, int q_stride, con
   float* part_ml = workspace + size_t(n_decode) * nq * n_splits * HD;
   if ((page_size & (page_size - 1)) == 0)
     attention_decode_kernel<DT, true, false><<<dim3(n_splits, decode_sets(nq, nkv), n_decode), 256, 0, s>>>(
-        (const uint16_t*)q, q_stride, (const uint16_t*)k_pool, (const uint16_t*)v_pool, block_tables, max_blocks, q_start,
-        ctx_len, decode_seqs, nullptr, part_o, part_ml, n_splits, nq, decode_sets(nq, nkv), nkv, page_size, num_pages, st,
-        scale * kLog2e);
+        (const uint16_t*)q, q_stride, (const uint16_t*)k_pool, (const uint16_t*)v_pool, block_tables, max_blocks,
+        chunk_mask(n_splits), q_start, ctx_len, decode_seqs, nullptr, part_o, part_ml, n_splits, nq, decode_sets(nq, nkv), nkv,
+        page_size, num_pages, st, scale * kLog2e);
   else
     attention_decode_kernel<DT, false, false><<<dim3(n_splits, decode_sets(nq, nkv), n_decode), 256, 0, s>>>(
-        (const uint16_t*)q, q_stride, (const uint16_t*)k_pool, (const uint16_t*)v_pool, block_tables, max_blocks, q_start,
-        ctx_len, decode_seqs, nullptr, part_o, part_ml, n_splits, nq, decode_sets(nq, nkv), nkv, page_size, num_pages, st,
-        scale * kLog2e);
+        (const uint16_t*)q, q_stride, (const uint16_t*)k_pool, (const uint16_t*)v_pool, block_tables, max_blocks,
+        chunk_mask(n_splits), q_start, ctx_len, decode_seqs, nullptr, part_o, part_ml, n_splits, nq, decode_sets(nq, nkv), nkv,
+        page_size, num_pages, st, scale * kLog2e);
   if (check_launch("sp_attention_decode_project (decode)")) return 1;
   const int tpw = project_tiles_per_wave(n_decode, nq, hidden);
   const dim3 grid(nq, (hidden + 64 * tpw - 1) / (64 * tpw), (n_decode + 15) / 16);
