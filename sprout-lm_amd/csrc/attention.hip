@@ -36,8 +36,8 @@ int attention_mfma_decode_project(hipStream_t s, const void* q, int q_stride, co
 
 using namespace sprout;
 
-// kernel_kind: 0 = the engine's choice, 1 = the float32-arithmetic path (on the matrix cores' float32 instruction where
-// they take the sizes), 2 = the float32-arithmetic kernel on the vector units and no other.
+// kernel_kind: 0 = the engine's choice, 1 = the float32-arithmetic path (on the matrix cores where they take the
+// sizes: their float32 instruction, or numbers in three bfloat16 parts), 2 = the float32-arithmetic kernel on the vector units and no other.
 static bool use_mfma(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind) {
   return kernel_kind == 0 && dtype == kBF16 && nkv > 0 && nq % nkv == 0 && attention_mfma_supports(hd, page_size, nq, nkv);
 }

@@ -276,7 +276,7 @@ int attention_split(hipStream_t s, const float* q, int q_stride, const float* k_
                     int nkv, int page_size, int num_pages, float scale);
 // Float32 storage goes to the matrix-core kernels of attention_f32.hip where they take the sizes: a step of
 // one-query sequences to the one that shares a sequence's keys out over blocks, any other to the one that walks
-// tiles of 32 queries.
+// tiles of 32 queries, or to attention_split.hip's where that takes the sizes.
 // `plain`: the caller asks for the float32-arithmetic kernel of this file and no other (a mask that only it knows).
 bool attention_generic_on_matrix_cores(int dtype, int nq, int nkv, int hd, int page_size, bool plain) {
   return !plain && dtype == kF32 && attention_f32_decode_takes(hd, page_size, nq, nkv);

@@ -2,6 +2,7 @@
 // float32 operands, on v_mfma_f32_32x32x2_f32 (true 32-bit products and sums; no reduced-precision mode).  The
 // kernel is the pipelined tiled product of gemm_pipe.h with float operands; K must be a multiple of 32 (rows of
 // whole 128-byte slices).  Everything else (few tokens, other K, mixed operand types) stays on the FMA kernels.
+// Callers with a workspace take products of 256 tokens and more to gemm_split.hip first.
 #include "gemm_pipe.h"
 
 namespace sprout {
