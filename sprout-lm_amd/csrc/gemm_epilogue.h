@@ -30,7 +30,7 @@ struct RopeArgs {
   uint16_t* second;
   int split;
   long long out_stride, second_stride;
-  // the plain float32 modes: elements from one row of the output to the next (0: N)
+  // split_t operands: elements from one row of the output to the next
   long long row_stride;
   // split_t operands: what the rows of x and of w were multiplied by, as powers of two (and odd rows by -1)
   const int32_t *x_exp, *w_exp;
@@ -44,15 +44,16 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // `turn` is LDS that no wave of the block reads or fills any more, at least waves * 32 * (32 WN + 4) floats;
-// it is used only when K is split over blocks (gridDim.z > 1).
-template <int WM, int WN, int MODE, typename TB, int WAVES_N = 2>
+// it is used only when K is split over blocks (gridDim.z > 1).  STRIDED: rows of the output lie rope.row_stride apart (asked
+// for at run time, the stride cost every product of a few hundred tokens 0.2 us).
+template <int WM, int WN, int MODE, typename TB, int WAVES_N = 2, bool STRIDED = false>
 __device__ __forceinline__ void tile_epilogue(floatx16 (&acc)[WM][WN], float* turn_all, const TB* __restrict__ bias,
                                               void* __restrict__ out, int T, int N, int t0, int n0,
                                               const RopeArgs& rope = RopeArgs{}) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int li = lane & 31, lk = lane >> 5;
-  const long long stride = rope.row_stride ? rope.row_stride : N;
+  const std::conditional_t<STRIDED, long long, int> stride = STRIDED ? rope.row_stride : N;
   if (MODE == kRope) {
     // Tile columns come in groups of 64: 32 dimensions of a head's first half (tile column 2 m of a wave) and
     // their rotation partners, half a head further on (tile column 2 m + 1), so that a lane holds both of a pair.
