@@ -378,8 +378,9 @@ int attention_generic(hipStream_t s, int dtype, const void* q, int q_stride, con
     return attention_f32_decode(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, ctx_len, tiles, n_tiles,
                                 out, nq, nkv, hd, page_size, num_pages, st, scale, max_tile_ctx, workspace);
   if (attention_generic_on_matrix_cores(dtype, nq, nkv, hd, page_size, plain)) {
-    // scores as they are under a softmax over every earlier key: the kernel of parts
-    if (attention_split_takes(hd, page_size) && st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && !st.sinks && !st.bias && !st.gate &&
+    // scores as they are under a softmax over every earlier key: the kernel of parts (it masks before it scales, and takes the
+    // largest product for the largest score: a scale that is not positive needs the other order, which the tiles' kernel has)
+    if (attention_split_takes(hd, page_size) && scale > 0.f && st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && !st.sinks && !st.bias && !st.gate &&
         (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pool) | reinterpret_cast<uintptr_t>(v_pool) |
          reinterpret_cast<uintptr_t>(out)) % 16 == 0 && q_stride % 4 == 0)
       return attention_split(s, (const float*)q, q_stride, (const float*)k_pool, (const float*)v_pool, block_tables, max_blocks, q_start,

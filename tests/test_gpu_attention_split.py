@@ -52,3 +52,39 @@ def test_split_attention(case):
             for got in (out, plain):
                 assert ((got[row:row + n, 64 * h:64 * h + 64].double() - want).abs() <= limit).all(), (case, i, h)
         row += n
+
+
+def prompt(seed, nq=4, nkv=2, ctx=600, n=40, page=16):
+    """Queries, pools, tables and batch of one prompt's last n tokens; the rows of keys [nkv, ctx, 64] and values [nkv, 64, ctx] that
+    `fill` writes into the pools."""
+    from sprout_lm_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    q, keys, values = (torch.randn(*s, device=DEV, generator=g) for s in ((n, nq * 64), (nkv, ctx, 64), (nkv, 64, ctx)))
+    pages = -(-ctx // page)
+    tables = torch.randperm(pages, device=DEV, generator=g).int()[None]
+
+    def run(scale=0.125):
+        k, v = torch.zeros(pages, nkv, page, 64, device=DEV), torch.zeros(pages, nkv, 64, page, device=DEV)
+        pad = torch.zeros(nkv, pages * page - ctx, 64, device=DEV)
+        k[tables[0].long()] = torch.cat([keys, pad], 1).view(nkv, pages, page, 64).permute(1, 0, 2, 3)
+        v[tables[0].long()] = torch.cat([values, pad.transpose(1, 2)], 2).view(nkv, 64, pages, page).permute(2, 0, 1, 3)
+        out = torch.full_like(q, float("nan"))
+        ops.attention(q, nq * 64, k, v, tables, ops.AttentionBatch.build([n], [ctx], DEV), out, nq, nkv, 64, None, scale)
+        return out.view(n, nq, 64).double()
+
+    def want(scale=0.125):
+        x, kk, vv = q.view(n, nq, 64).double(), keys.double().repeat_interleave(nq // nkv, 0), values.double().repeat_interleave(nq // nkv, 0)
+        hidden = torch.arange(ctx, device=DEV)[None] > torch.arange(ctx - n, ctx, device=DEV)[:, None]
+        # (a sum of products, number by number: an infinity times a zero is NaN here as there)
+        scores = torch.stack([(x[i, :, None] * kk).sum(-1) for i in range(n)]) * scale
+        weights = scores.masked_fill(hidden[:, None], float("-inf")).softmax(-1)
+        return torch.stack([(weights[i, :, None] * vv).sum(-1) for i in range(n)])
+
+    return q.view(n, nq, 64), keys, values, run, want
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.125, -2.0, 0.7])
+def test_scales_that_are_not_positive(scale):
+    q, keys, values, run, want = prompt(1)
+    # a few units of 2^-23 of sums of unit numbers, of scores up to |scale| 64
+    assert (run(scale) - want(scale)).abs().max() <= 1e-5 * max(1.0, abs(scale) * 8)
