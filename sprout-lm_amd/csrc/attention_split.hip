@@ -12,6 +12,13 @@
 // (2.7e-8 of the results' size at 4,095 keys), where a later average over tokens keeps it and loses the rest of the error: the
 // weights of odd rows have their sign changed, so that half the rows end above.
 //
+// What three parts cannot hold: infinities (inf - inf is NaN), numbers that round beyond bfloat16's largest, and the last bits of
+// numbers below 2^-110, whose third parts end in bfloat16's subnormal numbers.  The first two end as NaN in the row's sums; values of
+// the third kind end as results below kTinyResult.  A wave that finds one of them at the end of its walk walks again by itself, from
+// the pools on the float32 instruction and with every maximum exact, as attention_f32.hip's kernel does.  The look at the sums is 50
+// instructions a wave: no time beyond noise in any size measured (a walk of the block again, through LDS, put its check's three
+// barriers behind every block: 3 to 10 % of these launches).
+//
 // A block of four waves takes 32 queries of four heads of a key/value head, a wave a head; stages of 64 keys are loaded into
 // registers while the one before is used, split there and written to LDS as three planes each (48 KB), key rows and value
 // rows of 128 bytes in the layout of attention_rows.hip, whose tile products these are.  Two blocks run on a CU.  The matrix
@@ -26,6 +33,7 @@ namespace sprout {
 namespace {
 
 constexpr int kSplitKeys = 64, kPlane = 64 * 128, kSplitTable = 2048;
+constexpr float kTinyResult = 0x1p-100f;
 
 __device__ __forceinline__ int split_swz(int row) { return (row ^ (row >> 3)) & 7; }
 
@@ -53,6 +61,11 @@ __device__ __forceinline__ floatx16 mfma_parts(const uint4 (&a)[3], const uint4 
   c = mfma32(as_bf16x8(a[1]), as_bf16x8(b[0]), c);
   c = mfma32(as_bf16x8(a[0]), as_bf16x8(b[1]), c);
   return mfma32(as_bf16x8(a[0]), as_bf16x8(b[0]), c);
+}
+__device__ __forceinline__ float min3_of_magnitudes(float a, float b, float c) {
+  float least;
+  asm("v_min3_f32 %0, |%1|, |%2|, |%3|" : "=v"(least) : "v"(a), "v"(b), "v"(c));
+  return least;
 }
 __device__ __forceinline__ float max_over_row(float x) {      // the other half of a row's keys lies in lane ^ 32
   const unsigned u = __float_as_uint(x);
@@ -214,8 +227,85 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
       l += sum;
     }
   }
+  if (!live) return;
   l += __shfl_xor(l, 32, 64);
-  if (!live || li >= nvalid) return;
+  // sums that are not finite, or (zeros aside) results below kTinyResult
+  float total = l, least = INFINITY;
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+      total += fabsf(o[dt][r]);
+      total += fabsf(o[dt][r + 1]);
+      least = min3_of_magnitudes(least, o[dt][r], o[dt][r + 1]);
+    }
+  bool beyond = !(total < INFINITY);
+  if (least < kTinyResult * l) {
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) beyond |= (o[dt][r] != 0.f) & (fabsf(o[dt][r]) < kTinyResult * l);
+  }
+  if (__builtin_amdgcn_ballot_w64(beyond && li < nvalid) != 0) {
+    const float* row = q + size_t(qs + q_off + min(li, nvalid - 1)) * q_stride + head * HD + 8 * lk;
+    const int in_run = (li & ~12) | ((li & 4) << 1) | ((li & 8) >> 1);      // the key of row li of 32
+    m = kNoKeyYet;
+    l = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+#pragma unroll 1
+    for (int first = lo; first <= hi; first += 32) {
+      const int key = min(first + in_run, hi);
+      const float* krow = kbase + ((page_at(key) << page_shift) + (key & page_mask)) * HD + 8 * lk;
+      floatx16 s;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll 1
+      for (int d = 0; d < HD; d += 16)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s = mfma32_f32(krow[d + j], row[d + j], s);
+      float top = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if (first + 8 * lk + 16 * (r / 8) + r % 8 > pos) s[r] = -INFINITY;
+        top = vmax(top, s[r]);
+      }
+      const float mx = vmax(m, max_over_row(top * scale2)), alpha = __builtin_amdgcn_exp2f(m - mx);
+      m = mx;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        if (first + 16 * c > hi) break;      // (repeated values would have no weight, but an infinity among them would have a say)
+        float e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          e[j] = __builtin_amdgcn_exp2f(fmaf(s[8 * c + j], scale2, -m));
+          l += e[j];
+          e[j] = __uint_as_float(__float_as_uint(e[j]) ^ odd);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int kb = min(first + 16 * c + 8 * lk + 4 * u, hi & ~3);
+#pragma unroll
+          for (int dt = 0; dt < 2; ++dt) {
+            const float4 v = *reinterpret_cast<const float4*>(vbase + ((page_at(kb) * HD + 32 * dt + li) << page_shift) + (kb & page_mask));
+            o[dt] = mfma32_f32(v.x, e[4 * u], o[dt]);
+            o[dt] = mfma32_f32(v.y, e[4 * u + 1], o[dt]);
+            o[dt] = mfma32_f32(v.z, e[4 * u + 2], o[dt]);
+            o[dt] = mfma32_f32(v.w, e[4 * u + 3], o[dt]);
+          }
+        }
+      }
+    }
+    l += __shfl_xor(l, 32, 64);
+  }
+  if (li >= nvalid) return;
   float* dst;
   float factor = li & 1 ? -1.f : 1.f;
   if (n_splits > 1) {

@@ -88,3 +88,54 @@ def test_scales_that_are_not_positive(scale):
     q, keys, values, run, want = prompt(1)
     # a few units of 2^-23 of sums of unit numbers, of scores up to |scale| 64
     assert (run(scale) - want(scale)).abs().max() <= 1e-5 * max(1.0, abs(scale) * 8)
+
+
+def test_numbers_that_are_not_finite_and_at_the_ends_of_the_range():
+    inf = float("inf")
+    top = 3.4e38      # more than bfloat16's largest number
+
+    def check(change, seed, rel=1e-5):
+        q, keys, values, run, want = prompt(seed)
+        change(q, keys, values)
+        got, ref = run(), want()
+        assert torch.equal(got.isnan(), ref.isnan()), (change, (got.isnan() != ref.isnan()).nonzero()[:8])
+        good = ref.isfinite()
+        assert torch.equal(got[~good & ~ref.isnan()], ref[~good & ~ref.isnan()])
+        # a few units of 2^-23 of sums of numbers of one size: against the largest result of the head's dimension
+        error, size = ((x.where(good, torch.zeros(()).to(x))).abs().amax(0) for x in (got - ref, ref))
+        assert (error <= rel * size).all(), (change, (error > rel * size).nonzero()[:8])
+        return ref
+
+    def keys_of_minus_infinity(q, keys, values):      # every score of them is minus infinity: they weigh nothing
+        q[..., 3] = q[..., 3].abs() + 0.1
+        keys[:, 5:300:7, 3] = -inf
+
+    def one_infinite_key(q, keys, values):            # scores of both signs
+        keys[1, 100, 9] = inf
+
+    def infinite_values(q, keys, values):
+        values[0, 7, 33], values[0, 8, 34], values[0, 8, 35], values[1, 9, 36] = inf, inf, -inf, -inf
+
+    def queries(q, keys, values):
+        q[3, 1, 5], q[7, 2, 0], q[9, 3, 63] = inf, float("nan"), -inf
+
+    def nan_value(q, keys, values):
+        values[1, 4, 400] = float("nan")
+
+    def near_the_top(q, keys, values):
+        values[:, 2] *= top / 2000      # (the sums before they are divided by the weights' have to stay in the range themselves)
+        values[0, 2, 17] = top
+        q[..., 4] *= 1e-38
+        keys[:, 20:90, 4] = top
+
+    def tiny(q, keys, values):
+        values[:, 2] *= 2.0 ** -112
+        values[0, 3] *= 2.0 ** -120
+
+    assert check(keys_of_minus_infinity, 2).isfinite().all()
+    assert check(one_infinite_key, 3).isnan().any()
+    assert check(infinite_values, 4).isinf().any()
+    check(queries, 5)
+    check(nan_value, 6)
+    check(near_the_top, 7)
+    check(tiny, 8)
