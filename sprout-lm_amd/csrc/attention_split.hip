@@ -37,16 +37,6 @@ constexpr float kTinyResult = 0x1p-100f;
 
 __device__ __forceinline__ int split_swz(int row) { return (row ^ (row >> 3)) & 7; }
 
-// Two numbers into their three bfloat16 parts, packed.
-__device__ __forceinline__ void three_parts(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
-  p1 = pack_bf16x2(a, b);
-  a -= __uint_as_float(p1 << 16);
-  b -= __uint_as_float(p1 & 0xffff0000u);
-  p2 = pack_bf16x2(a, b);
-  a -= __uint_as_float(p2 << 16);
-  b -= __uint_as_float(p2 & 0xffff0000u);
-  p3 = pack_bf16x2(a, b);
-}
 __device__ __forceinline__ void three_parts8(const float (&f)[8], uint4 (&p)[3]) {
   three_parts(f[0], f[1], p[0].x, p[1].x, p[2].x);
   three_parts(f[2], f[3], p[0].y, p[1].y, p[2].y);

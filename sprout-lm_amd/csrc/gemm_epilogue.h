@@ -30,10 +30,8 @@ struct RopeArgs {
   uint16_t* second;
   int split;
   long long out_stride, second_stride;
-  // split_t operands: elements from one row of the output to the next
+  // STRIDED: elements from one row of the output to the next
   long long row_stride;
-  // split_t operands: what the rows of x and of w were multiplied by, as powers of two (and odd rows by -1)
-  const int32_t *x_exp, *w_exp;
 };
 
 // Orders a wave's LDS writes before its own later reads of what other lanes wrote (and the reverse).

@@ -80,14 +80,10 @@ __host__ __device__ inline bool pipe_tile_of(const PipeTiles& tiles, int block, 
 // v_mfma_f32_32x32x2_f32 (k-slot l / 32 of MFMA e is element 4 (l / 32) + e of the eight that a 32-byte slice of a
 // row holds, for both operands): true float32 products and sums, no reduced-precision mode, 1/8 of the bfloat16
 // rate per byte, so this form is bound by the matrix cores and not by its fetches.
-// split_t: float32 operands as pairs of float16 (gemm_split.hip): a step is 32 along K like float's, a row's 128 bytes hold
-// the 32 upper parts, then the 32 lower ones, and a number's product is upper.upper + upper.lower + lower.upper on
-// 32x32x16 MFMA; the sums are scaled back by the rows' exponents before the epilogue.
 // The grouped form (GROUPED): every group (an expert) has weights of its own, w_group_stride elements apart, and
 // multiplies the rows that a list of tiles gives it: tiles [n][3] = (group, first row, rows) with at most BM rows
 // each and n in *n_tiles; row r of the list reads operand row gather[r] / gather_div and writes output row r.  Block
 // b takes tile b / tiles_n and weight tile b % tiles_n.
-struct split_t { uint32_t bits; };
 struct PipeGroups {
   const int32_t* tiles;
   const int32_t* n_tiles;
@@ -102,7 +98,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
                                                         int N, int K, int k_per_split, RopeArgs rope, PipeGroups groups) {
   constexpr int NW = WAVES_M * WAVES_N;
   constexpr int ESZ = sizeof(TE), KSTEP = 128 / ESZ;    // elements of a tile row
-  constexpr bool SPLIT = std::is_same<TE, split_t>::value;
   static_assert(ESZ == 2 || (MODE != kSilu && MODE != kRope && MODE != kStore), "float32 operands store or add float32");
   constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N;
   constexpr int ROW = 128;                              // bytes of a tile row
@@ -202,30 +197,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
 
   auto multiply = [&](int buf) {
     const unsigned char* stage = pipe_lds + buf * STAGE;
-    if constexpr (SPLIT) {
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        uint4 b[WN][2];
-        const uint32_t xp = xrow0 + ((ks * 32) ^ xpos0), wp = wrow0 + ((ks * 32) ^ wpos0);
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            b[j][h] = *reinterpret_cast<const uint4*>(stage + (((j + h) & 1) ? (wp ^ 64) : wp) + j * 32 * ROW);
-#pragma unroll
-        for (int i = 0; i < WM; ++i) {
-          const uint4 hi = *reinterpret_cast<const uint4*>(stage + ((i & 1) ? (xp ^ 64) : xp) + i * 32 * ROW);
-          const uint4 lo = *reinterpret_cast<const uint4*>(stage + ((i & 1) ? xp : (xp ^ 64)) + i * 32 * ROW);
-#pragma unroll
-          for (int j = 0; j < WN; ++j) acc[i][j] = mfma32_f16(as_f16x8(b[j][0]), as_f16x8(hi), acc[i][j]);
-#pragma unroll
-          for (int j = 0; j < WN; ++j) acc[i][j] = mfma32_f16(as_f16x8(b[j][1]), as_f16x8(hi), acc[i][j]);
-#pragma unroll
-          for (int j = 0; j < WN; ++j) acc[i][j] = mfma32_f16(as_f16x8(b[j][0]), as_f16x8(lo), acc[i][j]);
-        }
-      }
-      return;
-    }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       uint4 a[WM], b[WN];
@@ -236,8 +207,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
 #pragma unroll
       for (int j = 0; j < WN; ++j)
         b[j] = *reinterpret_cast<const uint4*>(stage + ((j & 1) ? (wp ^ 64) : wp) + j * 32 * ROW);
-      if constexpr (SPLIT) {
-      } else if constexpr (ESZ == 2) {
+      if constexpr (ESZ == 2) {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -273,23 +243,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
       multiply(u);
     }
   }
-  if constexpr (SPLIT) {
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const int t = t0 + (wm * WM + i) * 32 + li, ex = rope.x_exp[min(t, T - 1)];
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int n = n0 + (wn * WN + j) * 32 + 8 * (r / 4) + 4 * lk + r % 4;
-          const float back = __builtin_amdgcn_ldexpf(acc[i][j][r], -(ex + rope.w_exp[min(n, N - 1)]));
-          acc[i][j][r] = (t ^ n) & 1 ? -back : back;
-        }
-    }
-  }
   if (MODE == kAccumulate && gridDim.z > 1) __syncthreads();   // the epilogue turns tiles round in this LDS
   static_assert(NW * 32 * (32 * WN + 4) * sizeof(float) <= size_t(STAGES) * STAGE, "the turning buffer must fit");
-  tile_epilogue<WM, WN, MODE, TB, WAVES_N, SPLIT>(acc, reinterpret_cast<float*>(pipe_lds), bias, out, T, N, t0, n0, rope);
+  tile_epilogue<WM, WN, MODE, TB, WAVES_N>(acc, reinterpret_cast<float*>(pipe_lds), bias, out, T, N, t0, n0, rope);
 }
 
 template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, int MODE, typename TB, typename TE = uint16_t>

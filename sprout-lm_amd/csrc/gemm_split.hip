@@ -1,52 +1,61 @@
-// float32 products of many tokens on the float16 matrix cores: out (float32) = or += a[T, K] . w[N, K]^T, K in 32s.
+// float32 products of many tokens on the bfloat16 matrix cores: out (float32) = or += a[T, K] . w[N, K]^T, K in 32s.
 //
-// v_mfma_f32_32x32x2_f32 gives 157 TFLOP/s, the float16 instruction sixteen times that.  A float32 number a is the sum of two
-// float16 numbers to its last bit or the one before: upper = rn(a), lower = rn(a - upper) leave at most 2^-23 |a|, on average
-// half of that where anything is left at all, and a . w = upper.upper + upper.lower + lower.upper leaves out a product of
-// 2^-22 at most: three products at sixteen times the rate.  All three are summed in float32 in one accumulator, sixteen
-// numbers of K an instruction instead of two, so that there are fewer roundings of the sums than before and those are what
-// the error of a long product is made of: relative error of the result against 64 bits (normal operands, the float32
-// instruction -> this): K = 896 5.4e-7 -> 3.4e-7, K = 4,864 1.25e-6 -> 7.8e-7.  Time, whole call (2,048 tokens): 9,728 rows of
-// 896 329 -> 132 us (of it 15 the split of the weights at 4.6 TB/s), 896 rows of 4,864 179 -> 97 us, 37,888 rows of 3,584
-// 4,150 -> 1,700 us (327 TFLOP/s of float32 products).
+// v_mfma_f32_32x32x2_f32 gives 157 TFLOP/s, the bfloat16 instruction sixteen times that.  A float32 number is the sum of three
+// bfloat16 numbers to its last bit (three_parts of mfma.h), and a product is taken as the six products of parts that reach 2^-24 of
+// it: a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1; what is left out is 2^-26 of it at most, less than the float32 product's own rounding.
+// a1 b1 is summed in one float32 accumulator and the other five, 2^-8 of its size, in a second: a result is rounded once for every
+// sixteen numbers of K and once where the two meet, where the float32 instruction rounds once for every number that is not zero
+// and at most once for every two.  Relative error of the result against 64 bits, float32 instruction -> this: normal operands,
+// K = 896 5.4e-7 -> 1.7e-7, 4,864 1.25e-6 -> 4.3e-7, 27,648 3.0e-6 -> 4.3e-7; weights with 1, 2, 8 and 64 numbers a row that are not
+// zero 2.5e-8 -> 2.6e-8, 3.1e-8 -> 2.6e-8, 5.4e-8 -> 2.9e-8, 1.4e-7 -> 5.7e-8; one number 2^100 times the others of its row against a
+// weight of zero 5.4e-7 -> 1.7e-7.  Time, whole call (2,048 tokens): 9,728 rows of 896 303 -> 235 us (of it 21 the splits, at 4.6
+// TB/s; the product 203, at 1.05 PFLOP/s of bfloat16 products), 896 rows of 4,864 182 -> 154, 37,888 rows of 3,584 4,268 -> 2,958.
 //
-// float16 has five bits of exponent, so every row is multiplied by a power of two that brings its largest number into
-// [2^14, 2^15): numbers down to 2^-17 of the row's largest keep a lower part of full width, and what is lost of smaller ones is
-// below 2^-40 of the largest.  Powers of two are exact, and the sums are multiplied back by them.  A row that
-// holds an infinity or NaN gives NaN where the float32 instruction gave an infinity or NaN.
+// (Pairs of float16 numbers took three products and half the time, but held 23 bits of 24, and numbers below 2^-17 of
+// their row's largest less and less of them: one number that stood 2^24 out of its row and met no weight left an error of 2e-5.)
 //
-// The instruction drops the bits below its sum's last place: every result lies a little (2e-8 of the results' size at K = 896,
-// 1.1e-7 at 4,864) below the true one, all to the same side, which the averages that attention takes over many tokens' values do
-// not lose as they lose the rest of the error.  So odd rows on either side change their sign and the results of an odd and an
-// even row change it back: the mean of the error over a row or a column of results goes to 1e-9, for an operation an element.
+// Every row is multiplied by a power of two that brings its largest number into [2^49, 2^50): numbers down to 2^-150 of it keep all
+// their bits, whatever the size of the row, and no sum overflows.  Powers of two are exact, and the sums are multiplied back
+// by them.  A row that is not finite passes as its bits (upper and lower sixteen in two parts): its results are taken number by
+// number behind the others, infinities and NaN as the float32 instruction gives them.
 //
-// The rows are split by a kernel of their own before the product (the activations with what stands before the product,
-// the norm or the gate, folded in; the weights into a workspace, a chunk of rows at a time, at the speed of memory), into the
-// 128-byte slices of 32 numbers (upper, then lower parts) that the pipelined kernel of gemm_pipe.h takes.
+// The instruction drops the bits below its sum's last place, so that results end a little below the true ones, all to the same
+// side, which the averages that attention takes over many tokens' values do not lose as they lose the rest of the error: odd rows
+// on either side change their sign, and the results of an odd and an even row change it back.
+//
+// The rows are split by a kernel of their own before the product (the activations with what stands before the product, the norm
+// or the gate, folded in; the weights into a workspace, a chunk of rows at a time, at the speed of memory): two rows together,
+// 32 numbers of K a step, a line of 128 bytes a part.  K beyond kMaxK is walked in pieces that add.
 #include "gemm_pipe.h"
 
 namespace sprout {
 
+float gemm_f32_time_us(int T, int N, int K);      // of the float32 instruction's kernel (gemm_f32.hip)
+
 namespace {
 
-constexpr int64_t kChunkBytes = int64_t(256) << 20;      // of split weights a launch multiplies
+constexpr int64_t kChunkBytes = int64_t(128) << 20;      // of split weights a launch multiplies
+constexpr int kMaxK = 5120;                              // numbers of a row at a time: a chunk of rows then fills the chip
+constexpr int kStep = 32, kStepBytes = 3 * 128;          // numbers of K a step, bytes of a step of two rows
+constexpr int kNotFinite = 1 << 20;                      // a row's exponent, where the row holds its numbers' bits
 
 enum { kRowsAsTheyAre = 0, kRowsGated = 1, kRowsNormed = 2 };
 
 struct SplitSource {
-  const float* a;              // [rows][K]; kRowsGated: [rows][2 K], gate then up
+  const float* a;              // [rows][length]; kRowsGated: [rows][2 length], gate then up
+  int length, first;           // of a row of the product, and the first of its numbers that is split
   const float* norm_w;         // kRowsNormed: a row is (a * scale) * norm_w, scale = 1 / rms
   float eps;
   int act;                     // kRowsGated
   float limit;
 };
 
-__device__ __forceinline__ float max4(float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
+__device__ __forceinline__ size_t row_at(int row, int K) { return size_t(row >> 1) * (size_t(K / kStep) * kStepBytes) + (row & 1) * 64; }
 
 // One row a wave (WAVES 1, four rows a block) or a block of four waves: bound by memory, a row's numbers stay in registers
-// between its largest and the split where eight pieces of 16 bytes a lane hold it, else they are formed again.
-template <int WAVES, int KIND, bool FITS>
-__global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, uint16_t* __restrict__ out, int32_t* __restrict__ exponents,
+// between its largest and the split (eight pieces of 16 bytes a lane).
+template <int WAVES, int KIND>
+__global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, unsigned char* __restrict__ out, int32_t* __restrict__ exponents,
                                                          int rows, int K) {
   constexpr int LANES = 64 * WAVES, PIECES = 8;
   __shared__ float scratch[16];
@@ -54,53 +63,50 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, uint16
   const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
   if (row >= rows) return;
   const int n4 = K / 4;
-  const float4* a = reinterpret_cast<const float4*>(src.a + size_t(row) * (KIND == kRowsGated ? 2 * K : K));
-  float factor = 1.f;
-  float4 kept[FITS ? PIECES : 1];
-  auto raw = [&](int i) { return a[i]; };
-  if (FITS && KIND != kRowsGated) {
+  const float* whole = src.a + size_t(row) * (KIND == kRowsGated ? 2 * src.length : src.length);
+  const float4* a = reinterpret_cast<const float4*>(whole + src.first);
+  float4 kept[PIECES];
+  if (KIND != kRowsGated) {
 #pragma unroll
-    for (int p = 0; p < (FITS ? PIECES : 0); ++p)
-      if (lane + p * LANES < n4) kept[p] = raw(lane + p * LANES);
+    for (int p = 0; p < PIECES; ++p)
+      if (lane + p * LANES < n4) kept[p] = a[lane + p * LANES];
   }
+  float factor = 1.f;
   if (KIND == kRowsNormed) {
     float squares = 0.f;
-    if (FITS) {
+    if (K == src.length) {
 #pragma unroll
-      for (int p = 0; p < (FITS ? PIECES : 0); ++p)
+      for (int p = 0; p < PIECES; ++p)
         if (lane + p * LANES < n4) squares += kept[p].x * kept[p].x + kept[p].y * kept[p].y + kept[p].z * kept[p].z + kept[p].w * kept[p].w;
     } else {
-      for (int i = lane; i < n4; i += LANES) { const float4 v = raw(i); squares += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; }
+      for (int i = lane; i < src.length / 4; i += LANES) {
+        const float4 v = reinterpret_cast<const float4*>(whole)[i];
+        squares += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+      }
     }
     squares = WAVES == 1 ? wave_sum(squares) : block_sum(squares, scratch);
-    factor = 1.0f / sqrtf(squares / float(K) + src.eps);
+    factor = 1.0f / sqrtf(squares / float(src.length) + src.eps);
   }
-  auto value = [&](int i, float4 v) {
-    if (KIND == kRowsNormed) {
-      const float4 w = reinterpret_cast<const float4*>(src.norm_w)[i];
-      return make_float4(v.x * factor * w.x, v.y * factor * w.y, v.z * factor * w.z, v.w * factor * w.w);
-    }
-    if (KIND == kRowsGated) {
-      const float4 g = a[i], u = a[i + n4];
-      v = make_float4(gated_value(g.x, u.x, src.act, src.limit), gated_value(g.y, u.y, src.act, src.limit),
-                      gated_value(g.z, u.z, src.act, src.limit), gated_value(g.w, u.w, src.act, src.limit));
-    }
-    return v;
-  };
   float top = 0.f;
   bool finite = true;
-  auto look = [&](float4 v) {
-    const float m = max4(v);
-    top = fmaxf(top, m);
-    // (a maximum drops a NaN: it is looked for by itself)
-    finite = finite && fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY && fabsf(v.z) < INFINITY && fabsf(v.w) < INFINITY;
-  };
-  if (FITS) {
 #pragma unroll
-    for (int p = 0; p < (FITS ? PIECES : 0); ++p)
-      if (lane + p * LANES < n4) { kept[p] = value(lane + p * LANES, kept[p]); look(kept[p]); }
-  } else {
-    for (int i = lane; i < n4; i += LANES) look(value(i, KIND == kRowsGated ? make_float4(0, 0, 0, 0) : raw(i)));
+  for (int p = 0; p < PIECES; ++p) {
+    const int i = lane + p * LANES;
+    if (i >= n4) continue;
+    if (KIND == kRowsNormed) {
+      const float4 v = kept[p], w = reinterpret_cast<const float4*>(src.norm_w + src.first)[i];
+      kept[p] = make_float4(v.x * factor * w.x, v.y * factor * w.y, v.z * factor * w.z, v.w * factor * w.w);
+    } else if (KIND == kRowsGated) {
+      const float4 g = a[i], u = reinterpret_cast<const float4*>(whole + src.length + src.first)[i];
+      kept[p] = make_float4(gated_value(g.x, u.x, src.act, src.limit), gated_value(g.y, u.y, src.act, src.limit),
+                            gated_value(g.z, u.z, src.act, src.limit), gated_value(g.w, u.w, src.act, src.limit));
+    }
+    const float f[4] = {fabsf(kept[p].x), fabsf(kept[p].y), fabsf(kept[p].z), fabsf(kept[p].w)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      top = fmaxf(top, f[c]);
+      finite = finite && f[c] < INFINITY;      // (a maximum drops a NaN: it is looked for by itself)
+    }
   }
   if (!finite) top = INFINITY;
   top = wave_max(top);
@@ -110,91 +116,267 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, uint16
     __syncthreads();
     top = fmaxf(fmaxf(scratch[0], scratch[1]), fmaxf(scratch[2], scratch[3]));
   }
+  const bool bits = !(top < INFINITY);
   int e = 0;
-  if (top > 0.f && top < INFINITY) e = 15 - __builtin_amdgcn_frexp_expf(top);      // top = m 2^x, m in [0.5, 1): m 2^15
-  if (lane == 0) exponents[row] = e;
-  const uint32_t odd = uint32_t(row & 1) << 31;      // odd rows change their sign (see above)
-  auto store = [&](int i, float4 v) {
-    uint16_t* dst = out + size_t(row) * 2 * K + size_t(i / 8) * 64 + 4 * (i % 8);
-    const float f[4] = {v.x, v.y, v.z, v.w};
-    uint16_t hi[4], lo[4];
+  if (top > 0.f && !bits) e = 50 - __builtin_amdgcn_frexp_expf(top);      // top = m 2^x, m in [0.5, 1): m 2^50
+  if (lane == 0) exponents[row] = bits ? kNotFinite : e;
+  const uint32_t odd = bits ? 0u : uint32_t(row & 1) << 31;      // odd rows change their sign (see above)
+  unsigned char* dst_row = out + row_at(row, K);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float x = __uint_as_float(__float_as_uint(__builtin_amdgcn_ldexpf(f[c], e)) ^ odd);
-      const _Float16 h = (_Float16)x;
-      hi[c] = __builtin_bit_cast(uint16_t, h);
-      lo[c] = __builtin_bit_cast(uint16_t, (_Float16)(x - (float)h));
+  for (int p = 0; p < PIECES; ++p) {
+    const int i = lane + p * LANES;
+    if (i >= n4) continue;
+    float f[4] = {kept[p].x, kept[p].y, kept[p].z, kept[p].w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f[c] = __uint_as_float(__float_as_uint(__builtin_amdgcn_ldexpf(f[c], e)) ^ odd);
+    uint2 part[3];
+    three_parts(f[0], f[1], part[0].x, part[1].x, part[2].x);
+    three_parts(f[2], f[3], part[0].y, part[1].y, part[2].y);
+    if (bits) {
+      const uint32_t u[4] = {__float_as_uint(kept[p].x), __float_as_uint(kept[p].y), __float_as_uint(kept[p].z), __float_as_uint(kept[p].w)};
+      part[0] = make_uint2((u[0] >> 16) | (u[1] & 0xffff0000u), (u[2] >> 16) | (u[3] & 0xffff0000u));
+      part[1] = make_uint2((u[0] & 0xffffu) | (u[1] << 16), (u[2] & 0xffffu) | (u[3] << 16));
     }
-    *reinterpret_cast<uint2*>(dst) = make_uint2(hi[0] | uint32_t(hi[1]) << 16, hi[2] | uint32_t(hi[3]) << 16);
-    *reinterpret_cast<uint2*>(dst + 32) = make_uint2(lo[0] | uint32_t(lo[1]) << 16, lo[2] | uint32_t(lo[3]) << 16);
-  };
-  if (FITS) {
+    unsigned char* dst = dst_row + size_t(i / 8) * kStepBytes + 8 * (i % 8);
 #pragma unroll
-    for (int p = 0; p < (FITS ? PIECES : 0); ++p)
-      if (lane + p * LANES < n4) store(lane + p * LANES, kept[p]);
-  } else {
-    for (int i = lane; i < n4; i += LANES) store(i, value(i, KIND == kRowsGated ? make_float4(0, 0, 0, 0) : raw(i)));
+    for (int c = 0; c < 3; ++c) *reinterpret_cast<uint2*>(dst + 128 * c) = part[c];
   }
 }
 
 template <int KIND>
-int launch_split(hipStream_t s, const SplitSource& src, uint16_t* out, int32_t* exponents, int rows, int K) {
-  if (K <= 2048) split_rows_kernel<1, KIND, true><<<(rows + 3) / 4, 256, 0, s>>>(src, out, exponents, rows, K);
-  else if (K <= 8192) split_rows_kernel<4, KIND, true><<<rows, 256, 0, s>>>(src, out, exponents, rows, K);
-  else split_rows_kernel<4, KIND, false><<<rows, 256, 0, s>>>(src, out, exponents, rows, K);
+int launch_split(hipStream_t s, const SplitSource& src, unsigned char* out, int32_t* exponents, int rows, int K) {
+  if (K <= 2048) split_rows_kernel<1, KIND><<<(rows + 3) / 4, 256, 0, s>>>(src, out, exponents, rows, K);
+  else split_rows_kernel<4, KIND><<<rows, 256, 0, s>>>(src, out, exponents, rows, K);
   return check_launch("sp_gemm_f32_split (rows)");
 }
 
-// Block shapes, blocks a CU holds, and microseconds of a step of 32 along K where few blocks run and where every CU is full,
-// measured over 200 to 2,048 tokens at 896 to 9,728 rows and K of 896 and 4,864; a block's start and end take 6 us, 3 us for
-// blocks that follow others.  (The model is within 20% of what it was fitted to, and the shape it takes within 10% of the best
-// there: 2,048 tokens by 9,728 rows of 896: 384 x 256 113 us, 64 x 128 125, 256 x 128 126, 128 x 128 140, 256 x 256 142;
-// 2,048 by 896 rows of 4,864: 64 x 128 73 us, 64 x 64 82, 128 x 128 108; 256 tokens by 896 rows of 4,864: 64 x 64 41, 64 x 128 66.)
-struct SplitShape { int bm, bn, per_cu; float light_us, full_us; };
-constexpr SplitShape kSplitShapes[] = {{384, 256, 1, 2.5f, 3.8f},   {256, 256, 1, 1.75f, 2.3f}, {256, 128, 1, 1.0f, 1.28f},
-                                       {128, 128, 1, 0.68f, 0.79f}, {64, 128, 2, 0.33f, 0.68f}, {64, 64, 2, 0.23f, 0.54f}};
+// Number k of a split row, as it was.
+__device__ float number_of(const unsigned char* __restrict__ parts, int row, int k, int K, int exponent) {
+  const uint16_t* p = reinterpret_cast<const uint16_t*>(parts + row_at(row, K) + size_t(k / kStep) * kStepBytes) + k % kStep;
+  const uint32_t p1 = p[0], p2 = p[64], p3 = p[128];
+  if (exponent == kNotFinite) return __uint_as_float(p1 << 16 | p2);
+  const float x = __uint_as_float(p1 << 16) + (__uint_as_float(p2 << 16) + __uint_as_float(p3 << 16));
+  return __builtin_amdgcn_ldexpf(row & 1 ? -x : x, -exponent);
+}
 
-int choose_split_shape(int T, int N, int K) {
+// The pipelined kernel of gemm_pipe.h (its ring, its waits, its numbering of tiles) with three parts an operand: a stage is 32 numbers
+// of K, BM + BN rows of three times 64 bytes, each part a plane of lines of two rows.  Piece c of 16 bytes of the row r & 1 of line
+// l = r / 2 lies at position (4 (r & 1) + c) ^ s(l) of it, s(l) = (l ^ l / 4) & 3: the 16 rows that a quarter of a wave reads
+// together lie on all banks, whether the LDS has 32 or 64, and s is the same 32 rows on.  A fetch of 1 KB is eight lines of a
+// plane, which are lines of memory.
+// What bounds it: a wave issues 12 WM WN matrix instructions a stage for 6 (WM + WN) KB from LDS; a block of 256 x 128 reads 72 KB
+// from L2 for 3,072 cycles of matrix instructions a SIMD, as the bfloat16 product of 384 x 256 reads 80.
+template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, int MODE, typename TB>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2 : 1)) void split_product_kernel(
+    const unsigned char* __restrict__ x, const unsigned char* __restrict__ w, const int32_t* __restrict__ x_exp,
+    const int32_t* __restrict__ w_exp, const TB* __restrict__ bias, float* out, int T, int N, int K, RopeArgs rope) {
+  constexpr int NW = WAVES_M * WAVES_N, BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N;
+  constexpr int STAGE = (BM + BN) * 192, XBYTES = BM * 192;
+  constexpr int LX = 3 * BM / (16 * NW), LW = 3 * BN / (16 * NW);      // load instructions per wave, stage and operand
+  static_assert(3 * BM % (16 * NW) == 0 && 3 * BN % (16 * NW) == 0, "every wave fills whole groups of 8 lines");
+  static_assert((STAGES - 2) * (LX + LW) <= 63, "vmcnt holds six bits");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char pipe_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int li = lane & 31, lk = lane >> 5;
+  int tile_n, tile_t;
+  if (!pipe_tile_of(pipe_tiles((T + BM - 1) / BM, (N + BN - 1) / BN), blockIdx.x, &tile_t, &tile_n)) return;
+  const int t0 = tile_t * BM, n0 = tile_n * BN;
+  const int steps = K / kStep;
+  typedef __attribute__((address_space(3))) unsigned char* lds_address_t;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_address_t)pipe_lds;
+  const uint32_t pitch = uint32_t(steps) * kStepBytes;      // of a line of two rows
+  const unsigned char *xbase = x + size_t(t0 / 2) * pitch, *wbase = w + size_t(n0 / 2) * pitch;
+  uint32_t xoff[LX], woff[LW];
+  // fetch u = NW j + wave of an operand: eight lines of part u / (rows / 16)
+  auto offset_of = [&](int u, int rows, int last_line) {
+    const int part = u / (rows / 16), line = (u % (rows / 16)) * 8 + (lane >> 3), piece = (lane & 7) ^ ((line ^ (line >> 2)) & 3);
+    return uint32_t(min(line, last_line)) * pitch + part * 128 + piece * 16;
+  };
+#pragma unroll
+  for (int j = 0; j < LX; ++j) xoff[j] = offset_of(NW * j + wave, BM, (T - 1 - t0) / 2);
+#pragma unroll
+  for (int j = 0; j < LW; ++j) woff[j] = offset_of(NW * j + wave, BN, (N - 1 - n0) / 2);
+  auto fetch = [&](int buf, int step) {
+    const unsigned char* xs = xbase + size_t(step) * kStepBytes;
+    const unsigned char* ws = wbase + size_t(step) * kStepBytes;
+    const uint32_t dst = lds0 + buf * STAGE + wave * 1024;
+#pragma unroll
+    for (int j = 0; j < LX; ++j) load_to_lds(xs, xoff[j], dst + NW * j * 1024);
+#pragma unroll
+    for (int j = 0; j < LW; ++j) load_to_lds(ws, woff[j], dst + XBYTES + NW * j * 1024);
+  };
+  // row 32 i + li of the wave's, pieces 2 ks + lk of a part
+  const uint32_t position = (li >> 1) * 128 + (((((li & 1) << 2) | lk) ^ (((li >> 1) ^ (li >> 3)) & 3)) << 4);
+  const uint32_t xrow = wm * WM * 2048 + position, wrow = XBYTES + wn * WN * 2048 + position;
+
+  floatx16 acc[WM][WN], low[WM][WN];      // sums of the first parts' products, and of the others
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.f;
+
+  auto multiply = [&](int buf) {
+    const unsigned char* stage = pipe_lds + buf * STAGE;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 b[WN][3];
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int h = 0; h < 3; ++h)
+          b[j][h] = as_bf16x8(*reinterpret_cast<const uint4*>(stage + (wrow ^ (ks * 32)) + h * (BN * 64) + j * 2048));
+#pragma unroll
+      for (int i = 0; i < WM; ++i) {
+        bf16x8 a[3];
+#pragma unroll
+        for (int h = 0; h < 3; ++h)
+          a[h] = as_bf16x8(*reinterpret_cast<const uint4*>(stage + (xrow ^ (ks * 32)) + h * (BM * 64) + i * 2048));
+#pragma unroll
+        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][0], a[2], low[i][j]);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) acc[i][j] = mfma32(b[j][0], a[0], acc[i][j]);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][2], a[0], low[i][j]);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][1], a[1], low[i][j]);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][0], a[1], low[i][j]);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][1], a[0], low[i][j]);
+      }
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < steps) fetch(s, s);
+  for (int s0 = 0; s0 < steps; s0 += STAGES) {
+#pragma unroll
+    for (int u = 0; u < STAGES; ++u) {
+      const int s = s0 + u;
+      if (s >= steps) break;
+      // every wave's loads of step s have landed, and every wave is done with step s - 1
+      if (steps - 1 - s >= STAGES - 2) wait_loads_then_barrier<(STAGES - 2) * (LX + LW)>();
+      else wait_loads_then_barrier<0>();
+      if (s + STAGES - 1 < steps) fetch((u + STAGES - 1) % STAGES, s + STAGES - 1);
+      multiply(u);
+    }
+  }
+  bool strange = false;
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    const int t = t0 + (wm * WM + i) * 32 + li, ex = x_exp[min(t, T - 1)];
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int n = n0 + (wn * WN + j) * 32 + 8 * (r / 4) + 4 * lk + r % 4, e = ex + w_exp[min(n, N - 1)];
+        const float back = __builtin_amdgcn_ldexpf(acc[i][j][r] + low[i][j][r], -e);
+        const bool beyond = e >= kNotFinite / 2;      // exponents of finite rows lie between -78 and 199
+        acc[i][j][r] = beyond ? 0.f : (t ^ n) & 1 ? -back : back;
+        strange |= beyond;
+      }
+  }
+  tile_epilogue<WM, WN, MODE, TB, WAVES_N, true>(acc, reinterpret_cast<float*>(pipe_lds), bias, out, T, N, t0, n0, rope);
+  if (!__syncthreads_or(strange)) return;
+  // results of rows that are not finite: bias, and what was there before, stand in the output; the sums are added to them
+  for (int at = threadIdx.x; at < BM * BN; at += 64 * NW) {
+    const int t = t0 + at / BN, n = n0 + at % BN;
+    if (t >= T || n >= N) continue;
+    const int ex = x_exp[t], ew = w_exp[n];
+    if (ex != kNotFinite && ew != kNotFinite) continue;
+    float sum = 0.f;
+    for (int k = 0; k < K; ++k) sum = fmaf(number_of(x, t, k, K, ex), number_of(w, n, k, K, ew), sum);
+    out[size_t(t) * rope.row_stride + n] += sum;
+  }
+}
+
+// Block shapes, blocks a CU holds, microseconds of a block's start and end, of a step of 32 along K on a CU by itself, and of one
+// where the chip is full.
+struct SplitShape { int bm, bn, per_cu; float start_us, light_us, full_us; };
+constexpr SplitShape kSplitShapes[] = {{256, 128, 1, 8.f, 1.75f, 2.35f}, {128, 64, 2, 3.f, 0.73f, 1.38f}, {64, 64, 2, 3.f, 0.44f, 0.80f}};
+
+int choose_split_shape(int T, int N, int K, float* time_us) {
   int best = 0;
-  float best_us = 0.f;
-  const float steps = float(K / 32);
+  const float steps = float(K / kStep);
   for (int i = 0; i < int(sizeof(kSplitShapes) / sizeof(kSplitShapes[0])); ++i) {
     const SplitShape& p = kSplitShapes[i];
     const long blocks = long((T + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), slots = 256 * p.per_cu;
     const long rounds = blocks / slots, rest = blocks % slots;
-    float us = float(rounds) * (3.f + steps * p.full_us) + 3.f;
-    if (rest) us += 3.f + steps * (p.light_us + (p.full_us - p.light_us) * float(rest) / float(slots));
-    if (i == 0 || us < best_us) { best = i; best_us = us; }
+    float us = float(rounds) * (p.start_us + steps * p.full_us) + 3.f;
+    const float shared = p.per_cu == 1 ? float(rest) / float(slots) : rest > 256 ? 1.f : 0.f;
+    if (rest) us += p.start_us + steps * (p.light_us + (p.full_us - p.light_us) * shared);
+    if (i == 0 || us < *time_us) { best = i; *time_us = us; }
   }
   return best;
 }
 
-template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, typename TB>
-int launch_product(hipStream_t s, const split_t* x, const split_t* w, const TB* bias, int mode, float* out, int T, int N, int K,
-                   const RopeArgs& args) {
-  if (mode == kAccumulate)
-    return launch_pipe_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kAccumulate, TB, split_t>(s, 1, x, w, bias, out, T, N, K, K, args);
-  return launch_pipe_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, TB, split_t>(s, 1, x, w, bias, out, T, N, K, K, args);
+struct Product {
+  const unsigned char *x, *w;
+  const int32_t *x_exp, *w_exp;
+  const void* bias;      // may be null
+  float* out;
+  int T, N, K;
+  long long out_stride;
+};
+
+template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, int MODE, typename TB>
+int launch_mode(hipStream_t s, const Product& p) {
+  constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N, lds = STAGES * (BM + BN) * 192;
+  static bool raised = false;
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_product_kernel<WM, WN, WAVES_M, WAVES_N, STAGES, MODE, TB>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) {
+      set_error("sp_gemm_f32_split: cannot raise the LDS limit: %s", hipGetErrorString(e));
+      return 1;
+    }
+    raised = true;
+  }
+  const PipeTiles tiles = pipe_tiles((p.T + BM - 1) / BM, (p.N + BN - 1) / BN);
+  RopeArgs args = {};
+  args.row_stride = p.out_stride;
+  split_product_kernel<WM, WN, WAVES_M, WAVES_N, STAGES, MODE, TB><<<8 * (tiles.own + tiles.run), 64 * WAVES_M * WAVES_N, lds, s>>>(
+      p.x, p.w, p.x_exp, p.w_exp, (const TB*)p.bias, p.out, p.T, p.N, p.K, args);
+  return check_launch("sp_gemm_f32_split");
 }
 
-template <typename TB>
-int product(hipStream_t s, int shape, const split_t* x, const split_t* w, const TB* bias, int mode, float* out, int T, int N, int K,
-            const RopeArgs& args) {
-  switch (shape) {
-    case 0: return launch_product<6, 2, 2, 4, 2, TB>(s, x, w, bias, mode, out, T, N, K, args);
-    case 1: return launch_product<4, 2, 2, 4, 2, TB>(s, x, w, bias, mode, out, T, N, K, args);
-    case 2: return launch_product<2, 2, 4, 2, 3, TB>(s, x, w, bias, mode, out, T, N, K, args);
-    case 3: return launch_product<2, 2, 2, 2, 4, TB>(s, x, w, bias, mode, out, T, N, K, args);
-    case 4: return launch_product<1, 2, 2, 2, 3, TB>(s, x, w, bias, mode, out, T, N, K, args);
-    default: return launch_product<1, 1, 2, 2, 4, TB>(s, x, w, bias, mode, out, T, N, K, args);
+template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES>
+int launch_product(hipStream_t s, const Product& p, bool add, int bias_dtype) {
+  if (p.bias && bias_dtype == kBF16)
+    return add ? launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kAccumulate, bf16_t>(s, p)
+               : launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, bf16_t>(s, p);
+  return add ? launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kAccumulate, float>(s, p)
+             : launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, float>(s, p);
+}
+
+int product(hipStream_t s, const Product& p, bool add, int bias_dtype) {
+  float time_us;
+  switch (choose_split_shape(p.T, p.N, p.K, &time_us)) {
+    case 0: return launch_product<2, 2, 4, 2, 2>(s, p, add, bias_dtype);
+    case 1: return launch_product<2, 1, 2, 2, 2>(s, p, add, bias_dtype);
+    default: return launch_product<1, 1, 2, 2, 3>(s, p, add, bias_dtype);
   }
 }
 
+// ... and of a split of `rows` rows of K numbers, at 4.6 TB/s.
+float split_time_us(int rows, int K) { return 4.f + float(rows) * float(K) * 10.f / 4.6e6f; }
+
 int64_t aligned(int64_t bytes) { return (bytes + 255) / 256 * 256; }
-// Rows of w of one launch: all of them, or as many whole tiles as the chunk holds.
-int chunk_rows(int N, int K) {
-  const int64_t rows = kChunkBytes / (int64_t(K) * 4) / 256 * 256;
-  return int(rows >= N ? N : rows);
+int64_t split_bytes(int rows, int K) { return aligned(int64_t((rows + 1) / 2) * (K / kStep) * kStepBytes); }
+// Numbers of K of one pass: all, or equal pieces of whole steps.
+int piece_of(int K) {
+  const int pieces = (K + kMaxK - 1) / kMaxK;
+  return ((K / kStep + pieces - 1) / pieces) * kStep;
+}
+// Rows of w of one launch: all of them; or of those that the chunk holds whole rounds of the largest blocks over the chip.
+int chunk_rows(int T, int N, int K) {
+  const int64_t rows = kChunkBytes / (int64_t(K) * 6) / 256 * 256;
+  if (rows >= N) return N;
+  const int token_tiles = (T + 255) / 256, round = token_tiles < 256 ? 256 / token_tiles * 128 : 256;
+  return int(rows >= round ? rows / round * round : rows);
 }
 
 }  // namespace
@@ -203,13 +385,33 @@ int chunk_rows(int N, int K) {
 
 using namespace sprout;
 
-// Bytes of workspace that sp_gemm_f32_split wants for T tokens by N rows of K, or 0 where it does not take the product or
-// the float32 instruction is as fast: the weights are split once a call, which few tokens do not pay for (whole call against the
-// float32 instruction: 200 tokens by 1,152 rows of 896 21.5 us against 20.7; 256 by 9,728 of 896 47 against 53, 256 by 896 of
-// 4,864 55 against 87; 2,048 by 9,728 of 896 132 against 329).
+// Bytes of workspace that sp_gemm_f32_split wants for T tokens by N rows of K, or 0 where it does not take the product.
 extern "C" int64_t sp_gemm_f32_split_bytes(int T, int N, int K) {
-  if (T < 256 || N < 1 || K < 64 || K % 32 || int64_t(K) * 4 * 384 >= (int64_t(1) << 31) || chunk_rows(N, K) < 1) return 0;
-  return aligned(int64_t(T) * K * 4) + aligned(int64_t(chunk_rows(N, K)) * K * 4) + aligned(int64_t(T) * 4) + aligned(int64_t(N) * 4);
+  if (T < 256 || N < 1 || K < 64 || K % kStep) return 0;
+  const int piece = piece_of(K);
+  return split_bytes(T, piece) + split_bytes(chunk_rows(T, N, piece), piece) + aligned(int64_t(T) * 4) + aligned(int64_t(N) * 4);
+}
+
+// Whether sp_gemm_f32_split is taken to be faster than the float32 instruction's kernel: the weights are split once a call, which
+// few tokens do not pay for, and small products pay for the launches (whole calls with the norm or the gate before them, float32
+// instruction -> this, us: 640 tokens by 9,728 rows of 896 129 -> 92, 2,048 303 -> 235; 896 rows of 4,864 at 1,500 tokens 176 -> 138, 2,048
+// 182 -> 154; 37,888 of 3,584 at 512 tokens 1,108 -> 1,216, at 1,024 2,170 -> 1,862, at 2,048 4,268 -> 2,958; 3,584 of 18,944 at 512
+// 645 -> 652, at 2,048 2,339 -> 1,654; 896 of 896 at 2,048 34 -> 43).  The two estimates were within a fifth of what was measured
+// over 124 products, and took none to the slower side by more than 3 %.
+extern "C" int sp_gemm_f32_split_pays(int T, int N, int K) {
+  if (sp_gemm_f32_split_bytes(T, N, K) == 0) return 0;
+  const int piece = piece_of(K), chunk = chunk_rows(T, N, piece);
+  float us = 0.f;
+  for (int k = 0; k < K; k += piece) {
+    const int width = min(K - k, piece);
+    us += split_time_us(T, width);
+    for (int n = 0; n < N; n += chunk) {
+      float time_us;
+      choose_split_shape(T, min(N - n, chunk), width, &time_us);
+      us += split_time_us(min(N - n, chunk), width) + time_us;
+    }
+  }
+  return us < gemm_f32_time_us(T, N, K);
 }
 
 // out[T, N] = or += rows . w^T + bias, everything float32; rows: `kind` 0: a [T, K]; 1: act(a[:, :K], a[:, K:]) of a [T, 2 K];
@@ -227,31 +429,30 @@ extern "C" int sp_gemm_f32_split(void* stream, int kind, const float* a, const f
               reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(workspace)) % 16 == 0,
              "sp_gemm_f32_split: operands must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  const int chunk = chunk_rows(N, K);
+  const int piece = piece_of(K), chunk = chunk_rows(T, N, piece);
   unsigned char* at = (unsigned char*)workspace;
-  uint16_t* xs = (uint16_t*)at; at += aligned(int64_t(T) * K * 4);
-  uint16_t* ws = (uint16_t*)at; at += aligned(int64_t(chunk) * K * 4);
+  unsigned char* xs = at; at += split_bytes(T, piece);
+  unsigned char* ws = at; at += split_bytes(chunk, piece);
   int32_t* x_exp = (int32_t*)at; at += aligned(int64_t(T) * 4);
   int32_t* w_exp = (int32_t*)at;
-  SplitSource src = {a, norm_w, eps, activation, limit};
-  if (kind == kRowsAsTheyAre ? launch_split<kRowsAsTheyAre>(s, src, xs, x_exp, T, K)
-      : kind == kRowsGated   ? launch_split<kRowsGated>(s, src, xs, x_exp, T, K)
-                             : launch_split<kRowsNormed>(s, src, xs, x_exp, T, K))
-    return 1;
-  RopeArgs args = {};
-  args.row_stride = N;
-  args.x_exp = x_exp;
-  for (int n = 0; n < N; n += chunk) {
-    const int rows = N - n < chunk ? N - n : chunk;
-    SplitSource wsrc = {};
-    wsrc.a = w + size_t(n) * K;
-    if (launch_split<kRowsAsTheyAre>(s, wsrc, ws, w_exp + n, rows, K)) return 1;
-    args.w_exp = w_exp + n;
-    const int shape = choose_split_shape(T, rows, K);
-    const int rc = bias && bias_dtype == kBF16
-        ? product<bf16_t>(s, shape, (const split_t*)xs, (const split_t*)ws, (const bf16_t*)bias + n, mode == 1 ? kAccumulate : kStoreF32, out + n, T, rows, K, args)
-        : product<float>(s, shape, (const split_t*)xs, (const split_t*)ws, bias ? (const float*)bias + n : nullptr, mode == 1 ? kAccumulate : kStoreF32, out + n, T, rows, K, args);
-    if (rc) return rc;
+  for (int k = 0; k < K; k += piece) {
+    const int width = K - k < piece ? K - k : piece;
+    const SplitSource src = {a, K, k, norm_w, eps, activation, limit};
+    if (kind == kRowsAsTheyAre ? launch_split<kRowsAsTheyAre>(s, src, xs, x_exp, T, width)
+        : kind == kRowsGated   ? launch_split<kRowsGated>(s, src, xs, x_exp, T, width)
+                               : launch_split<kRowsNormed>(s, src, xs, x_exp, T, width))
+      return 1;
+    for (int n = 0; n < N; n += chunk) {
+      const int rows = N - n < chunk ? N - n : chunk;
+      SplitSource wsrc = {};
+      wsrc.a = w + size_t(n) * K;
+      wsrc.length = K;
+      wsrc.first = k;
+      if (launch_split<kRowsAsTheyAre>(s, wsrc, ws, w_exp + n, rows, width)) return 1;
+      const void* rows_bias = !bias || k > 0 ? nullptr : bias_dtype == kBF16 ? (const void*)((const bf16_t*)bias + n) : (const void*)((const float*)bias + n);
+      const Product p = {xs, ws, x_exp, w_exp + n, rows_bias, out + n, T, rows, width, N};
+      if (const int rc = product(s, p, mode == 1 || k > 0, bias_dtype)) return rc;
+    }
   }
   return 0;
 }

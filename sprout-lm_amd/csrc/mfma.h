@@ -27,13 +27,6 @@ __device__ __forceinline__ floatx16 mfma32_f32(float a, float b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-// v_mfma_f32_32x32x16_f16: the layout of mfma32 with float16 operands.
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ f16x8 as_f16x8(uint4 v) { return __builtin_bit_cast(f16x8, v); }
-__device__ __forceinline__ floatx16 mfma32_f16(f16x8 a, f16x8 b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 __device__ __forceinline__ uint4 ldg128(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 
@@ -42,6 +35,17 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 // Two floats to two bfloat16 (round to nearest even) in one instruction.
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
+}
+// Two floats into three bfloat16 parts each, packed: a = a1 + a2 + a3 to the last bit (eight bits and a sign a part), where a3 does not
+// underflow.
+__device__ __forceinline__ void three_parts(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
+  p1 = pack_bf16x2(a, b);
+  a -= __uint_as_float(p1 << 16);
+  b -= __uint_as_float(p1 & 0xffff0000u);
+  p2 = pack_bf16x2(a, b);
+  a -= __uint_as_float(p2 << 16);
+  b -= __uint_as_float(p2 & 0xffff0000u);
+  p3 = pack_bf16x2(a, b);
 }
 
 }  // namespace sprout

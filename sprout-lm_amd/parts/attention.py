@@ -147,7 +147,7 @@ class Attention(Mixer):
                          kind=ctx.attention_kind, project=project, scores=self.scores, softcap=self.softcap):
             return
         if not ops.gemm_f32_split(attn, self.w_o, residual, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=self.b_o,
-                                  accumulate=True):
+                                  accumulate=True, if_faster=True):
             ops.gemm(attn, self.w_o, residual, bias=self.b_o, accumulate=True)
 
     def forward(self, ctx, h, residual, cache):
@@ -182,7 +182,7 @@ class Attention(Mixer):
         """Many tokens on the float32 path: the norm is folded into the projections' operand."""
         qkv, w, b, nkv = self._projections(ctx, residual.shape[0], cache)
         if not ops.gemm_f32_split(residual, w, qkv, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=b,
-                                  norm=(fold.weight, fold.eps)):
+                                  norm=(fold.weight, fold.eps), if_faster=True):
             return False
         self._rotate_and_attend(ctx, qkv, nkv, residual, cache)
         return True

@@ -74,13 +74,12 @@ class GatedMLP(FeedForward):
     def _split_f32(self, ctx, residual, fold) -> bool:
         """Many tokens on the float32 path: the norm is folded into the first product's operand, the gate into the second's."""
         T = residual.shape[0]
-        if min(ops.gemm_f32_split_bytes(T, 2 * self.inner, self.hidden), ops.gemm_f32_split_bytes(T, self.hidden, self.inner)) == 0:
-            return False
         scratch = lambda n: ctx.buffer("f32_split", (n,), torch.uint8)
         gu = ctx.buffer("gate_up", (T, 2 * self.inner), ctx.act_dtype)
-        if not ops.gemm_f32_split(residual, self.w_gate_up, gu, scratch, norm=(fold.weight, fold.eps)):
+        if not ops.gemm_f32_split(residual, self.w_gate_up, gu, scratch, norm=(fold.weight, fold.eps), if_faster=True):
             return False
-        if not ops.gemm_f32_split(gu, self.w_down, residual, scratch, accumulate=True, activation=self.activation, limit=self.limit):
+        if not ops.gemm_f32_split(gu, self.w_down, residual, scratch, accumulate=True, activation=self.activation, limit=self.limit,
+                                  if_faster=True):
             act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
             ops.silu_mul(gu, act, activation=self.activation, limit=self.limit)
             ops.gemm(act, self.w_down, residual, accumulate=True)

@@ -1,15 +1,15 @@
-"""float32 products of many tokens as products of float16 pairs, against float64 products of the same numbers."""
+"""float32 products of many tokens as products of bfloat16 parts, against float64 products of the same numbers."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# What the pairs, the three products and the float32 sums may lose of a sum of K products, against the sum of their
-# magnitudes: each operand is a pair to 2^-23, the product of the lower parts (2^-22) is left out, and 3 K / 16 sums of
-# sixteen products round to 2^-24 of the running sum each (their errors add up in the worst case only: a quarter of that).
+# What the parts, the six products and the float32 sums may lose of a sum of K products, against the sum of their magnitudes: the
+# products that are left out are 2^-25 together, the K / 16 sums of sixteen first parts' products round to 2^-24 of the running sum
+# each (their errors add up in the worst case only), the sums of the others to 2^-32, and two more where they meet and pieces add.
 def bound(K):
-    return 3 * 2.0 ** -22 + 3 * K / 16 * 2.0 ** -24 / 4
+    return 2.0 ** -25 + (K / 16 + 2) * 2.0 ** -24 + 5 * K / 16 * 2.0 ** -32
 
 
 def rows(T, K, seed, span=0):
@@ -25,10 +25,10 @@ def scratch(n):
     return torch.empty(n, dtype=torch.uint8, device=DEV)
 
 
-# one and several tiles of every block shape with remainders, one step and an odd number of steps of K, rows in and beyond a
-# wave's and a block's registers, weights of more than a chunk
+# one and several tiles of every block shape with remainders, one step and an odd number of steps of K, rows that a wave and that a
+# block splits, K in one piece and in several (the last of them shorter), weights of more than a chunk
 @pytest.mark.parametrize("T,N,K", [(256, 64, 64), (257, 1, 96), (300, 129, 896), (513, 4865, 160), (260, 896, 4864),
-                                   (2048, 1152, 896), (1025, 2432, 2080), (2048, 9728, 96), (256, 70, 8256), (256, 9001, 8192)])
+                                   (2048, 1152, 896), (1025, 2432, 2080), (2048, 9728, 96), (256, 70, 8256), (256, 9001, 8192), (2048, 5000, 5120)])
 @pytest.mark.parametrize("kind", ["rows", "norm", "gate"])
 def test_split_products(T, N, K, kind):
     from sprout_lm_amd import ops
@@ -97,3 +97,71 @@ def test_the_error_has_no_side(K):
     assert abs(float(error.mean())) <= 7 * spread / (2048 * 896) ** 0.5
     assert float(error.mean(0).square().mean().sqrt()) <= 2 * spread / 2048 ** 0.5
     assert float(error.mean(1).square().mean().sqrt()) <= 2 * spread / 896 ** 0.5
+
+
+def spread(x, w, out):
+    """2-norm of the error over the 2-norm of the result, against 64 bits."""
+    want = x.double() @ w.double().t()
+    return float((out.double() - want).norm() / want.norm())
+
+
+def both(x, w):
+    """Errors of this product and of the float32 instruction's."""
+    from sprout_lm_amd import ops
+    out, plain = (torch.empty(x.shape[0], w.shape[0], device=DEV) for _ in range(2))
+    assert ops.gemm_f32_split(x, w, out, scratch)
+    ops.gemm(x, w, plain)
+    return spread(x, w, out), spread(x, w, plain)
+
+
+@pytest.mark.parametrize("power", [0, 18, 24, 40, 100])
+@pytest.mark.parametrize("against", ["its inverse", "zero"])
+def test_a_number_that_stands_far_out_of_its_row(power, against):
+    """It meets a weight that takes it back, or none: the others must keep all their bits beside it."""
+    x, w = rows(300, 896, 11), rows(200, 896, 12)
+    x[:, 5] *= 2.0 ** power
+    w[:, 5] *= 0.0 if against == "zero" else 2.0 ** -power
+    got, plain = both(x, w)
+    assert got <= plain
+    x, w = rows(200, 896, 12), rows(300, 896, 11)      # and among the weights
+    w[:, 5] *= 2.0 ** power
+    x[:, 5] *= 0.0 if against == "zero" else 2.0 ** -power
+    got, plain = both(x.repeat(2, 1), w)
+    assert got <= plain
+
+
+@pytest.mark.parametrize("count", [1, 2, 4, 8, 64])
+def test_few_products_carry_the_result(count):
+    """Weights with `count` numbers a row that are not zero: no worse than the float32 instruction, a quarter more for the spread of
+    so few roundings."""
+    x, w = rows(512, 896, 21), torch.zeros(1024, 896, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(22)
+    at = torch.rand(1024, 896, device=DEV, generator=g).argsort(-1)[:, :count]
+    w.scatter_(1, at, torch.randn(1024, count, device=DEV, generator=g))
+    got, plain = both(x, w)
+    assert got <= 1.25 * plain
+
+
+@pytest.mark.parametrize("mode", ["store", "add"])
+def test_infinities_stay_infinities(mode):
+    from sprout_lm_amd import ops
+    x, w = rows(300, 160, 31), rows(190, 160, 32)
+    inf = float("inf")
+    x[5, 7], x[9, 0], x[11, 3], x[11, 4], x[299, 159] = inf, float("nan"), inf, inf, -inf
+    w[4, 95], w[189, 7], w[60, 30], w[61] = -inf, inf, float("nan"), 0.0
+    out, plain = torch.ones(300, 190, device=DEV), torch.ones(300, 190, device=DEV)
+    bias = torch.randn(190, device=DEV)
+    assert ops.gemm_f32_split(x, w, out, scratch, bias=bias, accumulate=mode == "add")
+    ops.gemm(x, w, plain, bias=bias, accumulate=mode == "add")
+    assert torch.equal(out.isnan(), plain.isnan()), (out.isnan() != plain.isnan()).nonzero()[:8]
+    assert plain.isinf().sum() > 300
+    assert torch.equal(out[out.isinf()], plain[out.isinf()]) and torch.equal(out.isinf(), plain.isinf())
+
+
+def test_where_the_split_product_is_taken_for_the_faster_way():
+    """Where it is not, the call is refused and nothing is written."""
+    from sprout_lm_amd import ops
+    for T, N, K, faster in [(2048, 9728, 896, True), (2048, 896, 4864, True), (640, 896, 896, False), (256, 64, 64, False)]:
+        out = torch.zeros(T, N, device=DEV)
+        assert ops.gemm_f32_split(rows(T, K, 1), rows(N, K, 2), out, scratch, if_faster=True) == faster
+        assert bool(out.any()) == faster
