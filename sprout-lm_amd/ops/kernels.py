@@ -583,19 +583,21 @@ def gemm_f32_split_bytes(T: int, N: int, K: int) -> int:
     return library().sp_gemm_f32_split_bytes(T, N, K)
 
 
+def gemm_f32_split_pays(T: int, N: int, K: int) -> bool:
+    """Whether `gemm_f32_split` takes the product of T tokens by N rows of K and is taken to be faster than `gemm`."""
+    return bool(library().sp_gemm_f32_split_pays(T, N, K))
+
+
 def gemm_f32_split(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, workspace, bias: torch.Tensor | None = None,
-                   accumulate: bool = False, norm=None, activation: str | None = None, limit: float = 0.0, if_faster: bool = False) -> bool:
+                   accumulate: bool = False, norm=None, activation: str | None = None, limit: float = 0.0) -> bool:
     """out = (or, with accumulate, +=) rows @ w.T (+ bias), everything float32, for many tokens; rows = a, or rmsnorm(a) * weight
     with `norm` = (weight, eps), or act(a[:, :K]) * a[:, K:] with an `activation`.  `workspace`: bytes -> a uint8 tensor.
-    Returns False (and does nothing) where the kernel does not take the product or, with `if_faster`, where `gemm` is taken to be
-    the faster way."""
+    Returns False (and does nothing) where the kernel does not take the product."""
     T, (N, K) = a.shape[0], w.shape
     if not (a.dtype == w.dtype == out.dtype == torch.float32) or tuple(out.shape) != (T, N) \
             or a.shape[1] != (K if activation is None else 2 * K):
         return False
     need = gemm_f32_split_bytes(T, N, K)
-    if need and if_faster and not library().sp_gemm_f32_split_pays(T, N, K):
-        return False
     if need == 0 or (a.data_ptr() | w.data_ptr() | out.data_ptr()) & 15:
         return False
     if norm is not None and (activation is not None or norm[0].dtype != torch.float32 or norm[0].numel() != K or norm[0].data_ptr() & 15):

@@ -146,8 +146,9 @@ class Attention(Mixer):
                          workspace=lambda n: ctx.buffer("attention_partials", (n,), torch.float32),
                          kind=ctx.attention_kind, project=project, scores=self.scores, softcap=self.softcap):
             return
-        if not ops.gemm_f32_split(attn, self.w_o, residual, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=self.b_o,
-                                  accumulate=True, if_faster=True):
+        if not (self._split_pays(ctx, attn, self.w_o)
+                and ops.gemm_f32_split(attn, self.w_o, residual, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=self.b_o,
+                                       accumulate=True)):
             ops.gemm(attn, self.w_o, residual, bias=self.b_o, accumulate=True)
 
     def forward(self, ctx, h, residual, cache):
@@ -178,11 +179,16 @@ class Attention(Mixer):
             b = None if b is None else b[: self.heads * self.head_dim]
         return qkv, w, b, nkv
 
+    @staticmethod
+    def _split_pays(ctx, rows, w) -> bool:
+        return ctx.act_dtype == torch.float32 and ops.gemm_f32_split_pays(rows.shape[0], *w.shape)
+
     def _split_f32(self, ctx, residual, cache, fold) -> bool:
         """Many tokens on the float32 path: the norm is folded into the projections' operand."""
         qkv, w, b, nkv = self._projections(ctx, residual.shape[0], cache)
-        if not ops.gemm_f32_split(residual, w, qkv, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=b,
-                                  norm=(fold.weight, fold.eps), if_faster=True):
+        if not (self._split_pays(ctx, residual, w)
+                and ops.gemm_f32_split(residual, w, qkv, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=b,
+                                       norm=(fold.weight, fold.eps))):
             return False
         self._rotate_and_attend(ctx, qkv, nkv, residual, cache)
         return True

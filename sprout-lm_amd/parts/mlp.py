@@ -55,10 +55,12 @@ class GatedMLP(FeedForward):
         if fold is None or fold.kind != "rms":       # the one prologue the product kernels have
             return False
         if ctx.act_dtype == torch.float32 and self.fuse_input_norm_f32:
+            if ops.gemm_f32_split_pays(T, 2 * self.inner, self.hidden) and self._split_f32(ctx, residual, fold):
+                return True
             act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
             if not ops.gate_up_silu_f32(self.w_gate_up, residual, act, activation=self.activation, norm_weight=fold.weight,
                                         eps=fold.eps, limit=self.limit):
-                return self._split_f32(ctx, residual, fold)
+                return False
             ops.gemm(act, self.w_down, residual, accumulate=True)
             return True
         if ctx.act_dtype != torch.bfloat16 or T > 64 or not self._fused(T, True):
@@ -72,14 +74,15 @@ class GatedMLP(FeedForward):
         return True
 
     def _split_f32(self, ctx, residual, fold) -> bool:
-        """Many tokens on the float32 path: the norm is folded into the first product's operand, the gate into the second's."""
+        """Many tokens on the float32 path: the norm is folded into the first product's operand, and where the second is taken too
+        the gate into its own; the gated rows then have no tensor."""
         T = residual.shape[0]
         scratch = lambda n: ctx.buffer("f32_split", (n,), torch.uint8)
         gu = ctx.buffer("gate_up", (T, 2 * self.inner), ctx.act_dtype)
-        if not ops.gemm_f32_split(residual, self.w_gate_up, gu, scratch, norm=(fold.weight, fold.eps), if_faster=True):
+        if not ops.gemm_f32_split(residual, self.w_gate_up, gu, scratch, norm=(fold.weight, fold.eps)):
             return False
-        if not ops.gemm_f32_split(gu, self.w_down, residual, scratch, accumulate=True, activation=self.activation, limit=self.limit,
-                                  if_faster=True):
+        if not (ops.gemm_f32_split_pays(T, self.hidden, self.inner)
+                and ops.gemm_f32_split(gu, self.w_down, residual, scratch, accumulate=True, activation=self.activation, limit=self.limit)):
             act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
             ops.silu_mul(gu, act, activation=self.activation, limit=self.limit)
             ops.gemm(act, self.w_down, residual, accumulate=True)

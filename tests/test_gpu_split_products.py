@@ -158,10 +158,33 @@ def test_infinities_stay_infinities(mode):
     assert torch.equal(out[out.isinf()], plain[out.isinf()]) and torch.equal(out.isinf(), plain.isinf())
 
 
-def test_where_the_split_product_is_taken_for_the_faster_way():
-    """Where it is not, the call is refused and nothing is written."""
+
+def test_the_step_takes_no_tensor_that_it_does_not_use():
+    """A gated feed-forward of 2,048 tokens at 0.5B sizes: the norm and the gate are folded, so that neither the normed rows nor the
+    gated ones have a tensor; and what the whole of it takes is less than half as much again as rows and gate took before the parts."""
     from sprout_lm_amd import ops
-    for T, N, K, faster in [(2048, 9728, 896, True), (2048, 896, 4864, True), (640, 896, 896, False), (256, 64, 64, False)]:
-        out = torch.zeros(T, N, device=DEV)
-        assert ops.gemm_f32_split(rows(T, K, 1), rows(N, K, 2), out, scratch, if_faster=True) == faster
-        assert bool(out.any()) == faster
+    from sprout_lm_amd.engine.batch import StepContext, Workspace
+    from sprout_lm_amd.parts.mlp import GatedMLP
+    from sprout_lm_amd.parts.norm import RMSNorm
+    T, H, I = 2048, 896, 4864
+    assert ops.gemm_f32_split_pays(T, 2 * I, H) and ops.gemm_f32_split_pays(T, H, I)
+    mlp, norm = GatedMLP(H, I), RMSNorm(H, 1e-6)
+    gate, up, down = rows(I, H, 1), rows(I, H, 2), rows(H, I, 3)
+    mlp.bind(dict(zip(mlp.names, (gate, up, down))))
+    norm.bind({"weight": torch.ones(H, device=DEV)})
+    ctx = StepContext(Workspace(torch.device(DEV)), torch.float32)
+    residual = rows(T, H, 4)
+    x = torch.nn.functional.rms_norm(residual.double(), (H,), eps=1e-6)
+    want = residual.double() + (torch.nn.functional.silu(x @ gate.double().t()) * (x @ up.double().t())) @ down.double().t()
+    assert mlp.forward_from_residual(ctx, norm, residual)
+    assert float((residual.double() - want).norm() / want.norm()) < 2e-6
+    held = {name for name, _ in ctx.workspace._flat}
+    assert held == {"gate_up", "f32_split"}
+    assert sum(t.numel() * t.element_size() for t in ctx.workspace._flat.values()) <= 1.5 * 4 * T * (3 * I + H)
+
+
+@pytest.mark.parametrize("H,I,kv", [(896, 4864, 128), (3584, 18944, 512), (5120, 27648, 1024)])
+def test_workspace_of_the_largest_steps(H, I, kv):
+    """Split operands of a step of 2,048 tokens: 200 MB at most, whatever the sizes."""
+    from sprout_lm_amd import ops
+    assert max(ops.gemm_f32_split_bytes(2048, n, k) for n, k in ((2 * I, H), (H, I), (H + 2 * kv, H), (H, H))) <= 200e6
