@@ -28,9 +28,10 @@ size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, 
   return splits <= 1 ? 0 : size_t(n_tiles) * 32 * nq * splits * (hd + 2);
 }
 
+// (In whole 16 bytes: a prompt's parts, written and read as float4, lie behind it in a mixed step's workspace.)
 size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_ctx) {
   const size_t splits = (max_ctx + kDecodeChunk - 1) / kDecodeChunk;
-  return splits <= 1 ? 0 : size_t(n_decode) * nq * splits * (hd + 2);
+  return splits <= 1 ? 0 : (size_t(n_decode) * nq * splits * (hd + 2) + 3) / 4 * 4;
 }
 
 int attention_mfma_wide(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,

@@ -18,7 +18,9 @@ def attention(kind, q, k, v, tables, batch, nq, nkv, **options):
 # in the first and in the last of a stage's steps; more page numbers than LDS holds
 CASES = [(64, 8, 8, [(1024, 1024)]), (48, 8, 32, [(700, 700), (331, 300), (33, 33), (9, 1)]), (24, 2, 64, [(2049, 2049)]),
          (14, 2, 16, [(4129, 2048)]), (14, 2, 16, [(4224, 2017), (2100, 31)]), (14, 2, 16, [(33001, 250)]),
-         (7, 1, 8, [(16384, 1000), (200, 200)]), (64, 8, 8, [(33000, 2048)]), (56, 8, 16, [(4096, 4096 - 2048), (130, 130)])]
+         (7, 1, 8, [(16384, 1000), (200, 200)]), (64, 8, 8, [(33000, 2048)]), (56, 8, 16, [(4096, 4096 - 2048), (130, 130)]),
+         # a one-query sequence whose parts are no whole number of sixteen bytes, before the prompt's in the workspace
+         (7, 1, 16, [(700, 1), (16384, 1000)])]
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
@@ -44,3 +46,32 @@ def test_rows_attention(case):
     size = attention(1, q, k, v.abs(), *args[3:])
     # weights rounded to bfloat16 (2^-9 of each, on both sides of the quotient's numerator only) and both results rounded
     assert ((got - want).abs() <= 2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-6).all()
+
+
+def test_keys_and_values_that_are_not_finite():
+    """As the general kernel has it: a key whose score is minus infinity weighs nothing, an infinite value is one for every row that
+    sees it, NaN stays with the rows and dimensions it reaches.  All before the first query, so that every row sees them."""
+    from sprout_lm_amd import ops
+    nq, nkv, page, ctx, n = 14, 2, 16, 4129, 2048
+    inf = float("inf")
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    pages = -(-ctx // page)
+    k, v, q = rand(pages, nkv, page, 64), rand(pages, nkv, 64, page), rand(n, nq, 64)
+    tables = torch.arange(pages, device=DEV, dtype=torch.int32)[None].contiguous()
+    q[..., 3] = q[..., 3].abs() + 0.1
+    k[5, :, 7, 3], k[40, 0, 0, 3] = -inf, -inf                  # scores of minus infinity
+    v[9, 0, 11, 2], v[60, 1, 12, 15], v[61, 1, 12, 0] = inf, inf, -inf
+    v[80, 1, 40, 8] = float("nan")
+    q[100, 3, 9] = float("nan")
+    q, k, v = q.view(n, -1).bfloat16(), k.bfloat16(), v.bfloat16()
+    results = [attention(kind, q, k, v, tables, ops.AttentionBatch.build([n], [ctx], DEV), nq, nkv) for kind in (0, 1)]
+    got, want = (x.view(n, nq, 64) for x in results)
+    assert got[100, 3].isnan().all()      # (the general kernel's row of a query that is NaN has zeros)
+    got[100, 3] = want[100, 3] = 0.0
+    assert torch.equal(got.isnan(), want.isnan()) and want.isinf().sum() == 7 * (n - 1) + 6
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    good = want.isfinite()
+    assert good.float().mean() > 0.95
+    # as above, of values of unit size
+    assert ((got - want)[good].abs() <= 2.0 ** -8 * 4 + 2.0 ** -8 * want[good].abs()).all()

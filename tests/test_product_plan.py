@@ -135,3 +135,12 @@ def test_blocks_are_numbered_so_that_every_tile_runs_once_and_the_xcds_share_the
     with pytest.raises(ops.KernelError):
         ops.pipe_tiles(0, 5)
 
+
+
+def test_parts_of_prompts_lie_at_whole_sixteen_bytes_of_a_mixed_step_s_workspace():
+    """They come behind the one-query sequences' parts and are read and written sixteen bytes at a time; those in turn are as many
+    floats as heads, sequences and chunks give, 1,386 here."""
+    lib = ops.library()
+    for nq, nkv, hd, n_decode, ctx in [(7, 1, 64, 1, 700), (5, 5, 16, 3, 257), (14, 2, 64, 8, 4096), (3, 1, 80, 5, 1100)]:
+        decode = lib.sp_attention_workspace_floats(1, hd, 16, nq, nkv, 0, n_decode, ctx, 0, 0)
+        assert decode % 4 == 0 and 0 <= decode - n_decode * nq * -(-ctx // 256) * (hd + 2) < 4
