@@ -1155,7 +1155,7 @@ static int decode_sets(int nq, int nkv) {
   return nkv * (G / rows);
 }
 
-constexpr int kMaxPrefillSplits = 32;   // the merge kernel holds one split per lane; 64 would do as well
+constexpr int kMaxPrefillSplits = 32;   // (more parts of a walk than that and their merge costs more than they save)
 
 static bool staged_prefill(int page_size) { return page_size >= 8 && (page_size & (page_size - 1)) == 0; }
 
@@ -1213,6 +1213,7 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
 int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; its splits are 0 where it is not the faster one.
 int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
+bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk);
 int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
                           const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                           const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int max_tile_ctx, int splits, uint16_t* out,
@@ -1236,7 +1237,8 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       int page_shift = 0;
       while ((1 << page_shift) < page_size) ++page_shift;
       const bool plain = st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && st.keep <= 0 && !st.sinks && !st.bias && !st.gate;
-      const int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
+      int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
+      if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk)) rows_splits = 0;
       const int splits = rows_splits ? rows_splits : attention_prefill_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx);
       const int stages = (max_tile_ctx + kStageKeys - 1) / kStageKeys;
       const int per_split = (stages + splits - 1) / splits;

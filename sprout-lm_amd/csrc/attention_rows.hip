@@ -141,8 +141,13 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   constexpr int HD = 64;
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];      // two stages, then the page numbers
   int32_t* s_table = reinterpret_cast<int32_t*>(ring + 2 * kRowsStageBytes);
-  // tiles are listed in order of position; the last ones walk the most keys, so they start first
-  const int tile = n_tiles - 1 - int(blockIdx.x);
+  // Tiles are listed in order of position; the last ones walk the most keys, so they start first.  Two blocks run on a CU, the second
+  // 256 blocks behind the first: where the blocks of a part of the keys fill the 256 in whole numbers, those behind take the tiles the
+  // other way round, so that a CU has a long walk and a short one (1,024 queries over 4,096 keys beside eight prompts of 128, 14 heads
+  // in 2 groups: 51 -> 40 us, the paired walks of attention_mfma.h 46; over 32,768 beside five of 256 276 -> 188).
+  const unsigned part = gridDim.x * gridDim.y;
+  const bool turned = 256 % part == 0 && (blockIdx.z * part / 256 & 1);
+  const int tile = turned ? int(blockIdx.x) : n_tiles - 1 - int(blockIdx.x);
   const int seq = tiles[2 * tile], q_off = tiles[2 * tile + 1];
   const int G = nq / nkv, sets = (G + 7) / 8, g = blockIdx.y / sets, first_head = (blockIdx.y % sets) * 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, li = lane & 31, lk = lane >> 5;
@@ -335,6 +340,21 @@ int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, i
   const long blocks = long(n_tiles) * nkv * sets;
   if (blocks * max(1, max_tile_ctx / 2048) < 256) return 0;
   return max(1, min(int(512 / blocks), max_tile_ctx / (blocks >= 256 ? 4096 : 1024)));
+}
+
+// Whether this kernel is the slower one all the same: one walk among many short ones bounds the launch where it is longer than three
+// times a CU's share of all walks, and a block of this kernel walks alone at 0.0203 us a key where the blocks of attention_mfma.h share
+// its keys out over four waves a head (us a walk, fitted to 250 mixes of 32 to 1,024 queries over 2,048 to 32,768 keys with prompts of 64 to
+// 1,024, which it leaves within 5 % of the faster kernel but for three of 9 to 13 %; 24 heads in 2 groups, 256 queries over 16,384 beside seven prompts of 300: 340 us here, 165 there; 64 in 8 groups, 32 queries over
+// 32,768 beside eight of 128: 662 and 578, but over 4,096 90 and 100).
+bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk) {
+  const int G = nq / nkv, sets = (G + 7) / 8, there = attention_prefill_splits(n_tiles, nq, nkv, 64, page_size, max_tile_ctx);
+  const float longest = float(max_tile_ctx) / float(splits);
+  if (longest <= 3.f * float(n_tiles) * float(nkv * sets) * float(mean_tile_walk) / 256.f) return false;
+  StagedShape shape = staged_shape(nq, nkv, 64, n_tiles);
+  staged_paired(n_tiles, nq, nkv, 64, there, max_tile_ctx, mean_tile_walk, &shape);
+  const float per_key = shape.hpb == 4 ? 0.0184f : shape.hpb == 2 ? 0.0088f : 0.0085f;
+  return 0.0203f * longest + (splits > 1 ? 15.f : 7.f) > per_key * float(max_tile_ctx) / float(there) + 24.f;
 }
 
 int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,

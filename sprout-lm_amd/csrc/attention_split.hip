@@ -316,7 +316,11 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
 
 }  // namespace
 
-// Heads of 64 and pages of a power of two of tokens, of whole pieces of 16 bytes.
+// Heads of 64 and pages of a power of two of tokens, of whole pieces of 16 bytes; any number of heads a group, also where three of a
+// block's waves then only carry stages (float32 instruction -> this, us, 2,048 tokens: 32 heads in 32 groups 422 -> 403, 16 in 16
+// 278 -> 237, 16 in 8 406 -> 133, 12 in 4 281 -> 86, 8 in 1 267 -> 59; 256 tokens: 36 to 39 -> 17 to 18 in all of them; 64 behind
+// 8,128: 1,080 -> 37 to 79; eight and 60 one-query sequences beside a prompt 169 -> 35 and 343 -> 158 under 14 heads in 2, 508 -> 480
+// under 16 in 16).
 bool attention_split_takes(int hd, int page_size) { return hd == 64 && page_size >= 4 && (page_size & (page_size - 1)) == 0; }
 
 // Blocks along the keys: as many as fill the chip's 512 places twice over, each with four stages at least.  (14 heads in 2
