@@ -16,8 +16,8 @@
 //
 // Every row is multiplied by a power of two that brings its largest number into [2^49, 2^50): numbers down to 2^-150 of it keep all
 // their bits, whatever the size of the row, and no sum overflows.  Powers of two are exact, and the sums are multiplied back
-// by them.  A row that is not finite passes as its bits (upper and lower sixteen in two parts): its results are taken number by
-// number behind the others, infinities and NaN as the float32 instruction gives them.
+// by them.  A row with an infinity passes as its bits (upper and lower sixteen in two parts): its results are taken number by
+// number behind the others, as the float32 instruction gives them.  A row with a NaN gives NaN, whatever it meets.
 //
 // The instruction drops the bits below its sum's last place, so that results end a little below the true ones, all to the same
 // side, which the averages that attention takes over many tokens' values do not lose as they lose the rest of the error: odd rows
@@ -38,6 +38,8 @@ constexpr int64_t kChunkBytes = int64_t(128) << 20;      // of split weights a l
 constexpr int kMaxK = 5120;                              // numbers of a row at a time: a chunk of rows then fills the chip
 constexpr int kStep = 32, kStepBytes = 3 * 128;          // numbers of K a step, bytes of a step of two rows
 constexpr int kNotFinite = 1 << 20;                      // a row's exponent, where the row holds its numbers' bits
+constexpr int kHasNan = 1 << 22;                         // ... and where one of them is NaN
+constexpr uint32_t kInfinityBits = 0x7f800000u;
 
 enum { kRowsAsTheyAre = 0, kRowsGated = 1, kRowsNormed = 2 };
 
@@ -59,6 +61,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, unsign
                                                          int rows, int K) {
   constexpr int LANES = 64 * WAVES, PIECES = 8;
   __shared__ float scratch[16];
+  __shared__ uint32_t tops[4];
   const int row = WAVES == 1 ? int(blockIdx.x) * 4 + (threadIdx.x >> 6) : int(blockIdx.x);
   const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
   if (row >= rows) return;
@@ -87,8 +90,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, unsign
     squares = WAVES == 1 ? wave_sum(squares) : block_sum(squares, scratch);
     factor = 1.0f / sqrtf(squares / float(src.length) + src.eps);
   }
-  float top = 0.f;
-  bool finite = true;
+  uint32_t top = 0;      // the bits of the largest magnitude: infinity's are above all numbers', NaN's above infinity's
 #pragma unroll
   for (int p = 0; p < PIECES; ++p) {
     const int i = lane + p * LANES;
@@ -101,25 +103,21 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, unsign
       kept[p] = make_float4(gated_value(g.x, u.x, src.act, src.limit), gated_value(g.y, u.y, src.act, src.limit),
                             gated_value(g.z, u.z, src.act, src.limit), gated_value(g.w, u.w, src.act, src.limit));
     }
-    const float f[4] = {fabsf(kept[p].x), fabsf(kept[p].y), fabsf(kept[p].z), fabsf(kept[p].w)};
+    const float f[4] = {kept[p].x, kept[p].y, kept[p].z, kept[p].w};
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      top = fmaxf(top, f[c]);
-      finite = finite && f[c] < INFINITY;      // (a maximum drops a NaN: it is looked for by itself)
-    }
+    for (int c = 0; c < 4; ++c) top = max(top, __float_as_uint(f[c]) & 0x7fffffffu);
   }
-  if (!finite) top = INFINITY;
-  top = wave_max(top);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) top = max(top, uint32_t(__shfl_xor(int(top), d, 64)));
   if (WAVES > 1) {
+    if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = top;
-    __syncthreads();
-    top = fmaxf(fmaxf(scratch[0], scratch[1]), fmaxf(scratch[2], scratch[3]));
+    top = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
   }
-  const bool bits = !(top < INFINITY);
+  const bool bits = top >= kInfinityBits;
   int e = 0;
-  if (top > 0.f && !bits) e = 50 - __builtin_amdgcn_frexp_expf(top);      // top = m 2^x, m in [0.5, 1): m 2^50
-  if (lane == 0) exponents[row] = bits ? kNotFinite : e;
+  if (top > 0 && !bits) e = 50 - __builtin_amdgcn_frexp_expf(__uint_as_float(top));      // top = m 2^x, m in [0.5, 1): m 2^50
+  if (lane == 0) exponents[row] = top > kInfinityBits ? kHasNan : bits ? kNotFinite : e;
   const uint32_t odd = bits ? 0u : uint32_t(row & 1) << 31;      // odd rows change their sign (see above)
   unsigned char* dst_row = out + row_at(row, K);
 #pragma unroll
@@ -286,9 +284,10 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
     const int t = t0 + at / BN, n = n0 + at % BN;
     if (t >= T || n >= N) continue;
     const int ex = x_exp[t], ew = w_exp[n];
-    if (ex != kNotFinite && ew != kNotFinite) continue;
-    float sum = 0.f;
-    for (int k = 0; k < K; ++k) sum = fmaf(number_of(x, t, k, K, ex), number_of(w, n, k, K, ew), sum);
+    if (max(ex, ew) < kNotFinite) continue;
+    const bool nan = max(ex, ew) == kHasNan;
+    float sum = nan ? __builtin_nanf("") : 0.f;
+    for (int k = 0; k < K && !nan; ++k) sum = fmaf(number_of(x, t, k, K, ex), number_of(w, n, k, K, ew), sum);
     out[size_t(t) * rope.row_stride + n] += sum;
   }
 }

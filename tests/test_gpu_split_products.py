@@ -158,6 +158,40 @@ def test_infinities_stay_infinities(mode):
     assert torch.equal(out[out.isinf()], plain[out.isinf()]) and torch.equal(out.isinf(), plain.isinf())
 
 
+@pytest.mark.parametrize("T,N,K", [(300, 190, 160), (512, 512, 4864), (260, 130, 8256)])
+def test_rows_with_a_nan_are_not_walked(T, N, K):
+    """NaN whatever they meet, infinities beside them too, on either side and in any piece of K; and in the time of finite rows, where
+    rows with an infinity are taken number by number (of all rows that would be 80 times the product itself)."""
+    from sprout_lm_amd import ops
+    x, w = rows(T, K, 41), rows(N, K, 42)
+    out, plain = torch.empty(T, N, device=DEV), torch.empty(T, N, device=DEV)
+
+    def best():
+        times = []
+        for _ in range(5):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            assert ops.gemm_f32_split(x, w, out, lambda n: kept)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    kept = scratch(ops.gemm_f32_split_bytes(T, N, K))
+    finite = best()
+    x[:, K - 1] = float("nan")
+    x[7] = float("nan")
+    x[9], w[3, 5] = 1.0, float("nan")
+    with_nan = best()
+    x[11, 0], w[4, 6] = float("inf"), float("-inf")
+    assert ops.gemm_f32_split(x, w, out, scratch)
+    ops.gemm(x, w, plain)
+    assert torch.equal(out.isnan(), plain.isnan()) and plain.isnan().sum() == (T - 1) * N + 1
+    good = ~plain.isnan()
+    assert torch.equal(out[good].isinf(), plain[good].isinf())
+    assert with_nan < 4 * finite + 0.2, (with_nan, finite)
+
+
 
 def test_the_step_takes_no_tensor_that_it_does_not_use():
     """A gated feed-forward of 2,048 tokens at 0.5B sizes: the norm and the gate are folded, so that neither the normed rows nor the
