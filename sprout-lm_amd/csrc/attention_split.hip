@@ -14,10 +14,13 @@
 //
 // What three parts cannot hold: infinities (inf - inf is NaN), numbers that round beyond bfloat16's largest, and the last bits of
 // numbers below 2^-110, whose third parts end in bfloat16's subnormal numbers.  The first two end as NaN in the row's sums; values of
-// the third kind end as results below kTinyResult.  A wave that finds one of them at the end of its walk walks again by itself, from
-// the pools on the float32 instruction and with every maximum exact, as attention_f32.hip's kernel does.  The look at the sums is 50
-// instructions a wave: no time beyond noise in any size measured (a walk of the block again, through LDS, put its check's three
-// barriers behind every block: 3 to 10 % of these launches).
+// the third kind end as results below kTinyResult; keys of the third kind matter beside queries above kLargeQuery only, and queries
+// of the third kind are looked for.  (What stays: a value above 2^100 under a weight below 2^-110.)  A wave that finds one of them at
+// the end of its walk walks again by itself, from the pools on the float32 instruction and with every maximum exact, as
+// attention_f32.hip's kernel does.  The look at the sums is 50 instructions a wave: no time beyond noise in any size measured (a walk
+// of the block again, through LDS, put its check's three barriers behind every block: 3 to 10 % of these launches); the look at the
+// queries 83.1 -> 86.8 us for 2,048 tokens under 14 heads (at the walk's start, where the first stage's loads wait for it, 87.5; at
+// its end from the queries' first parts 87.9).
 //
 // A block of four waves takes 32 queries of four heads of a key/value head, a wave a head; stages of 64 keys are loaded into
 // registers while the one before is used, split there and written to LDS as three planes each (48 KB), key rows and value
@@ -33,7 +36,7 @@ namespace sprout {
 namespace {
 
 constexpr int kSplitKeys = 64, kPlane = 64 * 128, kSplitTable = 2048;
-constexpr float kTinyResult = 0x1p-100f;
+constexpr float kTinyResult = 0x1p-100f, kLargeQuery = 0x1p60f, kTinyQuery = 0x1p-110f;
 
 __device__ __forceinline__ int split_swz(int row) { return (row ^ (row >> 3)) & 7; }
 
@@ -56,6 +59,11 @@ __device__ __forceinline__ float min3_of_magnitudes(float a, float b, float c) {
   float least;
   asm("v_min3_f32 %0, |%1|, |%2|, |%3|" : "=v"(least) : "v"(a), "v"(b), "v"(c));
   return least;
+}
+__device__ __forceinline__ float max3_of_magnitudes(float a, float b, float c) {
+  float most;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(most) : "v"(a), "v"(b), "v"(c));
+  return most;
 }
 __device__ __forceinline__ float max_over_row(float x) {      // the other half of a row's keys lies in lane ^ 32
   const unsigned u = __float_as_uint(x);
@@ -134,13 +142,17 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
   const uint32_t odd = uint32_t(li & 1) << 31;      // odd rows' sums are held with the other sign (see above)
   uint4 qp[4][3];
   floatx16 o[2];
-  float m = kNoKeyYet, l = 0.f;
+  float m = kNoKeyYet, l = 0.f, largest_q = 0.f, least_q = INFINITY;
   {
     const float* row = q + size_t(qs + q_off + min(li, nvalid - 1)) * q_stride + head * HD + 8 * lk;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const float4 a = *reinterpret_cast<const float4*>(row + 16 * ks), b = *reinterpret_cast<const float4*>(row + 16 * ks + 4);
       three_parts8({a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, qp[ks]);
+      largest_q = max3_of_magnitudes(max3_of_magnitudes(largest_q, a.x, a.y), a.z, a.w);
+      largest_q = max3_of_magnitudes(max3_of_magnitudes(largest_q, b.x, b.y), b.z, b.w);
+      least_q = min3_of_magnitudes(min3_of_magnitudes(least_q, a.x, a.y), a.z, a.w);
+      least_q = min3_of_magnitudes(min3_of_magnitudes(least_q, b.x, b.y), b.z, b.w);
     }
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
@@ -219,7 +231,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
   }
   if (!live) return;
   l += __shfl_xor(l, 32, 64);
-  // sums that are not finite, or (zeros aside) results below kTinyResult
+  // sums that are not finite, queries at the ends of the range, or (zeros aside) results below kTinyResult
   float total = l, least = INFINITY;
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
@@ -229,7 +241,13 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
       total += fabsf(o[dt][r + 1]);
       least = min3_of_magnitudes(least, o[dt][r], o[dt][r + 1]);
     }
-  bool beyond = !(total < INFINITY);
+  bool beyond = !(total < INFINITY) || largest_q > kLargeQuery;
+  if (least_q < kTinyQuery) {      // zeros, most often
+    const float* row = q + size_t(qs + q_off + min(li, nvalid - 1)) * q_stride + head * HD + 8 * lk;
+#pragma unroll 1
+    for (int d = 0; d < HD; d += 16)
+      for (int j = 0; j < 8; ++j) beyond |= (row[d + j] != 0.f) & (fabsf(row[d + j]) < kTinyQuery);
+  }
   if (least < kTinyResult * l) {
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
