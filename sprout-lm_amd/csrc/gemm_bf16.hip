@@ -5,7 +5,7 @@
 // instruction), the few activations wait in LDS, and the product runs on 16x16x32 MFMA with the
 // weights as the A operand: D[n, t].  Small matrices are cut along K over several blocks, whose
 // partial sums are added into the float32 output with hardware atomics (accumulate mode only).
-#include "gemm_epilogue.h"
+#include "gemm_quad.h"
 #include "sprout_hip.h"
 
 namespace sprout {
@@ -157,7 +157,9 @@ int gemm_bf16_tiled(hipStream_t s, const void* a, const void* w, int bias_dtype,
                     int T, int N, int K);
 int gemm_decode_plain(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, int mode, void* out,
                       int T, int N, int K);
-bool gemm_pipe_takes(int T, int N, int K);
+int gemm_bf16_quad(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, int mode, void* out, int T, int N, int K);
+int gemm_bf16_quad_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
+                        const float* row_gate, long long row_gate_stride);
 int gemm_bf16_pipe(hipStream_t s, const void* a, const void* w, int bias_dtype, const void* bias, int mode, void* out,
                    int T, int N, int K);
 int gemm_bf16_pipe_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
@@ -186,6 +188,8 @@ int gemm_bf16(hipStream_t s, const void* a, const void* w, int bias_dtype, const
     if (bias && bias_dtype == kBF16) return skinny_shape<bf16_t>(s, a, w, bias, mode, out, T, N, K);
     return skinny_shape<float>(s, a, w, bias, mode, out, T, N, K);
   }
+  if (gemm_quad_takes(mode == kAccumulate ? kQuadAccumulate : kQuadStore, T, N, K) && quad_aligned(a, w, out))
+    return gemm_bf16_quad(s, a, w, bias_dtype, bias, mode, out, T, N, K);
   if (gemm_pipe_takes(T, N, K)) return gemm_bf16_pipe(s, a, w, bias_dtype, bias, mode, out, T, N, K);
   return gemm_bf16_tiled(s, a, w, bias_dtype, bias, mode, out, T, N, K);
 }
@@ -364,10 +368,12 @@ static int tiled_shape(hipStream_t s, const void* x, const void* w, const void* 
   return launch_tiled<1, 1, TB>(s, x, w, bias, mode, out, T, N, K, splits_for(blocks(64, 64)));
 }
 
-// out[T, I] = silu(x . w[:I]^T) * (x . w[I:]^T): the pipelined kernel where it takes the shape, else (T > 64)
+// out[T, I] = silu(x . w[:I]^T) * (x . w[I:]^T): the four-wave or the pipelined kernel where it takes the shape, else (T > 64)
 // this file's kernel with 128-token tiles, 64 gate + 64 up rows per block.
 int gemm_bf16_tiled_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
                          const float* row_gate, long long row_gate_stride) {
+  if (gemm_quad_takes(kQuadGated, T, 2 * I, K) && quad_aligned(x, w, out))
+    return gemm_bf16_quad_silu(s, x, w, out, T, I, K, act, limit, row_gate, row_gate_stride);
   if (gemm_pipe_takes(T, 2 * I, K)) return gemm_bf16_pipe_silu(s, x, w, out, T, I, K, act, limit, row_gate, row_gate_stride);
   SP_REQUIRE(act == kActSilu && !row_gate, "sp_gate_up_silu: the tiles for K=%d have the SiLU epilogue alone", K);
   dim3 grid((I + 63) / 64, (T + 127) / 128, 1);

@@ -24,8 +24,7 @@
 // A step of decoded tokens spends a few microseconds in each of these kernels, and a wave's every vector
 // instruction is four cycles of them: with K in whole steps of 64 (K64) the loads carry no bounds of their
 // own, whole steps are switched by scalar branches, and addresses are one base per pass plus constants.
-#include "mfma.h"
-#include "sprout_hip.h"
+#include "gemm_quad.h"
 
 namespace sprout {
 
@@ -610,7 +609,9 @@ extern "C" int sp_gemm_decode(void* stream, const void* x, const float* residual
 namespace sprout {
 int gemm_bf16_tiled_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
                          const float* row_gate, long long row_gate_stride);
-bool gemm_pipe_takes(int T, int N, int K);
+int gemm_bf16_quad_rope(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, void* q_out,
+                        const int32_t* positions, const float* inv_freq, const int32_t* slot_mapping, void* k_pool,
+                        void* v_pool, int T, int K, int nq, int nkv, int hd, int page_size, const float* table);
 bool gemm_pipe_rope_takes(int T, int N, int K, int hd);
 int gemm_bf16_pipe_rope(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, void* q_out,
                         const int32_t* positions, const float* inv_freq, const int32_t* slot_mapping, void* k_pool,
@@ -621,7 +622,7 @@ extern "C" int sp_fused_supported(int kind, int T, int N, int K, int hd, int rot
   if (kind == kEpiSilu ? (variant < 0 || variant >= kGateActs) : variant != 0) return 0;   // the one pairing (halves); the gate activations of common.h
   // the tiled kernel's gated epilogue (its pipelined form has every activation, the older tiles SiLU alone)
   if (kind == kEpiSilu && T > 64) return !norm && K % 8 == 0 && N % 2 == 0 && (variant == 0 || gemm_pipe_takes(T, N, K));
-  if (kind == kEpiRope && T > 64) return !norm && rotary_dim == hd && gemm_pipe_rope_takes(T, N, K, hd);   // and its rotating one
+  if (kind == kEpiRope && T > 64) return !norm && rotary_dim == hd && gemm_quad_takes(kQuadRotating, T, N, K, hd);   // and its rotating one
   if (!fused_shape_ok(T, K, norm != 0)) return 0;
   if (kind == kEpiRope) return hd % 16 == 0 && (rotary_dim == hd || rotary_dim == 0) && N % hd == 0;
   if (kind == kEpiSilu) return N % 32 == 0;
@@ -686,6 +687,8 @@ extern "C" int sp_gemm_joined_takes(int T, int N, int K) {
 }
 
 namespace sprout {
+int gemm_bf16_quad_store(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, bool f32, void* out, int T, int N, int K,
+                         const RopeArgs& epilogue);
 int gemm_bf16_pipe_joined(hipStream_t s, const void* a, const void* w, const float* bias, int act, void* out, long long out_stride,
                           int split, void* second, long long second_stride, int T, int N, int K);
 }
@@ -701,6 +704,15 @@ extern "C" int sp_gemm_joined(void* stream, const void* x, const void* w, const 
                  ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(second)) & 7) == 0,
              "sp_gemm_joined: null operand, or one that does not start at a multiple of 16 (8: results) bytes");
   hipStream_t s = (hipStream_t)stream;
+  if (T > 64 && gemm_quad_takes(kQuadStore, T, N, K)) {      // results in eights or, at the seam of the two products, in fours
+    RopeArgs epilogue = {};
+    epilogue.act = act;
+    epilogue.second = (uint16_t*)second;
+    epilogue.split = split;
+    epilogue.out_stride = out_stride;
+    epilogue.second_stride = second_stride;
+    return gemm_bf16_quad_store(s, x, w, kF32, bias, false, out, T, N, K, epilogue);
+  }
   if (T > 64) return gemm_bf16_pipe_joined(s, x, w, bias, act, out, out_stride, split, second, second_stride, T, N, K);
   FusedArgs a = {};
   a.x = (const uint16_t*)x; a.w = (const uint16_t*)w; a.bias = bias; a.out = out; a.act = act;
@@ -723,7 +735,11 @@ extern "C" int sp_qkv_rope_cache(void* stream, const void* x, const float* resid
              "sp_qkv_rope_cache: shape T=%d K=%d hd=%d rotary=%d is not taken", T, K, hd, rotary_dim);
   SP_REQUIRE((x || residual) && w && q_out && positions && inv_freq && slot_mapping && k_pool && v_pool,
              "sp_qkv_rope_cache: null operand");
-  if (T > 64)   // many tokens: the pipelined tiled product with the rotation as its epilogue
+  // many tokens: the tiled product with the rotation as its epilogue
+  if (T > 64 && quad_aligned(x, w, q_out) && quad_aligned(k_pool, v_pool, nullptr))
+    return gemm_bf16_quad_rope((hipStream_t)stream, x, w, bias_dtype, bias, q_out, positions, inv_freq, slot_mapping, k_pool,
+                               v_pool, T, K, nq, nkv, hd, page_size, cos_sin);
+  if (T > 64)
     return gemm_bf16_pipe_rope((hipStream_t)stream, x, w, bias_dtype, bias, q_out, positions, inv_freq, slot_mapping, k_pool,
                                v_pool, T, K, nq, nkv, hd, page_size, cos_sin);
   FusedArgs a = {};

@@ -1,0 +1,85 @@
+// The four-wave tiled product that adds to its output, and the choice between the block shapes.  The kernel is in gemm_quad.h;
+// the stores and the gated and rotating epilogues are instantiated in gemm_quad_store.hip and gemm_quad_epilogues.hip, so that
+// the parts compile side by side.
+#include "gemm_quad.h"
+
+namespace sprout {
+
+bool gemm_quad_takes(int kind, int T, int N, int K, int hd) {
+  if (T <= 64 || !gemm_pipe_takes(T, N, K)) return false;
+  if (kind == kQuadGated) return N % 16 == 0;
+  if (kind == kQuadRotating) return hd % 64 == 0 && N % hd == 0;
+  return N % 8 == 0;
+}
+
+// What was measured of the block shapes, fitted over 56 products (weights of 896 to 37,888 rows and K of 896 to 18,944, 80 to 2,048
+// tokens) with every shape and split: microseconds a step of 64 along K on a full chip, and, where two blocks share a CU, of one that
+// has a CU to itself.
+struct QuadShape { int wm, wn, buffers, per_cu; };
+static const QuadShape kQuadShapes[] = {
+#define SPROUT_QUAD_ROW(I, WM, WN, NA) {WM, WN, NA, quad_shares_cu<WM, WN, NA> ? 2 : 1},
+    SPROUT_QUAD_SHAPES(SPROUT_QUAD_ROW)
+#undef SPROUT_QUAD_ROW
+};
+static const float kStepUs[] = {0.36f, 0.77f, 0.35f, 0.85f, 0.48f, 0.68f, 0.80f, 0.66f, 0.86f, 0.77f, 0.81f, 0.96f, 0.93f, 1.06f, 1.06f, 1.19f, 1.33f};
+static const float kAloneUs[] = {0.24f, 0.45f, 0.35f, 0.50f, 0.48f, 0.68f, 0.80f, 0.66f, 0.86f, 0.77f, 0.81f, 0.96f, 0.93f, 1.06f, 1.06f, 1.19f, 1.33f};
+
+// The estimate: rounds of blocks on the XCD that holds the most (blocks are numbered as pipe_tiles says), a block being its steps
+// (longer by 7 % each beyond 20 where two blocks share a CU) and its two ends; a last round that does not fill the chip runs
+// somewhat faster, fewer blocks share the caches.  Memory: the weights once at 5.4 TB/s, the tokens once an XCD at 9 TB/s together;
+// it adds to the blocks' time where both are alike (fourth powers).  A split's float atomics cost 1.9 us a million, the sums
+// read and written without a split 1.4.  Over the 56 products the choice takes 2 % longer than the best of all shapes and splits
+// (mean; 25 % at worst).
+void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
+  const int steps = K / 64;
+  const float memory = float(N) * float(K) * 2.f / 5.4e6f + 16.f * float(T) * float(K) / 9e6f, memory2 = memory * memory;
+  float best = 1e30f;
+  *shape = 3;
+  *splits = 1;
+  for (int c = 0; c < int(sizeof(kQuadShapes) / sizeof(kQuadShapes[0])); ++c) {
+    const QuadShape& p = kQuadShapes[c];
+    if (kind == kQuadRotating && p.wn != 2 && p.wn % 4 != 0) continue;     // a lane holds both of a pair
+    const int bm = 32 * p.wm, bn = 32 * p.wn, slots = 32 * p.per_cu;
+    const PipeTiles tiles = pipe_tiles((T + bm - 1) / bm, (N + bn - 1) / bn);
+    for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (sp > 1 && (kind != kQuadAccumulate || steps / sp < 4)) break;
+      const int k_steps = (steps + sp - 1) / sp;
+      if ((steps + k_steps - 1) / k_steps != sp) continue;
+      const int blocks = (tiles.full * tiles.tiles_t + tiles.run) * sp, full = blocks / slots, rest = blocks % slots;
+      const float ends = 0.14f * float(p.wm * p.wn) + 0.95f;
+      const float block = k_steps * kStepUs[c] * (p.per_cu == 2 && k_steps > 20 ? 1.07f : 1.f) + ends, alone = k_steps * kAloneUs[c] + ends;
+      float t = full * block;
+      if (rest > 32) t += fmaxf(alone, block * (0.81f + 0.19f * float(rest - 32) / 32.f));
+      else if (rest) t += alone * (0.79f + 0.21f * float(rest) / 32.f);
+      t = sqrtf(sqrtf(t * t * t * t + memory2 * memory2));
+      if (sp > 1) t += 1.9e-6f * float(T) * float(N) * sp;
+      else if (kind == kQuadAccumulate) t += 1.4e-6f * float(T) * float(N);
+      if (t < best) { best = t; *shape = c; *splits = sp; }
+    }
+  }
+}
+
+int gemm_bf16_quad_store(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, bool f32, void* out, int T, int N, int K,
+                         const RopeArgs& epilogue);
+
+int gemm_bf16_quad(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, int mode, void* out, int T, int N, int K) {
+  if (mode == kAccumulate) return quad_run<kAccumulate>(s, kQuadAccumulate, x, w, bias, bias_dtype, out, T, N, K);
+  return gemm_bf16_quad_store(s, x, w, bias_dtype, bias, mode == kStoreF32, out, T, N, K, RopeArgs{});
+}
+
+}  // namespace sprout
+
+// What the four-wave product would do with T x N x K: kind 0 store, 1 accumulate, 2 gated (N = 2 I rows of w), 3 rotating (head size
+// hd).  plan = {block rows, block columns, splits of K, buffers of x}.  Returns 1 where it does not take the product, else 0.  Runs
+// nothing: for tests and tools.
+extern "C" int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan) {
+  using namespace sprout;
+  if (T < 1 || N < 1 || K < 1 || kind < 0 || kind > 3 || !plan || (kind == kQuadRotating && hd < 1) || !gemm_quad_takes(kind, T, N, K, hd)) return 1;
+  int shape, splits;
+  quad_choice(kind, T, N, K, &shape, &splits);
+  plan[0] = 32 * kQuadShapes[shape].wm;
+  plan[1] = 32 * kQuadShapes[shape].wn;
+  plan[2] = splits;
+  plan[3] = kQuadShapes[shape].buffers;
+  return 0;
+}

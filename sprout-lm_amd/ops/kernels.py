@@ -869,6 +869,16 @@ def pipe_plan(kind: int, T: int, N: int, K: int, hd: int = 0):
     return tuple(plan)
 
 
+def quad_plan(kind: int, T: int, N: int, K: int, hd: int = 0):
+    """(block rows, block columns, splits of K, buffers of the activations) that the product on four waves a block would
+    take for T x N x K, or None where `pipe_plan`'s kernel or another has the product.  Runs nothing and needs no GPU."""
+    import ctypes
+    plan = (ctypes.c_int * 4)()
+    if library().sp_quad_plan(kind, T, N, K, hd, plan):
+        return None
+    return tuple(plan)
+
+
 def pipe_tiles(tiles_t: int, tiles_n: int) -> list:
     """For every block of the tiled product's launch over tiles_t token tiles and tiles_n weight tiles, in the order
     of the blocks (block b runs on XCD b % 8): (token tile, weight tile), or None for a block with nothing to do.

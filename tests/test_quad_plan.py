@@ -1,0 +1,52 @@
+"""The choice of block shape of the product on four waves a block, asked of the library without running a kernel (no GPU)."""
+import itertools
+
+import pytest
+
+from sprout_lm_amd import ops
+from tests.test_gpu_quad_products import ROTATING_SIZES, SIZES
+
+SHAPES = {(64, 64, 4), (96, 128, 2), (128, 64, 4), (128, 128, 2), (128, 128, 4), (128, 192, 2), (160, 192, 2), (192, 128, 2), (192, 192, 2),
+          (256, 128, 3), (128, 256, 2), (160, 256, 2), (320, 128, 2), (192, 256, 2), (256, 192, 2), (288, 192, 2), (256, 256, 2)}
+KINDS = [ops.PLAN_STORE, ops.PLAN_ACCUMULATE, ops.PLAN_GATED]
+
+
+@pytest.fixture(autouse=True, scope="module")
+def built_library():
+    try:
+        ops.library()
+    except Exception as e:      # no compiler here: nothing to ask
+        pytest.skip(f"the kernel library cannot be built or loaded here: {e}")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_plan_invariants(kind):
+    for T, N, K in itertools.product([1, 64, 65, 100, 264, 777, 2048, 8192], [8, 16, 130, 900, 1152, 37888, 151936], [64, 70, 192, 3584, 27648]):
+        plan = ops.quad_plan(kind, T, N, K)
+        if T <= 64 or K % 64 or N % (16 if kind == ops.PLAN_GATED else 8) or N * K * 2 >= 1 << 32:
+            assert plan is None, (T, N, K)          # other kernels' products
+            continue
+        rows, cols, splits, buffers = plan
+        assert (rows, cols, buffers) in SHAPES, (T, N, K, plan)
+        assert buffers * rows * 128 + (buffers + 1) * cols * 128 <= 160 * 1024
+        # only float atomics join partial sums; every split has a step
+        assert splits == 1 or (kind == ops.PLAN_ACCUMULATE and K // 64 // splits >= 4), (T, N, K, plan)
+
+
+def test_rotation_takes_heads_of_whole_sixty_fours():
+    for T, (nq, nkv, hd, K) in itertools.product([64, 65, 264, 2048], [(14, 2, 64, 896), (28, 4, 128, 3584), (3, 1, 48, 896), (2, 2, 192, 64)]):
+        plan = ops.quad_plan(ops.PLAN_ROTATING, T, (nq + 2 * nkv) * hd, K, hd)
+        assert (plan is None) == (T <= 64 or hd % 64 != 0), (T, nq, nkv, hd, K, plan)
+        assert plan is None or (plan[:2] + plan[3:] in SHAPES and plan[1] != 192 and plan[2] == 1)
+
+
+def test_kernel_tests_reach_every_block_shape():
+    for kind in KINDS:
+        seen = {}
+        for T, N, K in SIZES[kind]:
+            plan = ops.quad_plan(kind, T, N, K)
+            seen.setdefault((plan[0], plan[1], plan[3]), set()).add(plan[2] > 1)
+        assert set(seen) == SHAPES, SHAPES - set(seen)
+        assert kind != ops.PLAN_ACCUMULATE or sum(True in s for s in seen.values()) >= 8
+    rotating = {p[:2] + p[3:] for p in (ops.quad_plan(ops.PLAN_ROTATING, T, (nq + 2 * nkv) * hd, K, hd) for T, nq, nkv, hd, K in ROTATING_SIZES)}
+    assert rotating == {s for s in SHAPES if s[1] != 192}
