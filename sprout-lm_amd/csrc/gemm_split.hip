@@ -4,12 +4,13 @@
 // bfloat16 numbers to its last bit (three_parts of mfma.h), and a product is taken as the six products of parts that reach 2^-24 of
 // it: a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1; what is left out is 2^-26 of it at most, less than the float32 product's own rounding.
 // a1 b1 is summed in one float32 accumulator and the other five, 2^-8 of its size, in a second: a result is rounded once for every
-// sixteen numbers of K and once where the two meet, where the float32 instruction rounds once for every number that is not zero
+// thirty-two numbers of K and once where the two meet, where the float32 instruction rounds once for every number that is not zero
 // and at most once for every two.  Relative error of the result against 64 bits, float32 instruction -> this: normal operands,
 // K = 896 5.4e-7 -> 1.7e-7, 4,864 1.25e-6 -> 4.3e-7, 27,648 3.0e-6 -> 4.3e-7; weights with 1, 2, 8 and 64 numbers a row that are not
 // zero 2.5e-8 -> 2.6e-8, 3.1e-8 -> 2.6e-8, 5.4e-8 -> 2.9e-8, 1.4e-7 -> 5.7e-8; one number 2^100 times the others of its row against a
-// weight of zero 5.4e-7 -> 1.7e-7.  Time, whole call (2,048 tokens): 9,728 rows of 896 303 -> 235 us (of it 21 the splits, at 4.6
-// TB/s; the product 203, at 1.05 PFLOP/s of bfloat16 products), 896 rows of 4,864 182 -> 154, 37,888 rows of 3,584 4,268 -> 2,958.
+// weight of zero 5.4e-7 -> 1.7e-7.  Time, whole call (2,048 tokens): 9,728 rows of 896 320 -> 202 us (of it 21 the splits, at 4.6
+// TB/s; the product 170, at 1.26 PFLOP/s of bfloat16 products, where 32x32x16 on blocks with one barrier between whole steps took
+// 202), 896 rows of 4,864 163 -> 124, 37,888 rows of 3,584 4,095 -> 2,513.
 //
 // (Pairs of float16 numbers took three products and half the time, but held 23 bits of 24, and numbers below 2^-17 of
 // their row's largest less and less of them: one number that stood 2^24 out of its row and met no weight left an error of 2e-5.)
@@ -18,7 +19,7 @@
 // their bits, whatever the size of the row, and no sum overflows.  Powers of two are exact, and the sums are multiplied back
 // by them.  A row with an infinity passes as its bits (upper and lower sixteen in two parts): its results are taken number by
 // number behind the others, as the float32 instruction gives them; a row with a NaN gives NaN, whatever it meets (896
-// rows of 4,864, 2,048 tokens, whole call: 159 us; one token with a NaN 1,390 -> 166, 32 of them 2,560 -> 169; with an infinity 1,360).
+// rows of 4,864, 2,048 tokens, whole call: 124 us; with a token that has a NaN 122, with an infinity 567).
 //
 // The instruction drops the bits below its sum's last place, so that results end a little below the true ones, all to the same
 // side, which the averages that attention takes over many tokens' values do not lose as they lose the rest of the error: odd rows
@@ -149,165 +150,315 @@ int launch_split(hipStream_t s, const SplitSource& src, unsigned char* out, int3
   return check_launch("sp_gemm_f32_split (rows)");
 }
 
-// Number k of a split row, as it was.
-__device__ float number_of(const unsigned char* __restrict__ parts, int row, int k, int K, int exponent) {
-  const uint16_t* p = reinterpret_cast<const uint16_t*>(parts + row_at(row, K) + size_t(k / kStep) * kStepBytes) + k % kStep;
-  const uint32_t p1 = p[0], p2 = p[64], p3 = p[128];
-  if (exponent == kNotFinite) return __uint_as_float(p1 << 16 | p2);
-  const float x = __uint_as_float(p1 << 16) + (__uint_as_float(p2 << 16) + __uint_as_float(p3 << 16));
-  return __builtin_amdgcn_ldexpf(row & 1 ? -x : x, -exponent);
+// Numbers k .. k + 7 of a split row, as they were (k in eights).
+__device__ __forceinline__ void numbers_of(const unsigned char* __restrict__ parts, int row, int k, int K, int exponent, float (&v)[8]) {
+  const unsigned char* p = parts + row_at(row, K) + size_t(k / kStep) * kStepBytes + 2 * (k % kStep);
+  const uint4 q[3] = {ldg128(p), ldg128(p + 128), ldg128(p + 256)};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    uint32_t part[3];
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      const uint32_t two = e < 2 ? q[h].x : e < 4 ? q[h].y : e < 6 ? q[h].z : q[h].w;
+      part[h] = e & 1 ? two >> 16 : two & 0xffffu;
+    }
+    const float x = __uint_as_float(part[0] << 16) + (__uint_as_float(part[1] << 16) + __uint_as_float(part[2] << 16));
+    v[e] = exponent == kNotFinite ? __uint_as_float(part[0] << 16 | part[1]) : __builtin_amdgcn_ldexpf(row & 1 ? -x : x, -exponent);
+  }
 }
 
-// The pipelined kernel of gemm_pipe.h (its ring, its waits, its numbering of tiles) with three parts an operand: a stage is 32 numbers
-// of K, BM + BN rows of three times 64 bytes, each part a plane of lines of two rows.  Piece c of 16 bytes of the row r & 1 of line
-// l = r / 2 lies at position (4 (r & 1) + c) ^ s(l) of it, s(l) = (l ^ l / 4) & 3: the 16 rows that a quarter of a wave reads
-// together lie on all banks, whether the LDS has 32 or 64, and s is the same 32 rows on.  A fetch of 1 KB is eight lines of a
-// plane, which are lines of memory.
-// What bounds it: a wave issues 12 WM WN matrix instructions a stage for 6 (WM + WN) KB from LDS; a block of 256 x 128 reads 72 KB
-// from L2 for 3,072 cycles of matrix instructions a SIMD, as the bfloat16 product of 384 x 256 reads 80.
-template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, int MODE, typename TB>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2 : 1)) void split_product_kernel(
+template <int WM, int WN, int STAGES> constexpr int split_lds = STAGES * 32 * (WM + WN) * 192;
+template <int WM, int WN, int STAGES> constexpr bool split_shares_cu = split_lds<WM, WN, STAGES> <= 80 * 1024;
+
+// Four waves in two rows of two, each WM x WN tiles of 16 x 16 (see gemm_quad.h: 16x16x32, the instruction that takes the least power
+// a product, what else a wave has to do dealt out between its products).  A stage is 32 numbers of K, BM + BN rows of three times 64
+// bytes, each part a plane of lines of two rows.  Piece c of 16 bytes of the row r & 1 of line l = r / 2 lies at position
+// (4 (r & 1) + c) ^ s(l) of it, s(l) = (l ^ l / 4) & 3: the 16 rows that a quarter of a wave reads together lie on all banks, whether
+// the LDS has 32 or 64.  A fetch of 1 KB is eight lines of a plane, which are lines of memory.
+//
+// A wave walks its 16-row tiles i of x: 6 WN products each, with w's parts of the step in registers and x's read AHEAD tiles before
+// their use; at tile WM - AHEAD the reads pass to the next step, so there the wave has read all of this one: the barrier that says that
+// the next step has landed also frees this step's stage, and the loads into it follow one by one between the products.
+// What bounds it: matrix instructions, 6 WM WN of 16 cycles a stage and SIMD, at the clock that their power leaves; a block of
+// 256 x 128 reads 72 KB from L2 for 3,072 cycles.
+template <int WM, int WN, int STAGES, int MODE>
+__global__ __launch_bounds__(256, (split_shares_cu<WM, WN, STAGES> ? 2 : 1)) void split_product_kernel(
     const unsigned char* __restrict__ x, const unsigned char* __restrict__ w, const int32_t* __restrict__ x_exp,
-    const int32_t* __restrict__ w_exp, const TB* __restrict__ bias, float* out, int T, int N, int K, RopeArgs rope) {
-  constexpr int NW = WAVES_M * WAVES_N, BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N;
+    const int32_t* __restrict__ w_exp, const void* __restrict__ bias, int bias_dtype, float* out, int T, int N, int K, long long out_stride) {
+  constexpr int BM = 32 * WM, BN = 32 * WN;
   constexpr int STAGE = (BM + BN) * 192, XBYTES = BM * 192;
-  constexpr int LX = 3 * BM / (16 * NW), LW = 3 * BN / (16 * NW);      // load instructions per wave, stage and operand
-  static_assert(3 * BM % (16 * NW) == 0 && 3 * BN % (16 * NW) == 0, "every wave fills whole groups of 8 lines");
-  static_assert((STAGES - 2) * (LX + LW) <= 63, "vmcnt holds six bits");
+  constexpr int LX = 3 * BM / 64, LW = 3 * BN / 64, L = LX + LW;       // load instructions per wave, stage and operand
+  static_assert(3 * BM % 64 == 0 && 3 * BN % 64 == 0, "every wave fills whole groups of 8 lines");
+  static_assert((STAGES - 2) * L <= 63, "vmcnt holds six bits");
+  static_assert(split_lds<WM, WN, STAGES> <= 160 * 1024, "a CU's LDS");
+  constexpr bool AGPR = !split_shares_cu<WM, WN, STAGES>;
+  constexpr int SETS = WM % 4 == 0 ? 4 : WM % 3 == 0 ? 3 : 2, AHEAD = SETS == 2 ? 1 : 2;
+  static_assert(WM % SETS == 0, "a tile's registers are the same in every step");
   extern __shared__ __attribute__((aligned(1024))) unsigned char pipe_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int li = lane & 31, lk = lane >> 5;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int li = lane & 15, lq = lane >> 4;
   int tile_n, tile_t;
   if (!pipe_tile_of(pipe_tiles((T + BM - 1) / BM, (N + BN - 1) / BN), blockIdx.x, &tile_t, &tile_n)) return;
   const int t0 = tile_t * BM, n0 = tile_n * BN;
   const int steps = K / kStep;
   typedef __attribute__((address_space(3))) unsigned char* lds_address_t;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_address_t)pipe_lds;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_address_t)pipe_lds + wave * 1024;
   const uint32_t pitch = uint32_t(steps) * kStepBytes;      // of a line of two rows
-  const unsigned char *xbase = x + size_t(t0 / 2) * pitch, *wbase = w + size_t(n0 / 2) * pitch;
-  uint32_t xoff[LX], woff[LW];
-  // fetch u = NW j + wave of an operand: eight lines of part u / (rows / 16)
+  const unsigned char *xs = x + size_t(t0 / 2) * pitch, *ws = w + size_t(n0 / 2) * pitch;      // the next step to be asked for
+  uint32_t off[L];
+  // fetch u = 4 j + wave of an operand: eight lines of part u / (rows / 16)
   auto offset_of = [&](int u, int rows, int last_line) {
     const int part = u / (rows / 16), line = (u % (rows / 16)) * 8 + (lane >> 3), piece = (lane & 7) ^ ((line ^ (line >> 2)) & 3);
     return uint32_t(min(line, last_line)) * pitch + part * 128 + piece * 16;
   };
 #pragma unroll
-  for (int j = 0; j < LX; ++j) xoff[j] = offset_of(NW * j + wave, BM, (T - 1 - t0) / 2);
+  for (int j = 0; j < LX; ++j) off[j] = offset_of(4 * j + wave, BM, (T - 1 - t0) / 2);
 #pragma unroll
-  for (int j = 0; j < LW; ++j) woff[j] = offset_of(NW * j + wave, BN, (N - 1 - n0) / 2);
-  auto fetch = [&](int buf, int step) {
-    const unsigned char* xs = xbase + size_t(step) * kStepBytes;
-    const unsigned char* ws = wbase + size_t(step) * kStepBytes;
-    const uint32_t dst = lds0 + buf * STAGE + wave * 1024;
-#pragma unroll
-    for (int j = 0; j < LX; ++j) load_to_lds(xs, xoff[j], dst + NW * j * 1024);
-#pragma unroll
-    for (int j = 0; j < LW; ++j) load_to_lds(ws, woff[j], dst + XBYTES + NW * j * 1024);
+  for (int j = 0; j < LW; ++j) off[LX + j] = offset_of(4 * j + wave, BN, (N - 1 - n0) / 2);
+  auto load = [&](uint32_t stage, int j) __attribute__((always_inline)) {
+    if (j < LX) load_to_lds(xs, off[j], lds0 + stage + 4096 * j);
+    else load_to_lds(ws, off[j], lds0 + stage + XBYTES + 4096 * (j - LX));
   };
-  // row 32 i + li of the wave's, pieces 2 ks + lk of a part
-  const uint32_t position = (li >> 1) * 128 + (((((li & 1) << 2) | lk) ^ (((li >> 1) ^ (li >> 3)) & 3)) << 4);
-  const uint32_t xrow = wm * WM * 2048 + position, wrow = XBYTES + wn * WN * 2048 + position;
 
-  floatx16 acc[WM][WN], low[WM][WN];      // sums of the first parts' products, and of the others
+  floatx4 acc[WM][WN], low[WM][WN];      // sums of the first parts' products, and of the others
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
-    for (int j = 0; j < WN; ++j)
+    for (int j = 0; j < WN; ++j) acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (AGPR) {
+    // the compiler does not know the products below for matrix instructions: the zeros are written well ahead of them
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.f;
-
-  auto multiply = [&](int buf) {
-    const unsigned char* stage = pipe_lds + buf * STAGE;
+    for (int i = 0; i < WM; ++i)
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 b[WN][3];
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-#pragma unroll
-        for (int h = 0; h < 3; ++h)
-          b[j][h] = as_bf16x8(*reinterpret_cast<const uint4*>(stage + (wrow ^ (ks * 32)) + h * (BN * 64) + j * 2048));
-#pragma unroll
-      for (int i = 0; i < WM; ++i) {
-        bf16x8 a[3];
-#pragma unroll
-        for (int h = 0; h < 3; ++h)
-          a[h] = as_bf16x8(*reinterpret_cast<const uint4*>(stage + (xrow ^ (ks * 32)) + h * (BM * 64) + i * 2048));
-#pragma unroll
-        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][0], a[2], low[i][j]);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = mfma32(b[j][0], a[0], acc[i][j]);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][2], a[0], low[i][j]);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][1], a[1], low[i][j]);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][0], a[1], low[i][j]);
-#pragma unroll
-        for (int j = 0; j < WN; ++j) low[i][j] = mfma32(b[j][1], a[0], low[i][j]);
+      for (int j = 0; j < WN; ++j) {
+        asm volatile("" : "+a"(acc[i][j]));
+        asm volatile("" : "+a"(low[i][j]));
       }
+    asm volatile("s_nop 7" : : : "memory");
+  }
+
+#pragma unroll
+  for (int p = 0; p < STAGES; ++p)
+    if (p < steps) {
+#pragma unroll
+      for (int j = 0; j < L; ++j) load(p * STAGE, j);
+      xs += kStepBytes;
+      ws += kStepBytes;
+    }
+  if (steps >= STAGES) wait_loads_then_barrier<(STAGES - 1) * L>();
+  else wait_loads_then_barrier<0>();
+
+  // row li of tile i of the wave's, piece lq of a part; s(8 i + l) = s(l) ^ 2 (i & 1)
+  const uint32_t position = (li >> 1) * 128 + (((((li & 1) << 2) | lq) ^ (((li >> 1) ^ (li >> 3)) & 3)) << 4);
+  const uint32_t xrow = wm * WM * 1024 + position, wrow = XBYTES + wn * WN * 1024 + position;
+  bf16x8 a[SETS][3], b[WN][3];
+  auto read_x = [&](int i, uint32_t stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 3; ++h)
+      a[i % SETS][h] = as_bf16x8(*reinterpret_cast<const uint4*>(pipe_lds + stage + (xrow ^ (((wm * WM + i) & 1) << 5)) + h * (BM * 64) + i * 1024));
+  };
+  auto read_w = [&](int j, int h, uint32_t stage) __attribute__((always_inline)) {
+    b[j][h] = as_bf16x8(*reinterpret_cast<const uint4*>(pipe_lds + stage + (wrow ^ (((wn * WN + j) & 1) << 5)) + h * (BN * 64) + j * 1024));
+  };
+  auto mul = [&](floatx4& sum, bf16x8 wp, bf16x8 xp) __attribute__((always_inline)) {
+    if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(sum) : "v"(wp), "v"(xp));
+    else sum = mfma16(wp, xp, sum);
+  };
+
+  // One step from `stage`; the next step's operands are read from `next`, later loads go into `stage` once it is free.  A tile takes
+  // w's parts in their order, three products with the first, two with the second, one with the third: the step's last tile has done
+  // with the first two before its end, and they are read for the next step there, the third in the next step's first tile.
+  // LOADS: a step is left to be asked for; MORE: a step follows; ON_THE_WAY: loads of later steps than it.
+  auto walk = [&](auto loads, auto more, auto on_the_way, uint32_t stage, uint32_t next) __attribute__((always_inline)) {
+    constexpr int FREE = WM - AHEAD, PRODUCTS = 6 * WN * AHEAD;      // products from the barrier to the end of the step
+    constexpr bool LOADS = decltype(loads)::value, MORE = decltype(more)::value;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      if (i == FREE && MORE) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(decltype(on_the_way)::value) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (i + AHEAD < WM) read_x(i + AHEAD, stage);
+      else if (MORE) read_x(i + AHEAD - WM, next);
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int jj = 0; jj < WN; ++jj) {
+          const int j = (q & 1) ? WN - 1 - jj : jj;
+          const int m = (i - FREE) * 6 * WN + q * WN + jj;           // products since the barrier
+          if (i == 0 && q == 0) read_w(j, 2, stage);
+          if (i == WM - 1 && MORE && q == 3) read_w(jj, 0, next);
+          if (i == WM - 1 && MORE && q == 5) read_w(jj, 1, next);
+          if (LOADS && m >= 0 && m % 2 == 0 && m / 2 < L) load(stage, m / 2);      // one for every two products from the barrier on
+          if (q == 0) mul(low[i][j], b[j][0], a[i % SETS][2]);
+          else if (q == 1) mul(acc[i][j], b[j][0], a[i % SETS][0]);
+          else if (q == 2) mul(low[i][j], b[j][0], a[i % SETS][1]);
+          else if (q == 3) mul(low[i][j], b[j][1], a[i % SETS][1]);
+          else if (q == 4) mul(low[i][j], b[j][1], a[i % SETS][0]);
+          else mul(low[i][j], b[j][2], a[i % SETS][0]);
+          if (m & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (LOADS) {
+#pragma unroll
+      for (int j = PRODUCTS / 2; j < L; ++j) load(stage, j);
+      xs += kStepBytes;
+      ws += kStepBytes;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) read_x(i, 0);
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < WN; ++j) read_w(j, h, 0);
+  uint32_t stage = 0;
+  auto after = [&](uint32_t v) { return v == (STAGES - 1) * STAGE ? 0u : v + STAGE; };
+  int s = 0;
+  for (; s + STAGES < steps; ++s) {
+    const uint32_t next = after(stage);
+    walk(yes, yes, std::integral_constant<int, (STAGES - 2) * L>{}, stage, next);
+    stage = next;
+  }
+  auto tail = [&](auto behind) __attribute__((always_inline)) {       // a step with `behind` more behind it
+    constexpr int BEHIND = decltype(behind)::value;
+    if (steps - 1 - s == BEHIND) {
+      const uint32_t next = after(stage);
+      walk(no, yes, std::integral_constant<int, (BEHIND - 1) * L>{}, stage, next);
+      stage = next;
+      ++s;
     }
   };
+  if constexpr (STAGES > 3) tail(std::integral_constant<int, 3>{});
+  if constexpr (STAGES > 2) tail(std::integral_constant<int, 2>{});
+  tail(std::integral_constant<int, 1>{});
+  walk(no, no, std::integral_constant<int, 0>{}, stage, 0);
+  if constexpr (AGPR) {
+    asm volatile("s_nop 15\n\ts_nop 15" : : : "memory");      // the last products' sums are read after enough wait states
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
-    if (s < steps) fetch(s, s);
-  for (int s0 = 0; s0 < steps; s0 += STAGES) {
+    for (int i = 0; i < WM; ++i)
 #pragma unroll
-    for (int u = 0; u < STAGES; ++u) {
-      const int s = s0 + u;
-      if (s >= steps) break;
-      // every wave's loads of step s have landed, and every wave is done with step s - 1
-      if (steps - 1 - s >= STAGES - 2) wait_loads_then_barrier<(STAGES - 2) * (LX + LW)>();
-      else wait_loads_then_barrier<0>();
-      if (s + STAGES - 1 < steps) fetch((u + STAGES - 1) % STAGES, s + STAGES - 1);
-      multiply(u);
-    }
-  }
-  bool strange = false;
-#pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    const int t = t0 + (wm * WM + i) * 32 + li, ex = x_exp[min(t, T - 1)];
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int n = n0 + (wn * WN + j) * 32 + 8 * (r / 4) + 4 * lk + r % 4, e = ex + w_exp[min(n, N - 1)];
-        const float back = __builtin_amdgcn_ldexpf(acc[i][j][r] + low[i][j][r], -e);
-        const bool beyond = e >= kNotFinite / 2;      // exponents of finite rows lie between -78 and 199
-        acc[i][j][r] = beyond ? 0.f : (t ^ n) & 1 ? -back : back;
-        strange |= beyond;
+      for (int j = 0; j < WN; ++j) {
+        asm volatile("" : "+a"(acc[i][j]));
+        asm volatile("" : "+a"(low[i][j]));
       }
   }
-  tile_epilogue<WM, WN, MODE, TB, WAVES_N, true>(acc, reinterpret_cast<float*>(pipe_lds), bias, out, T, N, t0, n0, rope);
+
+  // lane (li, lq) holds out[t = tile row li][n = 4 lq + r of tile column j].  The sums there are asked for a tile of tokens ahead of the stores.
+  const int nbase = n0 + wn * WN * 16 + 4 * lq;
+  const bool fours = (out_stride & 3) == 0;
+  int ew[WN][4];
+  float add[WN][4];
+#pragma unroll
+  for (int j = 0; j < WN; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ew[j][r] = w_exp[min(nbase + 16 * j + r, N - 1)];
+#pragma unroll
+  for (int j = 0; j < WN; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = min(nbase + 16 * j + r, N - 1);
+      add[j][r] = !bias ? 0.f : bias_dtype == kBF16 ? to_float(reinterpret_cast<const bf16_t*>(bias)[n]) : reinterpret_cast<const float*>(bias)[n];
+    }
+  int ex[WM];
+#pragma unroll
+  for (int i = 0; i < WM; ++i) ex[i] = x_exp[min(t0 + (wm * WM + i) * 16 + li, T - 1)];
+  float4 there[2][WN];
+  auto fetch = [&](int i) __attribute__((always_inline)) {
+    const float* row = out + size_t(min(t0 + (wm * WM + i) * 16 + li, T - 1)) * out_stride;
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+      if (MODE == kAccumulate && fours && nbase + 16 * j + 4 <= N) there[i & 1][j] = *reinterpret_cast<const float4*>(row + nbase + 16 * j);
+  };
+  bool strange = false;
+  fetch(0);
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    if constexpr (AGPR) {
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        asm volatile("" : "+a"(acc[i][j]));
+        asm volatile("" : "+a"(low[i][j]));
+      }
+    }
+    if (i + 1 < WM) fetch(i + 1);
+    const int t = t0 + (wm * WM + i) * 16 + li;
+    float* row = out + size_t(min(t, T - 1)) * out_stride;
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const int n = nbase + 16 * j;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = ex[i] + ew[j][r];
+        const float back = __builtin_amdgcn_ldexpf(acc[i][j][r] + low[i][j][r], -e);
+        const bool beyond = e >= kNotFinite / 2;      // exponents of finite rows lie between -78 and 199
+        v[r] = (beyond ? 0.f : (t ^ (n + r)) & 1 ? -back : back) + add[j][r];
+        strange |= beyond;
+      }
+      if (t >= T || n >= N) continue;
+      if (fours && n + 4 <= N) {
+        if (MODE == kAccumulate) {
+          const float4 old = there[i & 1][j];
+          *reinterpret_cast<float4*>(row + n) = make_float4(old.x + v[0], old.y + v[1], old.z + v[2], old.w + v[3]);
+        } else {
+          *reinterpret_cast<float4*>(row + n) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+      } else {
+        for (int r = 0; r < 4 && n + r < N; ++r) row[n + r] = MODE == kAccumulate ? row[n + r] + v[r] : v[r];
+      }
+    }
+  }
   if (!__syncthreads_or(strange)) return;
   // results of rows that are not finite: bias, and what was there before, stand in the output; the sums are added to them
-  for (int at = threadIdx.x; at < BM * BN; at += 64 * NW) {
+  for (int at = threadIdx.x; at < BM * BN; at += 256) {
     const int t = t0 + at / BN, n = n0 + at % BN;
     if (t >= T || n >= N) continue;
-    const int ex = x_exp[t], ew = w_exp[n];
-    if (max(ex, ew) < kNotFinite) continue;
-    const bool nan = max(ex, ew) == kHasNan;
+    const int et = x_exp[t], en = w_exp[n];
+    if (max(et, en) < kNotFinite) continue;
+    const bool nan = max(et, en) == kHasNan;
     float sum = nan ? __builtin_nanf("") : 0.f;
-    for (int k = 0; k < K && !nan; ++k) sum = fmaf(number_of(x, t, k, K, ex), number_of(w, n, k, K, ew), sum);
-    out[size_t(t) * rope.row_stride + n] += sum;
+    for (int k = nan ? K : 0; k < K; k += 8) {
+      float xv[8], wv[8];
+      numbers_of(x, t, k, K, et, xv);
+      numbers_of(w, n, k, K, en, wv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum = fmaf(xv[e], wv[e], sum);
+    }
+    out[size_t(t) * out_stride + n] += sum;
   }
 }
 
-// Block shapes, blocks a CU holds, microseconds of a block's start and end, of a step of 32 along K on a CU by itself, and of one
-// where the chip is full.
-struct SplitShape { int bm, bn, per_cu; float start_us, light_us, full_us; };
-constexpr SplitShape kSplitShapes[] = {{256, 128, 1, 8.f, 1.75f, 2.35f}, {128, 64, 2, 3.f, 0.73f, 1.38f}, {64, 64, 2, 3.f, 0.44f, 0.80f}};
+// The block shapes: X(index, WM, WN, STAGES), and what was measured of them, fitted over 35 products (256 to 2,048 tokens, 896 to
+// 18,944 rows, K of 896 to 4,864) on every shape: microseconds of a step of 32 along K on a full chip, and, where two blocks share a CU,
+// of one that has a CU to itself.
+#define SPROUT_SPLIT_SHAPES(X) X(0, 8, 4, 2) X(1, 6, 4, 2) X(2, 2, 4, 4) X(3, 4, 2, 2) X(4, 2, 2, 3) X(5, 2, 2, 4) X(6, 6, 2, 3)
+struct SplitShape { int wm, wn, per_cu; };
+constexpr SplitShape kSplitShapes[] = {
+#define SPROUT_SPLIT_ROW(I, WM, WN, STAGES) {WM, WN, split_shares_cu<WM, WN, STAGES> ? 2 : 1},
+    SPROUT_SPLIT_SHAPES(SPROUT_SPLIT_ROW)
+#undef SPROUT_SPLIT_ROW
+};
+constexpr float kSplitStepUs[] = {1.95f, 1.48f, 0.61f, 1.10f, 0.66f, 0.37f, 0.85f};
+constexpr float kSplitAloneUs[] = {1.95f, 1.48f, 0.61f, 0.69f, 0.38f, 0.37f, 0.85f};
 
+// Rounds of blocks on the XCD that holds the most, as in quad_choice (gemm_quad.hip); the choice takes 1 % longer than the best shape
+// over the 35 products (mean; 17 % at worst).
 int choose_split_shape(int T, int N, int K, float* time_us) {
   int best = 0;
   const float steps = float(K / kStep);
   for (int i = 0; i < int(sizeof(kSplitShapes) / sizeof(kSplitShapes[0])); ++i) {
     const SplitShape& p = kSplitShapes[i];
-    const long blocks = long((T + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn), slots = 256 * p.per_cu;
-    const long rounds = blocks / slots, rest = blocks % slots;
-    float us = float(rounds) * (p.start_us + steps * p.full_us) + 3.f;
-    const float shared = p.per_cu == 1 ? float(rest) / float(slots) : rest > 256 ? 1.f : 0.f;
-    if (rest) us += p.start_us + steps * (p.light_us + (p.full_us - p.light_us) * shared);
+    const PipeTiles tiles = pipe_tiles((T + 32 * p.wm - 1) / (32 * p.wm), (N + 32 * p.wn - 1) / (32 * p.wn));
+    const int blocks = tiles.full * tiles.tiles_t + tiles.run, slots = 32 * p.per_cu, full = blocks / slots, rest = blocks % slots;
+    const float ends = 0.41f * float(p.wm * p.wn) + 0.61f, block = steps * kSplitStepUs[i] + ends, alone = steps * kSplitAloneUs[i] + ends;
+    float us = 2.7f + full * block;
+    if (rest > 32) us += fmaxf(alone, block * (0.85f + 0.15f * float(rest - 32) / 32.f));
+    else if (rest) us += alone * (0.81f + 0.19f * float(rest) / 32.f);
     if (i == 0 || us < *time_us) { best = i; *time_us = us; }
   }
   return best;
@@ -317,17 +468,18 @@ struct Product {
   const unsigned char *x, *w;
   const int32_t *x_exp, *w_exp;
   const void* bias;      // may be null
+  int bias_dtype;
   float* out;
   int T, N, K;
   long long out_stride;
 };
 
-template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, int MODE, typename TB>
+template <int WM, int WN, int STAGES, int MODE>
 int launch_mode(hipStream_t s, const Product& p) {
-  constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N, lds = STAGES * (BM + BN) * 192;
+  constexpr int lds = split_lds<WM, WN, STAGES>;
   static bool raised = false;
   if (!raised) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_product_kernel<WM, WN, WAVES_M, WAVES_N, STAGES, MODE, TB>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_product_kernel<WM, WN, STAGES, MODE>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) {
       set_error("sp_gemm_f32_split: cannot raise the LDS limit: %s", hipGetErrorString(e));
@@ -335,30 +487,22 @@ int launch_mode(hipStream_t s, const Product& p) {
     }
     raised = true;
   }
-  const PipeTiles tiles = pipe_tiles((p.T + BM - 1) / BM, (p.N + BN - 1) / BN);
-  RopeArgs args = {};
-  args.row_stride = p.out_stride;
-  split_product_kernel<WM, WN, WAVES_M, WAVES_N, STAGES, MODE, TB><<<8 * (tiles.own + tiles.run), 64 * WAVES_M * WAVES_N, lds, s>>>(
-      p.x, p.w, p.x_exp, p.w_exp, (const TB*)p.bias, p.out, p.T, p.N, p.K, args);
+  const PipeTiles tiles = pipe_tiles((p.T + 32 * WM - 1) / (32 * WM), (p.N + 32 * WN - 1) / (32 * WN));
+  split_product_kernel<WM, WN, STAGES, MODE><<<8 * (tiles.own + tiles.run), 256, lds, s>>>(
+      p.x, p.w, p.x_exp, p.w_exp, p.bias, p.bias_dtype, p.out, p.T, p.N, p.K, p.out_stride);
   return check_launch("sp_gemm_f32_split");
 }
 
-template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES>
-int launch_product(hipStream_t s, const Product& p, bool add, int bias_dtype) {
-  if (p.bias && bias_dtype == kBF16)
-    return add ? launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kAccumulate, bf16_t>(s, p)
-               : launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, bf16_t>(s, p);
-  return add ? launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kAccumulate, float>(s, p)
-             : launch_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, float>(s, p);
-}
-
-int product(hipStream_t s, const Product& p, bool add, int bias_dtype) {
+int product(hipStream_t s, const Product& p, bool add) {
   float time_us;
   switch (choose_split_shape(p.T, p.N, p.K, &time_us)) {
-    case 0: return launch_product<2, 2, 4, 2, 2>(s, p, add, bias_dtype);
-    case 1: return launch_product<2, 1, 2, 2, 2>(s, p, add, bias_dtype);
-    default: return launch_product<1, 1, 2, 2, 3>(s, p, add, bias_dtype);
+#define SPROUT_SPLIT_CASE(I, WM, WN, STAGES) \
+    case I: return add ? launch_mode<WM, WN, STAGES, kAccumulate>(s, p) : launch_mode<WM, WN, STAGES, kStoreF32>(s, p);
+    SPROUT_SPLIT_SHAPES(SPROUT_SPLIT_CASE)
+#undef SPROUT_SPLIT_CASE
   }
+  set_error("sp_gemm_f32_split: no shape for %d tokens, %d rows, K = %d", p.T, p.N, p.K);
+  return 1;
 }
 
 // ... and of a split of `rows` rows of K numbers, at 4.6 TB/s.
@@ -393,11 +537,10 @@ extern "C" int64_t sp_gemm_f32_split_bytes(int T, int N, int K) {
 }
 
 // Whether sp_gemm_f32_split is taken to be faster than the float32 instruction's kernel: the weights are split once a call, which
-// few tokens do not pay for, and small products pay for the launches (whole calls with the norm or the gate before them, float32
-// instruction -> this, us: 640 tokens by 9,728 rows of 896 129 -> 92, 2,048 303 -> 235; 896 rows of 4,864 at 1,500 tokens 176 -> 138, 2,048
-// 182 -> 154; 37,888 of 3,584 at 512 tokens 1,108 -> 1,216, at 1,024 2,170 -> 1,862, at 2,048 4,268 -> 2,958; 3,584 of 18,944 at 512
-// 645 -> 652, at 2,048 2,339 -> 1,654; 896 of 896 at 2,048 34 -> 43).  The two estimates were within a fifth of what was measured
-// over 124 products, and took none to the slower side by more than 3 %.
+// few tokens do not pay for, and small products pay for the launches (float32 instruction's product -> whole calls with the norm or
+// the gate, us: 640 tokens by 9,728 rows of 896 101 -> 80, 2,048 320 -> 202; 896 rows of 4,864 at 1,500 tokens 164 -> 115, 2,048 163 -> 124;
+// 37,888 of 3,584 at 512 tokens 1,079 -> 1,050, at 1,024 2,120 -> 1,559, at 2,048 4,095 -> 2,513; 3,584 of 18,944 at 512 615 -> 546,
+// at 2,048 2,226 -> 1,457; at 2,048 tokens 1,152 of 896 46 -> 44, 896 of 896 36 -> 50, which is not taken).
 extern "C" int sp_gemm_f32_split_pays(int T, int N, int K) {
   if (sp_gemm_f32_split_bytes(T, N, K) == 0) return 0;
   const int piece = piece_of(K), chunk = chunk_rows(T, N, piece);
@@ -450,8 +593,8 @@ extern "C" int sp_gemm_f32_split(void* stream, int kind, const float* a, const f
       wsrc.first = k;
       if (launch_split<kRowsAsTheyAre>(s, wsrc, ws, w_exp + n, rows, width)) return 1;
       const void* rows_bias = !bias || k > 0 ? nullptr : bias_dtype == kBF16 ? (const void*)((const bf16_t*)bias + n) : (const void*)((const float*)bias + n);
-      const Product p = {xs, ws, x_exp, w_exp + n, rows_bias, out + n, T, rows, width, N};
-      if (const int rc = product(s, p, mode == 1 || k > 0, bias_dtype)) return rc;
+      const Product p = {xs, ws, x_exp, w_exp + n, rows_bias, bias_dtype, out + n, T, rows, width, N};
+      if (const int rc = product(s, p, mode == 1 || k > 0)) return rc;
     }
   }
   return 0;

@@ -222,3 +222,20 @@ def test_workspace_of_the_largest_steps(H, I, kv):
     """Split operands of a step of 2,048 tokens: 200 MB at most, whatever the sizes."""
     from sprout_lm_amd import ops
     assert max(ops.gemm_f32_split_bytes(2048, n, k) for n, k in ((2 * I, H), (H, I), (H + 2 * kv, H), (H, H))) <= 200e6
+
+
+# a product for every block shape of the four-wave kernel, with tiles of tokens and rows that are not whole
+@pytest.mark.parametrize("T,N,K", [(1025, 6001, 1920), (1300, 4098, 288), (321, 4098, 1920), (450, 4098, 64), (450, 2050, 96),
+                                   (256, 33, 64), (513, 4097, 384)])
+def test_every_block_shape(T, N, K):
+    from sprout_lm_amd import ops
+    a, w, bias = rows(T, K, T), rows(N, K, N), torch.randn(N, device=DEV)
+    size = a.double().abs() @ w.double().abs().t()
+    want = a.double() @ w.double().t() + bias.double()
+    limit = bound(K) * size + 2.0 ** -22 * bias.double().abs()
+    out = torch.full((T + 1, N), 7.0, device=DEV)
+    assert ops.gemm_f32_split(a, w, out[:T], scratch, bias=bias)
+    assert ((out[:T].double() - want).abs() <= limit).all() and (out[T] == 7).all()
+    acc = torch.ones(T + 1, N, device=DEV)
+    assert ops.gemm_f32_split(a, w, acc[:T], scratch, bias=bias, accumulate=True)
+    assert ((acc[:T].double() - 1 - want).abs() <= limit + 2.0 ** -23 * (1 + want.abs())).all() and (acc[T] == 1).all()
