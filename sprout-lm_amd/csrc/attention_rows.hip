@@ -7,9 +7,14 @@
 // (global_load_lds, asked for a whole stage ahead, one barrier a stage); every operand is read a phase before it is used: the
 // values before the scores are multiplied, the next keys before they are weighed.  Two blocks run on a CU.
 // What bounds it: per 32 keys a wave issues 16 matrix instructions (512 cycles) and 130 vector ones (700 cycles: a multiply-add,
-// an exponential at 9 cycles, a sum, half a maximum and half a conversion a score), and a wave alone on its SIMD takes their
-// sum, 1,450 cycles; two waves overlap in part.  14 heads of 64 in 2 groups, 2,048 queries over 32,768 keys: 511 -> 298 us
-// (780 TFLOP/s) with four parts of the keys, and 8 for their merge; over 8,192: 137 -> 92 + 8; two prompts of 2,048: 80 -> 52.
+// an exponential at 9 cycles, a sum, half a maximum and half a conversion a score); two waves on a SIMD overlap in part.  A stage's
+// loads ask for little beside: a page's place in the pools is in LDS as it is added, and a lane's share of it is its own for the whole walk
+// (with every place worked out from its key 130 vector instructions a stage, 8 % more time).  14 heads of 64 in 2 groups, 2,048 queries over
+// 32,768 keys: 511 -> 280 us (830 TFLOP/s) with four parts of the keys, and 8 for their merge; over 8,192: 137 -> 92 + 8; two prompts of
+// 2,048: 80 -> 52.
+// (One head's weights between the other's products, in one wave: the matrix cores and the vector unit then overlap within a wave too,
+// but the launch takes 5 % longer; four waves a CU with all registers to themselves: 450 us, the vector unit takes 2.7 cycles an
+// instruction from two waves and 5 from one.)
 // (Stages of 64 keys in a ring of three with operands read where they are used: 366 us; s_setprio around the matrix
 // instructions changed nothing.)
 //
@@ -166,8 +171,11 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   const int32_t* table = block_tables + size_t(seq) * max_blocks;
   const int first_page = lo >> page_shift, n_pages = hi >= lo ? (hi >> page_shift) - first_page + 1 : 0;
   const bool table_in_lds = n_pages <= kRowsTable;
+  // a page's place in either pool, in units of 512 numbers (it holds 8 tokens of 64 at least): 32 bits reach 4 TB
+  const uint32_t page_units = uint32_t(nkv) << page_shift >> 3;
+  auto place_of = [&](int page) __attribute__((always_inline)) { return uint32_t(min(max(page, 0), num_pages - 1)) * page_units; };
   if (table_in_lds)
-    for (int i = threadIdx.x; i < n_pages; i += 256) s_table[i] = table[first_page + i];
+    for (int i = threadIdx.x; i < n_pages; i += 256) s_table[i] = int32_t(place_of(table[first_page + i]));
   __syncthreads();
 
   const int stages = hi >= lo ? (hi - lo) / kRowsKeys + 1 : 0;
@@ -176,10 +184,11 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   const uint16_t* kbase = k_pool + (size_t(g) << page_shift) * HD;
   const uint16_t* vbase = v_pool + (size_t(g) << page_shift) * HD;
   const int page_mask = (1 << page_shift) - 1;
-  // What this lane fetches of a stage: of row r = 8 (4 j + wave) + lane / 8 the piece (lane % 8) ^ swz(r); key rows hold the key with
-  // bits 2 and 3 of their number swapped, value rows are dimensions.
-  int kkey[2], vkey[2];
-  uint32_t kcol[2], vrow[2];
+  // What this lane fetches of a run of 64 keys: of row r = 8 (4 j + wave) + lane / 8 the piece (lane % 8) ^ swz(r); key rows hold the key
+  // with bits 2 and 3 of their number swapped, value rows are dimensions.  A run begins at a multiple of 64, so a key's page and
+  // its place there are the run's and the lane's own, added: kplace and vplace, and page kpage (vpage) from the run's first.
+  int kkey[2], vkey[2], kcol[2], vrow[2], kpage[2], vpage[2];
+  const uint16_t *kplace[2], *vplace[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int r = 8 * (4 * j + wave) + (lane >> 3), piece = (lane & 7) ^ rows_swz(r);
@@ -187,27 +196,37 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
     kcol[j] = 8 * piece;
     vkey[j] = 8 * piece;
     vrow[j] = r;
+    kpage[j] = kkey[j] >> page_shift;
+    vpage[j] = vkey[j] >> page_shift;
+    kplace[j] = kbase + (kkey[j] & page_mask) * HD + kcol[j];
+    vplace[j] = vbase + (size_t(vrow[j]) << page_shift) + (vkey[j] & page_mask);
   }
   auto fetch_from = [&](int s, int buf, auto in_lds) __attribute__((always_inline)) {
-    auto page_at = [&](int key) __attribute__((always_inline)) {
-      int page;
-      if constexpr (decltype(in_lds)::value) page = s_table[(key >> page_shift) - first_page];
-      else page = table[key >> page_shift];
-      return size_t(min(max(page, 0), num_pages - 1)) * nkv;
+    auto page_at = [&](int page) __attribute__((always_inline)) {
+      if constexpr (decltype(in_lds)::value) return size_t(uint32_t(s_table[page - first_page])) << 9;
+      else return size_t(place_of(table[page])) << 9;
     };
 #pragma unroll
     for (int run = 0; run < 2; ++run) {
       const int key0 = lo + s * kRowsKeys + 64 * run;
       const uint32_t dst = lds0 + buf * kRowsStageBytes + run * 16384 + wave * 1024;
+      if (key0 + 63 <= hi) {
+        const int page0 = key0 >> page_shift, in_page = key0 & page_mask;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) lanes_to_lds(kplace[j] + (page_at(page0 + kpage[j]) + size_t(in_page * HD)), dst + j * 4096);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) lanes_to_lds(vplace[j] + (page_at(page0 + vpage[j]) + size_t(in_page)), dst + 8192 + j * 4096);
+        continue;
+      }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int key = min(key0 + kkey[j], hi);      // keys behind the walk's end repeat the last one: masked by position
-        lanes_to_lds(kbase + ((page_at(key) << page_shift) + (key & page_mask)) * HD + kcol[j], dst + j * 4096);
+        lanes_to_lds(kbase + page_at(key >> page_shift) + (key & page_mask) * HD + kcol[j], dst + j * 4096);
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int key = min(key0 + vkey[j], hi & ~7);
-        lanes_to_lds(vbase + ((page_at(key) * HD + vrow[j]) << page_shift) + (key & page_mask), dst + 8192 + j * 4096);
+        lanes_to_lds(vbase + page_at(key >> page_shift) + (size_t(vrow[j]) << page_shift) + (key & page_mask), dst + 8192 + j * 4096);
       }
     }
   };
