@@ -180,12 +180,12 @@ __device__ __forceinline__ void quad_epilogue(floatx4 (&acc)[WM][WN], float* tur
       constexpr int ACT = decltype(which)::value;
 #pragma unroll
       for (int i = 0; i < WM; ++i) {
-        take(i);
         const int t = t0 + (wm * WM + i) * 16 + li;
         if (t >= T) continue;
         const float row = rope.row_gate ? 1.0f / (1.0f + expf(-rope.row_gate[size_t(t) * rope.row_gate_stride])) : 1.0f;
         auto value = [&](float gate, float up) __attribute__((always_inline)) {
-          const float g = to_float(bf16_t{f32_to_bf16_bits(gate)}), u = to_float(bf16_t{f32_to_bf16_bits(up)});
+          const uint32_t both = pack_bf16x2(gate, up);
+          const float g = __uint_as_float(both << 16), u = __uint_as_float(both & 0xffff0000u);
           float v;
           if (ACT == kActSilu) v = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
           else if (ACT == kActGeluTanh) v = g * __builtin_amdgcn_rcpf(1.0f + __expf(gelu_tanh_exponent(g))) * u;
