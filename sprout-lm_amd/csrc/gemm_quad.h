@@ -542,8 +542,8 @@ inline int launch_quad(hipStream_t s, int splits, const uint16_t* x, const uint1
 
 enum QuadKind { kQuadStore = 0, kQuadAccumulate = 1, kQuadGated = 2, kQuadRotating = 3 };   // as sp_quad_plan counts them
 
-// Whether the four-wave kernel takes T x N x K (N: all weight rows): more tokens than the decode kernels', whole steps of 64
-// along K, outputs in whole eights of a row.
+// Whether the four-wave kernel takes T x N x K (N: all weight rows): more than 64 tokens, from 17 on where it is the faster one; whole
+// steps of 64 along K, outputs in whole eights of a row.
 bool gemm_quad_takes(int kind, int T, int N, int K, int hd = 0);
 // 16-byte stores: an output that is not so aligned stays with gemm_pipe's kernel.
 inline bool quad_aligned(const void* x, const void* w, const void* out) {

@@ -53,8 +53,8 @@ int sp_pipe_plan(int kind, int T, int N, int K, int hd, int* plan);
 // How that kernel numbers its blocks: tile_of[2 b], tile_of[2 b + 1] = token tile and weight tile of block b (which
 // runs on XCD b % 8), -1 for a block with nothing to do; returns the number of blocks.  Runs nothing.
 int sp_pipe_tiles(int tiles_t, int tiles_n, int* tile_of, int room);
-// The same of the product on four waves a block, which takes more than 64 tokens with outputs in whole eights (sp_pipe_plan's kernel
-// has the others): plan = {block rows, block columns, splits of K, buffers of x}.
+// The same of the product on four waves a block, which takes more than 64 tokens, and from 17 on where it is the faster one, with
+// outputs in whole eights (other kernels have the rest): plan = {block rows, block columns, splits of K, buffers of x}.
 int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan);
 int sp_gemm_decode(void* stream, const void* x, const float* residual, int norm_w_dtype, const void* norm_w, float eps,
                    const void* w, int bias_dtype, const void* bias, int mode, void* out, int T, int N, int K);

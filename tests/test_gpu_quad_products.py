@@ -12,13 +12,14 @@ STORE, ACCUMULATE, GATED = 0, 1, 2          # the kinds of sp_quad_plan
 _STORED = [(65, 8, 64), (65, 72, 128), (66, 264, 192), (97, 131 * 8, 256), (65, 20000, 64), (65, 13608, 1920), (193, 26664, 64), (97, 26664, 192),
            (193, 20000, 1920), (321, 20000, 1920), (777, 9736, 64), (777, 20000, 896), (130, 20000, 1920), (513, 13608, 192), (513, 20000, 384),
            (193, 26664, 1920), (2047, 4904, 384), (641, 20000, 896), (1300, 9736, 576), (289, 26664, 192)]
+_STORED_FEW = [(17, 4608, 3584), (33, 2056, 1536), (64, 40000, 896), (45, 4104, 896)]
 # a split of K in two and more on every shape but the largest
 _SPLIT = [(65, 8, 576), (65, 9736, 1920), (65, 4904, 4864), (97, 9736, 3584), (193, 9736, 4864), (130, 20000, 3584), (777, 4904, 4864),
-          (130, 9736, 4864), (161, 20000, 4864), (257, 13608, 4864)]
+          (130, 9736, 4864), (161, 20000, 4864), (257, 13608, 4864), (17, 3592, 3584), (45, 904, 4864), (64, 2568, 5120)]
 _GATED = [(65, 16, 64), (66, 528, 128), (65, 19472, 64), (65, 14400, 1920), (97, 40000, 64), (97, 19472, 256), (193, 19472, 1920), (321, 19472, 1920),
           (130, 40000, 64), (130, 53328, 192), (130, 19472, 1920), (161, 40000, 192), (321, 27216, 384), (193, 27216, 1920), (193, 40000, 384),
-          (193, 53328, 896), (777, 14400, 576), (289, 27216, 192)]
-SIZES = {STORE: _STORED, ACCUMULATE: _STORED + _SPLIT, GATED: _GATED}
+          (193, 53328, 896), (777, 14400, 576), (289, 27216, 192), (17, 9728, 896), (45, 9760, 896), (64, 17920, 1536)]
+SIZES = {STORE: _STORED + _STORED_FEW, ACCUMULATE: _STORED + _SPLIT, GATED: _GATED}
 ROTATING_SIZES = [(65, 1, 1, 64, 64), (193, 56, 8, 128, 64), (321, 56, 8, 64, 1920), (2047, 8, 8, 128, 64), (289, 64, 8, 128, 320),
                   (777, 56, 8, 128, 1920), (777, 64, 8, 128, 256), (513, 64, 8, 128, 1088), (2047, 64, 8, 64, 384), (2047, 8, 8, 128, 1920),
                   (1238, 64, 8, 128, 896), (2047, 28, 4, 128, 320), (70, 2, 1, 192, 128)]
@@ -31,7 +32,7 @@ def _operands(T, N, K):
     return x, w, torch.randn(N, device=DEV, generator=gen), x.float() @ w.float().T
 
 
-@pytest.mark.parametrize("T,N,K", _STORED)
+@pytest.mark.parametrize("T,N,K", _STORED + _STORED_FEW)
 def test_store(T, N, K):
     from sprout_lm_amd import ops
     x, w, bias, want = _operands(T, N, K)

@@ -23,14 +23,25 @@ def built_library():
 def test_plan_invariants(kind):
     for T, N, K in itertools.product([1, 64, 65, 100, 264, 777, 2048, 8192], [8, 16, 130, 900, 1152, 37888, 151936], [64, 70, 192, 3584, 27648]):
         plan = ops.quad_plan(kind, T, N, K)
-        if T <= 64 or K % 64 or N % (16 if kind == ops.PLAN_GATED else 8) or N * K * 2 >= 1 << 32:
+        if T <= 16 or K % 64 or N % (16 if kind == ops.PLAN_GATED else 8) or N * K * 2 >= 1 << 32:
             assert plan is None, (T, N, K)          # other kernels' products
+            continue
+        if T <= 64 and plan is None:
             continue
         rows, cols, splits, buffers = plan
         assert (rows, cols, buffers) in SHAPES, (T, N, K, plan)
         assert buffers * rows * 128 + (buffers + 1) * cols * 128 <= 160 * 1024
         # only float atomics join partial sums; every split has a step
         assert splits == 1 or (kind == ops.PLAN_ACCUMULATE and K // 64 // splits >= 4), (T, N, K, plan)
+
+
+def test_few_tokens_are_taken_where_measurements_say_so():
+    taken = lambda kind, T, N, K: ops.quad_plan(kind, T, N, K) is not None
+    assert taken(ops.PLAN_GATED, 17, 9728, 896) and not taken(ops.PLAN_GATED, 16, 9728, 896) and not taken(ops.PLAN_GATED, 64, 37888, 3584)
+    assert taken(ops.PLAN_ACCUMULATE, 45, 896, 4864) and not taken(ops.PLAN_ACCUMULATE, 24, 896, 4864)
+    assert taken(ops.PLAN_ACCUMULATE, 17, 3584, 3584) and not taken(ops.PLAN_ACCUMULATE, 64, 896, 896)
+    assert taken(ops.PLAN_STORE, 17, 151936, 896) and not taken(ops.PLAN_STORE, 64, 152064, 3584)
+    assert taken(ops.PLAN_STORE, 17, 4608, 3584) and not taken(ops.PLAN_STORE, 32, 7168, 5120) and taken(ops.PLAN_STORE, 33, 7168, 5120)
 
 
 def test_rotation_takes_heads_of_whole_sixty_fours():
