@@ -157,6 +157,7 @@ int gemm_bf16_tiled(hipStream_t s, const void* a, const void* w, int bias_dtype,
                     int T, int N, int K);
 int gemm_decode_plain(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, int mode, void* out,
                       int T, int N, int K);
+int decode_splits(int T, int N, int K, int* k_per_split);
 int gemm_bf16_quad(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, int mode, void* out, int T, int N, int K);
 int gemm_bf16_quad_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
                         const float* row_gate, long long row_gate_stride);
@@ -164,6 +165,19 @@ int gemm_bf16_pipe(hipStream_t s, const void* a, const void* w, int bias_dtype, 
                    int T, int N, int K);
 int gemm_bf16_pipe_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
                         const float* row_gate, long long row_gate_stride);
+
+// Large accumulating products of few rows stream their weights through the pipelined tiles (K split over blocks), whatever the
+// number of tokens (3,584 x 18,944: 25.4 against 27.7 us at one token, 26.0 against 29.7 at 8, 26.6 against 32.8 at 16); the others
+// split K between the waves of a block.
+// (up to 16 tokens only where the matrix is that large: 3,584 x 3,584 at 8 tokens is 8.2 us fused, 8.8 tiled)
+static bool streams_few(int T, int N, int K) { return size_t(N) * K >= (size_t(T > 16 ? 6 : 32) << 20) && gemm_pipe_takes(T, N, K); }
+
+bool gemm_cuts_k(int T, int N, int K) {
+  int shape, splits, k_per_split;
+  if (T <= 64 && !streams_few(T, N, K) && (N + 15) / 16 < 2048) return decode_splits(T, N, K, &k_per_split) > 1;
+  pipe_choice(T, N, K, true, &shape, &splits);
+  return splits > 1;
+}
 
 // mode 0 stores bfloat16 here; a float32 store of mode 0 is passed in as mode 2 by the caller.
 int gemm_bf16(hipStream_t s, const void* a, const void* w, int bias_dtype, const void* bias, int mode, int out_dtype,
@@ -176,11 +190,7 @@ int gemm_bf16(hipStream_t s, const void* a, const void* w, int bias_dtype, const
   if (gemm_quad_takes(mode == kAccumulate ? kQuadAccumulate : kQuadStore, T, N, K) && quad_aligned(a, w, out))
     return gemm_bf16_quad(s, a, w, bias_dtype, bias, mode, out, T, N, K);
   if (T <= 64) {
-    // Few rows.  Large accumulating products stream their weights through the pipelined tiles (K split over
-    // blocks), whatever the number of tokens (3,584 x 18,944: 25.4 against 27.7 us at one token, 26.0 against 29.7
-    // at 8, 26.6 against 32.8 at 16); the others split K between the waves of a block.
-    // (up to 16 tokens only where the matrix is that large: 3,584 x 3,584 at 8 tokens is 8.2 us fused, 8.8 tiled)
-    if (mode == kAccumulate && size_t(N) * K >= (size_t(T > 16 ? 6 : 32) << 20) && gemm_pipe_takes(T, N, K))
+    if (mode == kAccumulate && streams_few(T, N, K))
       return gemm_bf16_pipe(s, a, w, bias_dtype, bias, mode, out, T, N, K);
     if ((N + 15) / 16 < 2048) return gemm_decode_plain(s, a, w, bias_dtype, bias, mode, out, T, N, K);
     // Very wide (the output head): rows streamed per wave up to 16 tokens; with more, the streaming kernel stops

@@ -645,6 +645,24 @@ int gemm_decode_plain(hipStream_t s, const void* x, const void* w, int bias_dtyp
                       int T, int N, int K) {
   return sp_gemm_decode((void*)s, x, nullptr, 0, nullptr, 0.f, w, bias_dtype, bias, mode, out, T, N, K);
 }
+
+// The split of K of an accumulating product.  A CU pulls its blocks' weight rows at about the same rate however many blocks it
+// holds, so it is chosen for the CU that gets the most: blocks per CU (rounded up) x bytes per block, plus the float
+// atomics of the split (measured 2.7 us per million added floats), both in microseconds.  (8 tokens, against
+// a fixed aim of 768 blocks: 18,944 x 3,584 36 -> 31 us, 27,648 x 5,120 64 -> 55 us, 4,864 x 896 6.0 -> 5.5 us.)
+int decode_splits(int T, int N, int K, int* k_per_split) {
+  const int blocks = (N + 31) / 32;
+  int splits = 1;
+  *k_per_split = (K + 63) / 64 * 64;
+  float best = 1e30f;
+  for (int sp = 1; sp <= min(64, max(1, K / 256)); ++sp) {
+    const int k_per = ((K + sp - 1) / sp + 63) / 64 * 64, real = (K + k_per - 1) / k_per;
+    const float per_cu = float((blocks * real + 255) / 256) * 32.f * float(k_per) * 2.f;   // bytes
+    const float cost = per_cu / 20e3f + 2.7e-6f * float(T) * float(N) * float(real) + (real > 1 ? 0.3f : 0.f);
+    if (cost < best) { best = cost; splits = real; *k_per_split = k_per; }
+  }
+  return splits;
+}
 }  // namespace sprout
 
 // Plain product through the K-splitting kernel: out = x . w^T (+ bias), modes as sp_gemm.
@@ -662,19 +680,7 @@ extern "C" int sp_gemm_decode(void* stream, const void* x, const float* residual
   const int blocks = (N + 31) / 32;
   int splits = 1;
   a.k_per_split = (K + 63) / 64 * 64;
-  if (mode == kEpiAccumulate && !residual) {
-    // A CU pulls its blocks' weight rows at about the same rate however many blocks it holds, so the split of K
-    // is chosen for the CU that gets the most: blocks per CU (rounded up) x bytes per block, plus the float
-    // atomics of the split (measured 2.7 us per million added floats), both in microseconds.  (8 tokens, against
-    // a fixed aim of 768 blocks: 18,944 x 3,584 36 -> 31 us, 27,648 x 5,120 64 -> 55 us, 4,864 x 896 6.0 -> 5.5 us.)
-    float best = 1e30f;
-    for (int sp = 1; sp <= min(64, max(1, K / 256)); ++sp) {
-      const int k_per = ((K + sp - 1) / sp + 63) / 64 * 64, real = (K + k_per - 1) / k_per;
-      const float per_cu = float((blocks * real + 255) / 256) * 32.f * float(k_per) * 2.f;   // bytes
-      const float cost = per_cu / 20e3f + 2.7e-6f * float(T) * float(N) * float(real) + (real > 1 ? 0.3f : 0.f);
-      if (cost < best) { best = cost; splits = real; a.k_per_split = k_per; }
-    }
-  }
+  if (mode == kEpiAccumulate && !residual) splits = decode_splits(T, N, K, &a.k_per_split);
   hipStream_t s = (hipStream_t)stream;
   if (mode == kEpiStore) return fused_norm<kEpiStore>(s, a, residual != nullptr, blocks, splits);
   if (mode == kEpiAccumulate) return fused_norm<kEpiAccumulate>(s, a, residual != nullptr, blocks, splits);

@@ -549,6 +549,10 @@ bool gemm_quad_takes(int kind, int T, int N, int K, int hd = 0);
 inline bool quad_aligned(const void* x, const void* w, const void* out) {
   return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
 }
+// Whether the accumulating product of T x N x K on the other kernels, which take it at other alignments, is cut along K.  Its parts
+// are joined with float atomics, whose order differs from run to run and the sums' last bits with it: a product that comes out the
+// same in every run there does so on four waves too.
+bool gemm_cuts_k(int T, int N, int K);
 // Picks the shape and the split of K with the least estimated time.
 void quad_choice(int kind, int T, int N, int K, int* shape, int* splits);
 

@@ -49,6 +49,7 @@ static const float kAloneUs[] = {0.24f, 0.45f, 0.35f, 0.50f, 0.48f, 0.68f, 0.80f
 // (mean; 25 % at worst).
 void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
   const int steps = K / 64;
+  const bool cuts_k = kind == kQuadAccumulate && gemm_cuts_k(T, N, K);
   const float memory = float(N) * float(K) * 2.f / 5.4e6f + 16.f * float(T) * float(K) / 9e6f, memory2 = memory * memory;
   float best = 1e30f;
   *shape = 3;
@@ -59,7 +60,7 @@ void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
     const int bm = 32 * p.wm, bn = 32 * p.wn, slots = 32 * p.per_cu;
     const PipeTiles tiles = pipe_tiles((T + bm - 1) / bm, (N + bn - 1) / bn);
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
-      if (sp > 1 && (kind != kQuadAccumulate || steps / sp < 4)) break;
+      if (sp > 1 && (!cuts_k || steps / sp < 4)) break;
       const int k_steps = (steps + sp - 1) / sp;
       if ((steps + k_steps - 1) / k_steps != sp) continue;
       const int blocks = (tiles.full * tiles.tiles_t + tiles.run) * sp, full = blocks / slots, rest = blocks % slots;

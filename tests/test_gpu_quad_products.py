@@ -15,7 +15,8 @@ _STORED = [(65, 8, 64), (65, 72, 128), (66, 264, 192), (97, 131 * 8, 256), (65, 
 _STORED_FEW = [(17, 4608, 3584), (33, 2056, 1536), (64, 40000, 896), (45, 4104, 896)]
 # a split of K in two and more on every shape but the largest
 _SPLIT = [(65, 8, 576), (65, 9736, 1920), (65, 4904, 4864), (97, 9736, 3584), (193, 9736, 4864), (130, 20000, 3584), (777, 4904, 4864),
-          (130, 9736, 4864), (161, 20000, 4864), (257, 13608, 4864), (17, 3592, 3584), (45, 904, 4864), (64, 2568, 5120)]
+          (130, 9736, 4864), (161, 20000, 4864), (257, 13608, 4864), (17, 3592, 3584), (45, 904, 4864), (64, 2568, 5120),
+          (835, 2312, 5696), (434, 2592, 7680), (769, 2592, 7488), (1366, 3280, 7168), (1490, 1440, 5824), (1385, 3080, 6528)]
 _GATED = [(65, 16, 64), (66, 528, 128), (65, 19472, 64), (65, 14400, 1920), (97, 40000, 64), (97, 19472, 256), (193, 19472, 1920), (321, 19472, 1920),
           (130, 40000, 64), (130, 53328, 192), (130, 19472, 1920), (161, 40000, 192), (321, 27216, 384), (193, 27216, 1920), (193, 40000, 384),
           (193, 53328, 896), (777, 14400, 576), (289, 27216, 192), (17, 9728, 896), (45, 9760, 896), (64, 17920, 1536)]
@@ -60,6 +61,18 @@ def test_accumulate(T, N, K):
         full = before[:T] + (want if b is None else want + b.float())
         assert (out[:T] - full).abs().max().item() <= 2e-5 * max(1.0, math.sqrt(K) / 8) * (1 + full.abs().max().item())
         assert torch.equal(out[T], before[T])
+
+
+@pytest.mark.parametrize("T,N,K", [(2048, 3584, 18944), (2048, 1536, 8960), (200, 896, 896), (512, 3584, 3584)])
+def test_sums_in_one_part_repeat_bit_for_bit(T, N, K):
+    from sprout_lm_amd import ops
+    assert ops.quad_plan(ops.PLAN_ACCUMULATE, T, N, K)[2] == 1
+    x, w, _, _ = _operands(T, N, K)
+    before = torch.randn(T, N, device=DEV, generator=torch.Generator(device=DEV).manual_seed(3))
+    runs = [before.clone() for _ in range(4)]
+    for out in runs:
+        ops.gemm(x, w, out, accumulate=True)
+    assert all(torch.equal(runs[0], out) for out in runs[1:])
 
 
 @pytest.mark.parametrize("T,N,K", _GATED)

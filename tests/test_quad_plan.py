@@ -1,5 +1,6 @@
 """The choice of block shape of the product on four waves a block, asked of the library without running a kernel (no GPU)."""
 import itertools
+import random
 
 import pytest
 
@@ -33,6 +34,25 @@ def test_plan_invariants(kind):
         assert buffers * rows * 128 + (buffers + 1) * cols * 128 <= 160 * 1024
         # only float atomics join partial sums; every split has a step
         assert splits == 1 or (kind == ops.PLAN_ACCUMULATE and K // 64 // splits >= 4), (T, N, K, plan)
+
+
+def test_no_product_is_cut_that_the_other_kernels_leave_whole():
+    """Parts of K meet in float atomics, whose order no two runs share: sums that the eight-wave kernel gives the same bits in every
+    run (the down product of a prompt of 2,048 tokens at 7B sizes, the output product of 65 to 512 at 0.5B sizes) stay so."""
+    rng = random.Random(3)
+    sizes = list(itertools.product([65, 200, 512, 1500, 2048, 4096], [896, 1536, 3584, 5120], [896, 3584, 4864, 8960, 18944, 27648]))
+    sizes += [(round(17 * 2 ** rng.uniform(0, 7)), 8 * rng.randint(1, 2000), 64 * rng.randint(1, 400)) for _ in range(4000)]
+    cut = 0
+    for T, N, K in sizes:
+        plan = ops.quad_plan(ops.PLAN_ACCUMULATE, T, N, K)
+        if plan is None or plan[2] == 1:
+            continue
+        cut += 1
+        if T > 64 or N * K >= 6 << 20:          # the eight-wave kernel's, otherwise
+            assert ops.pipe_plan(ops.PLAN_ACCUMULATE, T, N, K)[2] > 1, (T, N, K, plan)
+    assert cut > 500
+    for T, N, K in [(58, 4992, 1024), (42, 6648, 640), (34, 4760, 1216)]:      # the kernel for few tokens takes these in one part
+        assert ops.quad_plan(ops.PLAN_ACCUMULATE, T, N, K)[2] == 1
 
 
 def test_few_tokens_are_taken_where_measurements_say_so():
