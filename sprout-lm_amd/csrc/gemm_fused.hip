@@ -612,10 +612,6 @@ int gemm_bf16_tiled_silu(hipStream_t s, const void* x, const void* w, void* out,
 int gemm_bf16_quad_rope(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, void* q_out,
                         const int32_t* positions, const float* inv_freq, const int32_t* slot_mapping, void* k_pool,
                         void* v_pool, int T, int K, int nq, int nkv, int hd, int page_size, const float* table);
-bool gemm_pipe_rope_takes(int T, int N, int K, int hd);
-int gemm_bf16_pipe_rope(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, void* q_out,
-                        const int32_t* positions, const float* inv_freq, const int32_t* slot_mapping, void* k_pool,
-                        void* v_pool, int T, int K, int nq, int nkv, int hd, int page_size, const float* table);
 }
 
 extern "C" int sp_fused_supported(int kind, int T, int N, int K, int hd, int rotary_dim, int norm, int variant) {
@@ -741,13 +737,13 @@ extern "C" int sp_qkv_rope_cache(void* stream, const void* x, const float* resid
              "sp_qkv_rope_cache: shape T=%d K=%d hd=%d rotary=%d is not taken", T, K, hd, rotary_dim);
   SP_REQUIRE((x || residual) && w && q_out && positions && inv_freq && slot_mapping && k_pool && v_pool,
              "sp_qkv_rope_cache: null operand");
-  // many tokens: the tiled product with the rotation as its epilogue
-  if (T > 64 && quad_aligned(x, w, q_out) && quad_aligned(k_pool, v_pool, nullptr))
+  // many tokens: the tiled product with the rotation as its epilogue, which loads and stores sixteen bytes at a time
+  if (T > 64) {
+    SP_REQUIRE(quad_aligned(x, w, q_out) && quad_aligned(k_pool, cos_sin, nullptr),
+               "sp_qkv_rope_cache: operands of %d tokens must start at multiples of 16 bytes", T);
     return gemm_bf16_quad_rope((hipStream_t)stream, x, w, bias_dtype, bias, q_out, positions, inv_freq, slot_mapping, k_pool,
                                v_pool, T, K, nq, nkv, hd, page_size, cos_sin);
-  if (T > 64)
-    return gemm_bf16_pipe_rope((hipStream_t)stream, x, w, bias_dtype, bias, q_out, positions, inv_freq, slot_mapping, k_pool,
-                               v_pool, T, K, nq, nkv, hd, page_size, cos_sin);
+  }
   FusedArgs a = {};
   a.x = (const uint16_t*)x; a.residual = residual; a.norm_w = norm_w; a.norm_w_bf16 = norm_w_dtype == kBF16; a.eps = eps;
   a.w = (const uint16_t*)w; a.bias = bias; a.bias_bf16 = bias_dtype == kBF16; a.out = q_out;

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
                                                         int N, int K, int k_per_split, RopeArgs rope, PipeGroups groups) {
   constexpr int NW = WAVES_M * WAVES_N;
   constexpr int ESZ = sizeof(TE), KSTEP = 128 / ESZ;    // elements of a tile row
-  static_assert(ESZ == 2 || (MODE != kSilu && MODE != kRope && MODE != kStore), "float32 operands store or add float32");
+  static_assert(ESZ == 2 || (MODE != kSilu && MODE != kStore), "float32 operands store or add float32");
   constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N;
   constexpr int ROW = 128;                              // bytes of a tile row
   constexpr int STAGE = (BM + BN) * ROW;                // bytes of a stage
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
 
   // ---- what this lane fetches: row 8 (NW j + wave) + lane / 8 of each operand tile, for j < LX (LW)
   const unsigned char* xbase = reinterpret_cast<const unsigned char*>(x + (GROUPED ? size_t(0) : size_t(t0) * K) + k_begin);
-  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(w + (MODE == kSilu || MODE == kRope ? size_t(0) : size_t(n0) * K) + k_begin);
+  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(w + (MODE == kSilu ? size_t(0) : size_t(n0) * K) + k_begin);
   uint32_t xoff[LX], woff[LW];
 #pragma unroll
   for (int j = 0; j < LX; ++j) {
@@ -162,12 +162,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
       // gate rows and the matching up rows, so that a lane ends with both of one index.
       const int gate = min(N - 1, tile_n * (BN / 2) + (r / 64) * 32 + (r & 31));
       row = ((r >> 5) & 1) ? N + gate : gate;
-    } else if (MODE == kRope) {
-      // Tile rows in runs of 32: 32 dimensions of a head's first half, then their rotation partners half a
-      // head further on, so that a lane ends with both of a pair.
-      const int half = rope.hd / 2, groups_per_head = half / 32;
-      const int group = tile_n * (BN / 64) + r / 64, head = group / groups_per_head, u = group % groups_per_head;
-      row = min(N - 1, head * rope.hd + 32 * u + (r & 31) + ((r >> 5) & 1) * half);
     } else {
       row = min(r, N - 1 - n0);
     }

@@ -45,16 +45,16 @@ int sp_gemm_f32_split(void* stream, int kind, const float* a, const float* norm_
 int sp_fused_supported(int kind, int T, int N, int K, int hd, int rotary_dim, int norm, int variant);
 // Whether folding the norm into the product (norm = 1 above) is faster than a norm kernel before it.
 int sp_fused_norm_pays(int T, int N, int K);
-// What the tiled product for many tokens would do with T x N x K, without running anything: kind 0 store,
-// 1 accumulate, 2 gated (N = 2 I), 3 rotating (head size hd); plan = {block rows, block columns, splits of K,
-// waves of a block}.
-// Returns 1 where that kernel (for kind 3 its rotating epilogue) does not take the product.
-int sp_pipe_plan(int kind, int T, int N, int K, int hd, int* plan);
+// What the tiled product on up to eight waves a block would do with T x N x K, without running anything: kind 0 store,
+// 1 accumulate, 2 gated (N = 2 I); plan = {block rows, block columns, splits of K, waves of a block}.
+// Returns 1 where that kernel does not take the product.
+int sp_pipe_plan(int kind, int T, int N, int K, int* plan);
 // How that kernel numbers its blocks: tile_of[2 b], tile_of[2 b + 1] = token tile and weight tile of block b (which
 // runs on XCD b % 8), -1 for a block with nothing to do; returns the number of blocks.  Runs nothing.
 int sp_pipe_tiles(int tiles_t, int tiles_n, int* tile_of, int room);
 // The same of the product on four waves a block, which takes more than 64 tokens, and from 17 on where it is the faster one, with
-// outputs in whole eights (other kernels have the rest): plan = {block rows, block columns, splits of K, buffers of x}.
+// outputs in whole eights that start at 16 bytes (other kernels have the rest), and is the only one to rotate (kind 3, head size hd):
+// plan = {block rows, block columns, splits of K, buffers of x}.
 int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan);
 int sp_gemm_decode(void* stream, const void* x, const float* residual, int norm_w_dtype, const void* norm_w, float eps,
                    const void* w, int bias_dtype, const void* bias, int mode, void* out, int T, int N, int K);
@@ -65,7 +65,8 @@ int sp_gemm_joined_takes(int T, int N, int K);
 int sp_gemm_joined(void* stream, const void* x, const void* w, const float* bias, int act, void* out, long long out_stride,
                    int split, void* second, long long second_stride, int T, int N, int K);
 // q, k, v projection (+ bias), rotation of q and k, q to q_out [T, nq * hd], k and v into the paged pools.
-// With more than 64 tokens (head sizes that are multiples of 64) the tiled product does it in its epilogue;
+// With more than 64 tokens (head sizes that are multiples of 64) the tiled product does it in its epilogue: x, w, q_out, k_pool
+// and cos_sin then start at multiples of 16 bytes;
 // cos_sin (may be null): the table of sp_rope_table for these positions, which saves it the sines and cosines.
 int sp_qkv_rope_cache(void* stream, const void* x, const float* residual, int norm_w_dtype, const void* norm_w,
                       float eps, const void* w, int bias_dtype, const void* bias, void* q_out,

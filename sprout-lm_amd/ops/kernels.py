@@ -858,13 +858,13 @@ def fused_norm_pays(T: int, N: int, K: int) -> bool:
 PLAN_STORE, PLAN_ACCUMULATE, PLAN_GATED, PLAN_ROTATING = 0, 1, 2, 3
 
 
-def pipe_plan(kind: int, T: int, N: int, K: int, hd: int = 0):
-    """(block rows, block columns, splits of K, waves of a block) that the tiled product for many tokens would take
-    for T x N x K, or None where that kernel (for PLAN_ROTATING its rotating epilogue) does not take the product.
-    Runs nothing and needs no GPU."""
+def pipe_plan(kind: int, T: int, N: int, K: int):
+    """(block rows, block columns, splits of K, waves of a block) that the tiled product on up to eight waves a block would take
+    for T x N x K, or None where that kernel does not take the product (PLAN_ROTATING: never).  It has what `quad_plan`'s kernel does
+    not take, or what does not start at 16 bytes.  Runs nothing and needs no GPU."""
     import ctypes
     plan = (ctypes.c_int * 4)()
-    if library().sp_pipe_plan(kind, T, N, K, hd, plan):
+    if library().sp_pipe_plan(kind, T, N, K, plan):
         return None
     return tuple(plan)
 
@@ -912,7 +912,8 @@ def qkv_rope_cache(w: torch.Tensor, bias, q_out: torch.Tensor, positions, inv_fr
 
     Activations are x (bfloat16) or rmsnorm(residual) * norm_weight computed inside the kernel.
     `table`: `rope_table` of these positions (float32 [T, hd / 2, 2]), which the many-token kernel reads
-    instead of computing sines and cosines."""
+    instead of computing sines and cosines.  That kernel wants x, w, q_out and k_pool to start at multiples of 16 bytes; where
+    one does not, the product and the rotation are kernels of their own."""
     _gpu(w, "qkv weight"); _gpu(q_out, "q output")
     N, K = w.shape
     xp, rp, nd, npt, T = _activations(x, residual, norm_weight, K, "qkv_rope_cache")
@@ -928,6 +929,15 @@ def qkv_rope_cache(w: torch.Tensor, bias, q_out: torch.Tensor, positions, inv_fr
         _gpu(table, "rotation table")
         if table.dtype != torch.float32 or tuple(table.shape) != (T, hd // 2, 2) or rotary_dim != hd:
             raise KernelError(f"qkv_rope_cache: the rotation table must be float32 [{T}, {hd // 2}, 2]")
+        if table.data_ptr() % 16:
+            table = table.clone()
+    if (T > 64 and any(p is not None and p.data_ptr() % 16 for p in (x, w, q_out, k_pool))
+            and fused_supported(FUSED_ROPE, T, N, K, hd, rotary_dim, residual is not None, variant=pairing)):
+        qkv = torch.empty(T, N, dtype=torch.bfloat16, device=w.device)
+        gemm(x, w, qkv, bias=bias)
+        rope_cache(qkv, positions, inv_freq, rotary_dim, nq, nkv, hd, slot_mapping, k_pool, v_pool, pairing=pairing)
+        q_out.copy_(qkv[:, :nq * hd])
+        return
     check(library().sp_qkv_rope_cache(_stream(), xp, rp, nd, npt, float(eps), w.data_ptr(),
                                       _code(bias, "bias") if bias is not None else 0, _ptr(bias), q_out.data_ptr(),
                                       positions.data_ptr(), inv_freq.data_ptr(), rotary_dim, slot_mapping.data_ptr(),

@@ -108,3 +108,36 @@ def test_outputs_that_do_not_start_at_sixteen_bytes():
     room32 = torch.zeros(200 * 264 + 2, device=DEV)
     ops.gemm(x, w, room32[2:].view(200, 264), accumulate=True)
     assert (room32[2:].view(200, 264) - want).abs().max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("shifted", ["x", "w", "q_out", "k_pool", "v_pool", "table"])
+@pytest.mark.parametrize("T,nq,nkv,hd,K", [(65, 2, 1, 64, 64), (512, 14, 2, 64, 896), (300, 28, 4, 128, 448)])
+def test_rotating_with_operands_that_do_not_start_at_sixteen_bytes(T, nq, nkv, hd, K, shifted):
+    """A caller that asks whether the product, the rotation and the cache write are one call asks by sizes alone; the call is taken
+    wherever its operands start, with the result of aligned ones: to the bit where the same kernel runs, else within the roundings
+    of the projections and the results to bfloat16."""
+    from sprout_lm_amd import ops
+    N, page, pages = (nq + 2 * nkv) * hd, 16, 40
+    assert ops.fused_supported(ops.FUSED_ROPE, T, N, K, hd, hd, False, variant="halves")
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    x, w, bias, _ = _operands(T, N, K)
+    positions = torch.randint(0, 5000, (T,), device=DEV, generator=gen, dtype=torch.int32)
+    slots = torch.randperm(page * pages, device=DEV, generator=gen)[:T].int()
+    inv_freq = 1e4 ** (-torch.arange(hd // 2, device=DEV).float() / (hd // 2))
+    table = torch.empty(T, hd // 2, 2, device=DEV)
+    ops.rope_table(positions, inv_freq, table)
+
+    def run(moved):
+        place = lambda name, v: torch.empty(v.numel() + 4, dtype=v.dtype, device=DEV)[(8 // v.element_size() if name == moved else 0):][:v.numel()].view(v.shape).copy_(v)
+        q_out, k, v = (torch.zeros(*shape, dtype=torch.bfloat16, device=DEV) for shape in ((T, nq * hd), (pages, nkv, page, hd), (pages, nkv, hd, page)))
+        args = {name: place(name, v) for name, v in dict(x=x, w=w, q_out=q_out, k_pool=k, v_pool=v, table=table).items()}
+        assert moved is None or args[moved].data_ptr() % 16 == 8
+        ops.qkv_rope_cache(args["w"], bias, args["q_out"], positions, inv_freq, hd, slots, args["k_pool"], args["v_pool"], nq, nkv, hd,
+                           x=args["x"], table=args["table"])
+        return args["q_out"], args["k_pool"], args["v_pool"]
+
+    for got, want in zip(run(shifted), run(None)):
+        if shifted in ("v_pool", "table"):
+            assert torch.equal(got, want)
+        else:
+            assert (got.float() - want.float()).abs().max().item() <= 2 ** -7 * (1 + want.float().abs().max().item())

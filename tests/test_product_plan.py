@@ -19,7 +19,6 @@ def built_library():
 
 SHAPES = {(256, 256), (256, 128), (128, 128), (64, 64), (64, 256), (64, 128), (384, 256), (256, 160)}
 PAIRED = {(256, 256), (256, 128), (128, 128), (64, 256), (64, 128), (384, 256)}    # an even number of tile columns a wave
-ROTATING = {(256, 128), (128, 128), (64, 128)}
 
 
 def sizes():
@@ -54,19 +53,11 @@ def test_products_the_kernel_does_not_take():
     assert ops.pipe_plan(ops.PLAN_STORE, 300, 100, 70) is None          # K is no multiple of 64
     assert ops.pipe_plan(ops.PLAN_STORE, 300, 100, 0) is None
     assert ops.pipe_plan(7, 300, 128, 128) is None
-    assert ops.pipe_plan(ops.PLAN_ROTATING, 64, 1152, 896, 64) is None  # up to 64 tokens: the decode kernels rotate
-    assert ops.pipe_plan(ops.PLAN_ROTATING, 300, 18 * 48, 896, 48) is None   # head sizes that are no multiple of 64
-
-
-def test_rotating_epilogue_shapes():
-    for T, (nq, nkv, hd, K) in itertools.product([65, 128, 256, 264, 512, 1024, 2048, 4096],
-                                                  [(14, 2, 64, 896), (28, 4, 128, 3584), (40, 8, 128, 5120), (4, 4, 128, 256)]):
-        plan = ops.pipe_plan(ops.PLAN_ROTATING, T, (nq + 2 * nkv) * hd, K, hd)
-        assert plan is None or (plan[:2] in ROTATING and plan[2] == 1 and plan[3] in (4, 8)), (T, nq, nkv, hd, K, plan)
+    assert ops.pipe_plan(ops.PLAN_ROTATING, 300, 1152, 896) is None     # the four-wave product rotates, and the decode kernels
 
 
 def test_decisions_that_measurements_settled():
-    """(kind, T, N, K[, hd]) -> plan: each of these was timed against the other shapes with operands from memory."""
+    """(kind, T, N, K) -> plan: each of these was timed against the other shapes with operands from memory."""
     settled = {
         (ops.PLAN_STORE, 2048, 37888, 3584): (256, 256, 1),       # fills the chip: the largest blocks
         (ops.PLAN_STORE, 2048, 4608, 3584): (256, 160, 1),        # 232 blocks where 256 x 256 make 144
@@ -76,13 +67,6 @@ def test_decisions_that_measurements_settled():
         (ops.PLAN_ACCUMULATE, 2048, 896, 896): (64, 64, 1),
         (ops.PLAN_GATED, 2048, 9728, 896): (384, 256, 1),
         (ops.PLAN_GATED, 256, 9728, 896): (128, 128, 1),
-        (ops.PLAN_ROTATING, 2048, 1152, 896, 64): (128, 128, 1),
-        (ops.PLAN_ROTATING, 1024, 1152, 896, 64): (64, 128, 1),
-        (ops.PLAN_ROTATING, 512, 1152, 896, 64): None,            # 64 x 64 and a rotation kernel after it
-        (ops.PLAN_ROTATING, 2048, 4608, 3584, 128): None,         # 256 x 160 and a rotation kernel after it
-        (ops.PLAN_ROTATING, 1024, 4608, 3584, 128): (256, 128, 1),
-        (ops.PLAN_ROTATING, 512, 4608, 3584, 128): (128, 128, 1),
-        (ops.PLAN_ROTATING, 256, 4608, 3584, 128): (64, 128, 1),
     }
     for args, want in settled.items():
         got = ops.pipe_plan(*args)
@@ -91,7 +75,7 @@ def test_decisions_that_measurements_settled():
 
 def test_kernel_tests_reach_every_block_shape():
     """The sizes that tests/test_gpu_kernels.py runs on the GPU, asked here for their plans: every block shape of the
-    plain, the gated and the rotating product is reached by at least one of them."""
+    plain and the gated product is reached by at least one of them."""
     import importlib
     kernels = importlib.import_module("tests.test_gpu_kernels")
     plain = {(rows, cols, waves, split) for rows, cols, waves, split in kernels.BLOCK_SHAPE_SIZES.values()}
@@ -99,12 +83,6 @@ def test_kernel_tests_reach_every_block_shape():
     for (accumulate, T, N, K), (rows, cols, waves, split) in kernels.BLOCK_SHAPE_SIZES.items():
         got = ops.pipe_plan(ops.PLAN_ACCUMULATE if accumulate else ops.PLAN_STORE, T, N, K)
         assert (got[0], got[1], got[3], got[2] > 1) == (rows, cols, waves, split), (T, N, K, got)
-    rotating = set()
-    for (T, nq, nkv, hd, K), shape in kernels.ROTATING_SHAPE_SIZES.items():
-        got = ops.pipe_plan(ops.PLAN_ROTATING, T, (nq + 2 * nkv) * hd, K, hd)
-        assert (got[0], got[1], got[3]) == shape, (T, nq, nkv, hd, K, got)
-        rotating.add(shape[:2])
-    assert rotating == ROTATING
     marks = [m for m in kernels.test_fused_gate_up_silu_and_normed_product.pytestmark
              if m.name == "parametrize" and m.args[0] == "T,I,K"]
     gated = {ops.pipe_plan(ops.PLAN_GATED, T, 2 * I, K)[:2] for T, I, K in marks[0].args[1] if T > 64 and K % 64 == 0}

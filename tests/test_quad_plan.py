@@ -69,6 +69,8 @@ def test_rotation_takes_heads_of_whole_sixty_fours():
         plan = ops.quad_plan(ops.PLAN_ROTATING, T, (nq + 2 * nkv) * hd, K, hd)
         assert (plan is None) == (T <= 64 or hd % 64 != 0), (T, nq, nkv, hd, K, plan)
         assert plan is None or (plan[:2] + plan[3:] in SHAPES and plan[1] != 192 and plan[2] == 1)
+        # a caller asks the library once for the folded call, by sizes
+        assert T <= 64 or ops.fused_supported(ops.FUSED_ROPE, T, (nq + 2 * nkv) * hd, K, hd, hd) == (plan is not None)
 
 
 def test_kernel_tests_reach_every_block_shape():
