@@ -64,6 +64,14 @@ def test_few_tokens_are_taken_where_measurements_say_so():
     assert taken(ops.PLAN_STORE, 17, 4608, 3584) and not taken(ops.PLAN_STORE, 32, 7168, 5120) and taken(ops.PLAN_STORE, 33, 7168, 5120)
 
 
+def test_outputs_of_few_columns_are_cut_rather_than_read_by_every_xcd():
+    """With less than 8 weight tiles an XCD reads its run of the tokens alone: 512 rows of w on blocks of 128 columns and in two parts
+    of K (48 us at 4,096 tokens, K = 8,192; 128 x 64 in one part, which every XCD reads all tokens for, 80)."""
+    for T, K, most in [(2048, 8192, 4), (3000, 4864, 3), (4096, 4864, 2), (4096, 8192, 2)]:
+        rows, cols, splits, _ = ops.quad_plan(ops.PLAN_ACCUMULATE, T, 512, K)
+        assert cols == 128 and 2 <= splits <= most, (T, K, rows, cols, splits)
+
+
 def test_rotation_takes_heads_of_whole_sixty_fours():
     for T, (nq, nkv, hd, K) in itertools.product([64, 65, 264, 2048], [(14, 2, 64, 896), (28, 4, 128, 3584), (3, 1, 48, 896), (2, 2, 192, 64)]):
         plan = ops.quad_plan(ops.PLAN_ROTATING, T, (nq + 2 * nkv) * hd, K, hd)
