@@ -5,20 +5,24 @@
 
 namespace sprout {
 
-// 17 to 64 tokens, where the weights are read from memory once and the other kernels do that as well: microseconds there -> here, a launch of a
-// captured graph with weights from memory, at 17, 32 (33) and 64 tokens.  Gated: 9,728 rows of 896 8.0 -> 6.8, 8.0 -> 6.9, 8.4 -> 7.6; 17,920 of
-// 1,536 17.2 -> 16.8, 17.9 -> 17.5, 21.0 -> 19.8; 37,888 of 3,584 54 -> 55, 55 -> 56, 59 -> 63.  Added: 896 of 896 3.5 -> 4.0, 4.1 -> 4.4, 4.0 -> 4.5;
-// 896 of 4,864 4.7 -> 4.8, 6.0 -> 5.4, 7.3 -> 6.0; 3,584 of 3,584 8.1 -> 6.7, 9.0 -> 7.5, 9.6 -> 8.6; 5,120 of 5,120 15.6 -> 12.7, 18.1 -> 13.5, 20.2 ->
-// 15.2; 3,584 of 18,944 25.8 -> 27.6, 26.9 -> 27.1, 30.0 -> 30.6.  Stored: 1,152 of 896 5.1 -> 5.8, 5.8 -> 5.8, 5.8 -> 5.9; 2,048 of 1,536 7.3 -> 8.0, 8.3 ->
-// 7.9, 11.3 -> 7.9; 4,608 of 3,584 15.1 -> 14.9, 20.9 -> 15.7, 22.6 -> 18.4; 7,168 of 5,120 22.6 -> 24.4, 24.1 -> 26.5, 33.4 -> 31.9; 151,936 of 896
-// 59.3 -> 55.3, 63.0 -> 61.0, 72.4 -> 70.8; 152,064 of 3,584 204 -> 195, 211 -> 209, 224 -> 235.
+// 17 to 64 tokens, where the weights are read from memory once and the other kernels do that as well.  Both were timed at ten numbers of
+// tokens from 17 to 64 on 325 matrices (a launch of a captured graph, weights from memory).  Time here over time there, on either side of
+// each line: mean, and the least and the most of the side that is taken.
+//   gated, up to 16,384 rows: below 64 M weights 0.76 (0.58 .. 0.96), above 0.99; more rows: K up to 1,536 0.96 (0.87 .. 1.04; beyond
+//     24,576 rows and 40 tokens 0.99), K above 1.07;
+//   added, 33 tokens and more: 4 to 64 M weights 0.85 (0.67 .. 1.08; the first 4 M of them 0.84), 2 to 4 M 0.94, more than 64 M 0.95 with
+//     1.15 among them; up to 32 tokens: from 6 M weights on, where the other kernel is the eight-wave one, 0.87 (0.67 .. 1.06; to 12 M
+//     0.83), 3 to 6 M 1.02;
+//   stored, 33 tokens and more: from 2 M weights on 0.70 (0.39 .. 0.94; to 4 M 0.76), less 1.00; up to 32 tokens: 8,192 rows and more,
+//     or 6,144 with K up to 4,096, from 8 M weights on 0.78 (0.53 .. 1.04), others 1.02 with 1.16 among them; heads of 32,768 rows and more:
+//     K up to 2,048 0.91 (0.82 .. 0.99), 2,560 to 3,584 1.02 with 1.19 among them.
 static bool quad_pays_for_few(int kind, int T, int N, int K) {
   const size_t weights = size_t(N) * K, million = 1000000;
-  if (kind == kQuadGated) return weights >= 8 * million && weights < 64 * million;
-  if (kind == kQuadAccumulate) return weights >= (T > 32 ? 4 : 12) * million && weights < 64 * million;
+  if (kind == kQuadGated) return N <= 16384 ? weights < 64 * million : K <= 1536 && (N <= 24576 || T <= 40);
+  if (kind == kQuadAccumulate) return weights >= (T > 32 ? 4 * million : size_t(6) << 20) && weights < 64 * million;
   if (kind != kQuadStore) return false;
-  if (N >= 32768) return K <= 1024;
-  return T > 32 ? weights >= 2 * million && weights < 64 * million : weights >= 8 * million && weights < 32 * million;
+  if (N >= 32768) return K <= 2048;
+  return T > 32 ? weights >= 2 * million : weights >= 8 * million && (N >= 8192 || (N >= 6144 && K <= 4096));
 }
 
 bool gemm_quad_takes(int kind, int T, int N, int K, int hd) {

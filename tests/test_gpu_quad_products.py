@@ -12,7 +12,7 @@ STORE, ACCUMULATE, GATED = 0, 1, 2          # the kinds of sp_quad_plan
 _STORED = [(65, 8, 64), (65, 72, 128), (66, 264, 192), (97, 131 * 8, 256), (65, 20000, 64), (65, 13608, 1920), (193, 26664, 64), (97, 26664, 192),
            (193, 20000, 1920), (321, 20000, 1920), (777, 9736, 64), (777, 20000, 896), (130, 20000, 1920), (513, 13608, 192), (513, 20000, 384),
            (193, 26664, 1920), (2047, 4904, 384), (641, 20000, 896), (1300, 9736, 576), (289, 26664, 192)]
-_STORED_FEW = [(17, 4608, 3584), (33, 2056, 1536), (64, 40000, 896), (45, 4104, 896)]
+_STORED_FEW = [(17, 6152, 2048), (33, 2056, 1536), (64, 40000, 896), (45, 4104, 896)]
 # a split of K in two and more on every shape but the largest
 _SPLIT = [(65, 8, 576), (65, 9736, 1920), (65, 4904, 4864), (97, 9736, 3584), (193, 9736, 4864), (130, 20000, 3584), (777, 4904, 4864),
           (130, 9736, 4864), (161, 20000, 4864), (257, 13608, 4864), (17, 3592, 3584), (45, 904, 4864), (64, 2568, 5120),

@@ -61,7 +61,15 @@ def test_few_tokens_are_taken_where_measurements_say_so():
     assert taken(ops.PLAN_ACCUMULATE, 45, 896, 4864) and not taken(ops.PLAN_ACCUMULATE, 24, 896, 4864)
     assert taken(ops.PLAN_ACCUMULATE, 17, 3584, 3584) and not taken(ops.PLAN_ACCUMULATE, 64, 896, 896)
     assert taken(ops.PLAN_STORE, 17, 151936, 896) and not taken(ops.PLAN_STORE, 64, 152064, 3584)
-    assert taken(ops.PLAN_STORE, 17, 4608, 3584) and not taken(ops.PLAN_STORE, 32, 7168, 5120) and taken(ops.PLAN_STORE, 33, 7168, 5120)
+    assert not taken(ops.PLAN_STORE, 32, 7168, 5120) and taken(ops.PLAN_STORE, 33, 7168, 5120)
+    # on either side of lines that are no preset's: gated products of many rows and a long K are 7 to 33 % longer on four waves
+    for T in (17, 33, 64):
+        assert not any(taken(ops.PLAN_GATED, T, n, k) for n in (18432, 22528, 28672) for k in (2048, 2560, 3072))
+        assert all(taken(ops.PLAN_GATED, T, n, k) for n in (2048, 8192, 16384) for k in (512, 2048, 3072))
+    assert taken(ops.PLAN_GATED, 40, 28672, 1024) and not taken(ops.PLAN_GATED, 48, 28672, 1024)
+    # stored products of up to 32 tokens and few rows are 2 to 16 % longer there
+    assert not any(taken(ops.PLAN_STORE, 24, n, k) for n in (1152, 3072, 4608) for k in (2048, 4096, 5120))
+    assert taken(ops.PLAN_STORE, 24, 6144, 4096) and taken(ops.PLAN_STORE, 24, 8192, 5120) and taken(ops.PLAN_STORE, 48, 12288, 8192)
 
 
 def test_outputs_of_few_columns_are_cut_rather_than_read_by_every_xcd():
