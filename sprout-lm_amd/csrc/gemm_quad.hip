@@ -47,11 +47,11 @@ static const float kAloneUs[] = {0.24f, 0.45f, 0.35f, 0.50f, 0.48f, 0.68f, 0.80f
 
 // The estimate: rounds of blocks on the XCD that holds the most (blocks are numbered as pipe_tiles says), a block being its steps
 // (longer by 7 % each beyond 20 where two blocks share a CU) and its two ends; a last round that does not fill the chip runs
-// somewhat faster, fewer blocks share the caches.  Memory: the weights once at 5.4 TB/s and, at 9 TB/s together, the tokens once an
+// somewhat faster, fewer blocks share the caches.  Memory: the weights once at 5.4 TB/s and, at 9 TB/s together (8 with two buffers of x), the tokens once an
 // XCD, or, where there are less than 8 weight tiles and an XCD has a run of their blocks, once a weight tile; it adds to the blocks'
 // time where both are alike (fourth powers).  A split's float atomics cost 1.9 us a million, the sums read and written without a split
-// 1.4.  Over 1,100 products (65 to 8,192 tokens, 512 to 6,144 weight rows, K of 896 to 18,944) the choice takes 1.4 % longer than the best
-// of all shapes and splits (mean; 25 % at worst), 10 % less than the eight-wave kernel, and more than 3 % longer than that one on 24 (10 %
+// 1.4.  Over 1,100 products (65 to 8,192 tokens, 512 to 6,144 weight rows, K of 896 to 18,944) the choice takes 1.3 % longer than the best
+// of all shapes and splits (mean; 25 % at worst), 10 % less than the eight-wave kernel, and more than 3 % longer than that one on 18 (10 %
 // at worst).  (With the tokens read once an XCD whatever the weight tiles: 4,096 tokens by 512 rows of 8,192 in one part on 128 x 64, 80 us,
 // where 128 x 128 in two takes 48 and the eight-wave kernel 50.)
 void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
@@ -65,7 +65,7 @@ void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
     if (kind == kQuadRotating && p.wn != 2 && p.wn % 4 != 0) continue;     // a lane holds both of a pair
     const int bm = 32 * p.wm, bn = 32 * p.wn, slots = 32 * p.per_cu;
     const PipeTiles tiles = pipe_tiles((T + bm - 1) / bm, (N + bn - 1) / bn);
-    const float memory = float(N) * float(K) * 2.f / 5.4e6f + float(tiles.full ? 8 : tiles.left) * 2.f * float(T) * float(K) / 9e6f;
+    const float memory = float(N) * float(K) * 2.f / 5.4e6f + float(tiles.full ? 8 : tiles.left) * 2.f * float(T) * float(K) / (p.buffers == 2 ? 8e6f : 9e6f);
     const float memory2 = memory * memory;
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (sp > 1 && (!cuts_k || steps / sp < 4)) break;
