@@ -54,17 +54,18 @@ def test_gemm_all_modes_odd_sizes(T, N, K, dtype):
     assert np.abs(acc.cpu().numpy() - (base + want)).max() <= 1e-5 * max(1, math.sqrt(K) / 8) * (1 + np.abs(want).max())
 
 
-# One product for every block shape of the tiled kernel, whole and with K split: (accumulate, T, N, K) -> (block rows,
+# One product for every block shape of the tiled kernel on up to eight waves, whole and with K split: (accumulate, T, N, K) -> (block rows,
 # block columns, waves, K split?).  The plan is asserted, so that a change of the cost model that moves a size to
-# another shape says so here instead of leaving a shape without a test.
+# another shape says so here instead of leaving a shape without a test; rows in whole eights are the four-wave kernel's
+# (tests/test_gpu_quad_products.py), so there are none here.
 BLOCK_SHAPE_SIZES = {
     (0, 65, 130, 64): (64, 64, 4, False), (1, 260, 130, 3584): (64, 64, 4, True),
-    (0, 130, 13400, 64): (64, 128, 4, False), (1, 260, 2000, 18944): (64, 128, 4, True),
-    (0, 264, 7000, 64): (128, 128, 8, False), (1, 65, 4608, 3584): (128, 128, 8, True),
-    (0, 1024, 4608, 448): (256, 128, 8, False), (1, 200, 2570, 18944): (256, 128, 8, True),
+    (0, 130, 13404, 64): (64, 128, 4, False), (1, 260, 2004, 18944): (64, 128, 4, True),
+    (0, 264, 7004, 64): (128, 128, 8, False), (1, 65, 4612, 3584): (128, 128, 8, True),
+    (0, 1024, 4612, 448): (256, 128, 8, False), (1, 200, 2570, 18944): (256, 128, 8, True),
     (0, 2056, 3590, 1088): (256, 160, 4, False), (1, 4104, 900, 9728): (256, 160, 4, True),
-    (0, 513, 13400, 64): (256, 256, 8, False), (1, 1034, 4030, 9728): (256, 256, 8, True),
-    (0, 1100, 13400, 64): (384, 256, 8, False), (1, 260, 13400, 9728): (384, 256, 8, True),
+    (0, 513, 13404, 64): (256, 256, 8, False), (1, 1034, 4030, 9728): (256, 256, 8, True),
+    (0, 1100, 13404, 64): (384, 256, 8, False), (1, 260, 13404, 9728): (384, 256, 8, True),
 }
 
 
@@ -72,8 +73,10 @@ BLOCK_SHAPE_SIZES = {
 def test_tiled_product_on_every_block_shape(case):
     from sprout_lm_amd import ops
     accumulate, T, N, K = case
-    rows, cols, splits, waves = ops.pipe_plan(ops.PLAN_ACCUMULATE if accumulate else ops.PLAN_STORE, T, N, K)
+    kind = ops.PLAN_ACCUMULATE if accumulate else ops.PLAN_STORE
+    rows, cols, splits, waves = ops.pipe_plan(kind, T, N, K)
     assert (rows, cols, waves, splits > 1) == BLOCK_SHAPE_SIZES[case], "this size has moved to another block shape"
+    assert ops.quad_plan(kind, T, N, K) is None, "this size is another kernel's"
     gen = torch.Generator(device=DEV).manual_seed(T + N)
     x = torch.randn(T, K, device=DEV, generator=gen).to(torch.bfloat16)
     w = (torch.randn(N, K, device=DEV, generator=gen) * K ** -0.5).to(torch.bfloat16)
@@ -724,11 +727,16 @@ def check_fused_qkv_rope_cache(T, nq, nkv, hd, K, page, norm):
         assert np.array_equal(kp2.float().cpu().numpy(), kp) and np.array_equal(vp2.float().cpu().numpy().transpose(0, 1, 3, 2), vp)
 
 
+# The gated product on every block shape of the kernel on up to eight waves, which has what is no whole eights: blocks of 384 x 256 for
+# many tokens, 64 x 128, 128 x 128, 256 x 128, 256 x 256, one of 384 x 256 for all tokens
+EIGHT_WAVE_GATED_SIZES = [(1100, 6700, 128), (130, 9476, 448), (200, 1004, 3584), (513, 4868, 896), (513, 18948, 896), (264, 18948, 448)]
+
+
 @pytest.mark.parametrize("T,I,K", [(t_, i_, k_) for t_ in [1, 8, 16, 33, 64, 65, 200, 513]
                                    for i_, k_ in [(4864, 896), (224, 96), (176, 240), (1000, 264), (331, 72), (160, 2312)]]
-                         + [(1100, 6700, 128), (2048, 4864, 896),   # blocks of 384 tokens
-                            (1024, 2432, 264), (200, 1000, 3584),   # blocks of 256 x 128 and 128 x 128 on eight waves
-                            (513, 18944, 896), (130, 9472, 448), (264, 18944, 448)])  # blocks of 256 x 256, of 64 x 128, one of 384
+                         # K in no whole steps, and on four waves a block
+                         + [(1024, 2432, 264), (2048, 4864, 896), (200, 1000, 3584), (513, 18944, 896), (130, 9472, 448), (264, 18944, 448)]
+                         + EIGHT_WAVE_GATED_SIZES)
 @pytest.mark.parametrize("norm", [False, True])
 def test_fused_gate_up_silu_and_normed_product(T, I, K, norm):
     from sprout_lm_amd import ops

@@ -62,14 +62,17 @@ def test_square_of_relu_feed_forward(dtype, T, hidden, inner):
 
 
 @pytest.mark.parametrize("T", [1, 16, 17, 64, 65, 300])
-@pytest.mark.parametrize("split,second,K,bias", [(0, 64, 64, False), (40, 96, 128, True), (136, 24, 192, False), (256, 260, 64, True)])
+@pytest.mark.parametrize("split,second,K,bias", [(0, 64, 64, False), (40, 96, 128, True), (136, 24, 192, False), (256, 260, 64, True),
+                                                 (44, 84, 128, True), (4, 60, 64, False), (132, 132, 192, True)])
 def test_two_products_of_one_input(T, split, second, K, bias):
-    """Rows of one matrix that go to two tensors, the second activated and between other columns, for few and many tokens."""
+    """Rows of one matrix that go to two tensors, the second activated and between other columns, for few and many tokens; a seam
+    in the middle of eight, and a first tensor that starts at 8 bytes."""
     from sprout_lm_amd import ops
     rng = np.random.default_rng(T + split)
     x, w = (rounded(rng.standard_normal(shape), torch.bfloat16) for shape in ((T, K), (split + second, K)))
     b = rng.standard_normal(split + second).astype(np.float32) if bias else None
-    out = torch.full((T, max(split, 4)), 7.0, dtype=torch.bfloat16, device=DEV)
+    room = torch.full((T * max(split, 4) + 4,), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = room[4 if split % 8 else 0:][:T * max(split, 4)].view(T, -1)
     rows = torch.full((T, second + 12), 7.0, dtype=torch.bfloat16, device=DEV)
     ops.gemm_joined(dev(x, torch.bfloat16), dev(w, torch.bfloat16), None if b is None else dev(b), out if split else None, split, rows, 8,
                     "relu_squared")

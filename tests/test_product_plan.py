@@ -1,5 +1,6 @@
-"""The tiled product's choice of block shape and split, asked of the library without running a kernel (no GPU):
-invariants over a sweep of sizes, and the decisions that measurements on the GPU settled."""
+"""The choice of block shape and split of the tiled product on up to eight waves a block, asked of the library without running a
+kernel (no GPU): invariants over a sweep of sizes, and the decisions that measurements on the GPU settled.  Where results are whole
+eights that start at 16 bytes another kernel has these products (tests/test_quad_plan.py)."""
 import itertools
 
 import pytest
@@ -57,7 +58,8 @@ def test_products_the_kernel_does_not_take():
 
 
 def test_decisions_that_measurements_settled():
-    """(kind, T, N, K) -> plan: each of these was timed against the other shapes with operands from memory."""
+    """(kind, T, N, K) -> plan: each of these was timed against the other shapes with operands from memory.  They hold where a
+    result does not start at 16 bytes, and at sizes beside these that are no whole eights."""
     settled = {
         (ops.PLAN_STORE, 2048, 37888, 3584): (256, 256, 1),       # fills the chip: the largest blocks
         (ops.PLAN_STORE, 2048, 4608, 3584): (256, 160, 1),        # 232 blocks where 256 x 256 make 144
@@ -81,12 +83,13 @@ def test_kernel_tests_reach_every_block_shape():
     plain = {(rows, cols, waves, split) for rows, cols, waves, split in kernels.BLOCK_SHAPE_SIZES.values()}
     assert {(r, c) for r, c, _, _ in plain} == SHAPES - {(64, 256)} and {s for _, _, _, s in plain} == {False, True}
     for (accumulate, T, N, K), (rows, cols, waves, split) in kernels.BLOCK_SHAPE_SIZES.items():
-        got = ops.pipe_plan(ops.PLAN_ACCUMULATE if accumulate else ops.PLAN_STORE, T, N, K)
+        kind = ops.PLAN_ACCUMULATE if accumulate else ops.PLAN_STORE
+        got = ops.pipe_plan(kind, T, N, K)
         assert (got[0], got[1], got[3], got[2] > 1) == (rows, cols, waves, split), (T, N, K, got)
-    marks = [m for m in kernels.test_fused_gate_up_silu_and_normed_product.pytestmark
-             if m.name == "parametrize" and m.args[0] == "T,I,K"]
-    gated = {ops.pipe_plan(ops.PLAN_GATED, T, 2 * I, K)[:2] for T, I, K in marks[0].args[1] if T > 64 and K % 64 == 0}
-    assert gated >= {(64, 128), (128, 128), (256, 128), (256, 256), (384, 256)}, gated
+        assert ops.quad_plan(kind, T, N, K) is None, (T, N, K)          # it is this kernel that runs
+    assert all(ops.quad_plan(ops.PLAN_GATED, T, 2 * I, K) is None for T, I, K in kernels.EIGHT_WAVE_GATED_SIZES)
+    gated = {ops.pipe_plan(ops.PLAN_GATED, T, 2 * I, K)[:2] for T, I, K in kernels.EIGHT_WAVE_GATED_SIZES}
+    assert gated == {(64, 128), (128, 128), (256, 128), (256, 256), (384, 256)}, gated
 
 
 def test_blocks_are_numbered_so_that_every_tile_runs_once_and_the_xcds_share_them():
