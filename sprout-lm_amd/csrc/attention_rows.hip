@@ -10,7 +10,7 @@
 // an exponential at 9 cycles, a sum, half a maximum and half a conversion a score); two waves on a SIMD overlap in part.  A stage's
 // loads ask for little beside: a page's place in the pools is in LDS as it is added, and a lane's share of it is its own for the whole walk
 // (with every place worked out from its key 130 vector instructions a stage, 8 % more time).  14 heads of 64 in 2 groups, 2,048 queries over
-// 32,768 keys: 511 -> 280 us (830 TFLOP/s) with four parts of the keys, and 8 for their merge; over 8,192: 137 -> 92 + 8; two prompts of
+// 32,768 keys: 511 -> 298 us (780 TFLOP/s; 292 on another machine) with four parts of the keys, and 8 for their merge; over 8,192: 137 -> 92 + 8; two prompts of
 // 2,048: 80 -> 52.
 // (One head's weights between the other's products, in one wave: the matrix cores and the vector unit then overlap within a wave too,
 // but the launch takes 5 % longer; four waves a CU with all registers to themselves: 450 us, the vector unit takes 2.7 cycles an

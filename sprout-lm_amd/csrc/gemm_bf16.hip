@@ -194,8 +194,8 @@ int gemm_bf16(hipStream_t s, const void* a, const void* w, int bias_dtype, const
       return gemm_bf16_pipe(s, a, w, bias_dtype, bias, mode, out, T, N, K);
     if ((N + 15) / 16 < 2048) return gemm_decode_plain(s, a, w, bias_dtype, bias, mode, out, T, N, K);
     // Very wide (the output head): rows streamed per wave up to 16 tokens; with more, the streaming kernel stops
-    // for every chunk of activations it stages, and the pipelined tiles are faster (151,936 x 896 at 64 tokens:
-    // 98 against 126 us, 152,064 x 3,584: 263 against 409; the same at 16 tokens and fewer).
+    // for every chunk of activations it stages, and the pipelined tiles are faster (152,064 x 3,584 at 64 tokens:
+    // 263 against 409 us; the same at 16 tokens and fewer).  Heads of K up to 2,048 do not come here.
     if (T > 16 && gemm_pipe_takes(T, N, K)) return gemm_bf16_pipe(s, a, w, bias_dtype, bias, mode, out, T, N, K);
     if (bias && bias_dtype == kBF16) return skinny_shape<bf16_t>(s, a, w, bias, mode, out, T, N, K);
     return skinny_shape<float>(s, a, w, bias, mode, out, T, N, K);

@@ -42,9 +42,9 @@ __device__ __forceinline__ void wait_loads_then_barrier() {
 
 // How the tiles of a product are numbered over the blocks of a launch (the kernel and its launch agree on it):
 // every XCD has `own` blocks for the weight tiles that are its own (`full` of them, token tiles in groups of `group`, the
-// last what is left), then `run` blocks of the `left` weight tiles that are dealt out.  No block among them is without a tile:
-// one that ends at once does not make its place free for the next, which may wait for a whole round (2,048 tokens, 3,584
-// rows of 3,584 on 160 x 192, 31 tiles and 6 such blocks on an XCD of 32 CUs: 97 us, without them 63).
+// last what is left), then `run` blocks of the `left` weight tiles that are dealt out, at most 7 of them in all without a tile.  No `own`
+// block is without one: a block that ends at once does not make its place free for the next, which may wait for a whole round (2,048
+// tokens, 3,584 rows of 3,584 on 160 x 192, 31 tiles and 6 such blocks on an XCD of 32 CUs: 97 us, without them 58).
 struct PipeTiles { int tiles_t, full, left, group, own, run; };
 __host__ __device__ inline PipeTiles pipe_tiles(int tiles_t, int tiles_n) {
   PipeTiles p;

@@ -1,7 +1,11 @@
 // The plain modes of the pipelined tiled product (store, accumulate, store float32), its shapes and the choice
 // between them.  The kernel itself is in gemm_pipe.h; the products with a bfloat16 bias are instantiated in
-// gemm_pipe_bias16.hip, the gated and the rotating epilogue in gemm_pipe_epilogues.hip, so that the parts compile
+// gemm_pipe_bias16.hip, the gated epilogue in gemm_pipe_epilogues.hip, so that the parts compile
 // side by side.
+//
+// Products of more than 64 tokens whose results are whole eights that start at 16 bytes are the four-wave kernel's (gemm_quad.h), and of
+// those of 17 to 64 tokens many (quad_pays_for_few): here are the others, among them everything of 16 tokens and fewer that is tiled.  The
+// times below compare this kernel's shapes with one another, at whatever size they were measured.
 #include "gemm_pipe.h"
 
 namespace sprout {
