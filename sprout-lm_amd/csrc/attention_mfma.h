@@ -449,34 +449,42 @@ constexpr int kStageKeys = 128;
 __device__ __forceinline__ constexpr int step_row(int r) { return (r & ~31) | ((r & 4) << 2) | (((r & 31) >> 3) << 2) | (r & 3); }
 constexpr int kMaxTableLds = 2048;    // page numbers held in LDS; longer tables are read from memory
 
-template <int DT, int NQT, int HPB, int WPT, bool AHEAD, bool PAIRED, bool SIG>
-__global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kernel(
-    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
-    const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
-    const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len,
-    const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages,
-    ScoreStage st, float scale2, int n_tiles) {
-  constexpr int HD = 16 * DT, HC = (DT + 1) / 2;
-  constexpr int THREADS = 64 * WPT * HPB;
-  constexpr int WAVE_KEYS = kStageKeys / WPT;          // keys of a stage that one wave of a team takes
+template <int DT, int NQT, int WPT>
+struct StagedLds {
   // Key row pitch in LDS (elements).  A 16-byte LDS read serves lanes {0-3, 12-15, 20-27} of each half-wave in
   // one pass and the other 16 in a second (measured with two lanes at a time on one bank), not 16 lanes in a
   // row: with 16 bytes of padding the rows of those lanes met two to a bank (8 cycles an instruction instead
   // of 4); 32 bytes of padding keep them apart while the row is a whole number of 64 bytes.
-  constexpr int KP = HD + (DT % 2 == 0 ? 16 : 8);
+  static constexpr int KP = 16 * DT + (DT % 2 == 0 ? 16 : 8);
   // Value row pitch: the stage's keys + 32 bytes, for the same reason.  A lane reads its eight keys of a step in
   // one piece of 16 bytes (4 cycles an instruction); as two pieces of 8 bytes 32 bytes apart the compiler made one
   // ds_read2_b64 of them, which took 16 cycles at the old pitch and 8 at the best (counted on the pattern alone).
-  constexpr int VP = kStageKeys + 16;
+  static constexpr int VP = kStageKeys + 16;
+  static constexpr int STAGE_BYTES = (kStageKeys * KP + 16 * DT * VP) * 2;
+  static constexpr int MERGE_BYTES = WPT * 16 * NQT * (16 * DT + 4) * 4;
+  __attribute__((aligned(16))) unsigned char stage[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
+  int32_t table[kMaxTableLds];
+};
+
+// The work of block (bx, by, bz): the tile (or pair of tiles), the heads, the part of the keys.
+template <int DT, int NQT, int HPB, int WPT, bool AHEAD, bool PAIRED, bool SIG>
+__device__ __forceinline__ void attention_prefill_staged_block(
+    StagedLds<DT, NQT, WPT>& lds, int bx, int by, int bz, const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
+    const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
+    const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len,
+    const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, float* __restrict__ part_o,
+    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages,
+    const ScoreStage& st, float scale2, int n_tiles) {
+  constexpr int HD = 16 * DT, HC = (DT + 1) / 2;
+  constexpr int THREADS = 64 * WPT * HPB;
+  constexpr int WAVE_KEYS = kStageKeys / WPT;          // keys of a stage that one wave of a team takes
+  constexpr int KP = StagedLds<DT, NQT, WPT>::KP, VP = StagedLds<DT, NQT, WPT>::VP;
   constexpr int KCHUNKS = kStageKeys * (HD / 8);      // 16-byte pieces of the stage's keys ...
   const int page_size = 1 << page_shift, page_mask = page_size - 1;   // pages are a power of two of tokens
   constexpr int CHUNKS = 2 * KCHUNKS;                 // ... and of its values
   constexpr int PER_THREAD = (CHUNKS + THREADS - 1) / THREADS;
-  constexpr int STAGE_BYTES = (kStageKeys * KP + HD * VP) * 2;
-  constexpr int MERGE_BYTES = WPT * 16 * NQT * (HD + 4) * 4;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
-  __shared__ int32_t s_table[kMaxTableLds];
+  unsigned char* smem = lds.stage;
+  int32_t* s_table = lds.table;
   uint16_t* ks = reinterpret_cast<uint16_t*>(smem);
   uint16_t* vs = ks + kStageKeys * KP;
 
@@ -486,12 +494,12 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kerne
   // step then takes as long as its longest tile, with most of the chip idle towards the end.)
 #pragma unroll
   for (int pass = 0; pass < (PAIRED ? 2 : 1); ++pass) {
-  const int tile = pass == 0 ? n_tiles - 1 - int(blockIdx.x) : int(blockIdx.x);
-  if (pass == 1 && tile >= n_tiles - 1 - int(blockIdx.x)) break;   // the middle tile of an odd number is taken once
+  const int tile = pass == 0 ? n_tiles - 1 - bx : bx;
+  if (pass == 1 && tile >= n_tiles - 1 - bx) break;   // the middle tile of an odd number is taken once
   const int seq = tiles[2 * tile], q_off = tiles[2 * tile + 1];
   // the block's HPB heads belong to one key/value head: its four-wave teams share the staged keys and values
   const int G = nq / nkv, teams_per_group = (G + HPB - 1) / HPB;
-  const int g = blockIdx.y / teams_per_group, first_head = (blockIdx.y % teams_per_group) * HPB;
+  const int g = by / teams_per_group, first_head = (by % teams_per_group) * HPB;
   const int team = threadIdx.x / (64 * WPT), wave = (threadIdx.x >> 6) % WPT, lane = threadIdx.x & 63, lr = lane & 15, lj = lane >> 4;
   const bool has_head = first_head + team < G;          // the last block of a group may have teams to spare
   const int h = g * G + min(first_head + team, G - 1);
@@ -539,7 +547,7 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kerne
     // a sink is a term of the denominator without a key: one wave of the team, in the block of the first split,
     // starts its running softmax from it (one lane of a row's four)
     start_row<SIG>(m[qt], lsum[qt]);
-    if (!SIG && st.sinks && wave == 0 && blockIdx.z == 0) {
+    if (!SIG && st.sinks && wave == 0 && bz == 0) {
       m[qt] = st.sinks[h] * kLog2e;
       lsum[qt] = lj == 0 ? 1.f : 0.f;
     }
@@ -549,7 +557,7 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kerne
 
   // With n_splits > 1 the stages of a tile are shared out between gridDim.z blocks, stages_per_split each
   // (the last block takes what is left, however long the sequence), and the blocks leave partial results.
-  const int split = blockIdx.z;
+  const int split = bz;
   int range_lo = (k_lo / kStageKeys) * kStageKeys, range_hi = k_hi;
   if (n_splits > 1) {
     range_lo = max(range_lo, split * stages_per_split * kStageKeys);
@@ -797,17 +805,31 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kerne
   }
 }
 
+template <int DT, int NQT, int HPB, int WPT, bool AHEAD, bool PAIRED, bool SIG>
+__global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kernel(
+    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
+    const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
+    const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len,
+    const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, float* __restrict__ part_o,
+    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages,
+    ScoreStage st, float scale2, int n_tiles) {
+  __shared__ StagedLds<DT, NQT, WPT> lds;
+  attention_prefill_staged_block<DT, NQT, HPB, WPT, AHEAD, PAIRED, SIG>(
+      lds, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, out,
+      part_o, part_ml, n_splits, stages_per_split, nq, nkv, page_shift, num_pages, st, scale2, n_tiles);
+}
+
 // Merges the partial results of the key splits of the prompt kernels: four dimensions a lane, as many (query row, head) pairs a
 // block as it has lanes for, four splits asked for at a time (one pair a wave, a dimension a lane and a split at a time: 2,048
 // rows of 14 heads of 64 in four splits, 29 MB, 14.4 -> 8.0 us).
 // part_o [tile][row][head][split][HD], part_ml [tile][row][head][split][2] = (maximum in log2 units, sum).
-template <int DT, int NQT, bool SIG, typename TO = bf16_t>
-__global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
-    const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ q_start,
+template <int DT, int NQT, bool SIG, typename TO>
+__device__ __forceinline__ void attention_prefill_merge_block(
+    int block, const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ q_start,
     const int32_t* __restrict__ q_len, const int32_t* __restrict__ tiles, TO* __restrict__ out, int n_splits,
-    int nq, ScoreStage st, int pairs) {
+    int nq, const ScoreStage& st, int pairs) {
   constexpr int HD = 16 * DT, ROWS = 16 * NQT, LANES = HD / 4, PER_BLOCK = 256 / LANES;
-  const int pair = int(blockIdx.x) * PER_BLOCK + int(threadIdx.x) / LANES, d = 4 * (threadIdx.x % LANES);
+  const int pair = block * PER_BLOCK + int(threadIdx.x) / LANES, d = 4 * (threadIdx.x % LANES);
   if (int(threadIdx.x) / LANES >= PER_BLOCK || pair >= pairs) return;
   const int h = pair % nq, row = pair / nq % ROWS, tile = pair / nq / ROWS;
   const int seq = tiles[2 * tile], q_off = tiles[2 * tile + 1];
@@ -843,24 +865,42 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
   else *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(num[0] * inv, num[1] * inv), pack_bf16x2(num[2] * inv, num[3] * inv));
 }
 
+template <int DT, int NQT, bool SIG, typename TO = bf16_t>
+__global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
+    const float* __restrict__ part_o, const float* __restrict__ part_ml, const int32_t* __restrict__ q_start,
+    const int32_t* __restrict__ q_len, const int32_t* __restrict__ tiles, TO* __restrict__ out, int n_splits,
+    int nq, ScoreStage st, int pairs) {
+  attention_prefill_merge_block<DT, NQT, SIG>(blockIdx.x, part_o, part_ml, q_start, q_len, tiles, out, n_splits, nq, st, pairs);
+}
+
 // ------------------------------------------------------------------------------------------ decode
 // Partial results of a block, for the merge kernel: part_o [seq][head][split][HD] (not yet divided),
 // part_ml [seq][head][split][2] = (running maximum in log2 units, sum).
+template <int DT>
+struct DecodeLds {
+  float o[4][16][16 * DT + 1];
+  float m[4][16], l[4][16];
+  int32_t table[kDecodeChunk / 4 + 4];      // the chunk's page numbers (pages of 4 tokens or more)
+};
+
+// The work of block (bx, by, bz): the chunk, the set of heads, the sequence.  256 threads, four whole waves.
 template <int DT, bool POW2, bool SIG>
-__global__ __launch_bounds__(256) void attention_decode_kernel(
-    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
+__device__ __forceinline__ void attention_decode_block(
+    DecodeLds<DT>& lds, int bx, int by, int bz, const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
     const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks, int mask,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ decode_seqs,
     uint16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int nq,
-    int nkv, int kv_stored, int page_size, int num_pages, ScoreStage st, float scale2) {
-  // nkv: the sets of query heads that a block takes at once (blockIdx.y); kv_stored: the key/value heads the pools
+    int nkv, int kv_stored, int page_size, int num_pages, const ScoreStage& st, float scale2) {
+  // nkv: the sets of query heads that a block takes at once (by); kv_stored: the key/value heads the pools
   // hold.  They are the same unless a key/value head serves more query heads than the 16 rows of a block: then
   // its heads are taken in nkv / kv_stored sets that read the same keys.
   constexpr int HD = 16 * DT, HC = (DT + 1) / 2;
-  __shared__ float s_o[4][16][HD + 1];
-  __shared__ float s_m[4][16], s_l[4][16];
-  __shared__ int32_t s_table[kDecodeChunk / 4 + 4];      // the chunk's page numbers (pages of 4 tokens or more)
-  const int g = blockIdx.y, di = blockIdx.z, split = chunk_of(blockIdx.x, di, mask);
+  const int tid = threadIdx.x & 255;
+  auto& s_o = lds.o;
+  auto& s_m = lds.m;
+  auto& s_l = lds.l;
+  auto& s_table = lds.table;
+  const int g = by, di = bz, split = chunk_of(bx, di, mask);
   const int seq = decode_seqs ? decode_seqs[di] : di;   // no list: the batch is one-query sequences only, in order
   const int chunk0 = split * kDecodeChunk;
   // The page numbers of this chunk do not depend on how long the sequence is: they are asked for together with
@@ -869,8 +909,8 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
   if (POW2) page_shift = 31 - __builtin_clz(page_size);
   const int table_first = POW2 ? chunk0 >> page_shift : chunk0 / page_size;
   const int table_count = (POW2 ? (chunk0 + kDecodeChunk - 1) >> page_shift : (chunk0 + kDecodeChunk - 1) / page_size) - table_first + 1;
-  if (int(threadIdx.x) < table_count)
-    s_table[threadIdx.x] = block_tables[size_t(seq) * max_blocks + min(table_first + int(threadIdx.x), max_blocks - 1)];
+  if (tid < table_count)
+    s_table[tid] = block_tables[size_t(seq) * max_blocks + min(table_first + tid, max_blocks - 1)];
   // without a list, sequence i's one query is row i
   const int q_row = decode_seqs ? q_start[seq] : seq;
   const int ctx = ctx_len[seq], pos = ctx - 1;
@@ -879,14 +919,14 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
   if (chunk0 > pos || (chunk0 + kDecodeChunk <= k_lo && chunk0 >= st.keep)) {
     // no visible key in this chunk: the merge kernel reads every chunk's (maximum, sum) without looking at
     // the context length, so an empty chunk says so itself
-    if (n_splits > 1 && threadIdx.x < G) {
-      const size_t slot = (size_t(di) * nq + g * G + threadIdx.x) * n_splits + split;
+    if (n_splits > 1 && tid < G) {
+      const size_t slot = (size_t(di) * nq + g * G + tid) * n_splits + split;
       part_ml[2 * slot] = kNoKeyYet;
       part_ml[2 * slot + 1] = 0.f;
     }
     return;
   }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lj = lane >> 4;
+  const int wave = tid >> 6, lane = tid & 63, lr = lane & 15, lj = lane >> 4;
 
   PagedKV kv;
   kv.page_size = page_size;
@@ -942,7 +982,7 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
     for (int r = 0; r < 4; ++r) s_o[wave][lr][16 * dt + 4 * lj + r] = o[0][dt][r];
   __syncthreads();
 
-  for (int i = threadIdx.x; i < G * HD; i += 256) {
+  for (int i = tid; i < G * HD; i += 256) {
     const int qh = i / HD, d = i % HD;
     float mx = -INFINITY;
 #pragma unroll
@@ -965,18 +1005,29 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
   }
 }
 
+template <int DT, bool POW2, bool SIG>
+__global__ __launch_bounds__(256) void attention_decode_kernel(
+    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool,
+    const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks, int mask,
+    const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ decode_seqs,
+    uint16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int nq,
+    int nkv, int kv_stored, int page_size, int num_pages, ScoreStage st, float scale2) {
+  __shared__ DecodeLds<DT> lds;
+  attention_decode_block<DT, POW2, SIG>(lds, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, k_pool, v_pool, block_tables, max_blocks, mask,
+                                        q_start, ctx_len, decode_seqs, out, part_o, part_ml, n_splits, nq, nkv, kv_stored, page_size,
+                                        num_pages, st, scale2);
+}
+
 // Merges the chunks of one (sequence, head): grid (decode sequences, heads); lane d of a wave sums
 // dimension d.  Everything a wave reads depends on its indices alone (empty chunks are marked as such by
 // the decode kernel), so a wave requests 16 chunks at once: one trip to memory.  With WAVES > 1 (long
 // contexts) the waves take turns of 16 chunks each and wave 0 joins their sums through LDS.
 template <int DT, int WAVES, bool SIG>
-__global__ __launch_bounds__(64 * WAVES) void attention_merge_kernel(const float* __restrict__ part_o,
-                                                                     const float* __restrict__ part_ml,
-                                                                     const int32_t* __restrict__ q_start,
-                                                                     const int32_t* __restrict__ decode_seqs,
-                                                                     uint16_t* __restrict__ out, int n_splits, int nq, ScoreStage st) {
+__device__ __forceinline__ void attention_merge_block(int di, int head, const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                      const int32_t* __restrict__ q_start, const int32_t* __restrict__ decode_seqs,
+                                                      uint16_t* __restrict__ out, int n_splits, int nq, const ScoreStage& st) {
   constexpr int HD = 16 * DT, PER_LANE = (HD + 63) / 64, GROUP = 16;
-  const int di = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = WAVES > 1 ? threadIdx.x >> 6 : 0;
   const int seq = decode_seqs ? decode_seqs[di] : di;
   const size_t base = (size_t(di) * nq + head) * n_splits;
   const int q_row = q_start[seq];
@@ -1037,6 +1088,75 @@ __global__ __launch_bounds__(64 * WAVES) void attention_merge_kernel(const float
     if (d < HD)
       out[size_t(q_row) * (size_t(nq) * HD) + head * HD + d] = f32_to_bf16_bits((SIG ? num[j] : den > 0.f ? num[j] / den : 0.f) * gate);
   }
+}
+
+template <int DT, int WAVES, bool SIG>
+__global__ __launch_bounds__(64 * WAVES) void attention_merge_kernel(const float* __restrict__ part_o,
+                                                                     const float* __restrict__ part_ml,
+                                                                     const int32_t* __restrict__ q_start,
+                                                                     const int32_t* __restrict__ decode_seqs,
+                                                                     uint16_t* __restrict__ out, int n_splits, int nq, ScoreStage st) {
+  attention_merge_block<DT, WAVES, SIG>(blockIdx.x, blockIdx.y, part_o, part_ml, q_start, decode_seqs, out, n_splits, nq, st);
+}
+
+// ------------------------------------------------------------------------------------------ both kinds in one launch
+// A step that answers some requests while it reads a prompt of another has few blocks of either kind, and each kind's launch and merge
+// is bound by its own latency, not by the chip: one launch holds the blocks of both, another both merges.  Prompt blocks come first, they
+// are the longer ones.  A block of 512 threads takes two of the one-query kernel's: waves that have ended no longer count at a barrier, and
+// a half that does not end passes as many barriers as the other.  Same keys, same order, same sums as in launches of their own.
+// (8 answers at 1,024..4,096 and 256 tokens behind 1,024, 28 heads of 128: four launches 52.4 us, two 45.5; 5 answers at 300..1,500
+// and 250 tokens, 14 heads of 64: 24.0 us, 15.2.)
+struct PromptPart {
+  const int32_t *q_len, *tiles;
+  float *part_o, *part_ml;
+  int nx, ny, nz, per_split, page_shift, n_tiles;       // nx * ny * nz blocks; nz: parts of the keys
+};
+struct DecodePart {
+  const int32_t* seqs;
+  float *part_o, *part_ml;
+  int n_splits, sets, n, mask;                          // n_splits * sets * n units
+};
+
+template <int DT, int HPB, int WPT, bool AHEAD, bool PAIRED>
+__global__ __launch_bounds__(64 * WPT * HPB) void attention_mixed_kernel(
+    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len,
+    uint16_t* __restrict__ out, int nq, int nkv, int num_pages, ScoreStage st, float scale2, PromptPart p, DecodePart d) {
+  constexpr int UNITS = WPT * HPB / 4;                  // one-query blocks a block takes
+  static_assert(WPT * HPB % 4 == 0, "whole one-query blocks");
+  union Lds {
+    StagedLds<DT, 2, WPT> prompt;
+    DecodeLds<DT> decode[UNITS];
+  };
+  __shared__ Lds lds;
+  const int prompt_blocks = p.nx * p.ny * p.nz, block = blockIdx.x;
+  if (block < prompt_blocks) {
+    attention_prefill_staged_block<DT, 2, HPB, WPT, AHEAD, PAIRED, false>(
+        lds.prompt, block % p.nx, block / p.nx % p.ny, block / (p.nx * p.ny), q, q_stride, k_pool, v_pool, block_tables, max_blocks,
+        q_start, p.q_len, ctx_len, p.tiles, out, p.part_o, p.part_ml, p.nz, p.per_split, nq, nkv, p.page_shift, num_pages, st, scale2,
+        p.n_tiles);
+    return;
+  }
+  const int half = UNITS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, unit = (block - prompt_blocks) * UNITS + half;
+  if (unit >= d.n_splits * d.sets * d.n) return;
+  attention_decode_block<DT, true, false>(lds.decode[half], unit % d.n_splits, unit / d.n_splits % d.sets, unit / (d.n_splits * d.sets), q,
+                                          q_stride, k_pool, v_pool, block_tables, max_blocks, d.mask, q_start, ctx_len, d.seqs, out,
+                                          d.part_o, d.part_ml, d.n_splits, nq, d.sets, nkv, 1 << p.page_shift, num_pages, st, scale2);
+}
+
+// Both merges; WAVES as in attention_merge_kernel (with one wave a pair of sequence and head, a block takes four).
+template <int DT, int WAVES>
+__global__ __launch_bounds__(256) void attention_mixed_merge_kernel(const int32_t* __restrict__ q_start, uint16_t* __restrict__ out, int nq,
+                                                                    ScoreStage st, PromptPart p, DecodePart d, int pairs, int prompt_blocks) {
+  const int block = blockIdx.x;
+  if (block < prompt_blocks) {
+    attention_prefill_merge_block<DT, 2, false>(block, p.part_o, p.part_ml, q_start, p.q_len, p.tiles, reinterpret_cast<bf16_t*>(out), p.nz,
+                                                nq, st, pairs);
+    return;
+  }
+  const int unit = WAVES > 1 ? block - prompt_blocks : (block - prompt_blocks) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (unit >= d.n * nq) return;
+  attention_merge_block<DT, WAVES, false>(unit / nq, unit % nq, d.part_o, d.part_ml, q_start, d.seqs, out, d.n_splits, nq, st);
 }
 
 // Merge of the chunks of one head, folded into that head's share of the output projection (decode steps):
@@ -1219,6 +1339,13 @@ int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const 
                           const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int max_tile_ctx, int splits, uint16_t* out,
                           float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2);
 size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_ctx);
+// attention_mixed.hip: a step's prompts and its one-query sequences in one launch.  Blocks of up to eight waves, head sizes up to 128,
+// softmax weights: blocks of 16 waves are those of long prompts, beside which the one-query blocks are little, and would hold
+// four of those each.
+constexpr bool mixed_instantiated(int dt, bool sig) { return !sig && dt <= 8; }
+int launch_mixed(hipStream_t s, int dt, int hpb, int wpt, bool paired, const uint16_t* q, int q_stride, const uint16_t* k_pool,
+                 const uint16_t* v_pool, const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* ctx_len,
+                 uint16_t* out, int nq, int nkv, int num_pages, const ScoreStage& st, float scale2, const PromptPart& p, const DecodePart& d);
 
 template <int DT, bool SIG>
 static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
@@ -1232,6 +1359,9 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
   const uint16_t *qp = (const uint16_t*)q, *kp = (const uint16_t*)k_pool, *vp = (const uint16_t*)v_pool;
   // the workspace holds the decode partials first, then the prefill partials
   float* prefill_ws = workspace ? workspace + attention_decode_workspace_floats(n_decode, nq, HD, max_decode_ctx) : nullptr;
+  const int decode_splits = max(1, (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk);
+  float* decode_o = workspace;
+  float* decode_ml = workspace ? workspace + size_t(n_decode) * nq * decode_splits * HD : nullptr;
   if (n_tiles > 0) {
     if (staged_prefill(page_size)) {
       int page_shift = 0;
@@ -1247,6 +1377,13 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       StagedShape shape = staged_shape(nq, nkv, HD, n_tiles);
       const bool paired = staged_paired(n_tiles, nq, nkv, HD, splits, max_tile_ctx, mean_tile_walk, &shape);
       const dim3 grid(paired ? (n_tiles + 1) / 2 : n_tiles, nkv * ((nq / nkv + shape.hpb - 1) / shape.hpb), splits);
+      if (mixed_instantiated(DT, SIG) && n_decode > 0 && !rows_splits && shape.hpb * shape.wpt <= 8) {
+        const int sets = decode_sets(nq, nkv);
+        return launch_mixed(s, DT, shape.hpb, shape.wpt, paired, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, ctx_len,
+                            (uint16_t*)out, nq, nkv, num_pages, st, scale2,
+                            PromptPart{q_len, tiles, part_o, part_ml, int(grid.x), int(grid.y), splits, per_split, page_shift, n_tiles},
+                            DecodePart{decode_seqs, decode_o, decode_ml, decode_splits, sets, n_decode, chunk_mask(decode_splits)});
+      }
 #define SP_STAGED(HPB, WPT, AHEAD, PAIRED)                                                                      \
   attention_prefill_staged_kernel<DT, NQT, HPB, WPT, AHEAD, PAIRED, SIG><<<grid, 64 * WPT * HPB, 0, s>>>(            \
       qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, (uint16_t*)out, part_o,   \
@@ -1284,9 +1421,8 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
     if (check_launch("sp_attention (prefill)")) return 1;
   }
   if (n_decode > 0) {
-    const int n_splits = max(1, (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk);
-    float* part_o = workspace;
-    float* part_ml = workspace ? workspace + size_t(n_decode) * nq * n_splits * HD : nullptr;
+    const int n_splits = decode_splits;
+    float *part_o = decode_o, *part_ml = decode_ml;
     if ((page_size & (page_size - 1)) == 0)
       attention_decode_kernel<DT, true, SIG><<<dim3(n_splits, decode_sets(nq, nkv), n_decode), 256, 0, s>>>(
           qp, q_stride, kp, vp, block_tables, max_blocks, chunk_mask(n_splits), q_start, ctx_len, decode_seqs, (uint16_t*)out,

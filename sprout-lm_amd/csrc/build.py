@@ -19,7 +19,7 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-ta
          "-packed-fp32-ops", "-Wno-unused-result"]
 # Attention rescales its MFMA accumulators with vector instructions at every step, and so does the delta rule's state;
 # kept in AGPRs each such step would cost a move out and a move back, so these kernels take the VGPR form of MFMA.
-FILE_FLAGS = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("attention_mfma.hip", "attention_mfma_sigmoid.hip",
+FILE_FLAGS = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("attention_mfma.hip", "attention_mfma_sigmoid.hip", "attention_mixed.hip",
                                                                               "attention_mfma_wide.hip", "attention_mfma_wide_sigmoid.hip", "attention_rows.hip", "attention_split.hip",
                                                                               "delta.hip")}
 
