@@ -449,6 +449,15 @@ constexpr int kStageKeys = 128;
 __device__ __forceinline__ constexpr int step_row(int r) { return (r & ~31) | ((r & 4) << 2) | (((r & 31) >> 3) << 2) | (r & 3); }
 constexpr int kMaxTableLds = 2048;    // page numbers held in LDS; longer tables are read from memory
 
+// Part `split` of a walk from key lo, the first of a stage of `keys` keys, to key hi: the tile's own stages in equal shares (the last parts
+// of a short walk are empty).  A tile's walk, not the step's longest context, is what is shared out: a recorded step knows that one as a
+// bucket that may be twice as long (2,048 queries over 20,000 keys, 14 heads of 64 in 2 groups, known as 32,768: 183 -> 174 us).
+__device__ __forceinline__ void share_of_walk(int& lo, int& hi, int keys, int split, int n_splits) {
+  const int stages = (hi - lo) / keys + 1, per = (stages + n_splits - 1) / n_splits;
+  lo += split * per * keys;
+  hi = min(hi, lo + per * keys - 1);
+}
+
 template <int DT, int NQT, int WPT>
 struct StagedLds {
   // Key row pitch in LDS (elements).  A 16-byte LDS read serves lanes {0-3, 12-15, 20-27} of each half-wave in
@@ -473,7 +482,7 @@ __device__ __forceinline__ void attention_prefill_staged_block(
     const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len,
     const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages,
+    float* __restrict__ part_ml, int n_splits, int nq, int nkv, int page_shift, int num_pages,
     const ScoreStage& st, float scale2, int n_tiles) {
   constexpr int HD = 16 * DT, HC = (DT + 1) / 2;
   constexpr int THREADS = 64 * WPT * HPB;
@@ -555,14 +564,10 @@ __device__ __forceinline__ void attention_prefill_staged_block(
     for (int dt = 0; dt < DT; ++dt) o[qt][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // With n_splits > 1 the stages of a tile are shared out between gridDim.z blocks, stages_per_split each
-  // (the last block takes what is left, however long the sequence), and the blocks leave partial results.
+  // With n_splits > 1 the stages of a tile are shared out between that many blocks, which leave partial results.
   const int split = bz;
   int range_lo = (k_lo / kStageKeys) * kStageKeys, range_hi = k_hi;
-  if (n_splits > 1) {
-    range_lo = max(range_lo, split * stages_per_split * kStageKeys);
-    if (split + 1 < n_splits) range_hi = min(range_hi, (split + 1) * stages_per_split * kStageKeys - 1);
-  }
+  if (n_splits > 1) share_of_walk(range_lo, range_hi, kStageKeys, split, n_splits);
   // A stage travels memory -> registers -> LDS.  With AHEAD the registers are asked for the next stage as soon
   // as this one lies in LDS, so its trip to memory runs while this one is being used (the registers stay
   // occupied meanwhile: worth it where there are few per thread).  (Two sets of registers, each asked for the stage
@@ -811,12 +816,12 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_prefill_staged_kerne
     const uint16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len,
     const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages,
+    float* __restrict__ part_ml, int n_splits, int nq, int nkv, int page_shift, int num_pages,
     ScoreStage st, float scale2, int n_tiles) {
   __shared__ StagedLds<DT, NQT, WPT> lds;
   attention_prefill_staged_block<DT, NQT, HPB, WPT, AHEAD, PAIRED, SIG>(
       lds, blockIdx.x, blockIdx.y, blockIdx.z, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, out,
-      part_o, part_ml, n_splits, stages_per_split, nq, nkv, page_shift, num_pages, st, scale2, n_tiles);
+      part_o, part_ml, n_splits, nq, nkv, page_shift, num_pages, st, scale2, n_tiles);
 }
 
 // Merges the partial results of the key splits of the prompt kernels: four dimensions a lane, as many (query row, head) pairs a
@@ -1109,7 +1114,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_merge_kernel(const float
 struct PromptPart {
   const int32_t *q_len, *tiles;
   float *part_o, *part_ml;
-  int nx, ny, nz, per_split, page_shift, n_tiles;       // nx * ny * nz blocks; nz: parts of the keys
+  int nx, ny, nz, page_shift, n_tiles;       // nx * ny * nz blocks; nz: parts of the keys
 };
 struct DecodePart {
   const int32_t* seqs;
@@ -1133,7 +1138,7 @@ __global__ __launch_bounds__(64 * WPT * HPB) void attention_mixed_kernel(
   if (block < prompt_blocks) {
     attention_prefill_staged_block<DT, 2, HPB, WPT, AHEAD, PAIRED, false>(
         lds.prompt, block % p.nx, block / p.nx % p.ny, block / (p.nx * p.ny), q, q_stride, k_pool, v_pool, block_tables, max_blocks,
-        q_start, p.q_len, ctx_len, p.tiles, out, p.part_o, p.part_ml, p.nz, p.per_split, nq, nkv, p.page_shift, num_pages, st, scale2,
+        q_start, p.q_len, ctx_len, p.tiles, out, p.part_o, p.part_ml, p.nz, nq, nkv, p.page_shift, num_pages, st, scale2,
         p.n_tiles);
     return;
   }
@@ -1279,8 +1284,6 @@ constexpr int kMaxPrefillSplits = 32;   // (more parts of a walk than that and t
 
 static bool staged_prefill(int page_size) { return page_size >= 8 && (page_size & (page_size - 1)) == 0; }
 
-// Blocks per tile and head along the keys.  A step with few queries over a long context (a portion of a long
-// prompt) has few tiles, each with a long walk: the walk is cut until the grid fills the chip about three times.
 // Teams of a block of the staged kernel: HPB heads of one key/value head, WPT waves each.  The heads share
 // every stage of keys and values, which the kernel otherwise fetches from L2 once per head -- and that
 // traffic, not the matrix cores, is what bounds it (measured ~8.5 TB/s at every size).  Head sizes up to 64:
@@ -1330,13 +1333,13 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
   return false;
 }
 
-int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
+int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; its splits are 0 where it is not the faster one.
 int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
 bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk);
 int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
                           const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
-                          const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int max_tile_ctx, int splits, uint16_t* out,
+                          const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int splits, uint16_t* out,
                           float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2);
 size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_ctx);
 // attention_mixed.hip: a step's prompts and its one-query sequences in one launch.  Blocks of up to eight waves, head sizes up to 128,
@@ -1369,9 +1372,7 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       const bool plain = st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && st.keep <= 0 && !st.sinks && !st.bias && !st.gate;
       int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
       if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk)) rows_splits = 0;
-      const int splits = rows_splits ? rows_splits : attention_prefill_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx);
-      const int stages = (max_tile_ctx + kStageKeys - 1) / kStageKeys;
-      const int per_split = (stages + splits - 1) / splits;
+      const int splits = rows_splits ? rows_splits : attention_prefill_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, n_decode > 0);
       float* part_o = splits > 1 ? prefill_ws : nullptr;
       float* part_ml = splits > 1 ? prefill_ws + size_t(n_tiles) * 16 * NQT * nq * splits * HD : nullptr;
       StagedShape shape = staged_shape(nq, nkv, HD, n_tiles);
@@ -1381,16 +1382,16 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
         const int sets = decode_sets(nq, nkv);
         return launch_mixed(s, DT, shape.hpb, shape.wpt, paired, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, ctx_len,
                             (uint16_t*)out, nq, nkv, num_pages, st, scale2,
-                            PromptPart{q_len, tiles, part_o, part_ml, int(grid.x), int(grid.y), splits, per_split, page_shift, n_tiles},
+                            PromptPart{q_len, tiles, part_o, part_ml, int(grid.x), int(grid.y), splits, page_shift, n_tiles},
                             DecodePart{decode_seqs, decode_o, decode_ml, decode_splits, sets, n_decode, chunk_mask(decode_splits)});
       }
 #define SP_STAGED(HPB, WPT, AHEAD, PAIRED)                                                                      \
   attention_prefill_staged_kernel<DT, NQT, HPB, WPT, AHEAD, PAIRED, SIG><<<grid, 64 * WPT * HPB, 0, s>>>(            \
       qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, (uint16_t*)out, part_o,   \
-      part_ml, splits, per_split, nq, nkv, page_shift, num_pages, st, scale2, n_tiles)
+      part_ml, splits, nq, nkv, page_shift, num_pages, st, scale2, n_tiles)
       // the same cases as staged_shape() and staged_paired()
       if (rows_splits) {
-        if (launch_attention_rows(s, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, n_tiles, max_tile_ctx,
+        if (launch_attention_rows(s, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, n_tiles,
                                   splits, (uint16_t*)out, part_o, part_ml, nq, nkv, page_shift, num_pages, scale2))
           return 1;
       } else if constexpr (DT > 8) {

@@ -12,18 +12,28 @@ bool attention_mfma_supports(int hd, int page_size, int nq, int nkv) {
 bool attention_mfma_decode_supports(int nq, int nkv) { return true; }
 int attention_mfma_tile_q(int hd) { return 32; }
 
-int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx) {
+// Blocks per tile and set of heads along the keys.  A step with few queries over a long context (a portion of a long prompt) has few
+// tiles, each with a long walk: it is cut until a CU has a block of eight waves, or five waves on four at head sizes up to 64, whose blocks
+// of four share a CU; beside one-query sequences, whose blocks take places of their own, four, and above 64 half as many.  A block more than
+// that on some of the CUs, and the step waits for those; every part's sums are written and read again.  Parts hold two stages at least, eight
+// where the tiles fill half of the chip (the walks of a prompt's first tokens are half as long as the longest).  us a launch and its merge
+// by the number of parts, the choice first: 28 heads of 128 in 4 groups, 256 queries behind 1,024: four 26.0, two 28.0, five 34.8; 200 behind
+// 1,500: four 25.7, three 27.5, six 34.1; 700 from the start: one 24.3, two 36.1; 256 behind 1,024 beside eight answers: two 28.1, one 37.4,
+// four 34.1; 14 heads of 64 in 2 groups, 250 behind 1,500: five 15.5, three 15.3, eight 18.6; 300 behind 8,700: four 37.8, six 43.1; 600 behind
+// 1,000: two 20.7, one 21.4, four 25.0; 250 behind 1,500 beside five answers: four 15.5, eight 19.5, one 25.2.
+int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers) {
   if (!staged_prefill(page_size)) return 1;
   const StagedShape shape = staged_shape(nq, nkv, hd, n_tiles);
   const int G = nq / nkv;
   const int blocks = n_tiles * nkv * ((G + shape.hpb - 1) / shape.hpb), stages = (max_tile_ctx + kStageKeys - 1) / kStageKeys;
-  const int enough = 2048 / (shape.wpt * shape.hpb);   // blocks that hold 2,048 waves: two rounds of the chip's CUs
-  if (blocks <= 0 || blocks >= enough || stages <= 4) return 1;
-  return max(1, min(min((enough * 3 / 2 + blocks - 1) / blocks, stages / 2), kMaxPrefillSplits));
+  const int places = 2048 / (shape.wpt * shape.hpb);
+  if (blocks <= 0 || blocks >= places || stages <= 4) return 1;
+  const int enough = hd > 64 ? (beside_answers ? places / 2 : places) : (beside_answers ? places : places * 5 / 4);
+  return max(1, min(min(enough / blocks, stages / (2 * blocks >= places ? 8 : 2)), kMaxPrefillSplits));
 }
 
-size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx) {
-  const size_t splits = max(attention_prefill_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx),
+size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers) {
+  const size_t splits = max(attention_prefill_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, beside_answers),
                             attention_rows_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx));
   return splits <= 1 ? 0 : size_t(n_tiles) * 32 * nq * splits * (hd + 2);
 }

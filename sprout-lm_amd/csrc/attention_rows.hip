@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool,
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
     const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ tiles, uint16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages, float scale2,
+    float* __restrict__ part_ml, int n_splits, int nq, int nkv, int page_shift, int num_pages, float scale2,
     int n_tiles) {
   constexpr int HD = 64;
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];      // two stages, then the page numbers
@@ -162,10 +162,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   const int pos0 = ctx - qlen + q_off, k_hi = pos0 + nvalid - 1;
   const int split = blockIdx.z;
   int lo = 0, hi = k_hi;
-  if (n_splits > 1) {
-    lo = split * stages_per_split * kRowsKeys;
-    if (split + 1 < n_splits) hi = min(hi, (split + 1) * stages_per_split * kRowsKeys - 1);
-  }
+  if (n_splits > 1) share_of_walk(lo, hi, kRowsKeys, split, n_splits);
   const int heads = max(0, min(2, G - first_head - 2 * wave)), head0 = g * G + first_head + 2 * wave;
 
   const int32_t* table = block_tables + size_t(seq) * max_blocks;
@@ -368,7 +365,7 @@ int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, i
 // queries over 16,384 beside seven prompts of 300: 340 us here, 165 there; 64 in 8 groups, 32 queries over 32,768 beside eight of 128:
 // 662 and 578, but over 4,096 90 and 100).
 bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk) {
-  const int G = nq / nkv, sets = (G + 7) / 8, there = attention_prefill_splits(n_tiles, nq, nkv, 64, page_size, max_tile_ctx);
+  const int G = nq / nkv, sets = (G + 7) / 8, there = attention_prefill_splits(n_tiles, nq, nkv, 64, page_size, max_tile_ctx, false);
   const float longest = float(max_tile_ctx) / float(splits);
   if (longest <= 3.f * float(n_tiles) * float(nkv * sets) * float(mean_tile_walk) / 256.f) return false;
   StagedShape shape = staged_shape(nq, nkv, 64, n_tiles);
@@ -379,9 +376,8 @@ bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, 
 
 int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
                           const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
-                          const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int max_tile_ctx, int splits, uint16_t* out,
+                          const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int splits, uint16_t* out,
                           float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2) {
-  const int stages = (max_tile_ctx + kRowsKeys - 1) / kRowsKeys, per_split = (stages + splits - 1) / splits;
   constexpr int lds = 2 * kRowsStageBytes + kRowsTable * 4;
   static bool raised = false;
   if (!raised) {
@@ -393,7 +389,7 @@ int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const 
     raised = true;
   }
   attention_rows_kernel<<<dim3(n_tiles, nkv * ((nq / nkv + 7) / 8), splits), 256, lds, s>>>(
-      q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, out, part_o, part_ml, splits, per_split,
+      q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, out, part_o, part_ml, splits,
       nq, nkv, page_shift, num_pages, scale2, n_tiles);
   return check_launch("sp_attention (prefill)");
 }

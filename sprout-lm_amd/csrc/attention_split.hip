@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
     const float* __restrict__ q, int q_stride, const float* __restrict__ k_pool, const float* __restrict__ v_pool,
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
     const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ tiles, float* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int n_splits, int stages_per_split, int nq, int nkv, int page_shift, int num_pages, float scale2,
+    float* __restrict__ part_ml, int n_splits, int nq, int nkv, int page_shift, int num_pages, float scale2,
     int n_tiles) {
   constexpr int HD = 64;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // three planes of keys, three of values, the page numbers
@@ -89,10 +89,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
   if (nvalid <= 0) return;
   const int pos0 = ctx - qlen + q_off, k_hi = pos0 + nvalid - 1, split = blockIdx.z;
   int lo = 0, hi = k_hi;
-  if (n_splits > 1) {
-    lo = split * stages_per_split * kSplitKeys;
-    if (split + 1 < n_splits) hi = min(hi, (split + 1) * stages_per_split * kSplitKeys - 1);
-  }
+  if (n_splits > 1) share_of_walk(lo, hi, kSplitKeys, split, n_splits);
   const bool live = in_group < G;      // a wave without a head walks along for its share of the stages
   const int head = g * G + min(in_group, G - 1);
 
@@ -341,12 +338,12 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(
 // under 16 in 16).
 bool attention_split_takes(int hd, int page_size) { return hd == 64 && page_size >= 4 && (page_size & (page_size - 1)) == 0; }
 
-// Blocks along the keys: as many as fill the chip's 512 places twice over, each with four stages at least.  (14 heads in 2
-// groups, 2,048 tokens: one 122 us, two 99, four 94, eight 96; 256 tokens behind 1,024: one 72, four 29, eight 25; 32 heads in 8
+// Blocks along the keys: as many as fill the chip's 512 places two and a half times, each with four stages at least.  (14 heads in 2
+// groups, 2,048 tokens: one 113 us, two 90, four 91, five 85, eight 90; 256 tokens behind 1,024: one 72, four 29, eight 25; 32 heads in 8
 // groups, 2,048 tokens: one 178, two 167, four 168.)
 int attention_split_splits(int n_tiles, int nq, int nkv, int max_tile_ctx) {
   const long blocks = long(n_tiles) * nkv * ((nq / nkv + 3) / 4);
-  return blocks < 1 ? 1 : max(1, min(min(int(1024 / blocks), max_tile_ctx / (4 * kSplitKeys)), 16));
+  return blocks < 1 ? 1 : max(1, min(min(int(1280 / blocks), max_tile_ctx / (4 * kSplitKeys)), 16));
 }
 
 size_t attention_split_workspace_floats(int n_tiles, int nq, int nkv, int hd, int max_tile_ctx) {
@@ -371,11 +368,10 @@ int attention_split(hipStream_t s, const float* q, int q_stride, const float* k_
   }
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
-  const int stages = (max_tile_ctx + kSplitKeys - 1) / kSplitKeys;
   float* part_ml = splits > 1 ? workspace + size_t(n_tiles) * 32 * nq * splits * 64 : nullptr;
   attention_split_kernel<<<dim3(n_tiles, nkv * ((nq / nkv + 3) / 4), splits), 256, kLds, s>>>(
       q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, out, workspace, part_ml, splits,
-      (stages + splits - 1) / splits, nq, nkv, page_shift, num_pages, scale * kLog2e, n_tiles);
+      nq, nkv, page_shift, num_pages, scale * kLog2e, n_tiles);
   if (check_launch("sp_attention (float32, parts)")) return 1;
   if (splits > 1) {
     const int pairs = n_tiles * 32 * nq;

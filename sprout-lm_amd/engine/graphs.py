@@ -193,7 +193,7 @@ class _PortionGraph:
 
     _uids = itertools.count(1)
 
-    def __init__(self, runner, first, ctx_bucket: int, workspace):
+    def __init__(self, runner, first, ctx_bucket: int, tile_bucket: int, workspace):
         self.uid = next(self._uids)          # names this graph to the shared workspace
         self.runner = runner if isinstance(runner, weakref.ProxyTypes) else weakref.proxy(runner)
         cache = runner.cache
@@ -215,7 +215,8 @@ class _PortionGraph:
         # The logits are what the caller gets: they live in a tensor of this graph's own.
         self.shared_workspace = workspace
         self.ctx = context_from(first, views, len(cache.groups), OwnedNames(workspace, ("logits",), runner.device),
-                                runner.dtype, runner.attention_kind, max_decode_ctx=ctx_bucket, max_ctx=ctx_bucket)
+                                runner.dtype, runner.attention_kind, max_decode_ctx=ctx_bucket, max_ctx=ctx_bucket,
+                                max_tile_ctx=tile_bucket)
         self.ctx.host = {}
         self.copied = None
         self.graph = None
@@ -302,7 +303,9 @@ class DecodeGraphs:
         if not runner.parts.graph_safe_portions or not entries:
             return None
         bucket = self._context_bucket(max(e.seq.length + len(e.tokens) for e in entries))
-        key = (tuple((len(e.tokens), len(e.want)) for e in entries), bucket)
+        # the requests that bring several tokens have a bucket of their own, where it is another one
+        tile_bucket = self._context_bucket(max((e.seq.length + len(e.tokens) for e in entries if len(e.tokens) > 1), default=1))
+        key = (tuple((len(e.tokens), len(e.want)) for e in entries), bucket) + ((tile_bucket,) if tile_bucket != bucket else ())
         self.portion_steps += 1
         state = self.portion_graphs.pop(key, None)
         if state is None:
@@ -324,7 +327,7 @@ class DecodeGraphs:
         if state is None:
             if self._portion_workspace is None:
                 self._portion_workspace = KeptWorkspace(runner.device)
-            state = _PortionGraph(runner, step, bucket, self._portion_workspace)
+            state = _PortionGraph(runner, step, bucket, tile_bucket, self._portion_workspace)
         self.portion_graphs[key] = state
         state.last_used = self.portion_steps
         state.fill(step)

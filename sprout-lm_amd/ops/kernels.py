@@ -682,14 +682,16 @@ class AttentionBatch:
     """The device-side description of a step's sequences that `attention` reads."""
 
     def __init__(self, q_start, q_len, ctx_len, n_seqs: int, lists: dict, max_decode_ctx: int, max_ctx: int,
-                 mean_walk: int = 0):
+                 mean_walk: int = 0, max_tile_ctx: int | None = None):
         """`lists`: name -> (device int32 tensor, number of entries), names as in `attention_lists`;
         `max_decode_ctx`, `max_ctx`: the longest context among one-query sequences, and among all;
         `mean_walk`: the mean number of keys that a tile of queries walks, see `mean_tile_walk` (a hint for
-        how the kernels share out the work; unknown: 0)."""
+        how the kernels share out the work; unknown: 0); `max_tile_ctx`: the longest context among sequences with several
+        queries (a hint as well; by default the longest of all)."""
         self.q_start, self.q_len, self.ctx_len, self.n_seqs = q_start, q_len, ctx_len, n_seqs
         self.lists, self.max_decode_ctx, self.max_ctx = lists, max_decode_ctx, max_ctx
         self.mean_walk = mean_walk
+        self.max_tile_ctx = max_ctx if max_tile_ctx is None else max_tile_ctx
 
     @classmethod
     def build(cls, q_lens, ctx_lens, device) -> "AttentionBatch":
@@ -701,7 +703,7 @@ class AttentionBatch:
         decode_ctx = [c for c, q in zip(ctx_lens, q_lens) if q == 1]
         return cls(to(starts), to(q_lens), to(ctx_lens), len(q_lens), lists, max(decode_ctx, default=0),
                    max((int(c) for c in ctx_lens), default=0),
-                   mean_tile_walk(q_lens, ctx_lens))
+                   mean_tile_walk(q_lens, ctx_lens), max((int(c) for c, q in zip(ctx_lens, q_lens) if q > 1), default=0))
 
 
 def attention_plan(dtype: torch.dtype, hd: int, page_size: int, nq: int, nkv: int, kind: int = 0) -> tuple[int, bool]:
@@ -794,7 +796,7 @@ def attention(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torc
     if n_tiles and batch.max_ctx > block_tables.shape[1] * page_size:
         raise KernelError(f"attention: a context of {batch.max_ctx} tokens is longer than its block table "
                           f"({block_tables.shape[1]} pages of {page_size})")
-    max_tile_ctx = batch.max_ctx if n_tiles else 0
+    max_tile_ctx = (batch.max_ctx if every else batch.max_tile_ctx) if n_tiles else 0
     if one_query_each:
         n_decode = n_tiles
     need = library().sp_attention_workspace_floats(_code(q, "q"), hd, page_size, nq, nkv, kind, n_decode, max_decode_ctx,

@@ -1,5 +1,5 @@
-"""Steps that hold prompts and one-query sequences: one launch takes the blocks of both kinds and one their merges.  The keys, their
-order and the sums are those of the launches that steps of one kind have, so the result is the same bit for bit."""
+"""Steps that hold prompts and one-query sequences: one launch takes the blocks of both kinds and one their merges.  One-query sequences
+have the same keys in the same order as in a step of their own, and the same results bit for bit; a prompt's keys may lie in fewer parts."""
 import pytest
 import torch
 
@@ -45,4 +45,10 @@ def test_both_kinds_in_one_launch(nq, nkv, hd, page, seqs, options):
         mine = [i for i, (_, n) in enumerate(seqs) if (n == 1) == one]
         rows = [starts[i] + j for i in mine for j in range(seqs[i][1])]
         alone = _run(q, k, v, tables[mine].contiguous(), [seqs[i] for i in mine], rows, nq, nkv, hd, options)
-        assert torch.equal(got[rows], alone), (one, (got[rows].float() - alone.float()).abs().max().item())
+        if one:
+            assert torch.equal(got[rows], alone)
+            continue
+        # other parts, other maxima under the weights' rounding to bfloat16: a weight is off by 2^-9 of itself at most, the sum over keys of
+        # random values by 2^-9 / sqrt(3) of its size, the result by its own rounding, on either side; one of 2,048 keys missing is 0.022
+        a, b = (x.float().view(len(rows), nq, hd) for x in (got[rows], alone))
+        assert ((a - b).norm(dim=-1) <= 2 ** -6 * b.norm(dim=-1)).all()
