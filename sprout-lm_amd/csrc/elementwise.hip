@@ -84,6 +84,69 @@ __global__ void rmsnorm_rows_kernel(const float* __restrict__ x, const int32_t* 
   }
 }
 
+// The same where a product before it has left its sums in n_parts parts, [part][T][H], for the norm to join: x += their sum, taken in
+// order, first; rows given: only those rows are joined, and x stays as it is (the last norm of a step, behind which nobody reads it).
+// Bound by memory where there are many rows, by its chain of loads and sums where there are few (rows of 896: 2,048 without parts 5.0 us, with
+// two 7.3; 1,238 4.9, with three 6.3; 264 rows of 3,584 4.9, with eight and three 7.9).
+template <typename TW, typename TO, int PER>
+__global__ void rmsnorm_join_kernel(float* __restrict__ x, const float* __restrict__ parts, int n_parts, size_t part_stride,
+                                    const int32_t* __restrict__ rows, const TW* __restrict__ w, float eps, TO* __restrict__ out, int H) {
+  __shared__ float scratch[16];
+  const int r = blockIdx.x;
+  const size_t row = size_t(rows ? rows[r] : r) * H;
+  float4 v[PER], wv[PER], add[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = 4 * (threadIdx.x + j * blockDim.x);
+    v[j] = i < H ? load4(x + row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    wv[j] = i < H ? load4(w + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    add[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  for (int p0 = 0; p0 < n_parts; p0 += 4) {      // four parts are asked for at a time
+    float4 q[4][PER];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const int i = 4 * (threadIdx.x + j * blockDim.x);
+        q[u][j] = p0 + u < n_parts && i < H ? load4(parts + (p0 + u) * part_stride + row + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) add[j] = make_float4(add[j].x + q[u][j].x, add[j].y + q[u][j].y, add[j].z + q[u][j].z, add[j].w + q[u][j].w);
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    v[j] = make_float4(v[j].x + add[j].x, v[j].y + add[j].y, v[j].z + add[j].z, v[j].w + add[j].w);
+    sum = fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, fmaf(v[j].w, v[j].w, sum))));
+  }
+  sum = block_sum(sum, scratch);
+  const float scale = 1.0f / sqrtf(sum / float(H) + eps);
+  TO* o = out + size_t(r) * H;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = 4 * (threadIdx.x + j * blockDim.x);
+    if (i >= H) continue;
+    if (!rows) store4(x + row + i, v[j]);
+    store4(o + i, make_float4((v[j].x * scale) * wv[j].x, (v[j].y * scale) * wv[j].y, (v[j].z * scale) * wv[j].z, (v[j].w * scale) * wv[j].w));
+  }
+}
+
+// x += the parts' sum, n numbers in fours.
+__global__ void join_kernel(float* __restrict__ x, const float* __restrict__ parts, int n_parts, size_t n) {
+  const size_t i = 4 * (size_t(blockIdx.x) * blockDim.x + threadIdx.x);
+  if (i >= n) return;
+  float4 add = load4(parts + i);
+  for (int p = 1; p < n_parts; ++p) {
+    const float4 q = load4(parts + p * n + i);
+    add = make_float4(add.x + q.x, add.y + q.y, add.z + q.z, add.w + q.w);
+  }
+  const float4 v = load4(x + i);
+  store4(x + i, make_float4(v.x + add.x, v.y + add.y, v.z + add.z, v.w + add.w));
+}
+
 // ---------------------------------------------------------------- SiLU(gate) * up
 // row_gate (may be null): the token's row is also multiplied by sigmoid(row_gate[t * row_gate_stride]), float32.
 template <typename T>
@@ -380,6 +443,39 @@ extern "C" int sp_rmsnorm(void* stream, const float* x, const int32_t* rows, int
   else SP_REQUIRE(false, "sp_rmsnorm: unsupported dtypes w=%d out=%d", w_dtype, out_dtype);
 #undef SP_NORM
   return check_launch("sp_rmsnorm");
+}
+
+// sp_rmsnorm of x + the sum of parts [n_parts][T][H]; without rows (R = T) that sum also becomes x.  H in eights, up to 8,192.
+extern "C" int sp_rmsnorm_join(void* stream, float* x, const float* parts, int n_parts, int T, const int32_t* rows, int w_dtype, const void* w,
+                               float eps, int out_dtype, void* out, int R, int H) {
+  SP_REQUIRE(R >= 0 && T >= 1 && H > 0 && H % 8 == 0 && H <= 8192 && n_parts >= 1, "sp_rmsnorm_join: bad sizes R=%d H=%d parts=%d", R, H, n_parts);
+  SP_REQUIRE(rows || R == T, "sp_rmsnorm_join: %d of %d rows without a list", R, T);
+  SP_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(parts)) & 15) == 0, "sp_rmsnorm_join: sums must start at multiples of 16 bytes");
+  if (R == 0) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  const int threads = H >= 1024 ? 512 : 256, per = (H / 4 + threads - 1) / threads;
+  const size_t stride = size_t(T) * H;
+#define SP_NORM(TW, TO)                                                                                                          \
+  do {                                                                                                                           \
+    if (per == 1) rmsnorm_join_kernel<TW, TO, 1><<<R, threads, 0, s>>>(x, parts, n_parts, stride, rows, (const TW*)w, eps, (TO*)out, H);  \
+    else if (per == 2) rmsnorm_join_kernel<TW, TO, 2><<<R, threads, 0, s>>>(x, parts, n_parts, stride, rows, (const TW*)w, eps, (TO*)out, H); \
+    else rmsnorm_join_kernel<TW, TO, 4><<<R, threads, 0, s>>>(x, parts, n_parts, stride, rows, (const TW*)w, eps, (TO*)out, H);   \
+  } while (0)
+  if (w_dtype == kF32 && out_dtype == kF32) SP_NORM(float, float);
+  else if (w_dtype == kF32 && out_dtype == kBF16) SP_NORM(float, bf16_t);
+  else if (w_dtype == kBF16 && out_dtype == kF32) SP_NORM(bf16_t, float);
+  else if (w_dtype == kBF16 && out_dtype == kBF16) SP_NORM(bf16_t, bf16_t);
+  else SP_REQUIRE(false, "sp_rmsnorm_join: unsupported dtypes w=%d out=%d", w_dtype, out_dtype);
+#undef SP_NORM
+  return check_launch("sp_rmsnorm_join");
+}
+
+// x[i] += the sum of parts[p][i], n numbers, in fours.
+extern "C" int sp_join(void* stream, float* x, const float* parts, int n_parts, long long n) {
+  SP_REQUIRE(n >= 0 && n % 4 == 0 && n_parts >= 1 && (n == 0 || (x && parts)), "sp_join: bad arguments");
+  if (n == 0) return 0;
+  join_kernel<<<unsigned((n / 4 + 255) / 256), 256, 0, (hipStream_t)stream>>>(x, parts, n_parts, size_t(n));
+  return check_launch("sp_join");
 }
 
 extern "C" int sp_silu_mul(void* stream, int dtype, const void* gu, void* out, int T, int I, int activation, float limit,

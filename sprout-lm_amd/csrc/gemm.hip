@@ -13,6 +13,10 @@ int gemm_f32_skinny(hipStream_t s, const void* a, const void* w, int bias_dtype,
                     int T, int N, int K);
 int gemm_f32(hipStream_t s, const void* a, const void* w, int bias_dtype, const void* bias, int mode, void* out, int T,
              int N, int K);
+int quad_parts(int T, int N, int K);
+int gemm_bf16_quad_parts(hipStream_t s, const void* x, const void* w, float* out, int T, int N, int K);
+int f32_parts(int T, int N, int K);
+int gemm_f32_parts(hipStream_t s, const void* a, const void* w, void* out, int T, int N, int K);
 }  // namespace sprout
 
 using namespace sprout;
@@ -39,4 +43,20 @@ extern "C" int sp_gemm(void* stream, int a_dtype, const void* a, int w_dtype, co
     if (gemm_f32_takes(T, N, K, a, w, out)) return gemm_f32(s, a, w, bias_dtype, bias, mode, out, T, N, K);
   }
   return gemm_generic(s, a_dtype, a, w_dtype, w, bias_dtype, bias, mode, out_dtype, out, T, N, K);
+}
+
+// Parts of K in which a[T, K] . w[N, K]^T is better stored than added to a float32 sum, where the norm that reads the sum joins them
+// (sp_rmsnorm_join), or 0.  Nobody adds to another's sum then, so the sums are the same in every run.
+extern "C" int sp_gemm_parts_plan(int dtype, int T, int N, int K) {
+  if (T < 1 || N < 8 || N % 8 != 0 || N > 8192 || K < 64) return 0;
+  return dtype == kBF16 ? quad_parts(T, N, K) : dtype == kF32 ? f32_parts(T, N, K) : 0;
+}
+
+// out[p] (float32 [parts][T][N]) = the share of part p of K in a . w^T; parts as sp_gemm_parts_plan says.
+extern "C" int sp_gemm_parts(void* stream, int dtype, const void* a, const void* w, float* out, int parts, int T, int N, int K) {
+  SP_REQUIRE(parts > 1 && parts == sp_gemm_parts_plan(dtype, T, N, K), "sp_gemm_parts: %d parts are not the plan of T=%d N=%d K=%d", parts, T, N, K);
+  SP_REQUIRE(a && w && out && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) & 15) == 0,
+             "sp_gemm_parts: null operand, or one that does not start at a multiple of 16 bytes");
+  hipStream_t s = (hipStream_t)stream;
+  return dtype == kBF16 ? gemm_bf16_quad_parts(s, a, w, out, T, N, K) : gemm_f32_parts(s, a, w, out, T, N, K);
 }

@@ -32,6 +32,8 @@ struct RopeArgs {
   long long out_stride, second_stride;
   // STRIDED: elements from one row of the output to the next
   long long row_stride;
+  // the float32 store of the four-wave product: where not 0, the sums of every part of K go to out[part][T][N]
+  int parts;
 };
 
 // Orders a wave's LDS writes before its own later reads of what other lanes wrote (and the reverse).

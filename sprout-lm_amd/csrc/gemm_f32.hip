@@ -27,20 +27,40 @@ int choose_shape(int T, int N, float* least = nullptr) {
 }
 
 template <int WM, int WN, int WAVES_M, int WAVES_N, int STAGES, typename TB>
-int launch_f32(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K) {
+int launch_f32(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K, int parts) {
   if (mode == kAccumulate)
     return launch_pipe_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kAccumulate, TB, float>(s, 1, x, w, (const TB*)bias, out, T, N, K, K);
-  return launch_pipe_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, TB, float>(s, 1, x, w, (const TB*)bias, out, T, N, K, K);
+  const int k_per_part = (K / 32 + parts - 1) / parts * 32;
+  return launch_pipe_mode<WM, WN, WAVES_M, WAVES_N, STAGES, kStoreF32, TB, float>(s, parts, x, w, (const TB*)bias, out, T, N, K, k_per_part);
 }
 
 template <typename TB>
-int launch_shape(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K) {
-  switch (choose_shape(T, N)) {
-    case 0: return launch_f32<2, 2, 4, 2, 3, TB>(s, x, w, bias, mode, out, T, N, K);
-    case 1: return launch_f32<1, 2, 4, 2, 4, TB>(s, x, w, bias, mode, out, T, N, K);
-    case 2: return launch_f32<1, 2, 2, 2, 3, TB>(s, x, w, bias, mode, out, T, N, K);
-    default: return launch_f32<1, 1, 2, 2, 4, TB>(s, x, w, bias, mode, out, T, N, K);
+int launch_shape(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K, int shape,
+                 int parts = 1) {
+  switch (shape) {
+    case 0: return launch_f32<2, 2, 4, 2, 3, TB>(s, x, w, bias, mode, out, T, N, K, parts);
+    case 1: return launch_f32<1, 2, 4, 2, 4, TB>(s, x, w, bias, mode, out, T, N, K, parts);
+    case 2: return launch_f32<1, 2, 2, 2, 3, TB>(s, x, w, bias, mode, out, T, N, K, parts);
+    default: return launch_f32<1, 1, 2, 2, 4, TB>(s, x, w, bias, mode, out, T, N, K, parts);
   }
+}
+
+// Shape and parts of K of an accumulating product of few tiles whose parts are stored side by side.
+int choose_parts(int T, int N, int K, int* shape) {
+  const int steps = K / 32;
+  const float million = 1e-6f * float(T) * float(N);
+  int best_parts = 1;
+  float best = 1e30f;
+  for (int i = 0; i < 4; ++i)
+    for (int parts : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      const int per_part = (steps + parts - 1) / parts;
+      if (parts > 1 && (per_part < 4 || (steps + per_part - 1) / per_part != parts)) continue;
+      const long blocks = long((T + kShapes[i].bm - 1) / kShapes[i].bm) * ((N + kShapes[i].bn - 1) / kShapes[i].bn) * parts;
+      const float round = per_part * 0.6f * (kShapes[i].bm * kShapes[i].bn * kShapes[i].cost) / (64 * 64 * 1.25f);
+      const float t = float((blocks + 255) / 256) * round + (parts > 1 ? (0.7f * parts + 0.8f * (parts + 1)) * million : 1.4f * million);
+      if (t < best) { best = t; best_parts = parts; *shape = i; }
+    }
+  return best_parts;
 }
 
 }  // namespace
@@ -58,12 +78,27 @@ bool gemm_f32_takes(int T, int N, int K, const void* a, const void* w, const voi
          (reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
 }
 
+// Parts of K in which an accumulating product is better stored for the norm behind it to join, 0 where it is better added.  Rows alone give
+// few blocks: 160 tokens, 896 rows of 4,864 are 42 of 64 x 64 on 256 CUs.  From 256 tokens on the products in bfloat16 parts
+// (gemm_split.hip) take the norm as theirs.
+int f32_parts(int T, int N, int K) {
+  int shape;
+  if (T <= 16 || T >= 256 || K % 32 != 0 || int64_t(K) * 4 * 256 >= (int64_t(1) << 32)) return 0;
+  const int parts = choose_parts(T, N, K, &shape);
+  return parts > 1 && size_t(parts) * T * N <= (size_t(32) << 20) ? parts : 0;
+}
+int gemm_f32_parts(hipStream_t s, const void* a, const void* w, void* out, int T, int N, int K) {
+  int shape = 0;
+  const int parts = choose_parts(T, N, K, &shape);
+  return launch_shape<float>(s, (const float*)a, (const float*)w, nullptr, kStoreF32, (float*)out, T, N, K, shape, parts);
+}
+
 // mode: kAccumulate (out += ...) or anything else (out = ...); out is float32 either way.
 int gemm_f32(hipStream_t s, const void* a, const void* w, int bias_dtype, const void* bias, int mode, void* out, int T,
              int N, int K) {
   if (bias && bias_dtype == kBF16)
-    return launch_shape<bf16_t>(s, (const float*)a, (const float*)w, bias, mode, (float*)out, T, N, K);
-  return launch_shape<float>(s, (const float*)a, (const float*)w, bias, mode, (float*)out, T, N, K);
+    return launch_shape<bf16_t>(s, (const float*)a, (const float*)w, bias, mode, (float*)out, T, N, K, choose_shape(T, N));
+  return launch_shape<float>(s, (const float*)a, (const float*)w, bias, mode, (float*)out, T, N, K, choose_shape(T, N));
 }
 
 }  // namespace sprout

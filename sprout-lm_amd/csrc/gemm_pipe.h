@@ -135,6 +135,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, (WAVES_M * WAVES_N <= 4 ? 2
   const int n0 = tile_n * BN;
   const int k_begin = blockIdx.z * k_per_split, k_end = min(K, k_begin + k_per_split);
   const int steps = (k_end - k_begin) / KSTEP;
+  if (MODE == kStoreF32 && !GROUPED) out = reinterpret_cast<float*>(out) + size_t(blockIdx.z) * T * N;   // parts of K lie side by side
   typedef __attribute__((address_space(3))) unsigned char* lds_address_t;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_address_t)pipe_lds;   // the tiles' offset within the LDS
 

@@ -315,6 +315,18 @@ __device__ __forceinline__ void quad_epilogue(floatx4 (&acc)[WM][WN], float* tur
   }
 }
 
+// Which tile and which part of K block `block` of `blocks` takes where the parts are stored side by side: every XCD has an equal run of
+// all of them, numbered part by part and in a part weight tile by weight tile, so that an XCD reads its run's share of K and of the
+// weights alone.  (K in two parts, 2,048 tokens, 896 rows of 4,864 on 128 x 128: numbered as the other products are, where an XCD has
+// tiles of every part, 28.5 us, so 24.8; 1,238 tokens in four 21.8 and 18.9; 264 tokens, 3,584 rows of 18,944 in six 51.3 and 49.)
+__host__ __device__ inline void quad_part_of(int tiles_t, int tiles_n, int block, int blocks, int* tile_t, int* tile_n, int* part) {
+  const int xcd = block & 7, each = blocks >> 3, more = blocks & 7;
+  const int id = xcd * each + (xcd < more ? xcd : more) + (block >> 3);
+  *tile_t = id % tiles_t;
+  *tile_n = id / tiles_t % tiles_n;
+  *part = id / tiles_t / tiles_n;
+}
+
 // A block of 2 x 2 waves, each with WM x WN tiles of 16 x 16: BM = 32 WM tokens by BN = 32 WN weight rows.
 // Requires: K and the split multiples of 64, N of 8 (kSilu: N counts gate rows), 16-byte aligned operands, every
 // offset of a tile's row within 32 bits (gemm_pipe_takes).
@@ -333,11 +345,16 @@ __global__ __launch_bounds__(256, (quad_shares_cu<WM, WN, NA> ? 2 : 1)) void gem
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
   const int li = lane & 15, lq = lane >> 4;
-  int tile_n, tile_t;
-  const PipeTiles tiles = pipe_tiles((T + BM - 1) / BM, ((MODE == kSilu ? 2 * N : N) + BN - 1) / BN);
-  if (!pipe_tile_of(tiles, blockIdx.x, &tile_t, &tile_n)) return;
+  int tile_n, tile_t, part = blockIdx.z;
+  if (MODE == kStoreF32 && rope.parts > 0) {
+    quad_part_of((T + BM - 1) / BM, (N + BN - 1) / BN, blockIdx.x, gridDim.x, &tile_t, &tile_n, &part);
+    out = reinterpret_cast<float*>(out) + size_t(part) * T * N;
+  } else {
+    const PipeTiles tiles = pipe_tiles((T + BM - 1) / BM, ((MODE == kSilu ? 2 * N : N) + BN - 1) / BN);
+    if (!pipe_tile_of(tiles, blockIdx.x, &tile_t, &tile_n)) return;
+  }
   const int t0 = tile_t * BM, n0 = tile_n * BN;
-  const int k_begin = blockIdx.z * k_per_split, k_end = min(K, k_begin + k_per_split);
+  const int k_begin = part * k_per_split, k_end = min(K, k_begin + k_per_split);
   const int steps = (k_end - k_begin) / 64;
 
   // ---- what this lane fetches: row 8 (4 j + wave) + lane / 8 of each operand tile, for j < WM (WN)
@@ -530,6 +547,7 @@ inline int launch_quad(hipStream_t s, int splits, const uint16_t* x, const uint1
   const int k_per_split = (K / 64 + splits - 1) / splits * 64;
   const PipeTiles tiles = pipe_tiles((T + 32 * WM - 1) / (32 * WM), ((MODE == kSilu ? 2 * N : N) + 32 * WN - 1) / (32 * WN));
   dim3 grid(8 * (tiles.own + tiles.run), 1, (K + k_per_split - 1) / k_per_split);
+  if (MODE == kStoreF32 && rope.parts > 0) grid = dim3(((T + 32 * WM - 1) / (32 * WM)) * ((N + 32 * WN - 1) / (32 * WN)) * grid.z, 1, 1);
   gemm_quad_kernel<WM, WN, NA, MODE><<<grid, 256, lds, s>>>(x, w, bias, bias_dtype, out, T, N, K, k_per_split, rope);
   return check_launch("sp_gemm (four waves)");
 }
@@ -540,7 +558,7 @@ inline int launch_quad(hipStream_t s, int splits, const uint16_t* x, const uint1
   X(0, 2, 2, 4) X(1, 3, 4, 2) X(2, 4, 2, 4) X(3, 4, 4, 2) X(4, 4, 4, 4) X(5, 4, 6, 2) X(6, 5, 6, 2) X(7, 6, 4, 2) X(8, 6, 6, 2) \
   X(9, 8, 4, 3) X(10, 4, 8, 2) X(11, 5, 8, 2) X(12, 10, 4, 2) X(13, 6, 8, 2) X(14, 8, 6, 2) X(15, 9, 6, 2) X(16, 8, 8, 2)
 
-enum QuadKind { kQuadStore = 0, kQuadAccumulate = 1, kQuadGated = 2, kQuadRotating = 3 };   // as sp_quad_plan counts them
+enum QuadKind { kQuadStore = 0, kQuadAccumulate = 1, kQuadGated = 2, kQuadRotating = 3, kQuadParts = 4 };   // as sp_quad_plan counts them
 
 // Whether the four-wave kernel takes T x N x K (N: all weight rows): more than 64 tokens, from 17 on where it is the faster one; whole
 // steps of 64 along K, outputs in whole eights of a row.
@@ -553,8 +571,8 @@ inline bool quad_aligned(const void* x, const void* w, const void* out) {
 // are joined with float atomics, whose order differs from run to run and the sums' last bits with it: a product that comes out the
 // same in every run there does so on four waves too.
 bool gemm_cuts_k(int T, int N, int K);
-// Picks the shape and the split of K with the least estimated time.
-void quad_choice(int kind, int T, int N, int K, int* shape, int* splits);
+// Picks the shape and the split of K with the least estimated time, and returns that in microseconds.
+float quad_choice(int kind, int T, int N, int K, int* shape, int* splits);
 
 // The product on the shape that quad_choice picks (N as the kernel counts it: gate rows for kSilu).
 template <int MODE>

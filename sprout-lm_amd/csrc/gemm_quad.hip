@@ -54,9 +54,14 @@ static const float kAloneUs[] = {0.24f, 0.45f, 0.35f, 0.50f, 0.48f, 0.68f, 0.80f
 // of all shapes and splits (mean; 25 % at worst), 10 % less than the eight-wave kernel, and more than 3 % longer than that one on 18 (10 %
 // at worst).  (With the tokens read once an XCD whatever the weight tiles: 4,096 tokens by 512 rows of 8,192 in one part on 128 x 64, 80 us,
 // where 128 x 128 in two takes 48 and the eight-wave kernel 50.)
-void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
+//
+// Parts that are stored side by side and joined by the norm that reads them: their blocks are an equal run an XCD (quad_part_of), whose
+// operands are what the XCD reads, once each where the caches serve it; 0.7 us a million sums stored, and 5 TB/s for the norm to read all
+// parts and to write their sum.  Over 80 products (70 to 2,048 tokens, eight matrices of 896 to 5,120 rows) the choice takes 3 % longer than
+// the best of all shapes and parts, 10 % at worst.
+float quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
   const int steps = K / 64;
-  const bool cuts_k = kind == kQuadAccumulate && gemm_cuts_k(T, N, K);
+  const bool parts = kind == kQuadParts, cuts_k = parts || (kind == kQuadAccumulate && gemm_cuts_k(T, N, K));
   float best = 1e30f;
   *shape = 3;
   *splits = 1;
@@ -65,24 +70,47 @@ void quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
     if (kind == kQuadRotating && p.wn != 2 && p.wn % 4 != 0) continue;     // a lane holds both of a pair
     const int bm = 32 * p.wm, bn = 32 * p.wn, slots = 32 * p.per_cu;
     const PipeTiles tiles = pipe_tiles((T + bm - 1) / bm, (N + bn - 1) / bn);
-    const float memory = float(N) * float(K) * 2.f / 5.4e6f + float(tiles.full ? 8 : tiles.left) * 2.f * float(T) * float(K) / (p.buffers == 2 ? 8e6f : 9e6f);
-    const float memory2 = memory * memory;
+    const float caches = p.buffers == 2 ? 8e6f : 9e6f;
+    float memory = float(N) * float(K) * 2.f / 5.4e6f + float(tiles.full ? 8 : tiles.left) * 2.f * float(T) * float(K) / caches;
     for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (sp > 1 && (!cuts_k || steps / sp < 4)) break;
+      if (sp == 1 && parts) continue;
       const int k_steps = (steps + sp - 1) / sp;
       if ((steps + k_steps - 1) / k_steps != sp) continue;
-      const int blocks = (tiles.full * tiles.tiles_t + tiles.run) * sp, full = blocks / slots, rest = blocks % slots;
+      int blocks = (tiles.full * tiles.tiles_t + tiles.run) * sp;
+      if (parts) {
+        const int tiles_n = (N + bn - 1) / bn;
+        blocks = (tiles.tiles_t * tiles_n * sp + 7) / 8;
+        // what an XCD's run holds of one part: all token tiles and some weight tiles, or some token tiles of one weight tile
+        const float of_parts = fmaxf(1.f, float(sp) / 8.f), run = float(blocks) / of_parts;
+        const float rows = fminf(float(N), fminf(float(tiles_n), ceilf(run / tiles.tiles_t)) * bn), tokens = fminf(float(T), run * bm);
+        const float fetched = 16.f * of_parts * (rows + tokens) * float(K) / float(sp);
+        memory = float(N) * float(K) * 2.f / 5.4e6f + (fetched - float(N) * float(K) * 2.f) / caches;
+      }
+      const float memory2 = memory * memory;
+      const int full = blocks / slots, rest = blocks % slots;
       const float ends = 0.14f * float(p.wm * p.wn) + 0.95f;
       const float block = k_steps * kStepUs[c] * (p.per_cu == 2 && k_steps > 20 ? 1.07f : 1.f) + ends, alone = k_steps * kAloneUs[c] + ends;
       float t = full * block;
       if (rest > 32) t += fmaxf(alone, block * (0.81f + 0.19f * float(rest - 32) / 32.f));
       else if (rest) t += alone * (0.79f + 0.21f * float(rest) / 32.f);
       t = sqrtf(sqrtf(t * t * t * t + memory2 * memory2));
-      if (sp > 1) t += 1.9e-6f * float(T) * float(N) * sp;
+      if (parts) t += (0.7e-6f * sp + 0.8e-6f * (sp + 1)) * float(T) * float(N);
+      else if (sp > 1) t += 1.9e-6f * float(T) * float(N) * sp;
       else if (kind == kQuadAccumulate) t += 1.4e-6f * float(T) * float(N);
       if (t < best) { best = t; *shape = c; *splits = sp; }
     }
   }
+  return best;
+}
+
+// Parts of K in which the accumulating product is better stored for the norm behind it to join, 0 where it is better added: more than 64
+// tokens, at most 128 MiB of sums.
+int quad_parts(int T, int N, int K) {
+  int shape, parts, splits;
+  if (T <= 64 || !gemm_quad_takes(kQuadAccumulate, T, N, K) || K / 64 < 8) return 0;
+  const float stored = quad_choice(kQuadParts, T, N, K, &shape, &parts), added = quad_choice(kQuadAccumulate, T, N, K, &shape, &splits);
+  return stored < added && size_t(parts) * T * N <= (size_t(32) << 20) ? parts : 0;
 }
 
 int gemm_bf16_quad_store(hipStream_t s, const void* x, const void* w, int bias_dtype, const void* bias, bool f32, void* out, int T, int N, int K,
@@ -96,16 +124,25 @@ int gemm_bf16_quad(hipStream_t s, const void* x, const void* w, int bias_dtype, 
 }  // namespace sprout
 
 // What the four-wave product would do with T x N x K: kind 0 store, 1 accumulate, 2 gated (N = 2 I rows of w), 3 rotating (head size
-// hd).  plan = {block rows, block columns, splits of K, buffers of x}.  Returns 1 where it does not take the product, else 0.  Runs
+// hd), 4 parts side by side.  plan = {block rows, block columns, splits of K, buffers of x}.  Returns 1 where it does not take the product, else 0.  Runs
 // nothing: for tests and tools.
 extern "C" int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan) {
   using namespace sprout;
-  if (T < 1 || N < 1 || K < 1 || kind < 0 || kind > 3 || !plan || (kind == kQuadRotating && hd < 1) || !gemm_quad_takes(kind, T, N, K, hd)) return 1;
+  if (T < 1 || N < 1 || K < 1 || kind < 0 || kind > 4 || !plan || (kind == kQuadRotating && hd < 1) || !gemm_quad_takes(kind, T, N, K, hd)) return 1;
   int shape, splits;
   quad_choice(kind, T, N, K, &shape, &splits);
   plan[0] = 32 * kQuadShapes[shape].wm;
   plan[1] = 32 * kQuadShapes[shape].wn;
   plan[2] = splits;
   plan[3] = kQuadShapes[shape].buffers;
+  return 0;
+}
+
+// The tiles of a product in `parts` parts side by side, block by block: tile_of[3 b] = (token tile, weight tile, part) of block b of
+// tiles_t * tiles_n * parts.  Runs nothing: for tests.
+extern "C" int sp_quad_part_tiles(int tiles_t, int tiles_n, int parts, int* tile_of) {
+  if (tiles_t < 1 || tiles_n < 1 || parts < 1 || !tile_of) return 1;
+  const int blocks = tiles_t * tiles_n * parts;
+  for (int b = 0; b < blocks; ++b) sprout::quad_part_of(tiles_t, tiles_n, b, blocks, &tile_of[3 * b], &tile_of[3 * b + 1], &tile_of[3 * b + 2]);
   return 0;
 }

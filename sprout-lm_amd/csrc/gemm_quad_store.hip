@@ -9,4 +9,11 @@ int gemm_bf16_quad_store(hipStream_t s, const void* x, const void* w, int bias_d
   return quad_run<kStore>(s, kQuadStore, x, w, bias, bias_dtype, out, T, N, K, epilogue);
 }
 
+// The sums of every part of K, side by side (the plan is quad_parts').
+int gemm_bf16_quad_parts(hipStream_t s, const void* x, const void* w, float* out, int T, int N, int K) {
+  RopeArgs epilogue = {};
+  epilogue.parts = 1;
+  return quad_run<kStoreF32>(s, kQuadParts, x, w, nullptr, kF32, out, T, N, K, epilogue);
+}
+
 }  // namespace sprout

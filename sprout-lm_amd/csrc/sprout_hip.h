@@ -23,6 +23,15 @@ int sp_embed(void* stream, int table_dtype, const void* table, const int32_t* to
 int sp_rmsnorm(void* stream, const float* x, const int32_t* rows, int w_dtype, const void* w, float eps,
                int out_dtype, void* out, int R, int H);
 
+// A product whose sum is joined by the norm that reads it: sp_gemm_parts stores what each of `parts` (sp_gemm_parts_plan; 0: not this
+// way) parts of K contributes, float32 [parts][T][N]; sp_rmsnorm_join is sp_rmsnorm of x + their sum (which becomes x where no rows are
+// listed), sp_join that sum alone.
+int sp_gemm_parts_plan(int dtype, int T, int N, int K);
+int sp_gemm_parts(void* stream, int dtype, const void* a, const void* w, float* out, int parts, int T, int N, int K);
+int sp_rmsnorm_join(void* stream, float* x, const float* parts, int n_parts, int T, const int32_t* rows, int w_dtype, const void* w, float eps,
+                    int out_dtype, void* out, int R, int H);
+int sp_join(void* stream, float* x, const float* parts, int n_parts, long long n);
+
 // out = a[T, K] . w[N, K]^T (+ bias[N])
 // mode 0: store as out_dtype [T, N];  mode 1: out (float32 [T, N]) += result;  mode 2: store float32
 int sp_gemm(void* stream, int a_dtype, const void* a, int w_dtype, const void* w, int bias_dtype,
@@ -52,6 +61,7 @@ int sp_pipe_plan(int kind, int T, int N, int K, int* plan);
 // How that kernel numbers its blocks: tile_of[2 b], tile_of[2 b + 1] = token tile and weight tile of block b (which
 // runs on XCD b % 8), -1 for a block with nothing to do; returns the number of blocks.  Runs nothing.
 int sp_pipe_tiles(int tiles_t, int tiles_n, int* tile_of, int room);
+int sp_quad_part_tiles(int tiles_t, int tiles_n, int parts, int* tile_of);
 // The same of the product on four waves a block, which takes more than 64 tokens, and from 17 on where it is the faster one, with
 // outputs in whole eights that start at 16 bytes (other kernels have the rest), and is the only one to rotate (kind 3, head size hd):
 // plan = {block rows, block columns, splits of K, buffers of x}.

@@ -137,6 +137,9 @@ class StepContext:
         self.group_slots: list[torch.Tensor] = []
         self.extra = {}  # arrays that parts have registered (register_step_array), by name, on the device
         self.host = {}   # the same arrays on the host (numpy), for parts that plan on the CPU
+        self.owed = None   # parts of a product (`ops.gemm_parts`) that the next norm adds to the residual
+        self.joins = None  # the residual that such a product of the running part may be left to
+        self.settles = False   # whether whoever reads the residual next settles what is owed
         self.shared = {}   # what a part computes once per step for all layers (key chosen by the part)
 
     def buffer(self, name: str, shape, dtype) -> torch.Tensor:

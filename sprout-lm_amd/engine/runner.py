@@ -298,13 +298,20 @@ class ModelRunner:
             if kept_rows is not None:
                 kept_rows.copy_(residual)
                 ctx.shared["embedding"] = kept_rows
+            ctx.owed = ctx.joins = None
             for i, call in enumerate(self.plan.schedule):
-                self.parts.blocks[call.layer].forward(ctx, residual, self._slot_views(ctx, i))
+                block = self.parts.blocks[call.layer]
+                if ctx.owed is not None and not block.settles:
+                    ops.join(residual, ctx.owed)
+                    ctx.owed = None
+                ctx.settles = block.settles
+                block.forward(ctx, residual, self._slot_views(ctx, i))
+            ctx.settles = False
             n = ctx.n_logits
             logits = ctx.buffer("logits", (n, self.vocab_size), torch.float32)
             if n:
                 normed = ctx.buffer("final_normed", (n, H), self.dtype)
-                self.parts.final_norm.forward(ctx, residual, normed, rows=ctx.logit_rows)
+                self.parts.final_norm.forward_joining(ctx, residual, normed, rows=ctx.logit_rows)
                 self.parts.head.forward(ctx, normed, logits)
         return logits
 

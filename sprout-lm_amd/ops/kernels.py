@@ -2,6 +2,8 @@
 kernel that reads past a buffer can take the whole GPU down."""
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from .library import KernelError, check, library
@@ -576,6 +578,47 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: torch.Tensor
     check(library().sp_gemm(_stream(), _code(a, "gemm input"), a.data_ptr(), _code(w, "gemm weight"), w.data_ptr(),
                             _code(bias, "gemm bias") if bias is not None else 0, _ptr(bias), mode,
                             _code(out, "gemm output"), out.data_ptr(), T, N, K))
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_parts_plan(dtype: torch.dtype, T: int, N: int, K: int) -> int:
+    """Parts of K in which the product of T tokens by w [N, K], both of `dtype`, is better stored (`gemm_parts`) than added to a float32
+    sum, where the norm that reads that sum joins them (`rmsnorm_join`); 0 where it is better added."""
+    return library().sp_gemm_parts_plan(_CODES[dtype], T, N, K) if dtype in _CODES else 0
+
+
+def gemm_parts(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
+    """out[p] = what part p of K contributes to a @ w.T; out float32 [`gemm_parts_plan`, T, N]."""
+    _gpu(a, "gemm input"); _gpu(w, "gemm weight"); _gpu(out, "gemm output")
+    T, K = a.shape
+    N = w.shape[0]
+    if w.shape[1] != K or a.dtype != w.dtype or out.dtype != torch.float32 or out.dim() != 3 or tuple(out.shape[1:]) != (T, N):
+        raise KernelError(f"gemm_parts: shapes do not fit: a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
+    check(library().sp_gemm_parts(_stream(), _code(a, "gemm input"), a.data_ptr(), w.data_ptr(), out.data_ptr(), out.shape[0], T, N, K))
+
+
+def rmsnorm_join(x: torch.Tensor, parts: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor,
+                 rows: torch.Tensor | None = None) -> None:
+    """`rmsnorm` of x + the sum of `parts` (float32 [n, T, H], the shape of x).  Without rows that sum becomes x; with rows only theirs
+    is taken, and x stays as it is."""
+    _gpu(x, "norm input"); _gpu(parts, "parts"); _gpu(weight, "norm weight"); _gpu(out, "norm output")
+    R, H = out.shape
+    if (x.dtype != torch.float32 or parts.dtype != torch.float32 or tuple(parts.shape[1:]) != tuple(x.shape) or x.shape[1] != H
+            or weight.numel() != H or (rows is None and x.shape[0] != R)):
+        raise KernelError(f"rmsnorm_join: shapes do not fit: x {tuple(x.shape)} {x.dtype}, parts {tuple(parts.shape)}, weight {tuple(weight.shape)}, "
+                          f"out {tuple(out.shape)}")
+    if rows is not None:
+        _ints(rows, R, "norm rows")
+    check(library().sp_rmsnorm_join(_stream(), x.data_ptr(), parts.data_ptr(), parts.shape[0], x.shape[0], _ptr(rows), _code(weight, "norm weight"),
+                                    weight.data_ptr(), float(eps), _code(out, "norm output"), out.data_ptr(), R, H))
+
+
+def join(x: torch.Tensor, parts: torch.Tensor) -> None:
+    """x += the sum of `parts` (float32 [n, *x.shape])."""
+    _gpu(x, "sum"); _gpu(parts, "parts")
+    if x.dtype != torch.float32 or parts.dtype != torch.float32 or tuple(parts.shape[1:]) != tuple(x.shape) or x.numel() % 4:
+        raise KernelError(f"join: shapes do not fit: x {tuple(x.shape)} {x.dtype}, parts {tuple(parts.shape)}")
+    check(library().sp_join(_stream(), x.data_ptr(), parts.data_ptr(), parts.shape[0], x.numel()))
 
 
 def gemm_f32_split_bytes(T: int, N: int, K: int) -> int:

@@ -20,6 +20,10 @@ def _declare(lib):
         "sp_embed": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_float, c_void],
         "sp_rmsnorm": [c_void, c_void, c_void, c_int, c_void, c_float, c_int, c_void, c_int, c_int],
         "sp_gemm": [c_void, c_int, c_void, c_int, c_void, c_int, c_void, c_int, c_int, c_void, c_int, c_int, c_int],
+        "sp_gemm_parts_plan": [c_int] * 4,
+        "sp_gemm_parts": [c_void, c_int, c_void, c_void, c_void, c_int, c_int, c_int, c_int],
+        "sp_rmsnorm_join": [c_void, c_void, c_void, c_int, c_int, c_void, c_int, c_void, c_float, c_int, c_void, c_int, c_int],
+        "sp_join": [c_void, c_void, c_void, c_int, c_i64],
         "sp_gemm_f32_split": [c_void, c_int, c_void, c_void, c_float, c_int, c_float, c_void, c_int, c_void, c_int,
                               c_void, c_int, c_int, c_int, c_void, c_i64],
         "sp_rope_cache": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_int, c_int,
@@ -36,6 +40,7 @@ def _declare(lib):
         "sp_fused_norm_pays": [c_int] * 3,
         "sp_pipe_plan": [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int)],
         "sp_quad_plan": [c_int, c_int, c_int, c_int, c_int, ctypes.POINTER(c_int)],
+        "sp_quad_part_tiles": [c_int, c_int, c_int, ctypes.POINTER(c_int)],
         "sp_pipe_tiles": [c_int, c_int, ctypes.POINTER(c_int), c_int],
         "sp_gemm_decode": [c_void, c_void, c_void, c_int, c_void, c_float, c_void, c_int, c_void, c_int, c_void, c_int,
                            c_int, c_int],

@@ -9,7 +9,7 @@ from .. import ops
 from ..cache.spec import PagedKVSpec
 from ..config.base import ConfigError
 from ..weights.loader import TensorSpec
-from .base import Mixer, register_part
+from .base import Mixer, add_product, register_part
 
 
 @register_part("mixer", "attention")
@@ -27,6 +27,8 @@ class Attention(Mixer):
     """
 
     graph_safe = True
+
+    adds_last = True
 
     graph_safe_portions = True
 
@@ -149,7 +151,7 @@ class Attention(Mixer):
         if not (self._split_pays(ctx, attn, self.w_o)
                 and ops.gemm_f32_split(attn, self.w_o, residual, lambda n: ctx.buffer("f32_split", (n,), torch.uint8), bias=self.b_o,
                                        accumulate=True)):
-            ops.gemm(attn, self.w_o, residual, bias=self.b_o, accumulate=True)
+            add_product(ctx, attn, self.w_o, residual, bias=self.b_o)
 
     def forward(self, ctx, h, residual, cache):
         T = h.shape[0]

@@ -9,6 +9,9 @@ from __future__ import annotations
 
 from typing import Callable
 
+import torch
+
+from .. import ops
 from ..weights.loader import TensorSpec
 
 _REGISTRIES: dict[str, dict[str, type]] = {
@@ -97,10 +100,31 @@ class Part:
         return 0.0
 
 
+def add_product(ctx, x, w, residual, bias=None) -> None:
+    """residual += x @ w.T (+ bias), where nobody reads the residual before the norm that follows: where `ctx.joins` is this residual, the
+    product may be left to that norm in parts (`ctx.owed`, see `ops.gemm_parts`)."""
+    parts = 0
+    if bias is None and ctx.joins is residual and ctx.owed is None and (x.data_ptr() | w.data_ptr()) % 16 == 0 and x.dtype == w.dtype:
+        parts = ops.gemm_parts_plan(x.dtype, x.shape[0], *w.shape)
+    if parts:
+        owed = ctx.buffer("owed", (parts, x.shape[0], w.shape[0]), torch.float32)
+        ops.gemm_parts(x, w, owed)
+        ctx.owed = owed
+    else:
+        ops.gemm(x, w, residual, bias=bias, accumulate=True)
+
+
 class Norm(Part):
     def forward(self, ctx, x, out, rows=None):
         """out = norm(x[rows] or x).  x is the float32 residual stream, out has the activation dtype."""
         raise NotImplementedError
+
+    def forward_joining(self, ctx, x, out, rows=None):
+        """The same of x plus what is owed to it (`ctx.owed`, which is then settled: with `rows`, x itself stays without it)."""
+        owed, ctx.owed = ctx.owed, None
+        if owed is not None:
+            ops.join(x, owed)
+        return self.forward(ctx, x, out, rows)
 
     def fold(self):
         """How the norm can be computed inside the kernel of the product that follows it, or None if it
@@ -128,6 +152,8 @@ class PositionEncoding(Part):
 
 
 class Mixer(Part):
+    adds_last = False      # whether all that `forward` does to the residual is one `add_product`
+
     """Mixes information between the tokens of a sequence (attention, or anything with state)."""
 
     def forward(self, ctx, h, residual, cache):
@@ -174,6 +200,8 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    adds_last = False      # see Mixer.adds_last
+
     def forward(self, ctx, h, residual):
         """residual += feed_forward(h), token by token."""
         raise NotImplementedError
@@ -210,6 +238,8 @@ class StreamPart(Part):
 
 
 class Block(Part):
+    settles = False       # whether the block's first norm joins what a product before it has left (`ctx.owed`), and its own may be left
+
     """Arranges mixers, feed-forwards and their norms around the residual stream."""
 
     def parts(self) -> dict[str, Part]:

@@ -17,6 +17,8 @@ class PreNormBlock(Block):
 
     graph_safe_portions = True
 
+    settles = True
+
     def __init__(self, mixer_norm, mixer, ffn_norm=None, ffn=None, mixer_conv=None):
         self.mixer_norm, self.mixer, self.ffn_norm, self.ffn, self.mixer_conv = mixer_norm, mixer, ffn_norm, ffn, mixer_conv
 
@@ -32,19 +34,31 @@ class PreNormBlock(Block):
         T, H = residual.shape
         cache = caches.get("mixer")
         h = ctx.buffer("normed", (T, H), ctx.act_dtype)
+        # The next reader of the residual behind the mixer is this block's second norm, behind the feed-forward the norm of whatever
+        # follows, where that settles what is owed (`ctx.settles`): a last product may then be left to the norm in parts.
+        behind_mixer = residual if self.mixer.adds_last and ctx.settles else None
         if self.mixer_conv is not None:
-            self.mixer_norm.forward(ctx, residual, h)
+            self.mixer_norm.forward_joining(ctx, residual, h)
             mixed_in = ctx.buffer("normed_conv", (T, H), ctx.act_dtype)
             self.mixer_conv.forward(ctx, h, mixed_in, caches.get("mixer_conv"))
+            ctx.joins = behind_mixer
             self.mixer.forward(ctx, mixed_in, residual, cache)
-        elif not self.mixer.forward_from_residual(ctx, self.mixer_norm, residual, cache):
-            self.mixer_norm.forward(ctx, residual, h)
-            self.mixer.forward(ctx, h, residual, cache)
+        else:
+            ctx.joins = behind_mixer if ctx.owed is None else None
+            if ctx.owed is not None or not self.mixer.forward_from_residual(ctx, self.mixer_norm, residual, cache):
+                self.mixer_norm.forward_joining(ctx, residual, h)
+                ctx.joins = behind_mixer
+                self.mixer.forward(ctx, h, residual, cache)
+        ctx.joins = None
         if self.ffn is None:
             return
-        if not self.ffn.forward_from_residual(ctx, self.ffn_norm, residual):
-            self.ffn_norm.forward(ctx, residual, h)
+        behind_ffn = residual if self.ffn.adds_last and ctx.settles else None
+        ctx.joins = behind_ffn if ctx.owed is None else None
+        if ctx.owed is not None or not self.ffn.forward_from_residual(ctx, self.ffn_norm, residual):
+            self.ffn_norm.forward_joining(ctx, residual, h)
+            ctx.joins = behind_ffn
             self.ffn.forward(ctx, h, residual)
+        ctx.joins = None
 
 
 @register_part("block", "parallel")

@@ -5,7 +5,7 @@ import torch
 
 from .. import ops
 from ..weights.loader import TensorSpec
-from .base import FeedForward, register_part
+from .base import FeedForward, add_product, register_part
 
 
 @register_part("feed_forward", "gated_mlp")
@@ -15,6 +15,8 @@ class GatedMLP(FeedForward):
     g' * sigmoid(1.702 g') * (u' + 1); "relu": max(g, 0) * u; "gelu_tanh": gelu(g) * u, the tanh form)."""
 
     graph_safe = True
+
+    adds_last = True
 
     graph_safe_portions = True
 
@@ -61,7 +63,7 @@ class GatedMLP(FeedForward):
             if not ops.gate_up_silu_f32(self.w_gate_up, residual, act, activation=self.activation, norm_weight=fold.weight,
                                         eps=fold.eps, limit=self.limit):
                 return False
-            ops.gemm(act, self.w_down, residual, accumulate=True)
+            add_product(ctx, act, self.w_down, residual)
             return True
         if ctx.act_dtype != torch.bfloat16 or T > 64 or not self._fused(T, True):
             return False
@@ -70,7 +72,7 @@ class GatedMLP(FeedForward):
         act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
         ops.gate_up_silu(self.w_gate_up, act, residual=residual, norm_weight=fold.weight, eps=fold.eps,
                          activation=self.activation, limit=self.limit)
-        ops.gemm(act, self.w_down, residual, accumulate=True)
+        add_product(ctx, act, self.w_down, residual)
         return True
 
     def _split_f32(self, ctx, residual, fold) -> bool:
@@ -85,7 +87,7 @@ class GatedMLP(FeedForward):
                 and ops.gemm_f32_split(gu, self.w_down, residual, scratch, accumulate=True, activation=self.activation, limit=self.limit)):
             act = ctx.buffer("gated", (T, self.inner), ctx.act_dtype)
             ops.silu_mul(gu, act, activation=self.activation, limit=self.limit)
-            ops.gemm(act, self.w_down, residual, accumulate=True)
+            add_product(ctx, act, self.w_down, residual)
         return True
 
     def forward(self, ctx, h, residual, row_gate=None, row_gate_column: int = 0):
@@ -107,7 +109,7 @@ class GatedMLP(FeedForward):
             ops.gemm(h, self.w_gate_up, gu)
             ops.silu_mul(gu, act, activation=self.activation, limit=self.limit, row_gate=row_gate,
                          row_gate_column=row_gate_column)
-        ops.gemm(act, self.w_down, residual, accumulate=True)
+        add_product(ctx, act, self.w_down, residual)
 
 
 @register_part("feed_forward", "mlp")

@@ -36,6 +36,13 @@ class RMSNorm(Norm):
         ops.rmsnorm(x, self.weight, self.eps, out, rows)
         return out
 
+    def forward_joining(self, ctx, x, out, rows=None):
+        if ctx.owed is None:
+            return self.forward(ctx, x, out, rows)
+        owed, ctx.owed = ctx.owed, None
+        ops.rmsnorm_join(x, owed, self.weight, self.eps, out, rows)
+        return out
+
     def fold(self):
         return NormFold("rms", self.weight, self.eps)
 
