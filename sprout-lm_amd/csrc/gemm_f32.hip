@@ -145,7 +145,11 @@ struct SkinnyExtra {
   long long row_gate_stride;
 };
 
-template <int RT, int MODE, typename TB, bool NORM, int WAVES = 4>   // MODE: kStoreF32, kAccumulate, kSilu or kRope
+// STAGED (with NORM; up to 8 tokens of K up to 1,024): the block normalises its tokens' rows once, into LDS, from where the waves take them
+// as operands: a row is read from the caches once and not twice, and without it and the norm's weights a wave has registers to ask
+// for all its weights in one trip.  (8 tokens, 4,864 gate and up rows of 896: 15.4 -> 12.4 us; with the weights in
+// the caches 13.1 -> 10.7.  q/k/v of 14 + 2 + 2 heads of 64: 9.2 -> 8.3.)
+template <int RT, int MODE, typename TB, bool NORM, int WAVES = 4, bool STAGED = false>   // MODE: kStoreF32, kAccumulate, kSilu or kRope
 __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                               const TB* __restrict__ bias, float* __restrict__ out,
                                                               int T, int N, int K, int steps_per_block, SkinnyExtra extra) {
@@ -179,15 +183,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float
   const float* xrow = x + size_t(min(lr, T - 1)) * K + 4 * lj;
   const bool token = lr < T;
 
-  constexpr int U = RT <= 2 ? 8 : 4;      // steps requested together: what a wave has on its way
-  float4 wv[U][RT], xv[U], nv[U];
+  constexpr int U = STAGED ? 64 / WAVES : RT <= 2 ? 8 : 4;      // steps requested together: what a wave has on its way
+  float4 wv[U][RT], xv[STAGED ? 1 : U], nv[STAGED ? 1 : U];
   auto request = [&](int s) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = 16 * (s + u);
       const bool in = s + u < s1 && k + 4 * lj < K;
-      xv[u] = (in && token) ? *reinterpret_cast<const float4*>(xrow + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-      if (NORM) nv[u] = in ? *reinterpret_cast<const float4*>(extra.norm_w + k + 4 * lj) : make_float4(0.f, 0.f, 0.f, 0.f);
+      if (!STAGED) xv[u] = (in && token) ? *reinterpret_cast<const float4*>(xrow + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      if (NORM && !STAGED) nv[u] = in ? *reinterpret_cast<const float4*>(extra.norm_w + k + 4 * lj) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
         wv[u][rt] = in ? *reinterpret_cast<const float4*>(wrow[rt] + k) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -198,7 +202,39 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float
   // caches, and what returns from memory returns in the order asked for), the weights before anything is summed:
   // they are on their way meanwhile, and the rest of a longer row queues behind them.
   float scale = 1.f;
-  if (NORM) {
+  extern __shared__ float normed[];      // STAGED: [8][K + 4]
+  if constexpr (STAGED) {
+    static_assert(NORM && RT == 1, "normalised rows are what is staged");
+    constexpr int P = 8 * WAVES, NB = 256 / P;          // threads a token, all in one wave; 16-byte pieces a thread
+    const int t = threadIdx.x / P, part = threadIdx.x % P;
+    const float* row = x + size_t(min(t, T - 1)) * K;
+    float4 mine[NB], weight[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int k = 4 * (part + j * P);
+      mine[j] = k < K ? *reinterpret_cast<const float4*>(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int k = 4 * (part + j * P);
+      weight[j] = k < K ? *reinterpret_cast<const float4*>(extra.norm_w + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    request(s0);
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) sum = fmaf(mine[j].x, mine[j].x, fmaf(mine[j].y, mine[j].y, fmaf(mine[j].z, mine[j].z, fmaf(mine[j].w, mine[j].w, sum))));
+#pragma unroll
+    for (int o = P / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    scale = 1.0f / sqrtf(sum / float(K) + extra.eps);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int k = 4 * (part + j * P);
+      if (k < K)
+        *reinterpret_cast<float4*>(normed + t * (K + 4) + k) = make_float4((mine[j].x * scale) * weight[j].x, (mine[j].y * scale) * weight[j].y,
+                                                                           (mine[j].z * scale) * weight[j].z, (mine[j].w * scale) * weight[j].w);
+    }
+    __syncthreads();
+  } else if (NORM) {
     constexpr int P = 4 * WAVES, NB = 8;
     const int t = threadIdx.x / P, part = threadIdx.x % P;
     const float* row = x + size_t(min(t, T - 1)) * K;
@@ -243,15 +279,20 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (s + u >= s1) break;      // the same for the whole wave
-      if (NORM)
-        xv[u] = make_float4((xv[u].x * scale) * nv[u].x, (xv[u].y * scale) * nv[u].y, (xv[u].z * scale) * nv[u].z,
-                            (xv[u].w * scale) * nv[u].w);
+      float4 a;
+      if constexpr (STAGED) {
+        // (columns of tokens past the last one repeat the eighth row and are not used)
+        a = *reinterpret_cast<const float4*>(normed + min(lr, 7) * (K + 4) + min(16 * (s + u) + 4 * lj, K - 4));
+      } else {
+        a = xv[u];
+        if (NORM) a = make_float4((a.x * scale) * nv[u].x, (a.y * scale) * nv[u].y, (a.z * scale) * nv[u].z, (a.w * scale) * nv[u].w);
+      }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].x, xv[u].x, acc[rt], 0, 0, 0);
-        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].y, xv[u].y, acc[rt], 0, 0, 0);
-        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].z, xv[u].z, acc[rt], 0, 0, 0);
-        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].w, xv[u].w, acc[rt], 0, 0, 0);
+        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].x, a.x, acc[rt], 0, 0, 0);
+        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].y, a.y, acc[rt], 0, 0, 0);
+        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].z, a.z, acc[rt], 0, 0, 0);
+        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][rt].w, a.w, acc[rt], 0, 0, 0);
       }
     }
   }
@@ -351,33 +392,44 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float
   }
 }
 
-template <int RT, typename TB>
+template <int RT, typename TB, int WAVES>
 int launch_skinny(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K) {
   const int blocks_n = (N + 16 * RT - 1) / (16 * RT), steps = (K + 15) / 16;
   int splits = 1;
   if (mode == kAccumulate && blocks_n < 256) {
-    // rows alone give too few blocks: K is shared out too, while every wave keeps 8 steps or more
+    // rows alone give too few blocks: K is shared out too, while every wave of four keeps 8 steps or more
     splits = max(1, min((512 + blocks_n - 1) / blocks_n, steps / 32));
   }
   const int per_block = (steps + splits - 1) / splits;
   splits = (steps + per_block - 1) / per_block;
   dim3 grid(blocks_n, splits);
   if (mode == kAccumulate)
-    gemm_f32_skinny_kernel<RT, kAccumulate, TB, false><<<grid, 256, 0, s>>>(x, w, (const TB*)bias, out, T, N, K, per_block, SkinnyExtra{});
+    gemm_f32_skinny_kernel<RT, kAccumulate, TB, false, WAVES><<<grid, 64 * WAVES, 0, s>>>(x, w, (const TB*)bias, out, T, N, K, per_block, SkinnyExtra{});
   else
-    gemm_f32_skinny_kernel<RT, kStoreF32, TB, false><<<grid, 256, 0, s>>>(x, w, (const TB*)bias, out, T, N, K, per_block, SkinnyExtra{});
+    gemm_f32_skinny_kernel<RT, kStoreF32, TB, false, WAVES><<<grid, 64 * WAVES, 0, s>>>(x, w, (const TB*)bias, out, T, N, K, per_block, SkinnyExtra{});
   return check_launch("sp_gemm (float32, few tokens)");
 }
 
 template <typename TB>
 int skinny_shape(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K) {
+  // Eight waves share K where that brings a wave's steps down to the 8 that it asks for at once: matrices of up to 8 M weights, and heads of
+  // a short K (8 tokens, four waves -> eight, us: 896 rows of 4,864 7.86 -> 7.39, 896 of 896 6.43 -> 5.85, 1,152 of 896 5.86 -> 5.35, 2,560 of
+  // 2,560 12.1 -> 11.3, 151,936 of 896 138.7 -> 134.3).  Larger ones are bound by what the chip has on its way, and eight waves' sums cost
+  // them more than they save (1,536 of 8,960 21.0 -> 21.6, 4,608 of 3,584 30.0 -> 32.1, 5,120 of 5,120 44.2 -> 46.7, 32,000 of 256 10.5 -> 11.3).
   const int tiles = (N + 15) / 16;
-  if (tiles >= 4096) return launch_skinny<4, TB>(s, x, w, bias, mode, out, T, N, K);
-  if (tiles >= 1024) return launch_skinny<2, TB>(s, x, w, bias, mode, out, T, N, K);
-  return launch_skinny<1, TB>(s, x, w, bias, mode, out, T, N, K);
+  const bool eight = size_t(N) * K <= 8000000 || (tiles >= 4096 && K <= 2048);
+  if (tiles >= 4096)
+    return eight ? launch_skinny<4, TB, 8>(s, x, w, bias, mode, out, T, N, K) : launch_skinny<4, TB, 4>(s, x, w, bias, mode, out, T, N, K);
+  if (tiles >= 1024)
+    return eight ? launch_skinny<2, TB, 8>(s, x, w, bias, mode, out, T, N, K) : launch_skinny<2, TB, 4>(s, x, w, bias, mode, out, T, N, K);
+  return eight ? launch_skinny<1, TB, 8>(s, x, w, bias, mode, out, T, N, K) : launch_skinny<1, TB, 4>(s, x, w, bias, mode, out, T, N, K);
 }
 
 }  // namespace
+
+// STAGED: the rows that fit the LDS and a block's registers, all of a wave's weights in one trip.
+static bool staged_takes(int T, int K) { return T <= 8 && K <= 1024; }
+static int staged_bytes(int K) { return 8 * (K + 4) * 4; }
 
 // out[T, I] = silu(a . w[:I]^T) * (a . w[I:]^T) for up to 16 tokens, float32 throughout; a = x, or
 // rmsnorm(x) * norm_w where norm_w is given.
@@ -399,7 +451,10 @@ int gemm_f32_gated(hipStream_t s, const float* x, const float* norm_w, float eps
     if (norm_w) SP_GATED(2, true, pairs); else SP_GATED(2, false, pairs);
   } else {
     // few rows: tiles of 8 gate rows and their 8 up rows, twice the blocks
-    if (norm_w) SP_GATED(1, true, (I + 7) / 8); else SP_GATED(1, false, (I + 7) / 8);
+    if (norm_w && staged_takes(T, K))
+      gemm_f32_skinny_kernel<1, kSilu, float, true, 4, true><<<dim3((I + 7) / 8, 1), 256, staged_bytes(K), s>>>(x, w, nullptr, out, T, I, K, steps, extra);
+    else if (norm_w) SP_GATED(1, true, (I + 7) / 8);
+    else SP_GATED(1, false, (I + 7) / 8);
   }
 #undef SP_GATED
   return check_launch("sp_gate_up_silu_f32");
@@ -408,7 +463,9 @@ int gemm_f32_gated(hipStream_t s, const float* x, const float* norm_w, float eps
 template <typename TB, int WAVES>
 static int launch_qkv_waves(hipStream_t s, const float* x, const float* w, const void* bias, float* q_out, int T, int K,
                             const SkinnyExtra& extra, int N, int blocks, int steps) {
-  if (extra.norm_w)
+  if (extra.norm_w && staged_takes(T, K))
+    gemm_f32_skinny_kernel<1, kRope, TB, true, WAVES, true><<<dim3(blocks, 1), 64 * WAVES, staged_bytes(K), s>>>(x, w, (const TB*)bias, q_out, T, N, K, steps, extra);
+  else if (extra.norm_w)
     gemm_f32_skinny_kernel<1, kRope, TB, true, WAVES><<<dim3(blocks, 1), 64 * WAVES, 0, s>>>(x, w, (const TB*)bias, q_out, T, N, K, steps, extra);
   else
     gemm_f32_skinny_kernel<1, kRope, TB, false, WAVES><<<dim3(blocks, 1), 64 * WAVES, 0, s>>>(x, w, (const TB*)bias, q_out, T, N, K, steps, extra);
