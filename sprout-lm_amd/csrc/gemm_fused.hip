@@ -184,7 +184,14 @@ __device__ __forceinline__ int weight_row(const FusedArgs& a, int b, int i, int 
   return min(a.N - 1, row);
 }
 
-template <int TN, int EPI, bool NORM, int NT, bool K64, int UN>
+// STAGED (with NORM, K up to kStagedK): the block normalises its 8 or 16 rows once, into LDS, from where the waves take their operands; taken from
+// memory, a wave's come 16 rows apart, and the rows are what a block of few weights mostly reads.  (q/k/v of 14 + 2 + 2 heads of 64 at 896, us:
+// 64 tokens 6.53 -> 6.17, 32 5.94 -> 6.29, 16 5.84 -> 6.12, 8 5.49 -> 5.25, 4 5.06 -> 4.98, 1 4.92 -> 4.98; 8 + 2 + 2 of 128 at 1,024: 64 tokens 7.26
+// -> 6.36, 8 5.78 -> 5.31; the gated product 7.77 -> 7.76 at 8 tokens, 7.51 -> 7.73 at one.)
+constexpr int kStagedK = 1024;
+__host__ __device__ constexpr int staged_pitch(int K) { return K + 8; }      // bfloat16 numbers from one row to the next: banks shift by 4
+
+template <int TN, int EPI, bool NORM, int NT, bool K64, int UN, int STAGED = 0>
 __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
   static_assert(NT == 2 || EPI == kEpiRope || EPI == kEpiSilu, "one or three tiles a block only where rows are paired");
   static_assert(!NORM || TN == 1, "the norm prologue takes one tile of 16 tokens");
@@ -260,14 +267,38 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
     }
   };
   // The norm prologue's rows are requested right after the weights; both are then on their way together.
-  NormInputs<NORM ? UN : 1, K64> normed;
+  NormInputs<NORM && !STAGED ? UN : 1, K64> normed;
   auto request_rows = [&](int s0) {
     normed.request(norm_row + 64 * s0, norm_w0 + size_t(64 * s0) * (a.norm_w_bf16 ? 2 : 4), a.norm_w_bf16, steps - s0,
                    k_end - (k_begin + 16 * lj + 64 * s0), a.residual, a.norm_w);
   };
   // NORM: the rows first (they come from the caches and are needed first: their sum of squares is exchanged
   // between the waves while the weights, which take longest, are on their way)
-  if constexpr (NORM) request_rows(wave);
+  uint16_t* rows = reinterpret_cast<uint16_t*>(lds + 4 * NT * TN * 64);      // STAGED: [STAGED][staged_pitch(K)]
+  constexpr int P = STAGED ? 256 / STAGED : 64, PIECES = kStagedK / 4 / P;   // threads of a row, all in one wave; pieces of four numbers of a thread
+  const int piece = threadIdx.x % P;
+  float4 mine[STAGED ? PIECES : 1];
+  uint4 mine_w[STAGED ? PIECES : 1];                                         // four bfloat16 in x and y, or four float32
+  if constexpr (STAGED) {
+    const float* row = a.residual + size_t(min(t0 + int(threadIdx.x) / P, a.T - 1)) * a.K;
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int k = 4 * (piece + j * P);
+      mine[j] = k < a.K ? ldg_f4(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int k = min(4 * (piece + j * P), a.K - 4);
+      if (a.norm_w_bf16) {
+        const uint2 b = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.norm_w) + k);
+        mine_w[j] = make_uint4(b.x, b.y, 0, 0);
+      } else {
+        mine_w[j] = ldg128(reinterpret_cast<const float*>(a.norm_w) + k);
+      }
+    }
+  } else if constexpr (NORM) {
+    request_rows(wave);
+  }
   load_weights(wave);
   __builtin_amdgcn_sched_barrier(0);   // keep these requests ahead of everything below
   // What the epilogue reads per output (bias, position, rotation frequency, cache slot) is requested now
@@ -320,7 +351,28 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
   // steps each; rows longer than one pass (4 UN steps) are read once more for their squares.  The weights asked
   // for above are on their way meanwhile.
   float row_scale = 1.f;
-  if constexpr (NORM) {
+  if constexpr (STAGED) {
+    float square_sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j)
+      square_sum = fmaf(mine[j].x, mine[j].x, fmaf(mine[j].y, mine[j].y, fmaf(mine[j].z, mine[j].z, fmaf(mine[j].w, mine[j].w, square_sum))));
+#pragma unroll
+    for (int o = P / 2; o > 0; o >>= 1) square_sum += __shfl_xor(square_sum, o, 64);
+    const float scale = 1.0f / sqrtf(square_sum / float(a.K) + a.eps);
+    uint16_t* row = rows + int(threadIdx.x) / P * staged_pitch(a.K);
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int k = 4 * (piece + j * P);
+      const uint4 b = mine_w[j];
+      const float4 w = a.norm_w_bf16 ? make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16),
+                                                   __uint_as_float(b.y & 0xffff0000u))
+                                     : make_float4(__uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w));
+      if (k < a.K)
+        *reinterpret_cast<uint2*>(row + k) = make_uint2(pack_bf16x2((mine[j].x * scale) * w.x, (mine[j].y * scale) * w.y),
+                                                        pack_bf16x2((mine[j].z * scale) * w.z, (mine[j].w * scale) * w.w));
+    }
+    __syncthreads();
+  } else if constexpr (NORM) {
     float square_sum = normed.squares(steps - wave, k_end - (k_begin + 16 * lj + 64 * wave));
     for (int s0 = wave + 4 * UN; s0 < steps; s0 += 4 * UN) {
       NormInputs<UN, K64> further;
@@ -339,10 +391,18 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
   for (int s0 = wave; s0 < steps; s0 += 4 * UN) {
     if (s0 != wave) {
       load_weights(s0);
-      if constexpr (NORM) request_rows(s0);
+      if constexpr (NORM && !STAGED) request_rows(s0);
     }
     uint4 xb[UN][TN][2];
-    if constexpr (NORM) {
+    if constexpr (STAGED) {
+      // (columns of tokens past the block's rows repeat the last one; past the end of K the weights are zeros)
+      const uint16_t* row = rows + min(lr, STAGED - 1) * staged_pitch(a.K);
+#pragma unroll
+      for (int u = 0; u < UN; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          xb[u][0][h] = *reinterpret_cast<const uint4*>(row + min(16 * lj + 64 * (s0 + 4 * u) + 8 * h, a.K - 8));
+    } else if constexpr (NORM) {
       // Lane (lr, lj) needs 16 values of token lr per step, as the matrix cores take them.  They come straight
       // from the float32 residual, times the token's scale, times the norm's weights, rounded to bfloat16.
       normed.operands(a.norm_w_bf16, row_scale, xb);
@@ -493,14 +553,26 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
   }
 }
 
-static size_t fused_lds_bytes(int TN, bool norm, int NT = 2) {
-  return sizeof(float4) * 4 * NT * TN * 64 + (norm ? sizeof(float) * 4 * 16 : 0);
+static size_t fused_lds_bytes(int TN, bool norm, int NT = 2, int staged = 0, int K = 0) {
+  return sizeof(float4) * 4 * NT * TN * 64 + (staged ? size_t(staged) * staged_pitch(K) * 2 : norm ? sizeof(float) * 4 * 16 : 0);
 }
 
 template <int TN, int EPI, bool NORM, int NT, int UN>
 static int launch_fused_un(hipStream_t s, const FusedArgs& a, int blocks, int splits) {
   const size_t lds = fused_lds_bytes(TN, NORM, NT);     // at most 48 KB (four token tiles of three tiles)
   const dim3 grid(blocks, splits, (a.T + 16 * TN - 1) / (16 * TN));   // z: the tokens in tiles of 16 TN
+  if constexpr (NORM && EPI == kEpiRope) {
+    // several rows whose sums cost more than the way through LDS: 4 to 8 tokens, and more than 32 (blocks of 16 that share the CUs)
+    if (a.K <= kStagedK && a.T >= 4 && (a.T <= 8 || a.T > 32)) {      // at most 41 KB of LDS
+      const int staged = a.T <= 8 ? 8 : 16;
+      const size_t room = fused_lds_bytes(TN, true, NT, staged, a.K);
+      if (staged == 8 && a.K % 64 == 0) gemm_fused_kernel<TN, EPI, true, NT, true, UN, 8><<<grid, 256, room, s>>>(a);
+      else if (staged == 8) gemm_fused_kernel<TN, EPI, true, NT, false, UN, 8><<<grid, 256, room, s>>>(a);
+      else if (a.K % 64 == 0) gemm_fused_kernel<TN, EPI, true, NT, true, UN, 16><<<grid, 256, room, s>>>(a);
+      else gemm_fused_kernel<TN, EPI, true, NT, false, UN, 16><<<grid, 256, room, s>>>(a);
+      return check_launch("sp_gemm_fused");
+    }
+  }
   if (a.K % 64 == 0 && a.k_per_split % 64 == 0)
     gemm_fused_kernel<TN, EPI, NORM, NT, true, UN><<<grid, 256, lds, s>>>(a);
   else
