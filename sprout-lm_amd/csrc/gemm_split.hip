@@ -43,7 +43,7 @@ constexpr int kNotFinite = 1 << 20;                      // a row's exponent, wh
 constexpr int kHasNan = 1 << 22;                         // ... and where one of them is NaN
 constexpr uint32_t kInfinityBits = 0x7f800000u;
 
-enum { kRowsAsTheyAre = 0, kRowsGated = 1, kRowsNormed = 2 };
+enum { kRowsAsTheyAre = 0, kRowsGated = 1, kRowsNormed = 2, kRowsPaired = 3 };
 
 struct SplitSource {
   const float* a;              // [rows][length]; kRowsGated: [rows][2 length], gate then up
@@ -52,7 +52,12 @@ struct SplitSource {
   float eps;
   int act;                     // kRowsGated
   float limit;
+  int row0, half;              // kRowsPaired: the first split row, and the rows of a gate (see paired_row)
 };
+
+// A gated product's weights, gate rows then up rows (half of each, in sixteens), are split in pairs of sixteen: split row n of the
+// product is this row of them.  The two numbers that meet in an output are then in one lane of the product, in neighbouring tiles.
+__device__ __forceinline__ int paired_row(int n, int half) { return (n >> 5) * 16 + (n & 15) + ((n >> 4) & 1) * half; }
 
 __device__ __forceinline__ size_t row_at(int row, int K) { return size_t(row >> 1) * (size_t(K / kStep) * kStepBytes) + (row & 1) * 64; }
 
@@ -68,7 +73,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitSource src, unsign
   const int lane = WAVES == 1 ? threadIdx.x & 63 : threadIdx.x;
   if (row >= rows) return;
   const int n4 = K / 4;
-  const float* whole = src.a + size_t(row) * (KIND == kRowsGated ? 2 * src.length : src.length);
+  const float* whole = src.a + size_t(KIND == kRowsPaired ? paired_row(src.row0 + row, src.half) : row) * (KIND == kRowsGated ? 2 * src.length : src.length);
   const float4* a = reinterpret_cast<const float4*>(whole + src.first);
   float4 kept[PIECES];
   if (KIND != kRowsGated) {
@@ -181,10 +186,16 @@ template <int WM, int WN, int STAGES> constexpr bool split_shares_cu = split_lds
 // the next step has landed also frees this step's stage, and the loads into it follow one by one between the products.
 // What bounds it: matrix instructions, 6 WM WN of 16 cycles a stage and SIMD, at the clock that their power leaves; a block of
 // 256 x 128 reads 72 KB from L2 for 3,072 cycles.
+//
+// kSilu: w's rows in pairs of sixteen (paired_row), out [T, N / 2] the gated values of the two products, N in 32s, no bias.
+// Half the numbers are stored and read again, and the exponential and the division, which a split behind it hid under its reads, now
+// stand beside another block's products (2,048 tokens by 9,728 rows of 896: product 167 -> 169 us, the split of the rows that the
+// down product reads 22.7 -> 16.4).
 template <int WM, int WN, int STAGES, int MODE>
 __global__ __launch_bounds__(256, (split_shares_cu<WM, WN, STAGES> ? 2 : 1)) void split_product_kernel(
     const unsigned char* __restrict__ x, const unsigned char* __restrict__ w, const int32_t* __restrict__ x_exp,
-    const int32_t* __restrict__ w_exp, const void* __restrict__ bias, int bias_dtype, float* out, int T, int N, int K, long long out_stride) {
+    const int32_t* __restrict__ w_exp, const void* __restrict__ bias, int bias_dtype, float* out, int T, int N, int K, long long out_stride,
+    int act, float limit) {
   constexpr int BM = 32 * WM, BN = 32 * WN;
   constexpr int STAGE = (BM + BN) * 192, XBYTES = BM * 192;
   constexpr int LX = 3 * BM / 64, LW = 3 * BN / 64, L = LX + LW;       // load instructions per wave, stage and operand
@@ -388,18 +399,39 @@ __global__ __launch_bounds__(256, (split_shares_cu<WM, WN, STAGES> ? 2 : 1)) voi
     if (i + 1 < WM) fetch(i + 1);
     const int t = t0 + (wm * WM + i) * 16 + li;
     float* row = out + size_t(min(t, T - 1)) * out_stride;
-#pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const int n = nbase + 16 * j;
-      float v[4];
+    auto values = [&](int j, float (&v)[4]) __attribute__((always_inline)) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int e = ex[i] + ew[j][r];
         const float back = __builtin_amdgcn_ldexpf(acc[i][j][r] + low[i][j][r], -e);
         const bool beyond = e >= kNotFinite / 2;      // exponents of finite rows lie between -78 and 199
-        v[r] = (beyond ? 0.f : (t ^ (n + r)) & 1 ? -back : back) + add[j][r];
+        v[r] = (beyond ? 0.f : (t ^ (nbase + 16 * j + r)) & 1 ? -back : back) + add[j][r];
         strange |= beyond;
       }
+    };
+    if constexpr (MODE == kSilu) {
+#pragma unroll
+      for (int j = 0; j < WN; j += 2) {
+        const int n = nbase + 16 * j;      // of the gate rows of a pair, which is whole: N in 32s
+        float g[4], u[4];
+        values(j, g);
+        values(j + 1, u);
+        if (t >= T || n >= N) continue;
+        auto store = [&](int which) __attribute__((always_inline)) {
+          *reinterpret_cast<float4*>(row + (n >> 5) * 16 + (n & 15)) =
+              make_float4(gated_value(g[0], u[0], which, limit), gated_value(g[1], u[1], which, limit), gated_value(g[2], u[2], which, limit),
+                          gated_value(g[3], u[3], which, limit));
+        };
+        if (act == kActSilu) store(kActSilu);      // one choice for four numbers
+        else store(act);
+      }
+      continue;
+    }
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const int n = nbase + 16 * j;
+      float v[4];
+      values(j, v);
       if (t >= T || n >= N) continue;
       if (fours && n + 4 <= N) {
         if (MODE == kAccumulate) {
@@ -414,22 +446,41 @@ __global__ __launch_bounds__(256, (split_shares_cu<WM, WN, STAGES> ? 2 : 1)) voi
     }
   }
   if (!__syncthreads_or(strange)) return;
-  // results of rows that are not finite: bias, and what was there before, stand in the output; the sums are added to them
-  for (int at = threadIdx.x; at < BM * BN; at += 256) {
-    const int t = t0 + at / BN, n = n0 + at % BN;
-    if (t >= T || n >= N) continue;
-    const int et = x_exp[t], en = w_exp[n];
-    if (max(et, en) < kNotFinite) continue;
-    const bool nan = max(et, en) == kHasNan;
-    float sum = nan ? __builtin_nanf("") : 0.f;
-    for (int k = nan ? K : 0; k < K; k += 8) {
+  // results of rows that are not finite, number by number
+  auto by_number = [&](int t, int n, int et, int en, auto zero) {
+    auto sum = zero;
+    for (int k = 0; k < K; k += 8) {
       float xv[8], wv[8];
       numbers_of(x, t, k, K, et, xv);
       numbers_of(w, n, k, K, en, wv);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sum = fmaf(xv[e], wv[e], sum);
+      for (int e = 0; e < 8; ++e) sum = __builtin_elementwise_fma(decltype(zero)(xv[e]), decltype(zero)(wv[e]), sum);
     }
-    out[size_t(t) * out_stride + n] += sum;
+    return sum;
+  };
+  auto value = [&](int t, int n, int et) -> float {
+    const int en = w_exp[n];
+    if (max(et, en) == kHasNan) return __builtin_nanf("");
+    if (max(et, en) == kNotFinite) return by_number(t, n, et, en, 0.f);
+    return float(by_number(t, n, et, en, 0.0));      // a finite result that meets one that is not: its sums above are gone
+  };
+  if constexpr (MODE == kSilu) {
+    for (int at = threadIdx.x; at < BM * BN / 2; at += 256) {
+      const int t = t0 + at / (BN / 2), c = at % (BN / 2), n = n0 + (c >> 4) * 32 + (c & 15);
+      if (t >= T || n >= N) continue;
+      const int et = x_exp[t];
+      if (max(et, max(w_exp[n], w_exp[n + 16])) < kNotFinite) continue;
+      out[size_t(t) * out_stride + n0 / 2 + c] = gated_value(value(t, n, et), value(t, n + 16, et), act, limit);
+    }
+    return;
+  }
+  // ... bias, and what was there before, stand in the output; the sums are added to them
+  for (int at = threadIdx.x; at < BM * BN; at += 256) {
+    const int t = t0 + at / BN, n = n0 + at % BN;
+    if (t >= T || n >= N) continue;
+    const int et = x_exp[t];
+    if (max(et, w_exp[n]) < kNotFinite) continue;
+    out[size_t(t) * out_stride + n] += value(t, n, et);
   }
 }
 
@@ -472,6 +523,8 @@ struct Product {
   float* out;
   int T, N, K;
   long long out_stride;
+  int act;
+  float limit;
 };
 
 template <int WM, int WN, int STAGES, int MODE>
@@ -489,15 +542,16 @@ int launch_mode(hipStream_t s, const Product& p) {
   }
   const PipeTiles tiles = pipe_tiles((p.T + 32 * WM - 1) / (32 * WM), (p.N + 32 * WN - 1) / (32 * WN));
   split_product_kernel<WM, WN, STAGES, MODE><<<8 * (tiles.own + tiles.run), 256, lds, s>>>(
-      p.x, p.w, p.x_exp, p.w_exp, p.bias, p.bias_dtype, p.out, p.T, p.N, p.K, p.out_stride);
+      p.x, p.w, p.x_exp, p.w_exp, p.bias, p.bias_dtype, p.out, p.T, p.N, p.K, p.out_stride, p.act, p.limit);
   return check_launch("sp_gemm_f32_split");
 }
 
-int product(hipStream_t s, const Product& p, bool add) {
+int product(hipStream_t s, const Product& p, int mode) {
   float time_us;
   switch (choose_split_shape(p.T, p.N, p.K, &time_us)) {
 #define SPROUT_SPLIT_CASE(I, WM, WN, STAGES) \
-    case I: return add ? launch_mode<WM, WN, STAGES, kAccumulate>(s, p) : launch_mode<WM, WN, STAGES, kStoreF32>(s, p);
+    case I: return mode == kSilu ? launch_mode<WM, WN, STAGES, kSilu>(s, p) \
+                 : mode == kAccumulate ? launch_mode<WM, WN, STAGES, kAccumulate>(s, p) : launch_mode<WM, WN, STAGES, kStoreF32>(s, p);
     SPROUT_SPLIT_SHAPES(SPROUT_SPLIT_CASE)
 #undef SPROUT_SPLIT_CASE
   }
@@ -557,14 +611,20 @@ extern "C" int sp_gemm_f32_split_pays(int T, int N, int K) {
   return us < gemm_f32_time_us(T, N, K);
 }
 
+// Whether sp_gemm_f32_split takes the product as a gated one (mode 2): gate and up rows in sixteens, K in one piece (the values are
+// gated where the sums end).
+extern "C" int sp_gemm_f32_split_gates(int T, int N, int K) { return sp_gemm_f32_split_bytes(T, N, K) > 0 && N % 32 == 0 && piece_of(K) == K; }
+
 // out[T, N] = or += rows . w^T + bias, everything float32; rows: `kind` 0: a [T, K]; 1: act(a[:, :K], a[:, K:]) of a [T, 2 K];
-// 2: rmsnorm(a) * norm_w.  mode 1 adds into out.
+// 2: rmsnorm(a) * norm_w.  mode 1 adds into out; mode 2 (not of kind 1, without a bias): out[T, N / 2] = act(rows . first half of w) times
+// rows . second half.
 extern "C" int sp_gemm_f32_split(void* stream, int kind, const float* a, const float* norm_w, float eps, int activation, float limit,
                                  const float* w, int bias_dtype, const void* bias, int mode, float* out, int T, int N, int K, void* workspace, int64_t workspace_bytes) {
   const int64_t need = sp_gemm_f32_split_bytes(T, N, K);
   SP_REQUIRE(need > 0, "sp_gemm_f32_split: T=%d N=%d K=%d is not taken", T, N, K);
-  SP_REQUIRE(kind >= 0 && kind <= 2 && (kind != kRowsNormed || norm_w) && (mode == 0 || mode == 1), "sp_gemm_f32_split: unknown kind %d or mode %d", kind, mode);
+  SP_REQUIRE(kind >= 0 && kind <= 2 && (kind != kRowsNormed || norm_w) && mode >= 0 && mode <= 2, "sp_gemm_f32_split: unknown kind %d or mode %d", kind, mode);
   SP_REQUIRE(activation >= 0 && activation < kGateActs, "sp_gemm_f32_split: no kernel for activation %d", activation);
+  SP_REQUIRE(mode != 2 || (kind != kRowsGated && !bias && sp_gemm_f32_split_gates(T, N, K)), "sp_gemm_f32_split: T=%d N=%d K=%d kind %d is not taken as a gated product", T, N, K, kind);
   SP_REQUIRE(!bias || bias_dtype == kF32 || bias_dtype == kBF16, "sp_gemm_f32_split: unsupported bias dtype %d", bias_dtype);
   SP_REQUIRE(a && w && out && workspace && workspace_bytes >= need, "sp_gemm_f32_split: null operand, or a workspace of %lld bytes where %lld are needed",
              (long long)workspace_bytes, (long long)need);
@@ -588,13 +648,15 @@ extern "C" int sp_gemm_f32_split(void* stream, int kind, const float* a, const f
     for (int n = 0; n < N; n += chunk) {
       const int rows = N - n < chunk ? N - n : chunk;
       SplitSource wsrc = {};
-      wsrc.a = w + size_t(n) * K;
+      wsrc.a = mode == 2 ? w : w + size_t(n) * K;
       wsrc.length = K;
       wsrc.first = k;
-      if (launch_split<kRowsAsTheyAre>(s, wsrc, ws, w_exp + n, rows, width)) return 1;
+      wsrc.row0 = n;
+      wsrc.half = N / 2;
+      if (mode == 2 ? launch_split<kRowsPaired>(s, wsrc, ws, w_exp + n, rows, width) : launch_split<kRowsAsTheyAre>(s, wsrc, ws, w_exp + n, rows, width)) return 1;
       const void* rows_bias = !bias || k > 0 ? nullptr : bias_dtype == kBF16 ? (const void*)((const bf16_t*)bias + n) : (const void*)((const float*)bias + n);
-      const Product p = {xs, ws, x_exp, w_exp + n, rows_bias, bias_dtype, out + n, T, rows, width, N};
-      if (const int rc = product(s, p, mode == 1 || k > 0)) return rc;
+      const Product p = {xs, ws, x_exp, w_exp + n, rows_bias, bias_dtype, mode == 2 ? out + n / 2 : out + n, T, rows, width, mode == 2 ? N / 2 : N, activation, limit};
+      if (const int rc = product(s, p, mode == 2 ? kSilu : mode == 1 || k > 0 ? kAccumulate : kStoreF32)) return rc;
     }
   }
   return 0;

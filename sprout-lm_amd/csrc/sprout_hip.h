@@ -39,11 +39,13 @@ int sp_gemm(void* stream, int a_dtype, const void* a, int w_dtype, const void* w
 
 // float32 products of many tokens as six products of bfloat16 parts, three a number: out[T, N] = or (mode 1) += rows . w[N, K]^T (+ bias), all
 // float32, w split once a call.  rows, by `kind`: 0: a [T, K];  1: act(a[:, :K], a[:, K:]) of a [T, 2 K] (`activation`, `limit` as
-// for sp_gate_up_silu);  2: rmsnorm(a) * norm_w.
+// for sp_gate_up_silu);  2: rmsnorm(a) * norm_w.  mode 2 (kinds 0 and 2, no bias; where sp_gemm_f32_split_gates says so): out[T, N / 2] =
+// act(rows . w[:N / 2]^T) * (rows . w[N / 2:]^T).
 // sp_gemm_f32_split_bytes: the workspace it wants, 0 where it does not take the product.  sp_gemm_f32_split_pays: whether it is
 // taken to be the faster way (sp_gemm is the other).
 int64_t sp_gemm_f32_split_bytes(int T, int N, int K);
 int sp_gemm_f32_split_pays(int T, int N, int K);
+int sp_gemm_f32_split_gates(int T, int N, int K);
 int sp_gemm_f32_split(void* stream, int kind, const float* a, const float* norm_w, float eps, int activation, float limit,
                       const float* w, int bias_dtype, const void* bias, int mode, float* out, int T, int N, int K, void* workspace, int64_t workspace_bytes);
 

@@ -631,19 +631,28 @@ def gemm_f32_split_pays(T: int, N: int, K: int) -> bool:
     return bool(library().sp_gemm_f32_split_pays(T, N, K))
 
 
+def gemm_f32_split_gates(T: int, N: int, K: int) -> bool:
+    """Whether `gemm_f32_split` takes the product of T tokens by N rows (gate and up together) of K with `gates`."""
+    return bool(library().sp_gemm_f32_split_gates(T, N, K))
+
+
 def gemm_f32_split(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, workspace, bias: torch.Tensor | None = None,
-                   accumulate: bool = False, norm=None, activation: str | None = None, limit: float = 0.0) -> bool:
+                   accumulate: bool = False, norm=None, activation: str | None = None, limit: float = 0.0, gates: bool = False) -> bool:
     """out = (or, with accumulate, +=) rows @ w.T (+ bias), everything float32, for many tokens; rows = a, or rmsnorm(a) * weight
-    with `norm` = (weight, eps), or act(a[:, :K]) * a[:, K:] with an `activation`.  `workspace`: bytes -> a uint8 tensor.
+    with `norm` = (weight, eps), or act(a[:, :K]) * a[:, K:] with an `activation`.  With `gates` the activation is the result's
+    instead: out [T, N / 2] = act(rows @ w[:N / 2].T) * (rows @ w[N / 2:].T).  `workspace`: bytes -> a uint8 tensor.
     Returns False (and does nothing) where the kernel does not take the product."""
     T, (N, K) = a.shape[0], w.shape
-    if not (a.dtype == w.dtype == out.dtype == torch.float32) or tuple(out.shape) != (T, N) \
-            or a.shape[1] != (K if activation is None else 2 * K):
+    gated_rows = activation is not None and not gates
+    if not (a.dtype == w.dtype == out.dtype == torch.float32) or tuple(out.shape) != (T, N // 2 if gates else N) \
+            or a.shape[1] != (2 * K if gated_rows else K):
+        return False
+    if gates and (activation is None or accumulate or bias is not None or not gemm_f32_split_gates(T, N, K)):
         return False
     need = gemm_f32_split_bytes(T, N, K)
     if need == 0 or (a.data_ptr() | w.data_ptr() | out.data_ptr()) & 15:
         return False
-    if norm is not None and (activation is not None or norm[0].dtype != torch.float32 or norm[0].numel() != K or norm[0].data_ptr() & 15):
+    if norm is not None and (gated_rows or norm[0].dtype != torch.float32 or norm[0].numel() != K or norm[0].data_ptr() & 15):
         return False
     _gpu(a, "gemm input"); _gpu(w, "gemm weight"); _gpu(out, "gemm output")
     if norm is not None:
@@ -654,9 +663,9 @@ def gemm_f32_split(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, workspac
             raise KernelError(f"gemm: bias has {bias.numel()} values for {N} columns")
     scratch = workspace(need)
     check(library().sp_gemm_f32_split(
-        _stream(), 2 if norm is not None else 1 if activation is not None else 0, a.data_ptr(), _ptr(norm[0]) if norm else None,
+        _stream(), 2 if norm is not None else 1 if gated_rows else 0, a.data_ptr(), _ptr(norm[0]) if norm else None,
         float(norm[1]) if norm else 0.0, variant_code(GATE_ACTIVATIONS, activation, "gate activation") if activation else 0,
-        float(limit), w.data_ptr(), _code(bias, "gemm bias") if bias is not None else 0, _ptr(bias), int(accumulate),
+        float(limit), w.data_ptr(), _code(bias, "gemm bias") if bias is not None else 0, _ptr(bias), 2 if gates else int(accumulate),
         out.data_ptr(), T, N, K, scratch.data_ptr(), scratch.numel() * scratch.element_size()))
     return True
 

@@ -121,6 +121,8 @@ def _declare(lib):
     lib.sp_gemm_f32_split_bytes.restype = c_i64
     lib.sp_gemm_f32_split_pays.argtypes = [c_int] * 3
     lib.sp_gemm_f32_split_pays.restype = c_int
+    lib.sp_gemm_f32_split_gates.argtypes = [c_int] * 3
+    lib.sp_gemm_f32_split_gates.restype = c_int
     lib.sp_attention_workspace_floats.argtypes = [c_int] * 10
     lib.sp_attention_workspace_floats.restype = c_i64
     lib.sp_rglru_carry_floats.argtypes = [c_int] * 4

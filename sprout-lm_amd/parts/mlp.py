@@ -77,9 +77,17 @@ class GatedMLP(FeedForward):
 
     def _split_f32(self, ctx, residual, fold) -> bool:
         """Many tokens on the float32 path: the norm is folded into the first product's operand, and where the second is taken too
-        the gate into its own; the gated rows then have no tensor."""
+        the gate into the first one's end (into the second's operand where that does not take it)."""
         T = residual.shape[0]
         scratch = lambda n: ctx.buffer("f32_split", (n,), torch.uint8)
+        if ops.gemm_f32_split_gates(T, 2 * self.inner, self.hidden):
+            act = ctx.buffer("gate_up", (T, self.inner), ctx.act_dtype)      # of one number where the two have met
+            if ops.gemm_f32_split(residual, self.w_gate_up, act, scratch, norm=(fold.weight, fold.eps), activation=self.activation,
+                                  limit=self.limit, gates=True):
+                if not (ops.gemm_f32_split_pays(T, self.hidden, self.inner)
+                        and ops.gemm_f32_split(act, self.w_down, residual, scratch, accumulate=True)):
+                    add_product(ctx, act, self.w_down, residual)
+                return True
         gu = ctx.buffer("gate_up", (T, 2 * self.inner), ctx.act_dtype)
         if not ops.gemm_f32_split(residual, self.w_gate_up, gu, scratch, norm=(fold.weight, fold.eps)):
             return False

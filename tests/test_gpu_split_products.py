@@ -239,3 +239,48 @@ def test_every_block_shape(T, N, K):
     acc = torch.ones(T + 1, N, device=DEV)
     assert ops.gemm_f32_split(a, w, acc[:T], scratch, bias=bias, accumulate=True)
     assert ((acc[:T].double() - 1 - want).abs() <= limit + 2.0 ** -23 * (1 + want.abs())).all() and (acc[T] == 1).all()
+
+
+# tiles with remainders of every pair of sixteen, every block shape's ends, weights of more than a chunk; sums that are not finite
+# on either side of a gate
+@pytest.mark.parametrize("T,N,K", [(256, 32, 64), (257, 96, 96), (300, 160, 896), (2048, 9728, 96), (1025, 2464, 2080), (321, 4128, 1920), (450, 2080, 96),
+                                   (1300, 4128, 288), (600, 16384, 5120)])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "relu", "clamped_swish"])
+def test_gates_in_the_product(T, N, K, activation):
+    """The product of both halves is the plain one's, number by number, and so is what the gate makes of it."""
+    from sprout_lm_amd import ops
+    a, w, weight = rows(T, K, T + 1), (rows(N, K, N + 1) * K ** -0.5), 1 + 0.1 * torch.randn(K, device=DEV)
+    both, want = torch.empty(T, N, device=DEV), torch.empty(T, N // 2, device=DEV)
+    for options in ({"norm": (weight, 1e-6)}, {}):
+        assert ops.gemm_f32_split(a, w, both, scratch, **options)
+        ops.silu_mul(both, want, activation=activation, limit=7.0)
+        out = torch.full((T + 1, N // 2), 7.0, device=DEV)
+        assert ops.gemm_f32_split(a, w, out[:T], scratch, activation=activation, limit=7.0, gates=True, **options)
+        # the gate's exponential and division, two float32 functions of a few units each, may be contracted differently
+        assert ((out[:T] - want).abs() <= 2.0 ** -20 * want.abs()).all() and (out[T] == 7).all()
+
+
+def test_gates_of_numbers_that_are_not_finite():
+    from sprout_lm_amd import ops
+    a, w = rows(300, 96, 1), rows(160, 96, 2)
+    a[5, 7], a[9, 0], a[11, 3] = float("inf"), float("nan"), float("-inf")
+    w[4, 95], w[80 + 4, 1], w[17, 2], w[80 + 40, 5], w[79, 0] = float("-inf"), float("inf"), float("nan"), float("inf"), float("inf")
+    both, want, out = torch.empty(300, 160, device=DEV), torch.empty(300, 80, device=DEV), torch.empty(300, 80, device=DEV)
+    for activation in ("silu", "relu", "clamped_swish"):
+        assert ops.gemm_f32_split(a, w, both, scratch)
+        ops.silu_mul(both, want, activation=activation, limit=7.0)
+        assert ops.gemm_f32_split(a, w, out, scratch, activation=activation, limit=7.0, gates=True)
+        good = want.isfinite()
+        assert torch.equal(out.nan_to_num(nan=3.5, posinf=2.5, neginf=1.5)[~good], want.nan_to_num(nan=3.5, posinf=2.5, neginf=1.5)[~good])
+        # a finite half that meets one that is not is summed again, in 64 bits
+        assert ((out - want)[good].abs() <= 2.0 ** -18 * (1 + want[good].abs())).all()
+
+
+@pytest.mark.parametrize("T,N,K,why", [(300, 48, 96, "a gate of no whole sixteens"), (300, 160, 5152, "K in two pieces"), (255, 160, 96, "few tokens")])
+def test_gates_that_the_product_does_not_take(T, N, K, why):
+    from sprout_lm_amd import ops
+    a, w, out = rows(T, K, 1), rows(N, K, 2), torch.full((T, N // 2), 7.0, device=DEV)
+    assert not ops.gemm_f32_split_gates(T, N, K), why
+    assert not ops.gemm_f32_split(a, w, out, scratch, activation="silu", gates=True) and (out == 7).all()
+    a, w, out = rows(300, 96, 1), rows(160, 96, 2), torch.full((300, 80), 7.0, device=DEV)
+    assert not ops.gemm_f32_split(a, w, out, scratch, gates=True) and not ops.gemm_f32_split(a, w, out, scratch, activation="silu", gates=True, accumulate=True)
