@@ -193,7 +193,7 @@ class _PortionGraph:
 
     _uids = itertools.count(1)
 
-    def __init__(self, runner, first, ctx_bucket: int, tile_bucket: int, workspace):
+    def __init__(self, runner, first, ctx_bucket: int, workspace):
         self.uid = next(self._uids)          # names this graph to the shared workspace
         self.runner = runner if isinstance(runner, weakref.ProxyTypes) else weakref.proxy(runner)
         cache = runner.cache
@@ -216,7 +216,7 @@ class _PortionGraph:
         self.shared_workspace = workspace
         self.ctx = context_from(first, views, len(cache.groups), OwnedNames(workspace, ("logits",), runner.device),
                                 runner.dtype, runner.attention_kind, max_decode_ctx=ctx_bucket, max_ctx=ctx_bucket,
-                                max_tile_ctx=tile_bucket)
+                                max_tile_ctx=ctx_bucket)
         self.ctx.host = {}
         self.copied = None
         self.graph = None
@@ -303,9 +303,9 @@ class DecodeGraphs:
         if not runner.parts.graph_safe_portions or not entries:
             return None
         bucket = self._context_bucket(max(e.seq.length + len(e.tokens) for e in entries))
-        # the requests that bring several tokens have a bucket of their own, where it is another one
-        tile_bucket = self._context_bucket(max((e.seq.length + len(e.tokens) for e in entries if len(e.tokens) > 1), default=1))
-        key = (tuple((len(e.tokens), len(e.want)) for e in entries), bucket) + ((tile_bucket,) if tile_bucket != bucket else ())
+        # (No bucket for the prompts' own context beside it: a prompt read in portions beside longer answers would be recorded anew at
+        # every power of two that it passes, 30 ms each, for attention kernels that share out every tile's own walk anyway.)
+        key = (tuple((len(e.tokens), len(e.want)) for e in entries), bucket)
         self.portion_steps += 1
         state = self.portion_graphs.pop(key, None)
         if state is None:
@@ -327,7 +327,7 @@ class DecodeGraphs:
         if state is None:
             if self._portion_workspace is None:
                 self._portion_workspace = KeptWorkspace(runner.device)
-            state = _PortionGraph(runner, step, bucket, tile_bucket, self._portion_workspace)
+            state = _PortionGraph(runner, step, bucket, self._portion_workspace)
         self.portion_graphs[key] = state
         state.last_used = self.portion_steps
         state.fill(step)

@@ -239,6 +239,23 @@ def test_recorded_portions_at_real_layer_sizes_cross_a_context_bucket(tmp_path):
     print(f"recorded portions at real layer sizes: worst {worst:.2f} of the bound")
 
 
+def test_portions_beside_a_longer_answer_are_recorded_once(tmp_path):
+    """A prompt that passes 256 and 512 keys in equal portions beside a request that answers at more than 512: one shape, one graph."""
+    import sprout_lm_amd as S
+    from sprout_lm_amd.cli import PRESETS
+    from sprout_lm_amd.engine import ModelRunner
+    from sprout_lm_amd.weights import write_model_folder
+    raw = dict(PRESETS["qwen2.5-0.5b"], num_hidden_layers=2)
+    folder = str(tmp_path / "half_b")
+    write_model_folder(folder, S.config_from_dict(raw), seed=10, dtype=torch.bfloat16, std=0.02)
+    tokens = {"a": H.random_tokens(raw["vocab_size"], 607, 78), "b": H.random_tokens(raw["vocab_size"], 700, 79)}
+    runner = ModelRunner.from_folder(folder, "bfloat16", block_size=16, num_blocks=100, max_sequences=2)
+    seqs, fed = {r: runner.cache.create() for r in tokens}, {r: 0 for r in tokens}
+    fed_step(runner, seqs, tokens, fed, {"a": 600}, folder, "bfloat16", "the longer request")
+    ran = [fed_step(runner, seqs, tokens, fed, {"a": 1, "b": 100}, folder, "bfloat16", "a portion beside it")[0] for _ in range(7)]
+    assert ran == [False] + [True] * 6 and set(runner._graphs.portion_graphs) == {(((1, 1), (100, 1)), 1024)}
+
+
 def test_a_recorded_step_is_given_up_only_when_it_has_not_run_for_a_while(tmp_path):
     """Recording a step costs as much as dozens of steps.  With room for two recorded shapes, a third shape that
     keeps coming runs eagerly while both graphs are in use, and takes the place of the one that has not run for
