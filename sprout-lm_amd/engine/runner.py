@@ -12,6 +12,7 @@ from ..cache.spec import PagedKVSpec
 from ..config.base import token_id_list
 from .. import ops
 from ..models.plan import ModelPlan
+from ..parts.base import claims
 from ..registry import build_model_plan, load_config
 from ..weights.loader import load_named_tensors
 from ..weights.random_init import random_tensors
@@ -301,10 +302,11 @@ class ModelRunner:
             ctx.owed = ctx.joins = None
             for i, call in enumerate(self.plan.schedule):
                 block = self.parts.blocks[call.layer]
-                if ctx.owed is not None and not block.settles:
+                settles = claims(block, "settles")
+                if ctx.owed is not None and not settles:
                     ops.join(residual, ctx.owed)
                     ctx.owed = None
-                ctx.settles = block.settles
+                ctx.settles = settles
                 block.forward(ctx, residual, self._slot_views(ctx, i))
             ctx.settles = False
             n = ctx.n_logits

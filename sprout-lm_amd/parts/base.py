@@ -100,6 +100,12 @@ class Part:
         return 0.0
 
 
+def claims(part, name: str) -> bool:
+    """What the part's own class says of itself (`adds_last`, `settles`): a subclass may read or change the residual where its base
+    does not, and claims it anew if that still holds."""
+    return vars(type(part)).get(name, False)
+
+
 def add_product(ctx, x, w, residual, bias=None) -> None:
     """residual += x @ w.T (+ bias), where nobody reads the residual before the norm that follows: where `ctx.joins` is this residual, the
     product may be left to that norm in parts (`ctx.owed`, see `ops.gemm_parts`)."""
@@ -120,7 +126,7 @@ class Norm(Part):
         raise NotImplementedError
 
     def forward_joining(self, ctx, x, out, rows=None):
-        """The same of x plus what is owed to it (`ctx.owed`, which is then settled: with `rows`, x itself stays without it)."""
+        """The same of x plus what is owed to it (`ctx.owed`, which is then settled: with `rows`, x itself may stay without it)."""
         owed, ctx.owed = ctx.owed, None
         if owed is not None:
             ops.join(x, owed)
@@ -152,9 +158,9 @@ class PositionEncoding(Part):
 
 
 class Mixer(Part):
-    adds_last = False      # whether all that `forward` does to the residual is one `add_product`
-
     """Mixes information between the tokens of a sequence (attention, or anything with state)."""
+
+    adds_last = False      # whether all that `forward` does to the residual is one `add_product`
 
     def forward(self, ctx, h, residual, cache):
         """residual += mixer(h).  `cache` is this call's cache slot view (engine.batch.CacheSlotView), a dict of
@@ -238,9 +244,9 @@ class StreamPart(Part):
 
 
 class Block(Part):
-    settles = False       # whether the block's first norm joins what a product before it has left (`ctx.owed`), and its own may be left
-
     """Arranges mixers, feed-forwards and their norms around the residual stream."""
+
+    settles = False       # whether the block's first norm joins what a product before it has left (`ctx.owed`), and its own may be left
 
     def parts(self) -> dict[str, Part]:
         """The block's parts by the names under which the model plan gave them; everything the engine wants of a

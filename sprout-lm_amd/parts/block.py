@@ -4,7 +4,7 @@ from __future__ import annotations
 import torch
 
 from .. import ops
-from .base import Block, register_part
+from .base import Block, claims, register_part
 
 
 @register_part("block", "pre_norm")
@@ -36,7 +36,7 @@ class PreNormBlock(Block):
         h = ctx.buffer("normed", (T, H), ctx.act_dtype)
         # The next reader of the residual behind the mixer is this block's second norm, behind the feed-forward the norm of whatever
         # follows, where that settles what is owed (`ctx.settles`): a last product may then be left to the norm in parts.
-        behind_mixer = residual if self.mixer.adds_last and ctx.settles else None
+        behind_mixer = residual if claims(self.mixer, "adds_last") and ctx.settles else None
         if self.mixer_conv is not None:
             self.mixer_norm.forward_joining(ctx, residual, h)
             mixed_in = ctx.buffer("normed_conv", (T, H), ctx.act_dtype)
@@ -52,7 +52,7 @@ class PreNormBlock(Block):
         ctx.joins = None
         if self.ffn is None:
             return
-        behind_ffn = residual if self.ffn.adds_last and ctx.settles else None
+        behind_ffn = residual if claims(self.ffn, "adds_last") and ctx.settles else None
         ctx.joins = behind_ffn if ctx.owed is None else None
         if ctx.owed is not None or not self.ffn.forward_from_residual(ctx, self.ffn_norm, residual):
             self.ffn_norm.forward_joining(ctx, residual, h)

@@ -37,8 +37,8 @@ class RMSNorm(Norm):
         return out
 
     def forward_joining(self, ctx, x, out, rows=None):
-        if ctx.owed is None:
-            return self.forward(ctx, x, out, rows)
+        if ctx.owed is None or type(self).forward is not RMSNorm.forward:      # (a subclass with numbers of its own)
+            return super().forward_joining(ctx, x, out, rows)
         owed, ctx.owed = ctx.owed, None
         ops.rmsnorm_join(x, owed, self.weight, self.eps, out, rows)
         return out

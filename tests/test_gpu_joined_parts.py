@@ -91,3 +91,35 @@ def test_joining_norm(H, parts, T, dtype):
     assert torch.equal(joined, want) and torch.equal(out, norm)
     ops.join(x, owed)
     assert torch.equal(x, want)
+
+
+def test_a_subclass_does_not_inherit_the_claim():
+    """A class derived from a part that leaves its sums to the next norm may read the residual after them: it is not taken that way."""
+    from sprout_lm_amd.parts.base import claims
+    from sprout_lm_amd.parts.attention import Attention
+    from sprout_lm_amd.parts.block import PreNormBlock
+    from sprout_lm_amd.parts.mlp import GatedMLP
+    for base, name in ((Attention, "adds_last"), (GatedMLP, "adds_last"), (PreNormBlock, "settles")):
+        derived = type("Derived", (base,), {})
+        claimed = type("Claimed", (base,), {name: True})
+        assert [claims(c.__new__(c), name) for c in (base, derived, claimed)] == [True, False, True]
+
+
+@pytest.mark.gpu
+def test_a_norm_with_numbers_of_its_own_joins_first():
+    from sprout_lm_amd.engine.batch import StepContext, Workspace
+    from sprout_lm_amd.parts.norm import RMSNorm
+
+    class OnePlus(RMSNorm):
+        def forward(self, ctx, x, out, rows=None):
+            ops.rmsnorm(x, 1 + self.weight, self.eps, out, rows)
+            return out
+
+    x, owed, weight = torch.randn(5, 64, device=DEV), torch.randn(2, 5, 64, device=DEV), torch.randn(64, device=DEV)
+    want, out = torch.empty(5, 64, device=DEV), torch.empty(5, 64, device=DEV)
+    ops.rmsnorm(x + (owed[0] + owed[1]), 1 + weight, 1e-6, want)
+    norm, ctx = OnePlus(64, 1e-6), StepContext(Workspace(torch.device(DEV)), torch.float32)
+    norm.bind({"weight": weight})
+    ctx.owed = owed
+    norm.forward_joining(ctx, x, out)
+    assert torch.equal(out, want) and ctx.owed is None
