@@ -15,16 +15,17 @@ bool attention_mfma_supports(int hd, int page_size, int nq, int nkv);
 bool attention_mfma_decode_supports(int nq, int nkv);
 int attention_mfma_tile_q(int hd);
 size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_ctx);
-size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers);
+size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode,
+                                         long long one_query_keys);
 int attention_mfma(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                    const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                    const int32_t* ctx_len, const int32_t* tiles, int n_tiles, const int32_t* decode_seqs, int n_decode,
-                   int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, float* workspace, void* out, int nq, int nkv,
+                   int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, long long one_query_keys, float* workspace, void* out, int nq, int nkv,
                    int hd, int page_size, int num_pages, ScoreStage st, float scale);
 int attention_mfma_sigmoid(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                    const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                    const int32_t* ctx_len, const int32_t* tiles, int n_tiles, const int32_t* decode_seqs, int n_decode,
-                   int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, float* workspace, void* out, int nq, int nkv,
+                   int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, long long one_query_keys, float* workspace, void* out, int nq, int nkv,
                    int hd, int page_size, int num_pages, ScoreStage st, float scale);
 bool attention_decode_project_takes(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden);
 int attention_mfma_decode_project(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
@@ -58,24 +59,29 @@ extern "C" int sp_attention_plan(int dtype, int hd, int page_size, int nq, int n
 }
 
 static int64_t workspace_floats_of(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx,
-                                   int n_tiles, int max_tile_ctx) {
+                                   int n_tiles, int max_tile_ctx, int mean_tile_walk, long long one_query_keys) {
   const size_t decode = attention_mfma_decode_supports(nq, nkv)
                             ? attention_decode_workspace_floats(n_decode, nq, hd, max_decode_ctx) : 0;
-  return (int64_t)(decode + attention_prefill_workspace_floats(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, n_decode > 0));
+  return (int64_t)(decode + attention_prefill_workspace_floats(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk > 0 ? mean_tile_walk : max_tile_ctx,
+                                                               n_decode, one_query_keys));
 }
 
-extern "C" int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind,
-                                                 int n_decode, int max_decode_ctx, int n_tiles, int max_tile_ctx) {
+extern "C" int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int n_decode,
+                                                 int max_decode_ctx, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long one_query_keys) {
   if (!use_mfma(dtype, hd, page_size, nq, nkv, kernel_kind))   // (n_decode == n_tiles: every sequence brings one query)
     return (int64_t)attention_generic_workspace_floats(dtype, page_size, n_tiles, nq, nkv, hd, max_tile_ctx, n_decode > 0 && n_decode == n_tiles,
                                                        kernel_kind == 2);
-  return workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, n_tiles, max_tile_ctx);
+  return workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, n_tiles, max_tile_ctx, mean_tile_walk, one_query_keys);
+}
+extern "C" int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind,
+                                                 int n_decode, int max_decode_ctx, int n_tiles, int max_tile_ctx) {
+  return sp_attention_workspace_hinted(dtype, hd, page_size, nq, nkv, kernel_kind, n_decode, max_decode_ctx, n_tiles, max_tile_ctx, 0, 0);
 }
 
 extern "C" int sp_attention(void* stream, int dtype, const void* q, int q_stride, const void* k_pool,
                             const void* v_pool, const int32_t* block_tables, int max_blocks,
                             const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
-                            const int32_t* tiles, int n_tiles, int tile_q, int max_tile_ctx, int mean_tile_walk,
+                            const int32_t* tiles, int n_tiles, int tile_q, int max_tile_ctx, int mean_tile_walk, long long one_query_keys,
                             const int32_t* decode_seqs, int n_decode, int max_decode_ctx, float* workspace,
                             int64_t workspace_floats, void* out, int nq,
                             int nkv, int hd, int page_size, int num_pages, int window, float scale, int kernel_kind,
@@ -123,14 +129,15 @@ extern "C" int sp_attention(void* stream, int dtype, const void* q, int q_stride
   SP_REQUIRE(max_decode_ctx >= 0 && max_decode_ctx <= max_blocks * page_size,
              "sp_attention: decode context %d exceeds the block tables", max_decode_ctx);
   SP_REQUIRE(max_tile_ctx >= 0, "sp_attention: negative context length");
-  const int64_t need = workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, n_tiles, max_tile_ctx);
+  const int64_t need = workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, n_tiles, max_tile_ctx, mean_tile_walk,
+                                           one_query_keys);
   SP_REQUIRE(need == 0 || (workspace && workspace_floats >= need),
              "sp_attention: workspace of %lld floats is smaller than the %lld needed", (long long)workspace_floats,
              (long long)need);
   const auto launch = weight_bias ? attention_mfma_sigmoid : attention_mfma;
   return launch(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles,
                         n_tiles, decode_seqs, n_decode, max_decode_ctx, max_tile_ctx,
-                        mean_tile_walk > 0 ? mean_tile_walk : max_tile_ctx, workspace, out,
+                        mean_tile_walk > 0 ? mean_tile_walk : max_tile_ctx, one_query_keys, workspace, out,
                         nq, nkv, hd, page_size, num_pages, st, scale);
 }
 
@@ -162,7 +169,7 @@ extern "C" int sp_attention_decode_project(void* stream, const void* q, int q_st
   SP_REQUIRE(page_size > 0 && num_pages > 0 && max_blocks > 0 && max_decode_ctx <= max_blocks * page_size,
              "sp_attention_decode_project: decode context %d exceeds the block tables", max_decode_ctx);
   SP_REQUIRE(q_stride >= nq * hd, "sp_attention_decode_project: q row stride %d is smaller than %d", q_stride, nq * hd);
-  const int64_t need = workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, 0, 0);
+  const int64_t need = workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, 0, 0, 0, 0);
   SP_REQUIRE(workspace && workspace_floats >= need,
              "sp_attention_decode_project: workspace of %lld floats is smaller than the %lld needed",
              (long long)workspace_floats, (long long)need);

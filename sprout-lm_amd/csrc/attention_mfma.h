@@ -1333,7 +1333,7 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
   return false;
 }
 
-int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers);
+int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode, long long one_query_keys);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; its splits are 0 where it is not the faster one.
 int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
 bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk);
@@ -1354,7 +1354,7 @@ template <int DT, bool SIG>
 static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                        const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                        const int32_t* ctx_len, const int32_t* tiles, int n_tiles, const int32_t* decode_seqs,
-                       int n_decode, int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, float* workspace,
+                       int n_decode, int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, long long one_query_keys, float* workspace,
                        void* out, int nq, int nkv, int page_size, int num_pages, ScoreStage st, float scale) {
   constexpr int HD = 16 * DT;
   constexpr int NQT = 2;
@@ -1371,8 +1371,14 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       while ((1 << page_shift) < page_size) ++page_shift;
       const bool plain = st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && st.keep <= 0 && !st.sinks && !st.bias && !st.gate;
       int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
+      const int staged = attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, n_decode, one_query_keys);
       if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk)) rows_splits = 0;
-      const int splits = rows_splits ? rows_splits : attention_prefill_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, n_decode > 0);
+      int splits = rows_splits ? rows_splits : staged;
+      if (const int seen = st.window > 0 ? st.window : st.chunk; !rows_splits && seen > 0 && seen < max_tile_ctx - 32) {
+        // a walk is the rows' window long at most (the workspace was asked for without it: not more parts than that)
+        const int walk = seen + 32;
+        splits = min(splits, attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, walk, min(walk, mean_tile_walk), n_decode, one_query_keys));
+      }
       float* part_o = splits > 1 ? prefill_ws : nullptr;
       float* part_ml = splits > 1 ? prefill_ws + size_t(n_tiles) * 16 * NQT * nq * splits * HD : nullptr;
       StagedShape shape = staged_shape(nq, nkv, HD, n_tiles);

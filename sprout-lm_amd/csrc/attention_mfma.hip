@@ -12,28 +12,49 @@ bool attention_mfma_supports(int hd, int page_size, int nq, int nkv) {
 bool attention_mfma_decode_supports(int nq, int nkv) { return true; }
 int attention_mfma_tile_q(int hd) { return 32; }
 
-// Blocks per tile and set of heads along the keys.  A step with few queries over a long context (a portion of a long prompt) has few
-// tiles, each with a long walk: it is cut until a CU has a block of eight waves, or five waves on four at head sizes up to 64, whose blocks
-// of four share a CU; beside one-query sequences, whose blocks take places of their own, four, and above 64 half as many.  A block more than
-// that on some of the CUs, and the step waits for those; every part's sums are written and read again.  Parts hold two stages at least, eight
-// where the tiles fill half of the chip (the walks of a prompt's first tokens are half as long as the longest).  us a launch and its merge
-// by the number of parts, the choice first: 28 heads of 128 in 4 groups, 256 queries behind 1,024: four 26.0, two 28.0, five 34.8; 200 behind
-// 1,500: four 25.7, three 27.5, six 34.1; 700 from the start: one 24.3, two 36.1; 256 behind 1,024 beside eight answers: two 28.1, one 37.4,
-// four 34.1; 14 heads of 64 in 2 groups, 250 behind 1,500: five 15.5, three 15.3, eight 18.6; 300 behind 8,700: four 37.8, six 43.1; 600 behind
-// 1,000: two 20.7, one 21.4, four 25.0; 250 behind 1,500 beside five answers: four 15.5, eight 19.5, one 25.2.
-int attention_prefill_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers) {
-  if (!staged_prefill(page_size)) return 1;
+// Blocks per tile and set of heads along the keys: the number of parts with the least estimated time in microseconds.  A step with few
+// queries over a long context (a portion of a long prompt) has few tiles, each with a long walk.  `stage`: a block's 128 keys while
+// `places` blocks run at once (a CU holds one block of eight waves; of four waves as many as share it without taking longer); `ends`: its
+// queries, its waves' merge, its stores.  The one-query sequences beside them (one_query_keys keys in all) are blocks of hd / 16 us for 256 keys of
+// a set of heads that take the places which the last round of prompt blocks leaves free, and rounds behind it.  Every part costs the
+// merge what it writes and reads again, 0.8 us a million bytes.  max_tile_ctx is the longest walk, mean_tile_walk what tiles walk on average.
+// A part holds two stages at least.
+// Fitted to 1,555 steps (fifteen shapes of heads; 48 to 960 queries behind 0 to 30,720 keys, alone, beside one to 45 answers and beside short
+// prompts) timed with one to 24 parts: the choice takes 2.3 % longer than the best of them on average, 25 % or more at 10.  A rule by the number
+// of blocks alone (as many parts as give every CU a block, half as many beside answers) took 5 to 9 % longer on walks of up to 2,500
+// keys and 56 % on longer ones at 28 heads of 128 in 4 groups: 257 queries behind 30,720 beside eight answers one part 608 us, three
+// 219; 512 of them one 605, two 333; 640 alone one 604, three 425; 40 heads in 8 groups, 257 queries behind 30,720 one 586, eight 376.
+int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode, long long one_query_keys) {
+  if (!staged_prefill(page_size) || n_tiles < 1) return 1;
   const StagedShape shape = staged_shape(nq, nkv, hd, n_tiles);
-  const int G = nq / nkv;
-  const int blocks = n_tiles * nkv * ((G + shape.hpb - 1) / shape.hpb), stages = (max_tile_ctx + kStageKeys - 1) / kStageKeys;
-  const int places = 2048 / (shape.wpt * shape.hpb);
-  if (blocks <= 0 || blocks >= places || stages <= 4) return 1;
-  const int enough = hd > 64 ? (beside_answers ? places / 2 : places) : (beside_answers ? places : places * 5 / 4);
-  return max(1, min(min(enough / blocks, stages / (2 * blocks >= places ? 8 : 2)), kMaxPrefillSplits));
+  const int G = nq / nkv, blocks = n_tiles * nkv * ((G + shape.hpb - 1) / shape.hpb), stages = (max_tile_ctx + kStageKeys - 1) / kStageKeys;
+  if (blocks >= 2048 / (shape.wpt * shape.hpb) || stages <= 4) return 1;
+  const bool small = shape.wpt * shape.hpb == 4 && hd <= 128;      // blocks of four waves of which a CU holds several
+  const int places = !small ? 256 : hd <= 32 ? 1024 : hd <= 64 ? 768 : 512;
+  const float ends = small ? 2.f : 6.f;
+  const float stage = hd > 192 ? 6.f : hd > 128 ? 4.8f : small ? (hd <= 32 ? 0.8f : hd <= 64 ? 1.1f : 2.5f)
+                    : shape.hpb == 4 ? 2.3f : hd <= 64 ? 1.45f : 1.95f;
+  const float walked = fminf(1.f, float(max(1, mean_tile_walk)) / float(max_tile_ctx));
+  // (above a head size of 128 they have a launch of their own)
+  const float unit = float(hd) / 16.f, units_a_block = float(shape.wpt * shape.hpb) / 4.f;
+  const float units = hd > 128 ? 0.f : float(decode_sets(nq, nkv)) * (float(one_query_keys) / 256.f + 0.5f * float(n_decode)) / units_a_block;
+  const float merged = 0.8e-6f * float(n_tiles) * 32.f * float(nq) * float(hd + 2) * 4.f;
+  const int most = min(stages / 2, kMaxPrefillSplits);
+  int best = 1;
+  float least = 1e30f;
+  for (int parts = 1; parts <= most; ++parts) {
+    const float longest = ends + float((stages + parts - 1) / parts) * stage, mean = ends + float((stages + parts - 1) / parts) * stage * walked;
+    const int full = blocks * parts / places, rest = blocks * parts % places;
+    const float behind = rest ? fmaxf(0.f, units - float(places - rest) * floorf(mean / unit)) : units;
+    float us = fmaxf(longest, float(full + (rest > 0)) * mean + ceilf(behind / float(places)) * unit);
+    if (parts > 1) us += merged * float(parts);
+    if (us < least) least = us, best = parts;
+  }
+  return best;
 }
 
-size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, bool beside_answers) {
-  const size_t splits = max(attention_prefill_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, beside_answers),
+size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode, long long one_query_keys) {
+  const size_t splits = max(attention_prefill_parts(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, n_decode, one_query_keys),
                             attention_rows_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx));
   return splits <= 1 ? 0 : size_t(n_tiles) * 32 * nq * splits * (hd + 2);
 }
@@ -47,24 +68,24 @@ size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_c
 int attention_mfma_wide(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                         const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                         const int32_t* ctx_len, const int32_t* tiles, int n_tiles, const int32_t* decode_seqs, int n_decode,
-                        int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, float* workspace, void* out, int nq, int nkv,
+                        int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, long long one_query_keys, float* workspace, void* out, int nq, int nkv,
                         int hd, int page_size, int num_pages, ScoreStage st, float scale);
 
 int attention_mfma(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                    const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                    const int32_t* ctx_len, const int32_t* tiles, int n_tiles, const int32_t* decode_seqs, int n_decode,
-                   int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, float* workspace, void* out, int nq, int nkv,
+                   int max_decode_ctx, int max_tile_ctx, int mean_tile_walk, long long one_query_keys, float* workspace, void* out, int nq, int nkv,
                    int hd, int page_size, int num_pages, ScoreStage st, float scale) {
 #define SP_MFMA(DT)                                                                                              \
   case DT:                                                                                                       \
     return launch_mfma<DT, false>(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len,    \
-                           tiles, n_tiles, decode_seqs, n_decode, max_decode_ctx, max_tile_ctx, mean_tile_walk,  \
+                           tiles, n_tiles, decode_seqs, n_decode, max_decode_ctx, max_tile_ctx, mean_tile_walk, one_query_keys, \
                            workspace, out, nq, nkv, page_size, num_pages, st, scale)
   switch (hd / 16) {
     SP_MFMA(1); SP_MFMA(2); SP_MFMA(3); SP_MFMA(4); SP_MFMA(5); SP_MFMA(6); SP_MFMA(8);
     default:
       return attention_mfma_wide(s, q, q_stride, k_pool, v_pool, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, n_tiles,
-                                 decode_seqs, n_decode, max_decode_ctx, max_tile_ctx, mean_tile_walk, workspace, out, nq, nkv, hd,
+                                 decode_seqs, n_decode, max_decode_ctx, max_tile_ctx, mean_tile_walk, one_query_keys, workspace, out, nq, nkv, hd,
                                  page_size, num_pages, st, scale);
   }
 #undef SP_MFMA

@@ -125,12 +125,16 @@ int sp_rope_cache(void* stream, int dtype, void* qkv, const int32_t* positions, 
 // ctx_len among the sequences of the tile list (it only guides how a long walk over the keys is shared out
 // between blocks: a smaller value than the truth costs time, not correctness); mean_tile_walk: the mean over
 // the tiles of the keys a tile walks (likewise a hint, 0 if unknown: where the longest walk is much longer than
-// the mean, as in a prompt's first portion, a block takes a long and a short tile).
+// the mean, as in a prompt's first portion, a block takes a long and a short tile); one_query_keys: the sum of ctx_len over decode_seqs
+// (a hint as well, 0 if unknown: beside how much other work the walks are shared out).
 // window <= 0: all keys; else keys with position - key < window.
-// workspace: sp_attention_workspace_floats(...) floats of scratch for partial results.
+// workspace: sp_attention_workspace_hinted(...) floats of scratch for partial results, with the same hints (sp_attention_workspace_floats:
+// with both unknown).
 int sp_attention_plan(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int* plan);
 int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind,
                                       int n_decode, int max_decode_ctx, int n_tiles, int max_tile_ctx);
+int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int n_decode, int max_decode_ctx,
+                                      int n_tiles, int max_tile_ctx, int mean_tile_walk, long long one_query_keys);
 // scores: what stands between q . k and the softmax, numbered like the variants above: 0 = the scaled product and
 // nothing else; 1 = the scaled product s squashed to softcap * tanh(s / softcap).  sinks (null: none): one float per
 // query head whose exponential joins the softmax's denominator: a term without key or value, neither scaled nor
@@ -139,7 +143,7 @@ int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, 
 int sp_attention(void* stream, int dtype, const void* q, int q_stride, const void* k_pool,
                  const void* v_pool, const int32_t* block_tables, int max_blocks, const int32_t* q_start,
                  const int32_t* q_len, const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int tile_q,
-                 int max_tile_ctx, int mean_tile_walk, const int32_t* decode_seqs, int n_decode, int max_decode_ctx,
+                 int max_tile_ctx, int mean_tile_walk, long long one_query_keys, const int32_t* decode_seqs, int n_decode, int max_decode_ctx,
                  float* workspace, int64_t workspace_floats, void* out, int nq, int nkv, int hd, int page_size,
                  int num_pages, int window, float scale, int kernel_kind, int scores, float softcap, const float* sinks,
                  int mask_chunk, int keep_first, const float* weight_bias, const void* head_gate, long long head_gate_stride);

@@ -250,6 +250,7 @@ class StepArrays:
     max_ctx: int
     max_tile_ctx: int      # of the requests that bring several tokens
     mean_walk: int
+    one_query_keys: int    # the contexts of the requests that bring one token, together
     host: dict
 
     def named(self, name: str):
@@ -311,11 +312,12 @@ def step_arrays(entries: list[StepEntry], cache, table_tokens: int | None = None
             "state_slots": state_slots, "seq_of_token": seq_of_token, "first_pos": first_pos}
     return StepArrays(names, arrays, lists, T, len(entries), len(rows), max(q_lens, default=0), max(decode_ctx, default=0),
                       max((int(c) for c in ctx_len), default=0), max((int(c) for c, q in zip(ctx_len, q_lens) if q > 1), default=0),
-                      ops.mean_tile_walk(q_lens, ctx_len), host)
+                      ops.mean_tile_walk(q_lens, ctx_len), sum(decode_ctx), host)
 
 
 def context_from(step: StepArrays, dev: list, n_groups: int, workspace: Workspace, act_dtype, attention_kind: int = 0,
-                 max_decode_ctx: int | None = None, max_ctx: int | None = None, max_tile_ctx: int | None = None) -> StepContext:
+                 max_decode_ctx: int | None = None, max_ctx: int | None = None, max_tile_ctx: int | None = None,
+                 mean_walk: int | None = None) -> StepContext:
     """The step's context over the device copies `dev` of `step.arrays` (same order)."""
     ctx = StepContext(workspace, act_dtype, attention_kind)
     by_name = dict(zip(step.names, dev))
@@ -326,8 +328,9 @@ def context_from(step: StepArrays, dev: list, n_groups: int, workspace: Workspac
     on_device = {name: (by_name[name], len(step.lists[name])) for name in step.lists}
     ctx.attention = ops.AttentionBatch(ctx.q_start, ctx.q_len, ctx.ctx_len, step.n_seqs, on_device,
                                        step.max_decode_ctx if max_decode_ctx is None else max_decode_ctx,
-                                       step.max_ctx if max_ctx is None else max_ctx, step.mean_walk,
-                                       step.max_tile_ctx if max_tile_ctx is None else max_tile_ctx)
+                                       step.max_ctx if max_ctx is None else max_ctx,
+                                       step.mean_walk if mean_walk is None else mean_walk,
+                                       step.max_tile_ctx if max_tile_ctx is None else max_tile_ctx, step.one_query_keys)
     ctx.group_tables = [by_name[f"tables{g}"] for g in range(n_groups)]
     ctx.group_slots = [by_name[f"slots{g}"] for g in range(n_groups)]
     ctx.n_tokens, ctx.n_seqs, ctx.n_logits = step.n_tokens, step.n_seqs, step.n_logits

@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import gc
 import itertools
+import math
 import weakref
 
 import numpy as np
@@ -210,13 +211,15 @@ class _PortionGraph:
         views = [self.dev[o:o + n].view(a.shape) for o, n, a in zip(self.offsets, self.sizes, first.arrays)]
         # Descriptors of its own; the scratch tensors are shared with the other recorded steps of this kind (they
         # run one after the other on one stream, and `workspace` never frees or moves a tensor).  The longest
-        # context is known to the kernels as its bucket only (how a long walk is shared out follows it), and the
-        # step has no values on the host.
+        # context is known to the kernels as its bucket only, and the step has no values on the host.  How prompts'
+        # walks are shared out follows a length between the longest one's now and the bucket, which those of later
+        # portions lie between as well (256 tokens behind 1,024 beside answers at 4,096: as if 2,289 keys were read).
         # The logits are what the caller gets: they live in a tensor of this graph's own.
         self.shared_workspace = workspace
+        longest = math.isqrt(first.max_tile_ctx * ctx_bucket)
         self.ctx = context_from(first, views, len(cache.groups), OwnedNames(workspace, ("logits",), runner.device),
                                 runner.dtype, runner.attention_kind, max_decode_ctx=ctx_bucket, max_ctx=ctx_bucket,
-                                max_tile_ctx=ctx_bucket)
+                                max_tile_ctx=longest, mean_walk=first.mean_walk * longest // max(1, first.max_tile_ctx))
         self.ctx.host = {}
         self.copied = None
         self.graph = None

@@ -734,15 +734,16 @@ class AttentionBatch:
     """The device-side description of a step's sequences that `attention` reads."""
 
     def __init__(self, q_start, q_len, ctx_len, n_seqs: int, lists: dict, max_decode_ctx: int, max_ctx: int,
-                 mean_walk: int = 0, max_tile_ctx: int | None = None):
+                 mean_walk: int = 0, max_tile_ctx: int | None = None, one_query_keys: int = 0):
         """`lists`: name -> (device int32 tensor, number of entries), names as in `attention_lists`;
         `max_decode_ctx`, `max_ctx`: the longest context among one-query sequences, and among all;
         `mean_walk`: the mean number of keys that a tile of queries walks, see `mean_tile_walk` (a hint for
         how the kernels share out the work; unknown: 0); `max_tile_ctx`: the longest context among sequences with several
-        queries (a hint as well; by default the longest of all)."""
+        queries (a hint as well; by default the longest of all); `one_query_keys`: the sum of the one-query sequences'
+        contexts (a hint as well; unknown: 0)."""
         self.q_start, self.q_len, self.ctx_len, self.n_seqs = q_start, q_len, ctx_len, n_seqs
         self.lists, self.max_decode_ctx, self.max_ctx = lists, max_decode_ctx, max_ctx
-        self.mean_walk = mean_walk
+        self.mean_walk, self.one_query_keys = mean_walk, one_query_keys
         self.max_tile_ctx = max_ctx if max_tile_ctx is None else max_tile_ctx
 
     @classmethod
@@ -755,7 +756,8 @@ class AttentionBatch:
         decode_ctx = [c for c, q in zip(ctx_lens, q_lens) if q == 1]
         return cls(to(starts), to(q_lens), to(ctx_lens), len(q_lens), lists, max(decode_ctx, default=0),
                    max((int(c) for c in ctx_lens), default=0),
-                   mean_tile_walk(q_lens, ctx_lens), max((int(c) for c, q in zip(ctx_lens, q_lens) if q > 1), default=0))
+                   mean_tile_walk(q_lens, ctx_lens), max((int(c) for c, q in zip(ctx_lens, q_lens) if q > 1), default=0),
+                   sum(int(c) for c in decode_ctx))
 
 
 def attention_plan(dtype: torch.dtype, hd: int, page_size: int, nq: int, nkv: int, kind: int = 0) -> tuple[int, bool]:
@@ -851,8 +853,9 @@ def attention(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torc
     max_tile_ctx = (batch.max_ctx if every else batch.max_tile_ctx) if n_tiles else 0
     if one_query_each:
         n_decode = n_tiles
-    need = library().sp_attention_workspace_floats(_code(q, "q"), hd, page_size, nq, nkv, kind, n_decode, max_decode_ctx,
-                                                   n_tiles, max_tile_ctx)
+    hints = (int(batch.mean_walk), int(batch.one_query_keys))
+    need = library().sp_attention_workspace_hinted(_code(q, "q"), hd, page_size, nq, nkv, kind, n_decode, max_decode_ctx,
+                                                   n_tiles, max_tile_ctx, *hints)
     ws = None
     if need:
         ws = workspace(need) if workspace is not None else torch.empty(need, dtype=torch.float32, device=q.device)
@@ -876,7 +879,7 @@ def attention(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torc
     check(library().sp_attention(_stream(), _code(q, "q"), q.data_ptr(), q_stride, k_pool.data_ptr(), v_pool.data_ptr(),
                                  block_tables.data_ptr(), block_tables.shape[1], batch.q_start.data_ptr(),
                                  batch.q_len.data_ptr(), batch.ctx_len.data_ptr(), _ptr(tiles) if n_tiles else None,
-                                 n_tiles, tile_q, max_tile_ctx, int(batch.mean_walk),
+                                 n_tiles, tile_q, max_tile_ctx, *hints,
                                  _ptr(decode) if n_decode and decode is not None else None, n_decode,
                                  max_decode_ctx, _ptr(ws),
                                  need, out.data_ptr(), nq, nkv, hd, page_size, num_pages, int(window) if window else 0,

@@ -29,7 +29,7 @@ def _declare(lib):
         "sp_rope_cache": [c_void, c_int, c_void, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_int, c_int,
                           c_int, c_int, c_int, c_int, c_int],
         "sp_attention": [c_void, c_int, c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_void, c_void, c_void,
-                         c_int, c_int, c_int, c_int, c_void, c_int, c_int, c_void, c_i64, c_void, c_int, c_int, c_int, c_int,
+                         c_int, c_int, c_int, c_int, c_i64, c_void, c_int, c_int, c_void, c_i64, c_void, c_int, c_int, c_int, c_int,
                          c_int, c_int, c_float, c_int, c_int, c_float, c_void, c_int, c_int, c_void, c_void, c_i64],
         "sp_attention_decode_project_takes": [c_int] * 7,
         "sp_attention_decode_project": [c_void, c_void, c_int, c_void, c_void, c_void, c_int, c_void, c_void, c_void,
@@ -125,6 +125,8 @@ def _declare(lib):
     lib.sp_gemm_f32_split_gates.restype = c_int
     lib.sp_attention_workspace_floats.argtypes = [c_int] * 10
     lib.sp_attention_workspace_floats.restype = c_i64
+    lib.sp_attention_workspace_hinted.argtypes = [c_int] * 11 + [c_i64]
+    lib.sp_attention_workspace_hinted.restype = c_i64
     lib.sp_rglru_carry_floats.argtypes = [c_int] * 4
     lib.sp_rglru_carry_floats.restype = c_i64
     lib.sp_retention_scratch_floats.argtypes = [c_int] * 6
