@@ -16,7 +16,7 @@ bool attention_mfma_decode_supports(int nq, int nkv);
 int attention_mfma_tile_q(int hd);
 size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_ctx);
 size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode,
-                                         long long one_query_keys);
+                                         int max_decode_ctx, long long one_query_keys);
 int attention_mfma(hipStream_t s, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                    const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                    const int32_t* ctx_len, const int32_t* tiles, int n_tiles, const int32_t* decode_seqs, int n_decode,
@@ -63,7 +63,7 @@ static int64_t workspace_floats_of(int hd, int page_size, int nq, int nkv, int n
   const size_t decode = attention_mfma_decode_supports(nq, nkv)
                             ? attention_decode_workspace_floats(n_decode, nq, hd, max_decode_ctx) : 0;
   return (int64_t)(decode + attention_prefill_workspace_floats(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk > 0 ? mean_tile_walk : max_tile_ctx,
-                                                               n_decode, one_query_keys));
+                                                               n_decode, max_decode_ctx, one_query_keys));
 }
 
 extern "C" int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int n_decode,

@@ -1333,7 +1333,7 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
   return false;
 }
 
-int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode, long long one_query_keys);
+int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; its splits are 0 where it is not the faster one.
 int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
 bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk);
@@ -1346,6 +1346,29 @@ size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_c
 // softmax weights: blocks of 16 waves are those of long prompts, beside which the one-query blocks are little, and would hold
 // four of those each.
 constexpr bool mixed_instantiated(int dt, bool sig) { return !sig && dt <= 8; }
+// ... and where those blocks are not most of the step: in the prompts' blocks they get less of a CU than by themselves (LDS for 12 waves of
+// heads of 64 where their own launch runs 32), and where a block takes two of them, ragged batches of many chunks do not spread evenly.
+// `chunks`: blocks with keys in sight.  us in one launch and in their own, beside 33 queries: 16 heads of 64 in 8 groups (eight waves) 16 answers
+// at 3,000 to 4,096 (1,816 chunks) 35.8 and 36.0, 24 (2,728) 49 and 47, 64 (7,280) 109 and 97, 128 at 190 to 4,096 (5,608) 102 and 84; 28 heads of
+// 128 in 4 groups, 24 answers at 2,000 to 16,384 (2,648 of 64 a sequence) 1.29 times as long in one, 8 at 8,200 to 16,000 (1,480) 0.95 times, 192
+// at 1,500 to 2,048 (5,644 of 8) 1.01; 32 heads of 64 in 8 groups (four waves) 96 at 190 to 4,096 (4,200 of the launch's 12,288) 1.05, 32 (1,392)
+// 0.93, 192 at 1,500 to 2,048 (11,288 of 12,288) 0.97.
+static bool mixed_pays(int waves, int hd, int n_splits, long long chunks, long long launched) {
+  if (waves <= 4) return chunks <= 4096 || 2 * chunks > launched;
+  return chunks <= (n_splits > 32 ? 1024 : hd > 96 ? 4096 : 2048);
+}
+// Those blocks of n_decode sequences of keys_together keys; not known (0): as if every sequence were as long as the longest.
+static long long one_query_chunks(int nq, int nkv, int n_decode, int n_splits, long long keys_together) {
+  const long long whole = (long long)n_decode * n_splits;
+  return (keys_together > 0 ? min(whole, max((long long)n_decode, keys_together / kDecodeChunk + n_decode / 2)) : whole) * decode_sets(nq, nkv);
+}
+// The one-query blocks that share a launch with n_tiles tiles of prompts, 0 where they have their own.
+static long long chunks_beside(int hd, int nq, int nkv, int n_tiles, int n_decode, int max_decode_ctx, long long keys_together) {
+  const StagedShape shape = staged_shape(nq, nkv, hd, n_tiles);
+  const int n_splits = max(1, (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk);
+  const long long chunks = one_query_chunks(nq, nkv, n_decode, n_splits, keys_together);
+  return hd <= 128 && shape.hpb * shape.wpt <= 8 && mixed_pays(shape.hpb * shape.wpt, hd, n_splits, chunks, (long long)n_decode * n_splits * decode_sets(nq, nkv)) ? chunks : 0;
+}
 int launch_mixed(hipStream_t s, int dt, int hpb, int wpt, bool paired, const uint16_t* q, int q_stride, const uint16_t* k_pool,
                  const uint16_t* v_pool, const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* ctx_len,
                  uint16_t* out, int nq, int nkv, int num_pages, const ScoreStage& st, float scale2, const PromptPart& p, const DecodePart& d);
@@ -1371,20 +1394,21 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       while ((1 << page_shift) < page_size) ++page_shift;
       const bool plain = st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && st.keep <= 0 && !st.sinks && !st.bias && !st.gate;
       int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
-      const int staged = attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, n_decode, one_query_keys);
+      const long long beside = chunks_beside(HD, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys);
+      const int staged = attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside);
       if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk)) rows_splits = 0;
       int splits = rows_splits ? rows_splits : staged;
       if (const int seen = st.window > 0 ? st.window : st.chunk; !rows_splits && seen > 0 && seen < max_tile_ctx - 32) {
         // a walk is the rows' window long at most (the workspace was asked for without it: not more parts than that)
         const int walk = seen + 32;
-        splits = min(splits, attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, walk, min(walk, mean_tile_walk), n_decode, one_query_keys));
+        splits = min(splits, attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, walk, min(walk, mean_tile_walk), beside));
       }
       float* part_o = splits > 1 ? prefill_ws : nullptr;
       float* part_ml = splits > 1 ? prefill_ws + size_t(n_tiles) * 16 * NQT * nq * splits * HD : nullptr;
       StagedShape shape = staged_shape(nq, nkv, HD, n_tiles);
       const bool paired = staged_paired(n_tiles, nq, nkv, HD, splits, max_tile_ctx, mean_tile_walk, &shape);
       const dim3 grid(paired ? (n_tiles + 1) / 2 : n_tiles, nkv * ((nq / nkv + shape.hpb - 1) / shape.hpb), splits);
-      if (mixed_instantiated(DT, SIG) && n_decode > 0 && !rows_splits && shape.hpb * shape.wpt <= 8) {
+      if (mixed_instantiated(DT, SIG) && beside > 0 && !rows_splits && shape.hpb * shape.wpt <= 8) {
         const int sets = decode_sets(nq, nkv);
         return launch_mixed(s, DT, shape.hpb, shape.wpt, paired, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, ctx_len,
                             (uint16_t*)out, nq, nkv, num_pages, st, scale2,

@@ -15,8 +15,8 @@ int attention_mfma_tile_q(int hd) { return 32; }
 // Blocks per tile and set of heads along the keys: the number of parts with the least estimated time in microseconds.  A step with few
 // queries over a long context (a portion of a long prompt) has few tiles, each with a long walk.  `stage`: a block's 128 keys while
 // `places` blocks run at once (a CU holds one block of eight waves; of four waves as many as share it without taking longer); `ends`: its
-// queries, its waves' merge, its stores.  The one-query sequences beside them (one_query_keys keys in all) are blocks of hd / 16 us for 256 keys of
-// a set of heads that take the places which the last round of prompt blocks leaves free, and rounds behind it.  Every part costs the
+// queries, its waves' merge, its stores.  One-query blocks that share the launch (`beside`) take hd / 16 us for their 256 keys, in
+// the places which the last round of prompt blocks leaves free and in rounds behind it.  Every part costs the
 // merge what it writes and reads again, 0.8 us a million bytes.  max_tile_ctx is the longest walk, mean_tile_walk what tiles walk on average.
 // A part holds two stages at least.
 // Fitted to 1,555 steps (fifteen shapes of heads; 48 to 960 queries behind 0 to 30,720 keys, alone, beside one to 45 answers and beside short
@@ -24,7 +24,7 @@ int attention_mfma_tile_q(int hd) { return 32; }
 // of blocks alone (as many parts as give every CU a block, half as many beside answers) took 5 to 9 % longer on walks of up to 2,500
 // keys and 56 % on longer ones at 28 heads of 128 in 4 groups: 257 queries behind 30,720 beside eight answers one part 608 us, three
 // 219; 512 of them one 605, two 333; 640 alone one 604, three 425; 40 heads in 8 groups, 257 queries behind 30,720 one 586, eight 376.
-int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode, long long one_query_keys) {
+int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside) {
   if (!staged_prefill(page_size) || n_tiles < 1) return 1;
   const StagedShape shape = staged_shape(nq, nkv, hd, n_tiles);
   const int G = nq / nkv, blocks = n_tiles * nkv * ((G + shape.hpb - 1) / shape.hpb), stages = (max_tile_ctx + kStageKeys - 1) / kStageKeys;
@@ -35,9 +35,7 @@ int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size,
   const float stage = hd > 192 ? 6.f : hd > 128 ? 4.8f : small ? (hd <= 32 ? 0.8f : hd <= 64 ? 1.1f : 2.5f)
                     : shape.hpb == 4 ? 2.3f : hd <= 64 ? 1.45f : 1.95f;
   const float walked = fminf(1.f, float(max(1, mean_tile_walk)) / float(max_tile_ctx));
-  // (above a head size of 128 they have a launch of their own)
-  const float unit = float(hd) / 16.f, units_a_block = float(shape.wpt * shape.hpb) / 4.f;
-  const float units = hd > 128 ? 0.f : float(decode_sets(nq, nkv)) * (float(one_query_keys) / 256.f + 0.5f * float(n_decode)) / units_a_block;
+  const float unit = float(hd) / 16.f, units = float(beside) / (float(shape.wpt * shape.hpb) / 4.f);
   const float merged = 0.8e-6f * float(n_tiles) * 32.f * float(nq) * float(hd + 2) * 4.f;
   const int most = min(stages / 2, kMaxPrefillSplits);
   int best = 1;
@@ -53,8 +51,10 @@ int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size,
   return best;
 }
 
-size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode, long long one_query_keys) {
-  const size_t splits = max(attention_prefill_parts(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, n_decode, one_query_keys),
+size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, int n_decode,
+                                          int max_decode_ctx, long long one_query_keys) {
+  const long long beside = chunks_beside(hd, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys);
+  const size_t splits = max(attention_prefill_parts(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, beside),
                             attention_rows_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx));
   return splits <= 1 ? 0 : size_t(n_tiles) * 32 * nq * splits * (hd + 2);
 }
@@ -168,3 +168,11 @@ int attention_mfma_decode_project(hipStream_t s, const void* q, int q_stride, co
 }
 
 }  // namespace sprout
+
+// Whether a step's prompts and one-query sequences may share a launch (sp_attention takes it where no other kernel takes the prompts): 1 or
+// 0.  Runs nothing: for tests.
+extern "C" int sp_attention_mixed_pays(int hd, int nq, int nkv, int n_tiles, int n_decode, int max_decode_ctx, long long one_query_keys) {
+  using namespace sprout;
+  if (hd < 16 || hd > 128 || nkv < 1 || nq < nkv || nq % nkv || n_tiles < 1 || n_decode < 1 || max_decode_ctx < 1) return 0;
+  return chunks_beside(hd, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys) > 0;
+}

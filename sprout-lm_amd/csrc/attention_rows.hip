@@ -365,7 +365,7 @@ int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, i
 // queries over 16,384 beside seven prompts of 300: 340 us here, 165 there; 64 in 8 groups, 32 queries over 32,768 beside eight of 128:
 // 662 and 578, but over 4,096 90 and 100).
 bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk) {
-  const int G = nq / nkv, sets = (G + 7) / 8, there = attention_prefill_parts(n_tiles, nq, nkv, 64, page_size, max_tile_ctx, mean_tile_walk, 0, 0);
+  const int G = nq / nkv, sets = (G + 7) / 8, there = attention_prefill_parts(n_tiles, nq, nkv, 64, page_size, max_tile_ctx, mean_tile_walk, 0);
   const float longest = float(max_tile_ctx) / float(splits);
   if (longest <= 3.f * float(n_tiles) * float(nkv * sets) * float(mean_tile_walk) / 256.f) return false;
   StagedShape shape = staged_shape(nq, nkv, 64, n_tiles);

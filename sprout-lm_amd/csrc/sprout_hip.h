@@ -135,6 +135,7 @@ int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, 
                                       int n_decode, int max_decode_ctx, int n_tiles, int max_tile_ctx);
 int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int n_decode, int max_decode_ctx,
                                       int n_tiles, int max_tile_ctx, int mean_tile_walk, long long one_query_keys);
+int sp_attention_mixed_pays(int hd, int nq, int nkv, int n_tiles, int n_decode, int max_decode_ctx, long long one_query_keys);
 // scores: what stands between q . k and the softmax, numbered like the variants above: 0 = the scaled product and
 // nothing else; 1 = the scaled product s squashed to softcap * tanh(s / softcap).  sinks (null: none): one float per
 // query head whose exponential joins the softmax's denominator: a term without key or value, neither scaled nor

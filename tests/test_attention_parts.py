@@ -50,3 +50,16 @@ def test_a_part_holds_two_stages_and_there_are_32_at_most(lib):
             for behind in (0, 300, 600, 1100, 5000, 32000, 130000):
                 for parts in _asked(lib, nq, nkv, hd, queries, behind, 3, 700):
                     assert parts <= 32 and (parts == 1 or parts * 256 <= behind + queries + 127)
+
+
+def test_prompts_and_many_answers_have_launches_of_their_own(lib):
+    """Few one-query blocks go with the prompts' blocks, many do not: either side of the lines."""
+    pays = lambda hd, nq, nkv, tiles, answers, longest, keys: bool(lib.sp_attention_mixed_pays(hd, nq, nkv, tiles, answers, longest, keys))
+    assert pays(128, 28, 4, 4, 1, 63, 63) and pays(64, 14, 2, 4, 1, 256, 1)                       # one answer that has just begun
+    assert pays(64, 14, 2, 8, 5, 1500, 4000) and pays(128, 28, 4, 8, 8, 4096, 18000)            # the steps that gain
+    assert pays(64, 16, 8, 2, 16, 4096, 16 * 3400) and not pays(64, 16, 8, 2, 24, 4096, 24 * 3500)      # eight waves, heads of 64
+    assert not pays(64, 16, 8, 2, 128, 4096, 128 * 1300)
+    assert pays(128, 28, 4, 2, 8, 8192, 8 * 8000) and not pays(128, 28, 4, 2, 24, 16384, 24 * 7000)     # many chunks a sequence
+    assert pays(128, 28, 4, 2, 8, 32768, 8 * 2000)        # known as a bucket, though few of its chunks hold keys
+    assert pays(64, 32, 8, 2, 32, 4096, 32 * 1300) and not pays(64, 32, 8, 2, 128, 4096, 128 * 1300)    # four waves
+    assert not pays(64, 16, 8, 2, 128, 4096, 0)           # keys not known: all of them as long as the longest
