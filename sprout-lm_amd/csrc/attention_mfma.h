@@ -1336,7 +1336,7 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
 int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; its splits are 0 where it is not the faster one.
 int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
-bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk);
+bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk, int there);
 int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
                           const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
                           const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int splits, uint16_t* out,
@@ -1396,7 +1396,7 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
       const long long beside = chunks_beside(HD, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys);
       const int staged = attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside);
-      if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk)) rows_splits = 0;
+      if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk, staged)) rows_splits = 0;
       int splits = rows_splits ? rows_splits : staged;
       if (const int seen = st.window > 0 ? st.window : st.chunk; !rows_splits && seen > 0 && seen < max_tile_ctx - 32) {
         // a walk is the rows' window long at most (the workspace was asked for without it: not more parts than that)

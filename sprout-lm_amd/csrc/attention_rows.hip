@@ -360,12 +360,12 @@ int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, i
 
 // Whether this kernel is the slower one all the same: one walk among many short ones bounds the launch where it is longer than three
 // times a CU's share of all walks, and a block of this kernel walks alone at 0.0203 us a key where the blocks of attention_mfma.h share
-// its keys out over four waves a head.  Microseconds a walk, fitted to 250 mixes of 32 to 1,024 queries over 2,048 to 32,768 keys with
-// prompts of 64 to 1,024, which the rule leaves within 5 % of the faster kernel but for three of 9 to 13 % (24 heads in 2 groups, 256
-// queries over 16,384 beside seven prompts of 300: 340 us here, 165 there; 64 in 8 groups, 32 queries over 32,768 beside eight of 128:
-// 662 and 578, but over 4,096 90 and 100).
-bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk) {
-  const int G = nq / nkv, sets = (G + 7) / 8, there = attention_prefill_parts(n_tiles, nq, nkv, 64, page_size, max_tile_ctx, mean_tile_walk, 0);
+// its keys out over four waves a head, in `there` parts.  Timed on both kernels over 613 steps (eight shapes of heads; 32 to 1,024 queries behind
+// 2,048 to 32,000 keys, alone and with two or eight prompts of 64 to 1,024, alone and beside eight answers) the rule's choice takes 1.6 % longer than the faster
+// one on average, 55 of them more than 10 %; this kernel always 3.9 %, that one always 55 %.  The worst: 24 heads in 2 groups, 1,024 queries behind
+// 32,000 beside eight prompts of 300, 938 us here and 596 there, where the longest walk is not three times the share.
+bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk, int there) {
+  const int G = nq / nkv, sets = (G + 7) / 8;
   const float longest = float(max_tile_ctx) / float(splits);
   if (longest <= 3.f * float(n_tiles) * float(nkv * sets) * float(mean_tile_walk) / 256.f) return false;
   StagedShape shape = staged_shape(nq, nkv, 64, n_tiles);
