@@ -63,3 +63,10 @@ def test_prompts_and_many_answers_have_launches_of_their_own(lib):
     assert pays(128, 28, 4, 2, 8, 32768, 8 * 2000)        # known as a bucket, though few of its chunks hold keys
     assert pays(64, 32, 8, 2, 32, 4096, 32 * 1300) and not pays(64, 32, 8, 2, 128, 4096, 128 * 1300)    # four waves
     assert not pays(64, 16, 8, 2, 128, 4096, 0)           # keys not known: all of them as long as the longest
+
+
+def test_walks_count_in_fractions_for_the_kernel_of_two_heads_a_wave(lib):
+    """144 blocks that walk 3,768 keys fill the chip as 256 of 2,048 do (62 us against 123): three parts of 1,024 keys at least, which only that
+    kernel has here; 2,600 keys do not."""
+    assert _asked(lib, 48, 6, 64, 768, 3000) == [3, 3]
+    assert _asked(lib, 48, 6, 64, 768, 1832) == [1, 1]
