@@ -18,7 +18,7 @@ int attention_mfma_tile_q(int hd) { return 32; }
 // queries, its waves' merge, its stores.  One-query blocks that share the launch (`beside`) take hd / 16 us for their 256 keys, in
 // the places which the last round of prompt blocks leaves free and in rounds behind it.  Every part costs the
 // merge what it writes and reads again, 0.8 us a million bytes.  max_tile_ctx is the longest walk, mean_tile_walk what tiles walk on average.
-// A part holds two stages at least.
+// A part holds two stages at least, of wide heads one (8 heads of 256, 128 queries behind 512: five parts 22.5 us, two 34.7).
 // Fitted to 1,555 steps (fifteen shapes of heads; 48 to 960 queries behind 0 to 30,720 keys, alone, beside one to 45 answers and beside short
 // prompts) timed with one to 24 parts: the choice takes 2.3 % longer than the best of them on average, 25 % or more at 10.  A rule by the number
 // of blocks alone (as many parts as give every CU a block, half as many beside answers) took 5 to 9 % longer on walks of up to 2,500
@@ -37,7 +37,7 @@ int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size,
   const float walked = fminf(1.f, float(max(1, mean_tile_walk)) / float(max_tile_ctx));
   const float unit = float(hd) / 16.f, units = float(beside) / (float(shape.wpt * shape.hpb) / 4.f);
   const float merged = 0.8e-6f * float(n_tiles) * 32.f * float(nq) * float(hd + 2) * 4.f;
-  const int most = min(stages / 2, kMaxPrefillSplits);
+  const int most = min(hd > 128 ? stages : stages / 2, kMaxPrefillSplits);
   int best = 1;
   float least = 1e30f;
   for (int parts = 1; parts <= most; ++parts) {

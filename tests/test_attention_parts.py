@@ -44,12 +44,12 @@ def test_short_walks_and_full_chips_are_not_cut(lib):
     assert _asked(lib, 28, 4, 128, 320, 1024, 45, 2000)[1] == 1
 
 
-def test_a_part_holds_two_stages_and_there_are_32_at_most(lib):
+def test_a_part_holds_two_stages_or_one_of_wide_heads_and_there_are_32_at_most(lib):
     for nq, nkv, hd in ((28, 4, 128), (12, 4, 64), (8, 1, 256), (16, 1, 192), (3, 3, 80), (1, 1, 16)):
         for queries in (2, 33, 128, 500, 1000):
             for behind in (0, 300, 600, 1100, 5000, 32000, 130000):
                 for parts in _asked(lib, nq, nkv, hd, queries, behind, 3, 700):
-                    assert parts <= 32 and (parts == 1 or parts * 256 <= behind + queries + 127)
+                    assert parts <= 32 and (parts == 1 or parts * (128 if hd > 128 else 256) <= behind + queries + 127)
 
 
 def test_prompts_and_many_answers_have_launches_of_their_own(lib):
@@ -70,3 +70,7 @@ def test_walks_count_in_fractions_for_the_kernel_of_two_heads_a_wave(lib):
     kernel has here; 2,600 keys do not."""
     assert _asked(lib, 48, 6, 64, 768, 3000) == [3, 3]
     assert _asked(lib, 48, 6, 64, 768, 1832) == [1, 1]
+
+
+def test_short_walks_of_wide_heads_are_cut_into_single_stages(lib):
+    assert _asked(lib, 8, 1, 256, 48, 512) == [5, 5] and _asked(lib, 4, 4, 256, 48, 512, 8, 2048) == [5, 5]
