@@ -416,14 +416,23 @@ int launch_skinny(hipStream_t s, const float* x, const float* w, const void* bia
   return check_launch("sp_gemm (float32, few tokens)");
 }
 
+// Waves of a block that share K.  Eight where that brings a wave's steps of 16 down to the 8 that it asks for at once: K from 257 on, or from 129
+// with few rows, of matrices of up to 8 M weights, and of heads with K up to 2,048 (8 tokens, four waves -> eight, us: 896 rows of 4,864 7.86 ->
+// 7.39, 896 of 896 6.43 -> 5.85, 1,152 of 896 5.86 -> 5.35, 2,560 of 2,560 12.1 -> 11.3, 151,936 of 896 138.7 -> 134.3).  With shorter K four have no
+// more steps than that, and eight waves' sums cost more than they save (32,000 rows of 64 4.3 -> 5.7, of 128 6.4 -> 7.2, 15,000 of 256 6.5 -> 7.4); larger
+// matrices are bound by what the chip has on its way (1,536 of 8,960 21.0 -> 21.6, 4,608 of 3,584 30.0 -> 32.1, 5,120 of 5,120 44.2 -> 46.7).  Over 738
+// products (1, 8 and 16 tokens; 64 to 151,936 rows of 64 to 4,864) the choice takes 0.8 % longer than the better of the two, 9 % more than four
+// waves at worst (4,864 rows of 1,536).
+int skinny_waves(int N, int K) {
+  const int tiles = (N + 15) / 16;
+  if (K <= (tiles < 512 ? 128 : 256)) return 4;
+  return size_t(N) * K <= 8000000 || (tiles >= 4096 && K <= 2048) ? 8 : 4;
+}
+
 template <typename TB>
 int skinny_shape(hipStream_t s, const float* x, const float* w, const void* bias, int mode, float* out, int T, int N, int K) {
-  // Eight waves share K where that brings a wave's steps down to the 8 that it asks for at once: matrices of up to 8 M weights, and heads of
-  // a short K (8 tokens, four waves -> eight, us: 896 rows of 4,864 7.86 -> 7.39, 896 of 896 6.43 -> 5.85, 1,152 of 896 5.86 -> 5.35, 2,560 of
-  // 2,560 12.1 -> 11.3, 151,936 of 896 138.7 -> 134.3).  Larger ones are bound by what the chip has on its way, and eight waves' sums cost
-  // them more than they save (1,536 of 8,960 21.0 -> 21.6, 4,608 of 3,584 30.0 -> 32.1, 5,120 of 5,120 44.2 -> 46.7, 32,000 of 256 10.5 -> 11.3).
   const int tiles = (N + 15) / 16;
-  const bool eight = size_t(N) * K <= 8000000 || (tiles >= 4096 && K <= 2048);
+  const bool eight = skinny_waves(N, K) == 8;
   if (tiles >= 4096)
     return eight ? launch_skinny<4, TB, 8>(s, x, w, bias, mode, out, T, N, K) : launch_skinny<4, TB, 4>(s, x, w, bias, mode, out, T, N, K);
   if (tiles >= 1024)
@@ -550,6 +559,9 @@ extern "C" int sp_qkv_rope_cache_f32(void* stream, const float* x, const float* 
   if (bias && bias_dtype == kBF16) return launch_qkv<bf16_t>((hipStream_t)stream, x, w, bias, q_out, T, K, extra);
   return launch_qkv<float>((hipStream_t)stream, x, w, bias, q_out, T, K, extra);
 }
+
+// Waves a block with which sp_gemm takes up to 16 tokens in float32.  Runs nothing: for tests.
+extern "C" int sp_gemm_f32_waves(int N, int K) { return sprout::skinny_waves(N, K); }
 
 // The block shape and the parts of K that sp_gemm_parts takes for T x N x K in float32: plan = {block rows, block columns, parts}.  Returns 1 where
 // it does not take the product, else 0.  Runs nothing: for tests.

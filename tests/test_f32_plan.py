@@ -28,3 +28,11 @@ def test_parts_are_counted_on_the_fullest_xcd(lib):
             assert t * n * parts > 256 or fullest <= 32, (T, N, K, rows, columns, parts)
             taken += 1
     assert taken > 40
+
+
+def test_eight_waves_share_a_k_that_four_do_not_ask_for_at_once(lib):
+    for N, K in ((896, 4864), (896, 896), (1152, 896), (2560, 2560), (151936, 896), (9728, 512), (896, 192)):
+        assert lib.sp_gemm_f32_waves(N, K) == 8, (N, K)
+    # few steps a wave as it is, and matrices that are bound by what is on its way
+    for N, K in ((30000, 256), (32000, 64), (32000, 128), (15000, 256), (896, 128), (64, 64), (151936, 64), (1536, 8960), (5120, 5120), (65536, 2052)):
+        assert lib.sp_gemm_f32_waves(N, K) == 4, (N, K)
