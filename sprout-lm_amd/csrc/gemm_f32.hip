@@ -231,6 +231,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float
     for (int j = 0; j < NB; ++j) sum = fmaf(mine[j].x, mine[j].x, fmaf(mine[j].y, mine[j].y, fmaf(mine[j].z, mine[j].z, fmaf(mine[j].w, mine[j].w, sum))));
 #pragma unroll
     for (int o = P / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if (K % 16 != 0 && part == 0) *reinterpret_cast<float4*>(normed + t * (K + 4) + K) = make_float4(0.f, 0.f, 0.f, 0.f);
     scale = 1.0f / sqrtf(sum / float(K) + extra.eps);
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
@@ -287,8 +288,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_skinny_kernel(const float
       if (s + u >= s1) break;      // the same for the whole wave
       float4 a;
       if constexpr (STAGED) {
-        // (columns of tokens past the last one repeat the eighth row and are not used)
-        a = *reinterpret_cast<const float4*>(normed + min(lr, 7) * (K + 4) + min(16 * (s + u) + 4 * lj, K - 4));
+        // (columns of tokens past the last one repeat the eighth row and are not used; past the end of K both operands are zeros, this
+        // one's those behind its row: a weight's zero times a normed number that has overflowed would be NaN)
+        a = *reinterpret_cast<const float4*>(normed + min(lr, 7) * (K + 4) + min(16 * (s + u) + 4 * lj, K));
       } else {
         a = xv[u];
         if (NORM) a = make_float4((a.x * scale) * nv[u].x, (a.y * scale) * nv[u].y, (a.z * scale) * nv[u].z, (a.w * scale) * nv[u].w);

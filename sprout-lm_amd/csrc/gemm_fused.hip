@@ -360,6 +360,7 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
     for (int o = P / 2; o > 0; o >>= 1) square_sum += __shfl_xor(square_sum, o, 64);
     const float scale = 1.0f / sqrtf(square_sum / float(a.K) + a.eps);
     uint16_t* row = rows + int(threadIdx.x) / P * staged_pitch(a.K);
+    if (piece == 0) *reinterpret_cast<uint4*>(row + a.K) = make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < PIECES; ++j) {
       const int k = 4 * (piece + j * P);
@@ -395,13 +396,14 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
     }
     uint4 xb[UN][TN][2];
     if constexpr (STAGED) {
-      // (columns of tokens past the block's rows repeat the last one; past the end of K the weights are zeros)
+      // (columns of tokens past the block's rows repeat the last one; past the end of K both operands are zeros, this one's those
+      // behind its row: a weight's zero times a normed number that has overflowed would be NaN)
       const uint16_t* row = rows + min(lr, STAGED - 1) * staged_pitch(a.K);
 #pragma unroll
       for (int u = 0; u < UN; ++u)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          xb[u][0][h] = *reinterpret_cast<const uint4*>(row + min(16 * lj + 64 * (s0 + 4 * u) + 8 * h, a.K - 8));
+          xb[u][0][h] = *reinterpret_cast<const uint4*>(row + min(16 * lj + 64 * (s0 + 4 * u) + 8 * h, a.K));
     } else if constexpr (NORM) {
       // Lane (lr, lj) needs 16 values of token lr per step, as the matrix cores take them.  They come straight
       // from the float32 residual, times the token's scale, times the norm's weights, rounded to bfloat16.
