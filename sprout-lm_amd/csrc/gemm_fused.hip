@@ -555,6 +555,11 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(FusedArgs a) {
   }
 }
 
+// Several rows whose sums cost more than the way through LDS: 4 to 8 tokens, and more than 32 (blocks of 16 that share the CUs), of K from 769
+// on.  Staged over not, nine sizes of q/k/v, 4 to 8 and 33 to 64 tokens: K of 896 and 1,024 0.92 to 1.00 and 0.69 to 1.00, 768 0.96 to 1.00 and
+// 1.02, 576 and 520 0.96 to 1.04 and 1.10 to 1.14, 512 1.02 to 1.04 and 1.13 to 1.15, 256 1.04 and 1.22.
+static bool staged_rows_pay(int T, int K) { return K > 768 && K <= kStagedK && T >= 4 && (T <= 8 || T > 32); }
+
 static size_t fused_lds_bytes(int TN, bool norm, int NT = 2, int staged = 0, int K = 0) {
   return sizeof(float4) * 4 * NT * TN * 64 + (staged ? size_t(staged) * staged_pitch(K) * 2 : norm ? sizeof(float) * 4 * 16 : 0);
 }
@@ -564,8 +569,7 @@ static int launch_fused_un(hipStream_t s, const FusedArgs& a, int blocks, int sp
   const size_t lds = fused_lds_bytes(TN, NORM, NT);     // at most 48 KB (four token tiles of three tiles)
   const dim3 grid(blocks, splits, (a.T + 16 * TN - 1) / (16 * TN));   // z: the tokens in tiles of 16 TN
   if constexpr (NORM && EPI == kEpiRope) {
-    // several rows whose sums cost more than the way through LDS: 4 to 8 tokens, and more than 32 (blocks of 16 that share the CUs)
-    if (a.K <= kStagedK && a.T >= 4 && (a.T <= 8 || a.T > 32)) {      // at most 41 KB of LDS
+    if (staged_rows_pay(a.T, a.K)) {      // at most 41 KB of LDS
       const int staged = a.T <= 8 ? 8 : 16;
       const size_t room = fused_lds_bytes(TN, true, NT, staged, a.K);
       if (staged == 8 && a.K % 64 == 0) gemm_fused_kernel<TN, EPI, true, NT, true, UN, 8><<<grid, 256, room, s>>>(a);
@@ -858,3 +862,6 @@ extern "C" int sp_gate_up_silu(void* stream, const void* x, const float* residua
   a.rows_per_block = silu_rows_per_block(T, I, K, residual != nullptr);
   return fused_norm<kEpiSilu>((hipStream_t)stream, a, residual != nullptr, (I + a.rows_per_block - 1) / a.rows_per_block, 1);
 }
+
+// Whether the rotating product of T tokens and K normalises its rows into LDS.  Runs nothing: for tests.
+extern "C" int sp_staged_rows_pay(int T, int K) { return sprout::staged_rows_pay(T, K); }

@@ -63,6 +63,7 @@ int sp_pipe_plan(int kind, int T, int N, int K, int* plan);
 // How that kernel numbers its blocks: tile_of[2 b], tile_of[2 b + 1] = token tile and weight tile of block b (which
 // runs on XCD b % 8), -1 for a block with nothing to do; returns the number of blocks.  Runs nothing.
 int sp_pipe_tiles(int tiles_t, int tiles_n, int* tile_of, int room);
+int sp_staged_rows_pay(int T, int K);
 int sp_gemm_f32_waves(int N, int K);
 int sp_gemm_f32_parts_plan(int T, int N, int K, int* plan);
 int sp_quad_part_tiles(int tiles_t, int tiles_n, int parts, int* tile_of);

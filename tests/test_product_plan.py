@@ -125,3 +125,11 @@ def test_parts_of_prompts_lie_at_whole_sixteen_bytes_of_a_mixed_step_s_workspace
     for nq, nkv, hd, n_decode, ctx in [(7, 1, 64, 1, 700), (5, 5, 16, 3, 257), (14, 2, 64, 8, 4096), (3, 1, 80, 5, 1100)]:
         decode = lib.sp_attention_workspace_floats(1, hd, 16, nq, nkv, 0, n_decode, ctx, 0, 0)
         assert decode % 4 == 0 and 0 <= decode - n_decode * nq * -(-ctx // 256) * (hd + 2) < 4
+
+
+def test_rows_go_through_lds_where_there_are_several_of_a_long_k():
+    """Up to 768 numbers a row they gain nothing, and at 33 to 64 tokens lose up to a fifth; past 1,024 they have no room."""
+    pays = ops.library().sp_staged_rows_pay
+    assert all(pays(T, K) for T in (4, 8, 33, 45, 64) for K in (776, 896, 1016, 1024))
+    assert not any(pays(T, K) for T in (1, 3, 4, 8, 9, 16, 32, 33, 64) for K in (8, 256, 512, 576, 768, 1032, 3584))
+    assert not any(pays(T, 896) for T in (1, 2, 3, 9, 32))
