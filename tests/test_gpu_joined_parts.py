@@ -1,4 +1,4 @@
-"""Products whose sum the next norm joins from parts of K: the parts, the joining norm, and steps of a model that take this way."""
+"""Products whose sum the next norm joins from parts of K: the parts and the joining norm (tests/test_gpu_owed_parts.py has steps of a model)."""
 import math
 
 import pytest
