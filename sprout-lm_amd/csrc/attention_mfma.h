@@ -450,8 +450,8 @@ __device__ __forceinline__ constexpr int step_row(int r) { return (r & ~31) | ((
 constexpr int kMaxTableLds = 2048;    // page numbers held in LDS; longer tables are read from memory
 
 // Part `split` of a walk from key lo, the first of a stage of `keys` keys, to key hi: the tile's own stages in equal shares (the last parts
-// of a short walk are empty).  A tile's walk, not the step's longest context, is what is shared out: a recorded step knows that one as a
-// bucket that may be twice as long (2,048 queries over 20,000 keys, 14 heads of 64 in 2 groups, known as 32,768: 183 -> 174 us).
+// of a short walk are empty).  A tile's walk, not the step's longest context, is what is shared out: a recorded step knows that one up
+// to a bucket that may be twice as long (2,048 queries over 20,000 keys, 14 heads of 64 in 2 groups, known as 32,768: 183 -> 174 us).
 __device__ __forceinline__ void share_of_walk(int& lo, int& hi, int keys, int split, int n_splits) {
   const int stages = (hi - lo) / keys + 1, per = (stages + n_splits - 1) / n_splits;
   lo += split * per * keys;
@@ -1108,7 +1108,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_merge_kernel(const float
 // A step that answers some requests while it reads a prompt of another has few blocks of either kind, and each kind's launch and merge
 // is bound by its own latency, not by the chip: one launch holds the blocks of both, another both merges.  Prompt blocks come first, they
 // are the longer ones.  A block of 512 threads takes two of the one-query kernel's: waves that have ended no longer count at a barrier, and
-// a half that does not end passes as many barriers as the other.  Same keys, same order, same sums as in launches of their own.
+// a half that does not end passes as many barriers as the other.  One-query sequences have the same keys in the same order as in a launch of their
+// own, and the same sums; prompts the same as with as many parts.
 // (8 answers at 1,024..4,096 and 256 tokens behind 1,024, 28 heads of 128: four launches 52.4 us, two 45.5; 5 answers at 300..1,500
 // and 250 tokens, 14 heads of 64: 24.0 us, 15.2.)
 struct PromptPart {
