@@ -63,10 +63,14 @@ int sp_pipe_plan(int kind, int T, int N, int K, int* plan);
 // How that kernel numbers its blocks: tile_of[2 b], tile_of[2 b + 1] = token tile and weight tile of block b (which
 // runs on XCD b % 8), -1 for a block with nothing to do; returns the number of blocks.  Runs nothing.
 int sp_pipe_tiles(int tiles_t, int tiles_n, int* tile_of, int room);
+// ... and a product on four waves a block whose parts of K lie side by side: tile_of[3 b] = (token tile, weight tile, part) of block b.
+int sp_quad_part_tiles(int tiles_t, int tiles_n, int parts, int* tile_of);
+// Rules of products of few tokens, for tests; they run nothing.  Whether the rotating bfloat16 product normalises its rows into LDS; the waves
+// of a block of sp_gemm's float32 product of up to 16 tokens; the block shape and the parts of sp_gemm_parts in float32, plan = {block rows,
+// block columns, parts}, returning 1 where it does not take the product.
 int sp_staged_rows_pay(int T, int K);
 int sp_gemm_f32_waves(int N, int K);
 int sp_gemm_f32_parts_plan(int T, int N, int K, int* plan);
-int sp_quad_part_tiles(int tiles_t, int tiles_n, int parts, int* tile_of);
 // The same of the product on four waves a block, which takes more than 64 tokens, and from 17 on where it is the faster one, with
 // outputs in whole eights that start at 16 bytes (other kernels have the rest), and is the only one to rotate (kind 3, head size hd):
 // plan = {block rows, block columns, splits of K, buffers of x}.
@@ -138,6 +142,7 @@ int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, 
                                       int n_decode, int max_decode_ctx, int n_tiles, int max_tile_ctx);
 int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int n_decode, int max_decode_ctx,
                                       int n_tiles, int max_tile_ctx, int mean_tile_walk, long long one_query_keys);
+// Whether a step's prompts and its one-query sequences share a launch.  Runs nothing: for tests.
 int sp_attention_mixed_pays(int hd, int nq, int nkv, int n_tiles, int n_decode, int max_decode_ctx, long long one_query_keys);
 // scores: what stands between q . k and the softmax, numbered like the variants above: 0 = the scaled product and
 // nothing else; 1 = the scaled product s squashed to softcap * tanh(s / softcap).  sinks (null: none): one float per
