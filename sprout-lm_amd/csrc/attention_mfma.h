@@ -1335,13 +1335,12 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
 }
 
 int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
-// attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; its splits are 0 where it is not the faster one.
-int attention_rows_splits(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx);
-bool attention_rows_bound_by_one_walk(int n_tiles, int nq, int nkv, int splits, int page_size, int max_tile_ctx, int mean_tile_walk, int there);
-int launch_attention_rows(hipStream_t s, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
-                          const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len,
-                          const int32_t* ctx_len, const int32_t* tiles, int n_tiles, int splits, uint16_t* out,
-                          float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2);
+// attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; no parts where it is not the faster one.
+struct RowsPlan { int heads, sets, parts; };      // heads of a set, sets of all key/value heads, parts of a walk
+RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
+int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
+                          const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
+                          const int32_t* tiles, int n_tiles, uint16_t* out, float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2);
 size_t attention_decode_workspace_floats(int n_decode, int nq, int hd, int max_ctx);
 // attention_mixed.hip: a step's prompts and its one-query sequences in one launch.  Blocks of up to eight waves, head sizes up to 128,
 // softmax weights: blocks of 16 waves are those of long prompts, beside which the one-query blocks are little, and would hold
@@ -1394,12 +1393,10 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       int page_shift = 0;
       while ((1 << page_shift) < page_size) ++page_shift;
       const bool plain = st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && st.keep <= 0 && !st.sinks && !st.bias && !st.gate;
-      int rows_splits = DT == 4 && !SIG && plain ? attention_rows_splits(n_tiles, nq, nkv, HD, page_size, max_tile_ctx) : 0;
       const long long beside = chunks_beside(HD, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys);
-      const int staged = attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside);
-      if (rows_splits && attention_rows_bound_by_one_walk(n_tiles, nq, nkv, rows_splits, page_size, max_tile_ctx, mean_tile_walk, staged)) rows_splits = 0;
-      int splits = rows_splits ? rows_splits : staged;
-      if (const int seen = st.window > 0 ? st.window : st.chunk; !rows_splits && seen > 0 && seen < max_tile_ctx - 32) {
+      const RowsPlan rows = DT == 4 && !SIG && plain ? attention_rows_plan(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside) : RowsPlan{0, 0, 0};
+      int splits = rows.parts ? rows.parts : attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside);
+      if (const int seen = st.window > 0 ? st.window : st.chunk; !rows.parts && seen > 0 && seen < max_tile_ctx - 32) {
         // a walk is the rows' window long at most (the workspace was asked for without it: not more parts than that)
         const int walk = seen + 32;
         splits = min(splits, attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, walk, min(walk, mean_tile_walk), beside));
@@ -1409,7 +1406,7 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       StagedShape shape = staged_shape(nq, nkv, HD, n_tiles);
       const bool paired = staged_paired(n_tiles, nq, nkv, HD, splits, max_tile_ctx, mean_tile_walk, &shape);
       const dim3 grid(paired ? (n_tiles + 1) / 2 : n_tiles, nkv * ((nq / nkv + shape.hpb - 1) / shape.hpb), splits);
-      if (mixed_instantiated(DT, SIG) && beside > 0 && !rows_splits && shape.hpb * shape.wpt <= 8) {
+      if (mixed_instantiated(DT, SIG) && beside > 0 && !rows.parts && shape.hpb * shape.wpt <= 8) {
         const int sets = decode_sets(nq, nkv);
         return launch_mixed(s, DT, shape.hpb, shape.wpt, paired, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, ctx_len,
                             (uint16_t*)out, nq, nkv, num_pages, st, scale2,
@@ -1421,9 +1418,9 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, (uint16_t*)out, part_o,   \
       part_ml, splits, nq, nkv, page_shift, num_pages, st, scale2, n_tiles)
       // the same cases as staged_shape() and staged_paired()
-      if (rows_splits) {
-        if (launch_attention_rows(s, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, n_tiles,
-                                  splits, (uint16_t*)out, part_o, part_ml, nq, nkv, page_shift, num_pages, scale2))
+      if (rows.parts) {
+        if (launch_attention_rows(s, rows, qp, q_stride, kp, vp, block_tables, max_blocks, q_start, q_len, ctx_len, tiles, n_tiles,
+                                  (uint16_t*)out, part_o, part_ml, nq, nkv, page_shift, num_pages, scale2))
           return 1;
       } else if constexpr (DT > 8) {
         constexpr int kHeads = DT > 12 ? 2 : 4;

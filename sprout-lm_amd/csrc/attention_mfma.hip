@@ -55,7 +55,7 @@ size_t attention_prefill_workspace_floats(int n_tiles, int nq, int nkv, int hd, 
                                           int max_decode_ctx, long long one_query_keys) {
   const long long beside = chunks_beside(hd, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys);
   const size_t splits = max(attention_prefill_parts(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, beside),
-                            attention_rows_splits(n_tiles, nq, nkv, hd, page_size, max_tile_ctx));
+                            attention_rows_plan(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, beside).parts);
   return splits <= 1 ? 0 : size_t(n_tiles) * 32 * nq * splits * (hd + 2);
 }
 
