@@ -203,6 +203,20 @@ __device__ __forceinline__ void quad_epilogue(floatx4 (&acc)[WM][WN], float* tur
             for (int e = 0; e < 8; ++e) v[e] = value(acc[i][j + e / 4][e % 4], acc[i][j + 2 + e / 4][e % 4]);
             *reinterpret_cast<uint4*>(dst + n) = pack8(v);
           }
+        } else if constexpr (WN % 2 == 1) {
+          // a lane's four rows of a tile are two gate rows and the matching up rows: it ends with 2 WN neighbours
+          struct __attribute__((packed, aligned(4))) Run { uint32_t pair[WN]; };
+          const int n = n0 / 2 + wn * 8 * WN + 2 * WN * lq;
+          Run run;
+#pragma unroll
+          for (int j = 0; j < WN; ++j) run.pair[j] = pack_bf16x2(value(acc[i][j][0], acc[i][j][2]), value(acc[i][j][1], acc[i][j][3]));
+          if (n + 2 * WN <= N) {
+            *reinterpret_cast<Run*>(dst + n) = run;
+          } else {
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+              if (n + 2 * j < N) *reinterpret_cast<uint32_t*>(dst + n + 2 * j) = run.pair[j];
+          }
         } else {
           constexpr int G = WN / 2;
 #pragma unroll
@@ -338,7 +352,7 @@ __global__ __launch_bounds__(256, (quad_shares_cu<WM, WN, NA> ? 2 : 1)) void gem
   constexpr uint32_t ASZ = BM * ROW, BSZ = BN * ROW, B0 = NA * ASZ;
   constexpr int L = WM + WN;                            // a wave's loads of a step
   constexpr bool AGPR = !quad_shares_cu<WM, WN, NA>;
-  static_assert(WN % 2 == 0 && (MODE != kRope || WN == 2 || WN % 4 == 0), "tiles of w are paired");
+  static_assert((WN % 2 == 0 || MODE == kSilu) && (MODE != kRope || WN == 2 || WN % 4 == 0), "tiles of w are paired");
   static_assert(NA >= 2 && NA <= 4 && (NA - 1) * L <= 63, "vmcnt holds six bits");
   static_assert(quad_lds<WM, WN, NA> <= 160 * 1024, "a CU's LDS");
   extern __shared__ __attribute__((aligned(1024))) unsigned char pipe_lds[];
@@ -376,6 +390,10 @@ __global__ __launch_bounds__(256, (quad_shares_cu<WM, WN, NA> ? 2 : 1)) void gem
       if (WN % 4 == 0) {            // 32 gate rows, then the 32 up rows
         gate = tile_n * (BN / 2) + (r / 64) * 32 + neighbours8(r & 31);
         up = (r >> 5) & 1;
+      } else if (WN % 2 == 1) {     // two gate rows, then their two up rows, four times a tile
+        const int own = r % (16 * WN), tile = own / 16;
+        gate = tile_n * (BN / 2) + (r / (16 * WN)) * 8 * WN + 2 * WN * ((own >> 2) & 3) + 2 * tile + (own & 1);
+        up = (own >> 1) & 1;
       } else {                      // a wave's first half of tiles gate rows, its second half up rows
         constexpr int G = WN / 2;
         const int own = r % (16 * WN), tile = own / 16;
@@ -558,6 +576,9 @@ inline int launch_quad(hipStream_t s, int splits, const uint16_t* x, const uint1
   X(0, 2, 2, 4) X(1, 3, 4, 2) X(2, 4, 2, 4) X(3, 4, 4, 2) X(4, 4, 4, 4) X(5, 4, 6, 2) X(6, 5, 6, 2) X(7, 6, 4, 2) X(8, 6, 6, 2) \
   X(9, 8, 4, 3) X(10, 4, 8, 2) X(11, 5, 8, 2) X(12, 10, 4, 2) X(13, 6, 8, 2) X(14, 8, 6, 2) X(15, 9, 6, 2) X(16, 8, 8, 2)
 
+// Blocks of an odd number of tile columns a wave, of gated products alone: X(index, WM, WN, NA).  See gemm_quad_odd.hip.
+#define SPROUT_QUAD_ODD_SHAPES(X) X(0, 8, 5, 2) X(1, 10, 5, 2) X(2, 8, 7, 2) X(3, 9, 7, 2)
+
 enum QuadKind { kQuadStore = 0, kQuadAccumulate = 1, kQuadGated = 2, kQuadRotating = 3, kQuadParts = 4 };   // as sp_quad_plan counts them
 
 // Whether the four-wave kernel takes T x N x K (N: all weight rows): more than 64 tokens, from 17 on where it is the faster one; whole
@@ -573,6 +594,8 @@ inline bool quad_aligned(const void* x, const void* w, const void* out) {
 bool gemm_cuts_k(int T, int N, int K);
 // Picks the shape and the split of K with the least estimated time, and returns that in microseconds.
 float quad_choice(int kind, int T, int N, int K, int* shape, int* splits);
+// Whether a gated product of T tokens by N gate and up rows is better on blocks of an odd number of tile columns, and on which.
+bool quad_takes_odd(int T, int N, int K, int* shape);
 
 // The product on the shape that quad_choice picks (N as the kernel counts it: gate rows for kSilu).
 template <int MODE>

@@ -37,13 +37,13 @@ bool gemm_quad_takes(int kind, int T, int N, int K, int hd) {
 // tokens) with every shape and split: microseconds a step of 64 along K on a full chip, and, where two blocks share a CU, of one that
 // has a CU to itself.
 struct QuadShape { int wm, wn, buffers, per_cu; };
-static const QuadShape kQuadShapes[] = {
 #define SPROUT_QUAD_ROW(I, WM, WN, NA) {WM, WN, NA, quad_shares_cu<WM, WN, NA> ? 2 : 1},
-    SPROUT_QUAD_SHAPES(SPROUT_QUAD_ROW)
+static const QuadShape kQuadShapes[] = {SPROUT_QUAD_SHAPES(SPROUT_QUAD_ROW)};
+static const QuadShape kQuadOddShapes[] = {SPROUT_QUAD_ODD_SHAPES(SPROUT_QUAD_ROW)};
 #undef SPROUT_QUAD_ROW
-};
 static const float kStepUs[] = {0.36f, 0.77f, 0.35f, 0.85f, 0.48f, 0.68f, 0.80f, 0.66f, 0.86f, 0.77f, 0.81f, 0.96f, 0.93f, 1.06f, 1.06f, 1.19f, 1.33f};
 static const float kAloneUs[] = {0.24f, 0.45f, 0.35f, 0.50f, 0.48f, 0.68f, 0.80f, 0.66f, 0.86f, 0.77f, 0.81f, 0.96f, 0.93f, 1.06f, 1.06f, 1.19f, 1.33f};
+static const float kOddStepUs[] = {0.98f, 1.14f, 1.22f, 1.40f};
 
 // The estimate: rounds of blocks on the XCD that holds the most (blocks are numbered as pipe_tiles says), a block being its steps
 // (longer by 7 % each beyond 20 where two blocks share a CU) and its two ends; a last round that does not fill the chip runs
@@ -59,14 +59,13 @@ static const float kAloneUs[] = {0.24f, 0.45f, 0.35f, 0.50f, 0.48f, 0.68f, 0.80f
 // operands are what the XCD reads, once each where the caches serve it; 0.7 us a million sums stored, and 5 TB/s for the norm to read all
 // parts and to write their sum.  Over 80 products (70 to 2,048 tokens, eight matrices of 896 to 5,120 rows) the choice takes 3 % longer than
 // the best of all shapes and parts, 10 % at worst.
-float quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
+static float least_time(int kind, int T, int N, int K, const QuadShape* shapes, const float* step_us, const float* alone_us, int n_shapes, int* shape,
+                        int* splits) {
   const int steps = K / 64;
   const bool parts = kind == kQuadParts, cuts_k = parts || (kind == kQuadAccumulate && gemm_cuts_k(T, N, K));
   float best = 1e30f;
-  *shape = 3;
-  *splits = 1;
-  for (int c = 0; c < int(sizeof(kQuadShapes) / sizeof(kQuadShapes[0])); ++c) {
-    const QuadShape& p = kQuadShapes[c];
+  for (int c = 0; c < n_shapes; ++c) {
+    const QuadShape& p = shapes[c];
     if (kind == kQuadRotating && p.wn != 2 && p.wn % 4 != 0) continue;     // a lane holds both of a pair
     const int bm = 32 * p.wm, bn = 32 * p.wn, slots = 32 * p.per_cu;
     const PipeTiles tiles = pipe_tiles((T + bm - 1) / bm, (N + bn - 1) / bn);
@@ -90,7 +89,7 @@ float quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
       const float memory2 = memory * memory;
       const int full = blocks / slots, rest = blocks % slots;
       const float ends = 0.14f * float(p.wm * p.wn) + 0.95f;
-      const float block = k_steps * kStepUs[c] * (p.per_cu == 2 && k_steps > 20 ? 1.07f : 1.f) + ends, alone = k_steps * kAloneUs[c] + ends;
+      const float block = k_steps * step_us[c] * (p.per_cu == 2 && k_steps > 20 ? 1.07f : 1.f) + ends, alone = k_steps * alone_us[c] + ends;
       float t = full * block;
       if (rest > 32) t += fmaxf(alone, block * (0.81f + 0.19f * float(rest - 32) / 32.f));
       else if (rest) t += alone * (0.79f + 0.21f * float(rest) / 32.f);
@@ -102,6 +101,20 @@ float quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
     }
   }
   return best;
+}
+
+float quad_choice(int kind, int T, int N, int K, int* shape, int* splits) {
+  *shape = 3;
+  *splits = 1;
+  return least_time(kind, T, N, K, kQuadShapes, kStepUs, kAloneUs, int(sizeof(kQuadShapes) / sizeof(kQuadShapes[0])), shape, splits);
+}
+
+// Where the estimate says 2 % less: of 57 gated products (65 to 2,048 tokens at 0.5B, 7B and 32B sizes), each timed on every shape, the 17 that
+// this takes are 0.81 to 0.99 of the time (0.93 on average) and none is longer; without the margin one is, by 2.6 %.
+bool quad_takes_odd(int T, int N, int K, int* shape) {
+  int even, splits;
+  return least_time(kQuadGated, T, N, K, kQuadOddShapes, kOddStepUs, kOddStepUs, int(sizeof(kQuadOddShapes) / sizeof(kQuadOddShapes[0])), shape, &splits) <
+         0.98f * quad_choice(kQuadGated, T, N, K, &even, &splits);
 }
 
 // Parts of K in which the accumulating product is better stored for the norm behind it to join, 0 where it is better added: more than 64
@@ -123,8 +136,8 @@ int gemm_bf16_quad(hipStream_t s, const void* x, const void* w, int bias_dtype, 
 
 }  // namespace sprout
 
-// What the four-wave product would do with T x N x K: kind 0 store, 1 accumulate, 2 gated (N = 2 I rows of w), 3 rotating (head size
-// hd), 4 parts side by side.  plan = {block rows, block columns, splits of K, buffers of x}.  Returns 1 where it does not take the product, else 0.  Runs
+// What the four-wave product would do with T x N x K on blocks of an even number of tile columns a wave: kind 0 store, 1 accumulate, 2 gated (N = 2 I
+// rows of w; sp_quad_odd_plan says where others take its place), 3 rotating (head size hd), 4 parts side by side.  plan = {block rows, block columns, splits of K, buffers of x}.  Returns 1 where it does not take the product, else 0.  Runs
 // nothing: for tests and tools.
 extern "C" int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan) {
   using namespace sprout;
@@ -135,6 +148,18 @@ extern "C" int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan) {
   plan[1] = 32 * kQuadShapes[shape].wn;
   plan[2] = splits;
   plan[3] = kQuadShapes[shape].buffers;
+  return 0;
+}
+
+// Whether a gated product that the four-wave kernel takes (T tokens, N = 2 I rows of w) runs on blocks of an odd number of tile columns a wave: plan =
+// {block rows, block columns, buffers of x}.  Returns 1 where it does not, else 0.  Runs nothing: for tests.
+extern "C" int sp_quad_odd_plan(int T, int N, int K, int* plan) {
+  using namespace sprout;
+  int shape;
+  if (T < 1 || N < 1 || K < 1 || !plan || !gemm_quad_takes(kQuadGated, T, N, K, 0) || !quad_takes_odd(T, N, K, &shape)) return 1;
+  plan[0] = 32 * kQuadOddShapes[shape].wm;
+  plan[1] = 32 * kQuadOddShapes[shape].wn;
+  plan[2] = kQuadOddShapes[shape].buffers;
   return 0;
 }
 

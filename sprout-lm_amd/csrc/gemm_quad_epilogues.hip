@@ -2,6 +2,7 @@
 #include "gemm_quad.h"
 
 namespace sprout {
+int gemm_bf16_quad_odd_silu(int shape, hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, const RopeArgs& epilogue);
 
 // out[T, I] = silu(x . w[:I]^T) * (x . w[I:]^T): a block's weight rows are half gate rows, half the matching up rows.
 int gemm_bf16_quad_silu(hipStream_t s, const void* x, const void* w, void* out, int T, int I, int K, int act, float limit,
@@ -11,6 +12,8 @@ int gemm_bf16_quad_silu(hipStream_t s, const void* x, const void* w, void* out, 
   epilogue.limit = limit;
   epilogue.row_gate = row_gate;
   epilogue.row_gate_stride = row_gate_stride;
+  int shape;
+  if (quad_takes_odd(T, 2 * I, K, &shape)) return gemm_bf16_quad_odd_silu(shape, s, x, w, out, T, I, K, epilogue);
   return quad_run<kSilu>(s, kQuadGated, x, w, nullptr, kF32, out, T, I, K, epilogue);
 }
 

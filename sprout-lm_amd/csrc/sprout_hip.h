@@ -75,6 +75,8 @@ int sp_gemm_f32_parts_plan(int T, int N, int K, int* plan);
 // outputs in whole eights that start at 16 bytes (other kernels have the rest), and is the only one to rotate (kind 3, head size hd):
 // plan = {block rows, block columns, splits of K, buffers of x}.
 int sp_quad_plan(int kind, int T, int N, int K, int hd, int* plan);
+// Whether that gated product (N = 2 I rows) runs on blocks of an odd number of tile columns a wave instead.  Runs nothing: for tests.
+int sp_quad_odd_plan(int T, int N, int K, int* plan);
 int sp_gemm_decode(void* stream, const void* x, const float* residual, int norm_w_dtype, const void* norm_w, float eps,
                    const void* w, int bias_dtype, const void* bias, int mode, void* out, int T, int N, int K);
 // Two products of the same input in one (bfloat16 operands and results): with y = x . w^T + bias (float32 [N], may be null),

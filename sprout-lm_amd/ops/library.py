@@ -42,6 +42,7 @@ def _declare(lib):
         "sp_fused_norm_pays": [c_int] * 3,
         "sp_pipe_plan": [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int)],
         "sp_quad_plan": [c_int, c_int, c_int, c_int, c_int, ctypes.POINTER(c_int)],
+        "sp_quad_odd_plan": [c_int, c_int, c_int, ctypes.POINTER(c_int)],
         "sp_staged_rows_pay": [c_int, c_int],
         "sp_gemm_f32_waves": [c_int, c_int],
         "sp_gemm_f32_parts_plan": [c_int, c_int, c_int, ctypes.POINTER(c_int)],
