@@ -170,7 +170,7 @@ extern "C" int sp_attention_decode_project(void* stream, const void* q, int q_st
              "sp_attention_decode_project: decode context %d exceeds the block tables", max_decode_ctx);
   SP_REQUIRE(q_stride >= nq * hd, "sp_attention_decode_project: q row stride %d is smaller than %d", q_stride, nq * hd);
   const int64_t need = workspace_floats_of(hd, page_size, nq, nkv, n_decode, max_decode_ctx, 0, 0, 0, 0);
-  SP_REQUIRE(workspace && workspace_floats >= need,
+  SP_REQUIRE(need == 0 || (workspace && workspace_floats >= need),
              "sp_attention_decode_project: workspace of %lld floats is smaller than the %lld needed",
              (long long)workspace_floats, (long long)need);
   return attention_mfma_decode_project((hipStream_t)stream, q, q_stride, k_pool, v_pool, block_tables, max_blocks,

@@ -4,6 +4,8 @@
 
 namespace sprout {
 
+constexpr int kProjectColumns = 512;      // most columns of w_o that a set of heads has where attention and projection share a block
+
 bool attention_mfma_supports(int hd, int page_size, int nq, int nkv) {
   const int dt = hd / 16;
   const bool hd_ok = hd % 16 == 0 && (dt <= 6 || dt == 8 || dt == 10 || dt == 12 || dt == 16);
@@ -91,6 +93,130 @@ int attention_mfma(hipStream_t s, const void* q, int q_stride, const void* k_poo
 #undef SP_MFMA
 }
 
+// Attention of one-query sequences whose keys one block walks (64 a wave: up to 256 on four waves, 512 on eight), with the output projection behind it
+// in the same launch:
+//   residual[row(di), n] += sum over the heads of a set and d of attention[di, head, d] * w_o[n, head * HD + d]
+// grid (blocks of 64 rows of w_o, sets of heads, sequences).  A short context's attention is a few trips to memory and as long again in the launch
+// of the product behind it; here every block of rows walks its set's keys again (a set of 256 keys of 64 numbers is 64 KB out of the caches) and
+// its rows of w_o are in registers by the time the keys are weighed.  Each wave takes 16 rows and, with eight waves, half of the columns.
+// What bounds it is the chain: page numbers, keys, the waves' merge in LDS, sixteen matrix instructions, the adds.  One sequence of 79 keys, 14 heads
+// of 64 in 2 groups, a width of 896: 1.4 us a layer less than attention and product in launches of their own (5.1 and 3.2 us).
+template <int DT, int NW, bool POW2>
+__global__ __launch_bounds__(64 * NW) void attention_project_kernel(
+    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len,
+    const int32_t* __restrict__ decode_seqs, const uint16_t* __restrict__ w_o, float* __restrict__ residual, int hidden, int nq, int nkv,
+    int kv_stored, int page_size, int num_pages, ScoreStage st, float scale2) {
+  constexpr int HD = 16 * DT, HC = (DT + 1) / 2, KEYS = 64 * NW, SHARES = NW / 4, CHUNKS = kProjectColumns / 32 / SHARES;
+  __shared__ float s_o[NW][16][HD + 1];
+  __shared__ float s_m[NW][16], s_l[NW][16];
+  __shared__ int32_t s_table[KEYS / 4 + 4];
+  __shared__ __attribute__((aligned(16))) uint16_t xs[kProjectColumns];
+  __shared__ float sums[SHARES][64];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lj = lane >> 4;
+  const int g = blockIdx.y, di = blockIdx.z, seq = decode_seqs ? decode_seqs[di] : di, n_begin = blockIdx.x * 64;
+  const int G = nq / nkv, columns = G * HD;
+  const int pages = (KEYS - 1) / page_size + 1;
+  if (tid < pages) s_table[tid] = block_tables[size_t(seq) * max_blocks + min(tid, max_blocks - 1)];
+  const int q_row = decode_seqs ? q_start[seq] : seq;
+  const int pos = ctx_len[seq] - 1, k_lo = first_visible(pos, st.window, st.chunk);
+
+  PagedKV kv;
+  kv.page_size = page_size;
+  kv.num_pages = num_pages;
+  kv.page_stride = size_t(kv_stored) * page_size * HD;
+  kv.k = k_pool + size_t(g / (nkv / kv_stored)) * page_size * HD;
+  kv.v = v_pool + size_t(g / (nkv / kv_stored)) * page_size * HD;
+  kv.table = s_table;
+  kv.page_shift = POW2 ? 31 - __builtin_clz(page_size) : 0;
+  bf16x8 qop[1][HC];
+  int qpos[1] = {lr < G ? pos : -1}, qlo[1] = {k_lo};
+  const StepRule rule = step_rule(st, scale2);
+  load_q_operand<DT>(qop[0], lr < G ? q + size_t(q_row) * q_stride + (g * G + lr) * HD : nullptr);
+  __syncthreads();   // the page numbers are in LDS
+  const int w0 = wave * 64;
+  KVStep<DT> steps[2];
+  bool live[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    live[i] = w0 + 32 * i <= pos && w0 + 32 * i + 32 > k_lo;
+    if (live[i]) load_step<DT, POW2>(steps[i], kv, w0 + 32 * i, k_lo, pos);
+  }
+  // this wave's rows of w_o, asked for behind the keys: they are multiplied last
+  const int share = wave >> 2, tile = n_begin + 16 * (wave & 3);
+  uint4 wa[CHUNKS];
+  {
+    const uint16_t* wrow = w_o + size_t(min(tile + lr, hidden - 1)) * (size_t(nq) * HD) + g * columns;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int d = 32 * (c * SHARES + share) + 8 * lj;
+      wa[c] = d < columns ? ldg128(wrow + d) : make_uint4(0, 0, 0, 0);
+    }
+  }
+  floatx4 o[1][DT];
+  float m[1], lsum[1];
+  start_row<false>(m[0], lsum[0]);
+  if (st.sinks && wave == 0 && lr < G) {      // a term of the denominator without a key: in one lane of a row's four
+    m[0] = st.sinks[g * G + lr] * kLog2e;
+    lsum[0] = lj == 0 ? 1.f : 0.f;
+  }
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[0][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (live[i]) attend_step<DT, 1, false>(steps[i], qop, o, m, lsum, w0 + 32 * i, k_lo, qpos, qlo, rule, scale2, 0.f, pos);
+  float l = lsum[0];
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (lj == 0) { s_m[wave][lr] = m[0]; s_l[wave][lr] = l; }
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s_o[wave][lr][16 * dt + 4 * lj + r] = o[0][dt][r];
+  __syncthreads();
+  for (int i = tid; i < kProjectColumns; i += 64 * NW) {
+    const int qh = i / HD, d = i % HD;
+    float value = 0.f;
+    if (i < columns) {
+      float mx = -INFINITY, num = 0.f, den = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) mx = fmaxf(mx, s_m[w][qh]);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float f = exp2f(s_m[w][qh] - mx);
+        num += f * s_o[w][qh][d];
+        den += f * s_l[w][qh];
+      }
+      value = den > 0.f ? num / den : 0.f;
+    }
+    xs[i] = f32_to_bf16_bits(value);      // as where the attention output passes through memory
+  }
+  __syncthreads();
+  floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c)      // every column of the result is this sequence's
+    acc[c & 1] = mfma16(as_bf16x8(wa[c]), as_bf16x8(*reinterpret_cast<const uint4*>(&xs[32 * (c * SHARES + share) + 8 * lj])), acc[c & 1]);
+  if (lr == 0)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sums[share][16 * (wave & 3) + 4 * lj + r] = acc[0][r] + acc[1][r];
+  __syncthreads();
+  if (tid < 64 && n_begin + tid < hidden) {
+    float sum = sums[0][tid];
+    if (SHARES == 2) sum += sums[SHARES - 1][tid];
+    unsafeAtomicAdd(residual + size_t(q_row) * hidden + n_begin + tid, sum);
+  }
+}
+
+// Whether that kernel takes a step, on how many waves (0: no).  Where its blocks are at most the CUs.  us a step of 24 layers at 14 heads of 64
+// in 2 groups and a width of 896, with attention and product (or the merge that projects) in launches of their own and so:
+//   contexts of 79: one sequence 683 and 648, 4 706 and 662, 8 (224 blocks) 726 and 680, 16 (448) 771 and 768;
+//   of 250: one 702 and 667, 8 750 and 721, 16 797 and 835; of 400 on eight waves: one 704 and 692, 4 728 and 705, 8 752 and 730.
+static int project_waves(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
+  const int sets = decode_sets(nq, nkv);
+  if (hd > 64 || nq / sets * hd > kProjectColumns || max_decode_ctx > 512 || (long long)((hidden + 63) / 64) * sets * n_decode > 256) return 0;
+  return max_decode_ctx <= 256 ? 4 : 8;
+}
+
 // Decode steps whose chunks' merge is folded into the output projection.  Worth it where the merged partial
 // results, which every block of a head and a tile of 16 sequences reads again, stay small beside the rows of w_o
 // (measured at 14 heads of 64, a width of 896, contexts of 4,096, tokens a second with the fold against merge and
@@ -98,6 +224,7 @@ int attention_mfma(hipStream_t s, const void* q, int q_stride, const void* k_poo
 // sequences 27,400 against 26,660, 64 sequences 39,840 against 40,350).
 bool attention_decode_project_takes(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
   if (hd > 128 || !attention_mfma_supports(hd, page_size, nq, nkv) || !attention_mfma_decode_supports(nq, nkv)) return false;
+  if (n_decode >= 1 && max_decode_ctx >= 1 && hidden >= 16 && project_waves(hd, page_size, nq, nkv, n_decode, max_decode_ctx, hidden)) return true;
   const int n_splits = (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk;
   return n_decode >= 1 && n_decode <= 32 && n_splits > 1 && min(n_decode, 16) * n_splits <= 256 && hidden >= 16 &&
          hidden <= 2048;   // (wider: 28 heads of 128 at 3,584 +1%, 40 heads at 5,120 -0.5% with four tiles a wave)
@@ -122,6 +249,22 @@ static int launch_decode_project(hipStream_t s, const void* q, int q_stride, con
                                  float* workspace, const void* w_o, float* residual, int hidden, int nq, int nkv,
                                  int page_size, int num_pages, ScoreStage st, float scale) {
   constexpr int HD = 16 * DT;
+  if constexpr (DT <= 4) {
+    if (const int waves = project_waves(HD, page_size, nq, nkv, n_decode, max_decode_ctx, hidden)) {
+      const int sets = decode_sets(nq, nkv);
+      const dim3 grid((hidden + 63) / 64, sets, n_decode);
+#define SP_PROJECT(NW, POW2)                                                                                                            \
+  attention_project_kernel<DT, NW, POW2><<<grid, 64 * NW, 0, s>>>((const uint16_t*)q, q_stride, (const uint16_t*)k_pool,               \
+                                                                 (const uint16_t*)v_pool, block_tables, max_blocks, q_start, ctx_len,  \
+                                                                 decode_seqs, (const uint16_t*)w_o, residual, hidden, nq, sets, nkv,   \
+                                                                 page_size, num_pages, st, scale * kLog2e)
+      const bool pow2 = (page_size & (page_size - 1)) == 0;
+      if (waves == 4) { if (pow2) SP_PROJECT(4, true); else SP_PROJECT(4, false); }
+      else { if (pow2) SP_PROJECT(8, true); else SP_PROJECT(8, false); }
+#undef SP_PROJECT
+      return check_launch("sp_attention_decode_project (one block a context)");
+    }
+  }
   const int n_splits = (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk;
   float* part_o = workspace;
   float* part_ml = workspace + size_t(n_decode) * nq * n_splits * HD;

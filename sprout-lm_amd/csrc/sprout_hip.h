@@ -168,7 +168,8 @@ int sp_attention(void* stream, int dtype, const void* q, int q_stride, const voi
 // A step of one-query sequences only (bfloat16): attention with the output projection folded into the merge
 // of the key chunks: residual[q_start[seq], :] += attention(seq) . w_o^T with w_o [hidden, nq * hd] bfloat16
 // and residual float32 [rows, hidden].  sp_attention_decode_project_takes says whether a step is taken
-// (several chunks of keys, at most 64 sequences, a narrow model); the workspace is sp_attention's for the step.
+// (several chunks of keys, at most 32 sequences, a narrow model; or a short context and few sequences); the workspace is sp_attention's for the step
+// (none for contexts of one chunk).
 int sp_attention_decode_project_takes(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx,
                                       int hidden);
 int sp_attention_decode_project(void* stream, const void* q, int q_stride, const void* k_pool, const void* v_pool,

@@ -861,10 +861,10 @@ def attention(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool: torc
         ws = workspace(need) if workspace is not None else torch.empty(need, dtype=torch.float32, device=q.device)
         if ws.dtype != torch.float32 or ws.numel() < need:
             raise KernelError("attention: workspace too small")
-    if project is not None and kind == 0 and n_tiles == 0 and n_decode and need and q.dtype == torch.bfloat16 and not every:
+    if project is not None and kind == 0 and n_tiles == 0 and n_decode and q.dtype == torch.bfloat16 and not every and not keep_first:
         w_o, residual = project
         hidden = w_o.shape[0]
-        if (w_o.dtype == torch.bfloat16 and w_o.is_contiguous() and tuple(w_o.shape) == (hidden, nq * hd)
+        if (w_o.dtype == torch.bfloat16 and w_o.data_ptr() % 16 == 0 and w_o.is_contiguous() and tuple(w_o.shape) == (hidden, nq * hd)
                 and residual.dtype == torch.float32 and residual.is_contiguous() and residual.dim() == 2
                 and residual.shape[1] == hidden and residual.shape[0] >= T
                 and library().sp_attention_decode_project_takes(hd, page_size, nq, nkv, n_decode, max_decode_ctx, hidden)):

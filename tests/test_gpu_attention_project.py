@@ -1,0 +1,63 @@
+"""Attention of short contexts and the output projection in one launch: one to eight waves' keys, ragged batches, one key, pages of every kind,
+groups of one and of sixteen heads, widths that end within a block's rows; windows, sinks, capped scores, blocks of positions; and which steps take it."""
+import pytest
+import torch
+
+from sprout_lm_amd import ops
+from tests.test_gpu_kernels import run_attention
+
+DEV = "cuda"
+SIZES = [(14, 2, 64, 16, 896), (3, 1, 32, 8, 100), (4, 4, 16, 16, 264), (8, 1, 64, 4, 17), (6, 2, 48, 12, 300), (32, 2, 16, 32, 65)]
+CONTEXTS = [[1], [64], [65], [256], [79, 256, 1, 33], [257], [512], [511, 3, 300]]
+
+
+def takes(hd, page, nq, nkv, contexts, hidden):
+    return bool(ops.library().sp_attention_decode_project_takes(hd, page, nq, nkv, len(contexts), max(contexts), hidden))
+
+
+def test_which_steps():
+    try:
+        ops.library()
+    except Exception as e:      # no compiler here: nothing to ask
+        pytest.skip(f"the kernel library cannot be built or loaded here: {e}")
+    assert all(takes(hd, page, nq, nkv, c, hidden) for nq, nkv, hd, page, hidden in SIZES for c in CONTEXTS)
+    # as many blocks as CUs, a set's columns, a head's size: beyond them contexts of one chunk have launches of their own
+    assert takes(64, 16, 14, 2, [79] * 8, 896) and not takes(64, 16, 14, 2, [79] * 16, 896)
+    assert not takes(64, 16, 16, 1, [79], 896) and not takes(128, 16, 4, 2, [79], 896) and not takes(128, 16, 28, 4, [79], 3584)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nq,nkv,hd,page,hidden", SIZES)
+@pytest.mark.parametrize("contexts", CONTEXTS)
+@pytest.mark.parametrize("window", [None, 70])
+def test_short_contexts(nq, nkv, hd, page, hidden, contexts, window):
+    got, want = run_attention(torch.bfloat16, nq, nkv, hd, page, [(c, 1) for c in contexts], window=window, kind=0, seed=hidden, hidden=hidden)
+    assert not (got != got).any()
+    # weights and outputs of unit size rounded to bfloat16, a row of w_o of unit norm: as the steps of several chunks are tested
+    assert abs(got - want).max() <= 2e-2 * (1 + abs(want).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("options", [{"sinks": True}, {"scores": "capped", "softcap": 3.0}, {"mask_chunk": 48}, {"sinks": True, "window": 50}])
+@pytest.mark.parametrize("contexts", [[90, 7], [400]])
+def test_score_stages(options, contexts):
+    nq, nkv, hd, page, hidden = 14, 2, 64, 16, 896
+    g = torch.Generator(device=DEV).manual_seed(len(contexts))
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    options = dict(options)
+    window = options.pop("window", None)
+    if options.get("sinks"):
+        options["sinks"] = rand(nq)
+    T, pages = len(contexts), [-(-c // page) for c in contexts]
+    tables = torch.zeros(T, max(pages), dtype=torch.int32, device=DEV)
+    for i, n in enumerate(pages):
+        tables[i, :n] = torch.arange(sum(pages[:i]), sum(pages[:i]) + n, device=DEV)
+    q, k, v = rand(T, nq * hd).bfloat16(), rand(sum(pages), nkv, page, hd).bfloat16(), rand(sum(pages), nkv, hd, page).bfloat16()
+    w_o, before = (rand(hidden, nq * hd) * (nq * hd) ** -0.5).bfloat16(), rand(T, hidden)
+    batch = lambda: ops.AttentionBatch.build([1] * T, contexts, DEV)
+    residual, out = before.clone(), torch.full_like(q, float("nan"))
+    assert ops.attention(q, nq * hd, k, v, tables, batch(), out, nq, nkv, hd, window, 0.125, project=(w_o, residual), **options)
+    assert ops.attention(q, nq * hd, k, v, tables, batch(), out, nq, nkv, hd, window, 0.125, kind=1, **options) is False
+    want = out.float() @ w_o.float().T
+    # each of the 896 outputs is off by a rounding of at most 2^-8 of its size on either side, weighed by rows of w_o of unit norm
+    assert ((residual - before) - want).abs().max() <= 2 * 2.0 ** -8 * (out.float().abs() @ w_o.float().abs().T).max()
