@@ -1336,8 +1336,9 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
 
 int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; no parts where it is not the faster one.
-struct RowsPlan { int heads, sets, parts; };      // heads of a set, sets of all key/value heads, parts of a walk
+struct RowsPlan { int heads, sets, parts; bool shared; };      // heads of a set, sets of all key/value heads, parts of a walk, waves that share their rows
 RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
+RowsPlan attention_rows_choice(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
                           const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
                           const int32_t* tiles, int n_tiles, uint16_t* out, float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2);
@@ -1394,7 +1395,7 @@ static int launch_mfma(hipStream_t s, const void* q, int q_stride, const void* k
       while ((1 << page_shift) < page_size) ++page_shift;
       const bool plain = st.window <= 0 && st.chunk <= 0 && st.cap <= 0.f && st.keep <= 0 && !st.sinks && !st.bias && !st.gate;
       const long long beside = chunks_beside(HD, nq, nkv, n_tiles, n_decode, max_decode_ctx, one_query_keys);
-      const RowsPlan rows = DT == 4 && !SIG && plain ? attention_rows_plan(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside) : RowsPlan{0, 0, 0};
+      const RowsPlan rows = DT == 4 && !SIG && plain ? attention_rows_choice(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside) : RowsPlan{0, 0, 0, false};
       int splits = rows.parts ? rows.parts : attention_prefill_parts(n_tiles, nq, nkv, HD, page_size, max_tile_ctx, mean_tile_walk, beside);
       if (const int seen = st.window > 0 ? st.window : st.chunk; !rows.parts && seen > 0 && seen < max_tile_ctx - 32) {
         // a walk is the rows' window long at most (the workspace was asked for without it: not more parts than that)

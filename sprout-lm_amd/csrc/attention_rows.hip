@@ -178,6 +178,47 @@ __device__ __forceinline__ float rows_half(RowState& st, float scale2, const BET
   return sum[0] + sum[1];
 }
 
+// Each wave's sums and statistics of the block's 64 rows to LDS, once no wave reads its stages any more: four bytes of row r and dimension
+// 4 n .. of wave w at ((w * 64 + r) * 16 + (n ^ r % 16)) * 16, so that rows lie on different banks.
+__device__ __forceinline__ void join_waves(const RowState& st, unsigned char* ring, float2* ml, int wave, int lane) {
+  const int li = lane & 31, lk = lane >> 5;
+  __syncthreads();
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const int r = 32 * rt + li;
+    float l = st.l[rt];
+    l += __shfl_xor(l, 32, 64);
+    if (lk == 0) ml[64 * wave + r] = make_float2(st.m[rt], l);
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+        *reinterpret_cast<float4*>(ring + ((64 * wave + r) * 16 + ((8 * dt + 2 * a + lk) ^ (r & 15))) * 16) =
+            make_float4(st.o[rt][dt][4 * a], st.o[rt][dt][4 * a + 1], st.o[rt][dt][4 * a + 2], st.o[rt][dt][4 * a + 3]);
+  }
+  __syncthreads();
+}
+// Row r's dimensions 16 n .. over all waves, and what they are to be multiplied with.
+__device__ __forceinline__ void joined_row(const unsigned char* ring, const float2* ml, int r, int n, float (&sum)[16], float& inv) {
+  float2 of[4];
+  float mx = kNoKeyYet, den = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) of[w] = ml[64 * w + r], mx = fmaxf(mx, of[w].x);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float f = __builtin_amdgcn_exp2f(of[w].x - mx);
+    den += f * of[w].y;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float4 v = *reinterpret_cast<const float4*>(ring + ((64 * w + r) * 16 + ((4 * n + p) ^ (r & 15))) * 16);
+      sum[4 * p] += f * v.x, sum[4 * p + 1] += f * v.y, sum[4 * p + 2] += f * v.z, sum[4 * p + 3] += f * v.w;
+    }
+  }
+  inv = row_factor<false>(den);
+}
+
 // The shape of a launch.  An entry of the tile list stands for rows 256 n .. of its sequence and set, n counted by its place in the
 // sequence, which has at least as many tiles of 32 queries as blocks of rows: a set holds up to eight heads.  Entries beyond the last rows
 // have nothing to do.
@@ -187,12 +228,18 @@ struct RowsShape {
 };
 
 // NARROW: either pool is below 4 GB, so that a page's place is 32 bits of bytes.
-template <bool NARROW>
+// SHARED: the four waves of a block share 64 rows and the keys of a stage, 32 each, and their sums are joined in LDS.  A prompt has four times
+// the blocks, none of which walks its keys alone, so short walks fill the chip without parts that another launch joins.  What bounds it
+// is the longest walk's chain: 0.85 us a stage (loads of the stage after the next asked for in the middle of one, one barrier), 16 stages for
+// 2,048 tokens, and 7 before and behind it.  14 heads of 64 in 2 groups, 2,048 tokens 29.7 -> 22.9 us, 47 to 611 tokens five times 14.5 -> 12.0, 1,800
+// queries over 2,900 keys 49.6 -> 30.5; 32 heads in 8 groups, 1,024 tokens 19.6 -> 15.9.  (Keys and values waited for apart, with a step and
+// a half for their way and two barriers a stage: 27.5 us for the first.)
+template <bool NARROW, bool SHARED>
 __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool,
     const int32_t* __restrict__ block_tables, int max_blocks, RowsShape shape, uint16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2) {
-  constexpr int HD = 64;
+  constexpr int HD = 64, BLOCK_ROWS = SHARED ? 64 : kRowsBlock, SUBS = kRowsBlock / BLOCK_ROWS;      // blocks of an entry
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];      // two stages, then the pages' places
   uint32_t* s_table = reinterpret_cast<uint32_t*>(ring + 2 * kRowsStageBytes);
   auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
@@ -203,36 +250,49 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   // they start first; all sets and parts of an entry one after another, so that an XCD keeps to few of them where they come in eights.  Two blocks
   // run on a CU, the second 256 blocks behind the first: those behind take the entries the other way round, so that a CU has a long walk and a short
   // one (1,024 queries over 4,096 keys beside eight prompts of 128, 14 heads in 2 groups: 51 -> 40 us).
-  auto block_of_rows = [&](int e) { return e < shape.n_tiles && kRowsBlock * (shape.tiles[2 * e + 1] / 32) < shape.q_len[shape.tiles[2 * e]] * shape.heads; };
-  const int sets_parts = shape.sets * shape.parts;
-  int n_entries = 0;
-  for (int e = 0; e < shape.n_tiles; e += 64) n_entries += __builtin_popcountll(__builtin_amdgcn_ballot_w64(block_of_rows(e + lane)));
+  // What 64 entries of the list say, one a lane, is asked for together, the first 64 once: one by one they would be trips to memory of their own.
+  struct Entry { int seq, nth, qlen, ctx, qs; };
+  auto entry_of = [&](int e) __attribute__((always_inline)) {
+    Entry entry = {0, 0, 0, 0, 0};
+    if (e < shape.n_tiles) {
+      const int at = shape.tiles[2 * e];
+      entry = {at, shape.tiles[2 * e + 1] / 32, shape.q_len[at], shape.ctx_len[at], shape.q_start[at]};
+    }
+    return entry;
+  };
+  auto with_rows = [&](const Entry& entry) { return __builtin_amdgcn_ballot_w64(kRowsBlock * entry.nth < entry.qlen * shape.heads); };
+  const int sets_parts = shape.sets * shape.parts * SUBS;
+  const Entry first_entries = entry_of(lane);
+  int n_entries = __builtin_popcountll(with_rows(first_entries));
+  for (int e = 64; e < shape.n_tiles; e += 64) n_entries += __builtin_popcountll(with_rows(entry_of(e + lane)));
   const int n_blocks = n_entries * sets_parts;
   int id = blockIdx.x;
   if (id >= n_blocks) return;
   if (const int first = id & ~255, eights = min(256, n_blocks - first) / 8; id & 256 && id - first < 8 * eights)
     id = first + 8 * (eights - 1 - (id - first) / 8) + id % 8;
-  const int set = id % sets_parts % shape.sets, part = id % sets_parts / shape.sets;
-  int tile = 0;
+  const int set = id % sets_parts % shape.sets, of_set = id % sets_parts / shape.sets, part = SHARED ? 0 : of_set;
+  int tile = 0, seq = 0, nth = 0, qlen = 0, ctx = 0, qs = 0;
   for (int e = 0, left = n_entries - 1 - id / sets_parts; e < shape.n_tiles; e += 64) {      // entry number `left` of those with rows
-    const unsigned long long with = __builtin_amdgcn_ballot_w64(block_of_rows(e + lane));
+    const Entry entry = e == 0 ? first_entries : entry_of(e + lane);
+    const unsigned long long with = with_rows(entry);
     const int here = __builtin_popcountll(with);
     if (left < here) {
       const bool mine = (with >> lane & 1) && __builtin_popcountll(with & ((1ull << lane) - 1)) == left;
-      tile = e + __builtin_ctzll(__builtin_amdgcn_ballot_w64(mine));
+      const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(mine));
+      auto its = [&](int v) { return __builtin_amdgcn_readlane(v, from); };
+      tile = e + from, seq = its(entry.seq), nth = its(entry.nth), qlen = its(entry.qlen), ctx = its(entry.ctx), qs = its(entry.qs);
       break;
     }
     left -= here;
   }
-  const int seq = uniform(shape.tiles[2 * tile]), nth = uniform(shape.tiles[2 * tile + 1]) / 32;
   const int G = nq / nkv, heads = shape.heads, sets_of_group = shape.sets / nkv;
   const int g = set / sets_of_group, first_head = set % sets_of_group * heads;      // the last set of a group may have heads to spare
-  const int qlen = uniform(shape.q_len[seq]), ctx = uniform(shape.ctx_len[seq]), qs = uniform(shape.q_start[seq]);
   // row r of the sequence: query r / heads, head first_head + r % heads
-  const int rows = qlen * heads, row0 = kRowsBlock * nth;
-  const int pos0 = ctx - qlen, k_last = pos0 + (min(row0 + kRowsBlock, rows) - 1) / heads;
+  const int rows = qlen * heads, row0 = kRowsBlock * nth + (SHARED ? BLOCK_ROWS * (SUBS - 1 - of_set) : 0);
+  if (SHARED && row0 >= rows) return;
+  const int pos0 = ctx - qlen, k_last = pos0 + (min(row0 + BLOCK_ROWS, rows) - 1) / heads;
   int lo = 0, hi = k_last;
-  if (shape.parts > 1) share_of_walk(lo, hi, kRowsKeys, part, shape.parts);
+  if (!SHARED && shape.parts > 1) share_of_walk(lo, hi, kRowsKeys, part, shape.parts);
   const int stages = hi >= lo ? (hi - lo) / kRowsKeys + 1 : 0;
 
   typedef __attribute__((address_space(3))) unsigned char* lds_address_t;
@@ -324,9 +384,10 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   };
 
   // this wave's rows; one without any walks along for its share of the fetches
-  const int wave_row = row0 + 64 * wave;
-  const bool has_rows = wave_row < rows;
+  const int wave_row = SHARED ? row0 : row0 + 64 * wave;
+  const bool has_rows = SHARED || wave_row < rows;
   if (stages > 0) fetch(0, 0, places(0));
+  if (SHARED && stages > 1) fetch(1, 1, places(1));
   int pos[2], query[2], head[2];
   RowState st;
 #pragma unroll
@@ -351,16 +412,43 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   // the last key of the part that every row of the wave sees
   const int last_seen = min(has_rows ? pos0 + wave_row / heads : ctx, hi);
   const int steps = stages ? (hi - lo) / 32 + 1 : 0;      // of 32 keys, four a stage
-  rows_wait_then_barrier<0>();
-  if (stages > 1) fetch(1, 1, places(1));
-  // The keys of step `i` of the stage in buffer `buf`; its values.
+  if constexpr (SHARED) {
+    if (stages > 1) rows_wait_then_barrier<8>();      // the first stage has landed
+    else rows_wait_then_barrier<0>();
+  } else {
+    rows_wait_then_barrier<0>();
+    if (stages > 1) fetch(1, 1, places(1));
+  }
+  // The keys of step `i` of the stage in buffer `buf`; its values.  Where waves share a stage, this wave's step of it.
+  uint32_t my_keys[4], my_values[2][2];
+  if constexpr (SHARED) {
+    const uint32_t at = (wave >> 1) * 16384;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) my_keys[ks] = at + (wave & 1) * 4096 + (kaddr[ks] ^ ((wave & 1) * 64));
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) my_values[c][dt] = at + 8192 + dt * 4096 + li * 128 + ((((4 * (wave & 1) + 2 * c + lk) ^ swz(li)) << 4) ^ (dt * 64));
+  }
   auto keys = [&](int buf, int i) __attribute__((always_inline)) {
+    if constexpr (SHARED) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) st.k[ks] = *reinterpret_cast<const uint4*>(ring + buf * kRowsStageBytes + my_keys[ks]);
+      return;
+    }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
       st.k[ks] = *reinterpret_cast<const uint4*>(ring + buf * kRowsStageBytes + (i >> 1) * 16384 + (i & 1) * 4096 + (kaddr[ks] ^ ((i & 1) * 64)));
   };
   auto values = [&](int buf, int i) __attribute__((always_inline)) {
     // value row 32 dt + li, keys 32 i + 16 c + 8 lk ..
+    if constexpr (SHARED) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) st.v[c][dt] = *reinterpret_cast<const uint4*>(ring + buf * kRowsStageBytes + my_values[c][dt]);
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -400,6 +488,46 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
     settle(B, rows_half<1>(st, scale2, [] {}));
     __builtin_amdgcn_sched_barrier(0);
   };
+  if constexpr (SHARED) {
+    keys(0, 0);
+    rows_scores<0>(st);
+    int s = 0, buf = 0;
+    // A stage is a step: the one after the next is asked for in its middle, from places that were looked up at its start.
+    auto shared_step = [&](auto masked, bool more, bool another) __attribute__((always_inline)) {
+      constexpr bool MASKED = decltype(masked)::value;
+      const int first = s * kRowsKeys + 32 * wave;
+      const bool beyond = MASKED && first + 31 > last_seen;
+      const Pieces next = places(min(s + 2, stages - 1));
+      if (beyond) rows_mask<0>(st, first + 8 * lk, pos[0]);
+      settle(A, rows_half<0>(st, scale2, [&]() __attribute__((always_inline)) { values(buf, 0); }));
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        if (another) fetch(s + 2, buf, next);
+        keys(buf ^ 1, 0);
+      }
+      if (beyond) rows_mask<1>(st, first + 8 * lk, pos[1]);
+      settle(B, rows_half<1>(st, scale2, [] {}));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (; s + 2 < stages && s * kRowsKeys + 32 * wave + 31 <= last_seen; ++s, buf ^= 1) shared_step(std::false_type{}, true, true);
+    for (; s < stages; ++s, buf ^= 1) shared_step(std::true_type{}, s + 1 < stages, s + 2 < stages);
+    rows_sums<1>(st);
+    join_waves(st, ring, reinterpret_cast<float2*>(s_table), wave, lane);
+    // four lanes a row, 16 dimensions each
+    const int r = threadIdx.x >> 2, row = row0 + r, n = threadIdx.x & 3;
+    if (row >= rows) return;
+    const int h = first_head + row % heads;
+    if (h >= G) return;
+    float sum[16], inv;
+    joined_row(ring, reinterpret_cast<const float2*>(s_table), r, n, sum, inv);
+    uint16_t* dst = out + size_t(qs + row / heads) * (size_t(nq) * HD) + (g * G + h) * HD + 16 * n;
+#pragma unroll
+    for (int e = 0; e < 16; e += 8)
+      *reinterpret_cast<uint4*>(dst + e) = make_uint4(pack_bf16x2(sum[e] * inv, sum[e + 1] * inv), pack_bf16x2(sum[e + 2] * inv, sum[e + 3] * inv),
+                                                      pack_bf16x2(sum[e + 4] * inv, sum[e + 5] * inv), pack_bf16x2(sum[e + 6] * inv, sum[e + 7] * inv));
+    return;
+  }
   if (has_rows && steps > 0) {
     keys(0, 0);
     rows_scores<0>(st);
@@ -473,7 +601,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
 // Parts: two blocks a CU, each of eight stages at least, walks of less than 3,000 keys whole; where most tiles walk little beside a few long ones, those few
 // count.  Over 75 steps these cost 3 % more than the best of 1 to 32.
 RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside) {
-  RowsPlan plan = {0, 0, 0};
+  RowsPlan plan = {0, 0, 0, false};
   if (hd != 64 || !staged_prefill(page_size) || n_tiles < 1) return plan;
   const int G = nq / nkv, sets = (G + 7) / 8;
   plan.heads = (G + sets - 1) / sets;
@@ -487,23 +615,60 @@ RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size
   return plan;
 }
 
+// The launch for a step, between that one, the one whose waves share a block's rows (SHARED), and none.
+//
+// Both estimates in us.  Shared rows: 7 before and behind the walks; `chain`, the longest walk, at 0.85 a stage where its block has a CU's memory path
+// to itself, 1.2 beside another all along; `chip`, all stages on 512 places and 4.8 a round of blocks; where the places are taken once or
+// twice, what two blocks of a CU walk together.  Rows of their own: 12, 1.95 a stage of a part, all stages, and what the merge reads.  (Measured,
+// 14 heads in 2 groups: 2,048 tokens twice 34.8 and 43.1, 4,096 at once 52 and 61, 1,024 behind 7,168 60 and 52, 2,048 behind 30,720 314 and
+// 258; 32 heads in 8 groups: 2,048 tokens 37 and 43, twice 71 and 51.)
+// Beside the kernels of attention_mfma.h (where rows of their own do not pay) the lines are in blocks and stages: over 560 steps (ten shapes of
+// heads, one to eight prompts of 24 to 2,048 queries behind 0 to 30,000) those with 224 blocks of 64 rows and more took 0.32 to 1.02 of the time, with
+// fewer 0.8 to 1.4 and, from 150 and 1,000 stages on, 0.78 to 1.03; with one head a group and less than 600 stages up to 1.36; one long walk among
+// little else is what those cut.  Beside answers, which then have a launch of their own: from 250 blocks and 1,800 stages on 0.61 to 1.0, below to 1.6.
+// With this choice the steps take 0.84 of the time of before on average, the worst 1.03.
+RowsPlan attention_rows_choice(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside) {
+  RowsPlan rows = attention_rows_plan(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, beside);
+  if (hd != 64 || !staged_prefill(page_size) || n_tiles < 1) return rows;
+  const int G = nq / nkv;
+  RowsPlan shared = {0, 0, 1, true};
+  const int sets_of_group = (G + 7) / 8;
+  shared.heads = (G + sets_of_group - 1) / sets_of_group;
+  shared.sets = nkv * sets_of_group;
+  const float longest = ceilf(float(max(1, max_tile_ctx)) / kRowsKeys), mean = fminf(longest, float(max(1, mean_tile_walk)) / kRowsKeys);      // stages
+  const float blocks = 0.5f * float(n_tiles) * float(shared.heads) * float(shared.sets), stages = blocks * (mean + 0.5f);
+  const float rounds = floorf(blocks / 512.f), rest = blocks - 512.f * rounds;
+  const float of_rest = (rest > 256.f ? 1.22f : rest > 0.f ? 0.85f : 0.f) * (rounds > 0.f ? fmaxf(0.f, 2.f * mean - longest) : mean);
+  const float chain = (rounds > 0.f ? 1.2f : 0.85f) * longest, chip = fmaxf(0.65f / 256.f * stages + 4.8f / 512.f * blocks, 1.22f * rounds * mean + of_rest);
+  if (rows.parts) {
+    float us = 12.f + fmaxf(1.95f * ceilf(longest / float(rows.parts)), 0.55f / 256.f * stages);
+    if (rows.parts > 1) us += 2.f + 5.3e-5f * float(n_tiles) * 32.f * float(nq) * float(rows.parts);
+    return 1.05f * (7.f + fmaxf(chain, chip)) < us ? shared : rows;
+  }
+  if (beside > 0) return blocks >= 250.f && stages >= 1800.f && chain <= 8.f + 1.4f * chip ? shared : rows;
+  if (blocks < 224.f) return blocks >= 150.f && stages >= 1000.f && chain <= 12.f + 1.5f * chip ? shared : rows;
+  return (G > 1 || stages >= 600.f) && chain <= 12.f + (G > 1 ? 3.f : 1.6f) * chip ? shared : rows;
+}
+
 int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
                           const int32_t* block_tables, int max_blocks, const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
                           const int32_t* tiles, int n_tiles, uint16_t* out, float* part_o, float* part_ml, int nq, int nkv, int page_shift, int num_pages, float scale2) {
   constexpr int lds = 2 * kRowsStageBytes + kRowsTable * 4;
   const bool narrow = (size_t(num_pages) * nkv << page_shift) * 128 < (size_t(1) << 32);
-  auto kernel = narrow ? attention_rows_kernel<true> : attention_rows_kernel<false>;
-  static bool raised[2] = {false, false};
-  if (!raised[narrow]) {
+  const bool shared = plan.shared;
+  auto kernel = shared ? (narrow ? attention_rows_kernel<true, true> : attention_rows_kernel<false, true>)
+                       : (narrow ? attention_rows_kernel<true, false> : attention_rows_kernel<false, false>);
+  static bool raised[2][2] = {};
+  if (!raised[shared][narrow]) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) {
       set_error("sp_attention (prefill): cannot raise the LDS limit: %s", hipGetErrorString(e));
       return 1;
     }
-    raised[narrow] = true;
+    raised[shared][narrow] = true;
   }
   const RowsShape shape = {plan.heads, plan.sets, n_tiles, plan.parts, tiles, q_start, q_len, ctx_len};
-  kernel<<<n_tiles * plan.sets * plan.parts, 256, lds, s>>>(q, q_stride, k_pool, v_pool, block_tables, max_blocks, shape, out, part_o, part_ml,
+  kernel<<<n_tiles * plan.sets * plan.parts * (shared ? 4 : 1), 256, lds, s>>>(q, q_stride, k_pool, v_pool, block_tables, max_blocks, shape, out, part_o, part_ml,
                                                                  nq, nkv, page_shift, num_pages, scale2);
   return check_launch("sp_attention (prefill)");
 }
@@ -519,5 +684,18 @@ extern "C" int sp_attention_rows_plan(int hd, int page_size, int nq, int nkv, in
   plan[0] = p.heads;
   plan[1] = p.sets;
   plan[2] = p.parts;
+  return p.parts == 0;
+}
+
+// ... and what it does with them in the end: plan = {heads of a set, sets, parts, whether a block's waves share its rows}.  Returns 1 where the other
+// kernels take them, else 0.  Runs nothing: for tests.
+extern "C" int sp_attention_rows_choice(int hd, int page_size, int nq, int nkv, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long beside,
+                                        int* plan) {
+  if (nkv < 1 || nq < nkv || nq % nkv || page_size < 1 || n_tiles < 1 || max_tile_ctx < 1 || !plan) return 1;
+  const sprout::RowsPlan p = sprout::attention_rows_choice(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk > 0 ? mean_tile_walk : max_tile_ctx, beside);
+  plan[0] = p.heads;
+  plan[1] = p.sets;
+  plan[2] = p.parts;
+  plan[3] = p.shared;
   return p.parts == 0;
 }
