@@ -6,7 +6,7 @@ into a HIP graph (through torch's capture of the current stream, which our kerne
 replayed with new values in the same device buffers.  Sampling is part of the graph, so one
 descriptor upload, one graph launch and one small download make a step.
 
-Shapes are bucketed: the number of sequences to a power of two (missing ones are filled with
+Shapes are bucketed: the number of sequences to a power of two or, from 33 to 256, three quarters of it (missing ones are filled with
 one-token dummies that write no cache), the block-table width and the key splits of attention to a
 power-of-two context.  Nothing in a graph depends on the values of a step.
 
@@ -34,6 +34,16 @@ from .batch import (STEP_ARRAY_NAMES, CacheSlotView, KeptWorkspace, OwnedNames, 
 
 def _bucket(n: int, floor: int = 1) -> int:
     return max(floor, 1 << max(0, (n - 1)).bit_length())
+
+
+def sequence_rows(n: int) -> int:
+    """The rows of the recorded step that n requests run as: the bucket's, of 64 to 256 three quarters of them where those suffice.
+
+    Products take rows in tiles of 16, attention and sampling launch blocks for every one.  Requests at 190 to 4,096 tokens, us a step as one
+    of the whole bucket and so: 0.5B sizes 45 1,150 and 1,125, 70 1,575 and 1,501, 150 1,999 and 1,862; 7B sizes 45 4,882 and 4,630, 90 (to
+    2,000 tokens) 5,660 and 5,284."""
+    S = _bucket(n)
+    return S // 4 * 3 if 32 < S <= 256 and n <= S // 4 * 3 else S
 
 
 class _DecodeGraph:
@@ -101,6 +111,7 @@ class _DecodeGraph:
         self.sample_ws = torch.empty(max(1, ops.sample_workspace_floats(S, runner.vocab_size)), dtype=torch.float32,
                                      device=runner.device)
         self.graph = None
+        self.other = None          # the bucket's step of the other number of rows, once there is one (see sequence_rows)
         self.logits = None
         self._filled = -1          # number of real sequences at the last fill
         self._rows = [None] * S    # per row: which sequence and how many pages its table row holds
@@ -276,7 +287,7 @@ def _record(state) -> None:
 class DecodeGraphs:
     def __init__(self, runner, max_graphs: int = 32):
         self.runner = weakref.proxy(runner)
-        self.graphs: dict[tuple, _DecodeGraph] = {}      # (sequences, context bucket) -> recorded decode step
+        self.graphs: dict[tuple, _DecodeGraph] = {}      # (sequence bucket, context bucket) -> recorded decode step, that used last in front
         self.max_graphs = max_graphs
         self.replays = 0
         # steps with portions of prompts: (tokens and wanted places request by request, context bucket) -> graph
@@ -291,8 +302,8 @@ class DecodeGraphs:
     def _context_bucket(self, longest: int) -> int:
         return min(_bucket(longest, 256), -(-self.runner.max_positions // 256) * 256)
 
-    def _make_room(self) -> None:
-        if len(self.graphs) >= self.max_graphs:
+    def _make_room(self, held: int = 0) -> None:
+        while self.graphs and held + sum(1 + (g.other is not None) for g in self.graphs.values()) >= self.max_graphs:
             # the least recently used graph goes; a step launched ahead may still be running from it
             torch.cuda.current_stream().synchronize()
             self.graphs.pop(next(iter(self.graphs)))
@@ -356,20 +367,31 @@ class DecodeGraphs:
         """
         runner = self.runner
         n = len(entries)
-        S = _bucket(n)
+        S, rows = _bucket(n), sequence_rows(n)
         longest = max(e.seq.length for e in entries) + 1
         ctx_bucket = self._context_bucket(longest)
         key = (S, ctx_bucket)
-        state = self.graphs.pop(key, None)
+        state, other = self.graphs.pop(key, None), None
+        if state is not None:
+            if state.S != rows:           # the bucket's other step takes its place in front
+                state, other = state.other, state
+            else:
+                other = state.other
+            if other is not None:
+                other.other = None        # one names the other, not both each other: see __init__
         if state is None:
-            self._make_room()
-            state = _DecodeGraph(runner, S, ctx_bucket)
+            if other is not None and self.max_graphs < 2:
+                torch.cuda.current_stream().synchronize()      # see _make_room
+                other = None
+            self._make_room(other is not None)
+            state = _DecodeGraph(runner, rows, ctx_bucket)
+        state.other = other
         self.graphs[key] = state          # most recently used last
         previous, sources = (None, None) if feed is None else (feed[0].sampled, feed[1])
         state.fill(entries, params, counters, sources)
         state.launch(previous)
         self.replays += 1
-        pending = PendingDecode(state.sampled, n, self._host_tokens(S), state.logits)
+        pending = PendingDecode(state.sampled, n, self._host_tokens(rows), state.logits)
         for e in entries:
             runner.cache.commit(e.seq, e.seq.length + 1)
         return pending
