@@ -4,6 +4,7 @@
 
 namespace sprout {
 
+bool gemm_adds_parts(int T, int N, int K);      // gemm_bf16.hip
 constexpr int kProjectColumns = 512;      // most columns of w_o that a set of heads has where attention and projection share a block
 
 bool attention_mfma_supports(int hd, int page_size, int nq, int nkv) {
@@ -207,27 +208,37 @@ __global__ __launch_bounds__(64 * NW) void attention_project_kernel(
   }
 }
 
-// Whether that kernel takes a step, on how many waves (0: no).  Where its blocks are at most the CUs.  us a step of 24 layers at 14 heads of 64
-// in 2 groups and a width of 896, with attention and product (or the merge that projects) in launches of their own and so:
-//   contexts of 79: one sequence 683 and 648, 4 706 and 662, 8 (224 blocks) 726 and 680, 16 (448) 771 and 768;
-//   of 250: one 702 and 667, 8 750 and 721, 16 797 and 835; of 400 on eight waves: one 704 and 692, 4 728 and 705, 8 752 and 730.
-static int project_waves(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
-  const int sets = decode_sets(nq, nkv);
-  if (hd > 64 || nq / sets * hd > kProjectColumns || max_decode_ctx > 512 || (long long)((hidden + 63) / 64) * sets * n_decode > 256) return 0;
-  return max_decode_ctx <= 256 ? 4 : 8;
-}
-
 // Decode steps whose chunks' merge is folded into the output projection.  Worth it where the merged partial
 // results, which every block of a head and a tile of 16 sequences reads again, stay small beside the rows of w_o
 // (measured at 14 heads of 64, a width of 896, contexts of 4,096, tokens a second with the fold against merge and
 // projection kernels of their own: 8 sequences 8,250 against 7,930, 24 sequences 21,870 against 21,260, 32
 // sequences 27,400 against 26,660, 64 sequences 39,840 against 40,350).
+static bool merge_projects(int n_decode, int max_decode_ctx, int hidden) {
+  const int n_splits = (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk;
+  return n_decode <= 32 && n_splits > 1 && min(n_decode, 16) * n_splits <= 256 &&
+         hidden <= 2048;   // (wider: 28 heads of 128 at 3,584 +1%, 40 heads at 5,120 -0.5% with four tiles a wave)
+}
+
+// Whether the kernel above takes a step, on how many waves (0: no).  Where its blocks are at most the CUs.  us a step of 24 layers at 14 heads of 64
+// in 2 groups and a width of 896, with attention and product (or the merge that projects) in launches of their own and so:
+//   contexts of 79: one sequence 683 and 648, 4 706 and 662, 8 (224 blocks) 726 and 680, 16 (448) 771 and 768;
+//   of 250: one 702 and 667, 8 750 and 721, 16 797 and 835; of 400 on eight waves: one 704 and 692, 4 728 and 705, 8 752 and 730.
+// Over 24 other layouts (1 to 16 heads a set, 1 to 16 groups, heads of 32 to 64, widths of 128 to 8,192, 1 to 64 sequences) a layer's share takes 0.65 to 1.0 of
+// the time at contexts of up to 256.
+// Its sets add into the residual in whatever order they end, so where there are several it takes a step only if the launches of its own would add parts
+// in no fixed order either (the merge that projects, a product with K cut): a step that comes out the same bit for bit every time stays so.  (4 heads of 64
+// in 2 groups, a width of 256, contexts of 60: 6.4 us a layer and not 4.9; 14 in 2, 8,192 wide: 10.2 and not 7.5.)
+static int project_waves(int hd, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
+  const int sets = decode_sets(nq, nkv);
+  if (hd > 64 || nq / sets * hd > kProjectColumns || max_decode_ctx > 512 || (long long)((hidden + 63) / 64) * sets * n_decode > 256) return 0;
+  if (sets > 1 && !merge_projects(n_decode, max_decode_ctx, hidden) && !gemm_adds_parts(n_decode, hidden, nq * hd)) return 0;
+  return max_decode_ctx <= 256 ? 4 : 8;
+}
+
 bool attention_decode_project_takes(int hd, int page_size, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
   if (hd > 128 || !attention_mfma_supports(hd, page_size, nq, nkv) || !attention_mfma_decode_supports(nq, nkv)) return false;
-  if (n_decode >= 1 && max_decode_ctx >= 1 && hidden >= 16 && project_waves(hd, page_size, nq, nkv, n_decode, max_decode_ctx, hidden)) return true;
-  const int n_splits = (max_decode_ctx + kDecodeChunk - 1) / kDecodeChunk;
-  return n_decode >= 1 && n_decode <= 32 && n_splits > 1 && min(n_decode, 16) * n_splits <= 256 && hidden >= 16 &&
-         hidden <= 2048;   // (wider: 28 heads of 128 at 3,584 +1%, 40 heads at 5,120 -0.5% with four tiles a wave)
+  if (n_decode < 1 || max_decode_ctx < 1 || hidden < 16) return false;
+  return project_waves(hd, nq, nkv, n_decode, max_decode_ctx, hidden) || merge_projects(n_decode, max_decode_ctx, hidden);
 }
 
 // Tiles of 16 rows of w_o a wave takes in the folded kernel: one up to 16 sequences; with more, every tile of 16
@@ -250,7 +261,7 @@ static int launch_decode_project(hipStream_t s, const void* q, int q_stride, con
                                  int page_size, int num_pages, ScoreStage st, float scale) {
   constexpr int HD = 16 * DT;
   if constexpr (DT <= 4) {
-    if (const int waves = project_waves(HD, page_size, nq, nkv, n_decode, max_decode_ctx, hidden)) {
+    if (const int waves = project_waves(HD, nq, nkv, n_decode, max_decode_ctx, hidden)) {
       const int sets = decode_sets(nq, nkv);
       const dim3 grid((hidden + 63) / 64, sets, n_decode);
 #define SP_PROJECT(NW, POW2)                                                                                                            \

@@ -179,6 +179,18 @@ bool gemm_cuts_k(int T, int N, int K) {
   return splits > 1;
 }
 
+// Whether the accumulating product (rows that start at 16 bytes, as gemm_bf16() chooses its kernel) adds parts of K by float atomics, whose order no two
+// runs share.  Says no where it is not known.
+bool gemm_adds_parts(int T, int N, int K) {
+  if (K % 8 != 0) return false;
+  if (gemm_quad_takes(kQuadAccumulate, T, N, K)) {
+    int shape, splits;
+    quad_choice(kQuadAccumulate, T, N, K, &shape, &splits);
+    return splits > 1;
+  }
+  return (T <= 64 ? (N + 15) / 16 < 2048 || streams_few(T, N, K) : gemm_pipe_takes(T, N, K)) && gemm_cuts_k(T, N, K);
+}
+
 // mode 0 stores bfloat16 here; a float32 store of mode 0 is passed in as mode 2 by the caller.
 int gemm_bf16(hipStream_t s, const void* a, const void* w, int bias_dtype, const void* bias, int mode, int out_dtype,
               void* out, int T, int N, int K, bool* handled) {

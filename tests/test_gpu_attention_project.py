@@ -1,5 +1,6 @@
 """Attention of short contexts and the output projection in one launch: one to eight waves' keys, ragged batches, one key, pages of every kind,
-groups of one and of sixteen heads, widths that end within a block's rows; windows, sinks, capped scores, blocks of positions; and which steps take it."""
+groups of one and of sixteen heads, widths that end within a block's rows; windows, sinks, capped scores, blocks of positions; and which steps take it:
+none that launches of its own give the same bits every time."""
 import pytest
 import torch
 
@@ -7,7 +8,9 @@ from sprout_lm_amd import ops
 from tests.test_gpu_kernels import run_attention
 
 DEV = "cuda"
-SIZES = [(14, 2, 64, 16, 896), (3, 1, 32, 8, 100), (4, 4, 16, 16, 264), (8, 1, 64, 4, 17), (6, 2, 48, 12, 300), (32, 2, 16, 32, 65)]
+SIZES = [(14, 2, 64, 16, 896), (3, 1, 32, 8, 100), (32, 32, 16, 16, 120), (8, 1, 64, 4, 17), (12, 4, 48, 12, 300), (32, 2, 16, 32, 65)]
+# several sets of heads and a K that no product cuts: contexts of one chunk have launches of their own
+WHOLE = [(4, 4, 16, 16, 264), (6, 2, 48, 12, 300), (4, 2, 64, 16, 896), (4, 2, 32, 16, 8192)]
 CONTEXTS = [[1], [64], [65], [256], [79, 256, 1, 33], [257], [512], [511, 3, 300]]
 
 
@@ -23,6 +26,12 @@ def test_which_steps():
     assert all(takes(hd, page, nq, nkv, c, hidden) for nq, nkv, hd, page, hidden in SIZES for c in CONTEXTS)
     # as many blocks as CUs, a set's columns, a head's size: beyond them contexts of one chunk have launches of their own
     assert takes(64, 16, 14, 2, [79] * 8, 896) and not takes(64, 16, 14, 2, [79] * 16, 896)
+    for nq in range(1, 32):
+        for nkv in [n for n in range(2, nq + 1) if nq % n == 0]:
+            for hd in (16, 32, 48, 64):
+                # (a part of K holds 256 numbers at least)
+                assert nq * hd >= 512 or not any(takes(hd, 16, nq, nkv, [c] * n, w) for c in (1, 79, 256) for n in (1, 3, 8) for w in (16, 300, 896, 8192))
+    assert all(takes(hd, page, nq, nkv, c, hidden) == (max(c) > 256 and hidden <= 2048) for nq, nkv, hd, page, hidden in WHOLE for c in CONTEXTS)
     assert not takes(64, 16, 16, 1, [79], 896) and not takes(128, 16, 4, 2, [79], 896) and not takes(128, 16, 28, 4, [79], 3584)
 
 
@@ -61,3 +70,25 @@ def test_score_stages(options, contexts):
     want = out.float() @ w_o.float().T
     # each of the 896 outputs is off by a rounding of at most 2^-8 of its size on either side, weighed by rows of w_o of unit norm
     assert ((residual - before) - want).abs().max() <= 2 * 2.0 ** -8 * (out.float().abs() @ w_o.float().abs().T).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nq,nkv,hd,page,hidden", WHOLE)
+def test_steps_that_repeat_bit_for_bit(nq, nkv, hd, page, hidden):
+    g = torch.Generator(device=DEV).manual_seed(hidden)
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    contexts = [79, 256, 1]
+    T, pages = len(contexts), -(-256 // page)
+    q, k, v = rand(T, nq * hd).bfloat16(), rand(T * pages, nkv, page, hd).bfloat16(), rand(T * pages, nkv, hd, page).bfloat16()
+    w_o, before = (rand(hidden, nq * hd) * (nq * hd) ** -0.5).bfloat16(), rand(T, hidden)
+    tables = torch.arange(T * pages, device=DEV, dtype=torch.int32).view(T, pages)
+    batch = ops.AttentionBatch.build([1] * T, contexts, DEV)
+
+    def step():
+        residual, out = before.clone(), torch.full_like(q, float("nan"))
+        if not ops.attention(q, nq * hd, k, v, tables, batch, out, nq, nkv, hd, None, hd ** -0.5, project=(w_o, residual)):
+            ops.gemm(out, w_o, residual, accumulate=True)
+        return residual
+
+    first = step()
+    assert all(torch.equal(step(), first) for _ in range(40))
