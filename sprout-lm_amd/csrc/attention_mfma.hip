@@ -224,13 +224,17 @@ static bool merge_projects(int n_decode, int max_decode_ctx, int hidden) {
 //   contexts of 79: one sequence 683 and 648, 4 706 and 662, 8 (224 blocks) 726 and 680, 16 (448) 771 and 768;
 //   of 250: one 702 and 667, 8 750 and 721, 16 797 and 835; of 400 on eight waves: one 704 and 692, 4 728 and 705, 8 752 and 730.
 // Over 24 other layouts (1 to 16 heads a set, 1 to 16 groups, heads of 32 to 64, widths of 128 to 8,192, 1 to 64 sequences) a layer's share takes 0.65 to 1.0 of
-// the time at contexts of up to 256.
+// the time at contexts of up to 256.  On eight waves 0.75 to 0.98 at contexts of 300, at 500 0.84 to 1.02 and, where the model is narrow, so that the product's
+// launch is short, and most CUs walk 500 keys of 64 numbers each, to 1.18 (8 heads in 8 groups, 512 wide, 4 sequences 8.4 and 9.1; in one group, 32
+// sequences 9.2 and 10.9; with 160 blocks and fewer 0.84 to 0.99, but for 8 heads in one group and 3 to 6 sequences 1.03 to 1.09, 0.92 to 0.98 at 300).
 // Its sets add into the residual in whatever order they end, so where there are several it takes a step only if the launches of its own would add parts
 // in no fixed order either (the merge that projects, a product with K cut): a step that comes out the same bit for bit every time stays so.  (4 heads of 64
 // in 2 groups, a width of 256, contexts of 60: 6.4 us a layer and not 4.9; 14 in 2, 8,192 wide: 10.2 and not 7.5.)
 static int project_waves(int hd, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
   const int sets = decode_sets(nq, nkv);
-  if (hd > 64 || nq / sets * hd > kProjectColumns || max_decode_ctx > 512 || (long long)((hidden + 63) / 64) * sets * n_decode > 256) return 0;
+  const long long blocks = (long long)((hidden + 63) / 64) * sets * n_decode;
+  if (hd > 64 || nq / sets * hd > kProjectColumns || max_decode_ctx > 512 || blocks > 256) return 0;
+  if (max_decode_ctx > 256 && hidden < 768 && blocks * hd > 160 * 64) return 0;
   if (sets > 1 && !merge_projects(n_decode, max_decode_ctx, hidden) && !gemm_adds_parts(n_decode, hidden, nq * hd)) return 0;
   return max_decode_ctx <= 256 ? 4 : 8;
 }
@@ -322,6 +326,14 @@ int attention_mfma_decode_project(hipStream_t s, const void* q, int q_stride, co
 }
 
 }  // namespace sprout
+
+// On how many waves a block takes attention and output projection of a step of one-query sequences, 0 where they are launches of their own (or the
+// merge of the chunks projects).  Runs nothing: for tests.
+extern "C" int sp_attention_project_waves(int hd, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden) {
+  using namespace sprout;
+  if (hd < 16 || hd % 16 || nkv < 1 || nq < nkv || nq % nkv || n_decode < 1 || max_decode_ctx < 1 || hidden < 16) return 0;
+  return project_waves(hd, nq, nkv, n_decode, max_decode_ctx, hidden);
+}
 
 // Whether a step's prompts and one-query sequences may share a launch (sp_attention takes it where no other kernel takes the prompts): 1 or
 // 0.  Runs nothing: for tests.

@@ -148,6 +148,8 @@ int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, 
 int sp_attention_rows_plan(int hd, int page_size, int nq, int nkv, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long beside, int* plan);
 // ... and whether, in the end, a block's four waves share 64 of them.  Runs nothing: for tests.
 int sp_attention_rows_choice(int hd, int page_size, int nq, int nkv, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long beside, int* plan);
+// On how many waves a block takes attention and output projection of one-query sequences of short contexts, 0: in launches of their own.  Runs nothing: for tests.
+int sp_attention_project_waves(int hd, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden);
 // Whether a step's prompts and its one-query sequences share a launch.  Runs nothing: for tests.
 int sp_attention_mixed_pays(int hd, int nq, int nkv, int n_tiles, int n_decode, int max_decode_ctx, long long one_query_keys);
 // scores: what stands between q . k and the softmax, numbered like the variants above: 0 = the scaled product and

@@ -32,6 +32,7 @@ def _declare(lib):
                          c_int, c_int, c_int, c_int, c_i64, c_void, c_int, c_int, c_void, c_i64, c_void, c_int, c_int, c_int, c_int,
                          c_int, c_int, c_float, c_int, c_int, c_float, c_void, c_int, c_int, c_void, c_void, c_i64],
         "sp_attention_decode_project_takes": [c_int] * 7,
+        "sp_attention_project_waves": [c_int] * 6,
         "sp_attention_mixed_pays": [c_int] * 6 + [c_i64],
         "sp_attention_rows_plan": [c_int] * 7 + [c_i64, ctypes.POINTER(c_int)],
         "sp_attention_rows_choice": [c_int] * 7 + [c_i64, ctypes.POINTER(c_int)],
