@@ -1336,7 +1336,11 @@ static bool staged_paired(int n_tiles, int nq, int nkv, int hd, int splits, int 
 
 int attention_prefill_parts(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 // attention_rows.hip: more rows a wave, for plain softmax scores of heads of 64; no parts where it is not the faster one.
-struct RowsPlan { int heads, sets, parts; bool shared; };      // heads of a set, sets of all key/value heads, parts of a walk, waves that share their rows
+struct RowsPlan {
+  int heads, sets, parts;      // heads of a set, sets of all key/value heads, parts of a walk
+  bool shared;                 // a block's waves share its rows
+  bool direct = false;         // a block takes the entry of its own number
+};
 RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 RowsPlan attention_rows_choice(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside);
 int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,

@@ -34,6 +34,9 @@ namespace {
 
 // A stage: two runs of 64 keys, each 8 KB of key rows (64 keys of 128 bytes), then 8 KB of value rows (64 dimensions of 128 bytes).
 constexpr int kRowsBlock = 256, kRowsKeys = 128, kRowsStageBytes = 2 * 2 * 64 * 128, kRowsTable = 2048;
+// The longest list of tiles whose blocks an entry (a byte) and a group of 64 (four) fit where the stages lie afterwards.
+constexpr int kRowsEntries = 64 * (2 * kRowsStageBytes / (64 + 4));
+static_assert(kRowsEntries + kRowsEntries / 64 * 4 <= 2 * kRowsStageBytes && kRowsEntries % 64 == 0, "both lie in the stages' place");
 
 // 64 lanes x 16 bytes, each from an address of its own, into LDS at lds_address + 16 lane.
 __device__ __forceinline__ void lanes_to_lds(const void* address, uint32_t lds_address) {
@@ -221,9 +224,10 @@ __device__ __forceinline__ void joined_row(const unsigned char* ring, const floa
 
 // The shape of a launch.  An entry of the tile list stands for rows 256 n .. of its sequence and set, n counted by its place in the
 // sequence, which has at least as many tiles of 32 queries as blocks of rows: a set holds up to eight heads.  Entries beyond the last rows
-// have nothing to do.
+// have nothing to do.  (The list holds every tile of its sequences, each once.)
 struct RowsShape {
   int heads, sets, n_tiles, parts;      // heads of a set, sets of all key/value heads, entries of the tile list, parts of a walk
+  bool direct;                          // a block takes the entry of its own number, rows or not
   const int32_t *tiles, *q_start, *q_len, *ctx_len;
 };
 
@@ -250,7 +254,12 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
   // they start first; all sets and parts of an entry one after another, so that an XCD keeps to few of them where they come in eights.  Two blocks
   // run on a CU, the second 256 blocks behind the first: those behind take the entries the other way round, so that a CU has a long walk and a short
   // one (1,024 queries over 4,096 keys beside eight prompts of 128, 14 heads in 2 groups: 51 -> 40 us).
-  // What 64 entries of the list say, one a lane, is asked for together, the first 64 once: one by one they would be trips to memory of their own.
+  // What the list says of up to 256 entries, four a lane, is asked for together, and kept: one by one they would be trips to memory of their own.
+  // A longer list is read by the four waves, 1,024 entries in a trip, into LDS (`ring`, where no stage is yet): the blocks of each entry, and their sums
+  // over 64.  (With trips for 64 entries one behind the other, and all of them twice, a list of 512 entries took a block 24 us, those without rows too:
+  // 8 heads in 8 groups on shared rows, 256 prompts of 33 tokens 125 us and now 40, 32 of 1,024 272 and 119; 14 in 2, 256 of 64 37 and 32.)
+  // Sets of eight heads have no entries without rows: a block of a long list takes the entry of its own number (`direct`; 16 heads in 2 groups, 100
+  // prompts of 100 tokens 30 us and so 26.  With seven heads 256 prompts of 33, half of whose entries are without, 17 and so 25).
   struct Entry { int seq, nth, qlen, ctx, qs; };
   auto entry_of = [&](int e) __attribute__((always_inline)) {
     Entry entry = {0, 0, 0, 0, 0};
@@ -260,36 +269,127 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
     }
     return entry;
   };
-  auto with_rows = [&](const Entry& entry) { return __builtin_amdgcn_ballot_w64(kRowsBlock * entry.nth < entry.qlen * shape.heads); };
-  const int sets_parts = shape.sets * shape.parts * SUBS;
-  const Entry first_entries = entry_of(lane);
-  int n_entries = __builtin_popcountll(with_rows(first_entries));
-  for (int e = 64; e < shape.n_tiles; e += 64) n_entries += __builtin_popcountll(with_rows(entry_of(e + lane)));
-  const int n_blocks = n_entries * sets_parts;
+  auto blocks_of = [&](int nth, int qlen) { return min(max((qlen * shape.heads - kRowsBlock * nth + BLOCK_ROWS - 1) / BLOCK_ROWS, 0), SUBS); };
+  // over the wave: the sum of numbers 0 .. SUBS, and of those in the lanes before this one
+  auto sums = [&](int n, int& before) __attribute__((always_inline)) {
+    int all = 0;
+    before = 0;
+#pragma unroll
+    for (int bit = 0; 1 << bit <= SUBS; ++bit) {
+      const unsigned long long with = __builtin_amdgcn_ballot_w64(n >> bit & 1);
+      all += __builtin_popcountll(with) << bit;
+      before += int(__builtin_amdgcn_mbcnt_hi(uint32_t(with >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(with), 0))) << bit;
+    }
+    return all;
+  };
+  constexpr int KEPT = 4;
+  const bool listed_once = shape.n_tiles <= 64 * KEPT, direct = !SHARED && shape.direct;
+  const int groups = (shape.n_tiles + 63) / 64;
+  int* s_groups = reinterpret_cast<int*>(ring + kRowsEntries);
+  Entry kept[KEPT];
+  int here[KEPT], before[KEPT], all[KEPT], n_units = 0;
+  if (direct) {
+    n_units = shape.n_tiles;
+  } else if (groups == 1) {      // most steps: by itself, so that they run past what follows
+    kept[0] = entry_of(lane);
+    here[0] = blocks_of(kept[0].nth, kept[0].qlen);
+    n_units = sums(here[0], before[0]);
+  } else if (listed_once) {
+    int at[KEPT];
+#pragma unroll
+    for (int j = 0; j < KEPT; ++j) {
+      const int e = 64 * j + lane;
+      at[j] = 0, kept[j] = {0, 0, 0, 0, 0};
+      if (e < shape.n_tiles) at[j] = shape.tiles[2 * e], kept[j].nth = shape.tiles[2 * e + 1] / 32;
+    }
+#pragma unroll
+    for (int j = 0; j < KEPT; ++j)
+      if (64 * j + lane < shape.n_tiles) kept[j] = {at[j], kept[j].nth, shape.q_len[at[j]], shape.ctx_len[at[j]], shape.q_start[at[j]]};
+#pragma unroll
+    for (int j = 0; j < KEPT; ++j) {
+      here[j] = blocks_of(kept[j].nth, kept[j].qlen);
+      all[j] = sums(here[j], before[j]);
+      n_units += all[j];
+    }
+  } else {
+    for (int group0 = wave; group0 < groups; group0 += 16) {
+      int at[4], nth[4], qlen[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int e = 64 * (group0 + 4 * j) + lane, in = min(e, shape.n_tiles - 1);
+        at[j] = shape.tiles[2 * in], nth[j] = e == in ? shape.tiles[2 * in + 1] / 32 : 1 << 20;      // (beyond any sequence: without rows)
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qlen[j] = shape.q_len[at[j]];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (group0 + 4 * j >= groups) break;
+        const int n = blocks_of(nth[j], qlen[j]), of_group = sums(n, before[0]);
+        ring[64 * (group0 + 4 * j) + lane] = uint8_t(n);
+        if (lane == 0) s_groups[group0 + 4 * j] = of_group;
+      }
+    }
+    __syncthreads();
+    for (int group = lane; group < groups; group += 64) n_units += s_groups[group];
+#pragma unroll
+    for (int step = 1; step < 64; step *= 2) n_units += __shfl_xor(n_units, step, 64);
+    n_units = uniform(n_units);
+  }
+  const int sets_parts = shape.sets * shape.parts, n_blocks = n_units * sets_parts;
   int id = blockIdx.x;
   if (id >= n_blocks) return;
   if (const int first = id & ~255, eights = min(256, n_blocks - first) / 8; id & 256 && id - first < 8 * eights)
     id = first + 8 * (eights - 1 - (id - first) / 8) + id % 8;
-  const int set = id % sets_parts % shape.sets, of_set = id % sets_parts / shape.sets, part = SHARED ? 0 : of_set;
-  int tile = 0, seq = 0, nth = 0, qlen = 0, ctx = 0, qs = 0;
-  for (int e = 0, left = n_entries - 1 - id / sets_parts; e < shape.n_tiles; e += 64) {      // entry number `left` of those with rows
-    const Entry entry = e == 0 ? first_entries : entry_of(e + lane);
-    const unsigned long long with = with_rows(entry);
-    const int here = __builtin_popcountll(with);
-    if (left < here) {
-      const bool mine = (with >> lane & 1) && __builtin_popcountll(with & ((1ull << lane) - 1)) == left;
-      const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(mine));
-      auto its = [&](int v) { return __builtin_amdgcn_readlane(v, from); };
-      tile = e + from, seq = its(entry.seq), nth = its(entry.nth), qlen = its(entry.qlen), ctx = its(entry.ctx), qs = its(entry.qs);
-      break;
+  const int set = id % sets_parts % shape.sets, part = SHARED ? 0 : id % sets_parts / shape.sets;
+  int left = n_units - 1 - id / sets_parts, group = 0, tile = left, sub = 0;      // number `left` of the blocks of all entries
+  Entry entry;
+  if (direct) {
+    entry = entry_of(tile);
+    if (blocks_of(entry.nth, entry.qlen) == 0) return;
+  } else {
+    if (groups > 1 && listed_once) {
+#pragma unroll
+      for (int j = 0; j + 1 < KEPT; ++j)
+        if (group == j && left >= all[j]) {
+          left -= all[j];
+          group = j + 1, kept[0] = kept[j + 1], here[0] = here[j + 1], before[0] = before[j + 1];
+        }
+    } else if (groups > 1) {
+      for (int first = 0;; first += 64) {
+        const int sum = first + lane < groups ? s_groups[first + lane] : 0;
+        int upto = sum;
+#pragma unroll
+        for (int step = 1; step < 64; step *= 2) {
+          const int below = __shfl_up(upto, step, 64);
+          upto += lane >= step ? below : 0;
+        }
+        const int of_all = __builtin_amdgcn_readlane(upto, 63);
+        if (left < of_all) {
+          const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(left < upto));
+          group = first + from;
+          left -= __builtin_amdgcn_readlane(upto - sum, from);
+          break;
+        }
+        left -= of_all;
+      }
+      here[0] = ring[64 * group + lane];
+      sums(here[0], before[0]);
     }
-    left -= here;
+    const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(before[0] <= left && left < before[0] + here[0]));
+    tile = 64 * group + from;
+    sub = left - __builtin_amdgcn_readlane(before[0], from);
+    if (listed_once) {
+      auto its = [&](int v) { return __builtin_amdgcn_readlane(v, from); };
+      entry = {its(kept[0].seq), its(kept[0].nth), its(kept[0].qlen), its(kept[0].ctx), its(kept[0].qs)};
+    } else {
+      entry = entry_of(tile);
+    }
   }
+  const int seq = uniform(entry.seq), nth = uniform(entry.nth), qlen = uniform(entry.qlen), ctx = uniform(entry.ctx), qs = uniform(entry.qs);
   const int G = nq / nkv, heads = shape.heads, sets_of_group = shape.sets / nkv;
   const int g = set / sets_of_group, first_head = set % sets_of_group * heads;      // the last set of a group may have heads to spare
   // row r of the sequence: query r / heads, head first_head + r % heads
-  const int rows = qlen * heads, row0 = kRowsBlock * nth + (SHARED ? BLOCK_ROWS * (SUBS - 1 - of_set) : 0);
-  if (SHARED && row0 >= rows) return;
+  const int rows = qlen * heads, row0 = kRowsBlock * nth + BLOCK_ROWS * sub;
   const int pos0 = ctx - qlen, k_last = pos0 + (min(row0 + BLOCK_ROWS, rows) - 1) / heads;
   int lo = 0, hi = k_last;
   if (!SHARED && shape.parts > 1) share_of_walk(lo, hi, kRowsKeys, part, shape.parts);
@@ -602,7 +702,7 @@ __global__ __launch_bounds__(256, 2) void attention_rows_kernel(
 // count.  Over 75 steps these cost 3 % more than the best of 1 to 32.
 RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside) {
   RowsPlan plan = {0, 0, 0, false};
-  if (hd != 64 || !staged_prefill(page_size) || n_tiles < 1) return plan;
+  if (hd != 64 || !staged_prefill(page_size) || n_tiles < 1 || n_tiles > kRowsEntries) return plan;
   const int G = nq / nkv, sets = (G + 7) / 8;
   plan.heads = (G + sets - 1) / sets;
   plan.sets = nkv * sets;
@@ -611,6 +711,7 @@ RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size
   const bool cut = longest >= 3000;
   if (G < (cut ? 2 : 3) || (!cut && blocks < 192) || work < (G == 2 ? 3500 : beside > 0 ? 2200 : cut ? 1400 : 400)) return plan;
   const long long count = 2 * mean < longest ? max(1LL, blocks * mean / longest) : blocks;
+  plan.direct = n_tiles > 64 && plan.heads == 8;
   plan.parts = !cut ? 1 : int(max(1LL, min(min(512 / count, (longest + kRowsKeys - 1) / kRowsKeys / 8), (long long)kMaxPrefillSplits)));
   return plan;
 }
@@ -624,12 +725,16 @@ RowsPlan attention_rows_plan(int n_tiles, int nq, int nkv, int hd, int page_size
 // 258; 32 heads in 8 groups: 2,048 tokens 37 and 43, twice 71 and 51.)
 // Beside the kernels of attention_mfma.h (where rows of their own do not pay) the lines are in blocks and stages: over 560 steps (ten shapes of
 // heads, one to eight prompts of 24 to 2,048 queries behind 0 to 30,000) those with 224 blocks of 64 rows and more took 0.32 to 1.02 of the time, with
-// fewer 0.8 to 1.4 and, from 150 and 1,000 stages on, 0.78 to 1.03; with one head a group and less than 600 stages up to 1.36; one long walk among
+// fewer 0.8 to 1.4 and, from 150 and 1,000 stages on, 0.78 to 1.03; with one head a group and less than 600 stages up to 1.36, and with more than a round of
+// blocks whose walks are shorter than two stages on average 1.08 to 1.35 (256 prompts of 64 tokens 1.25, 32 of 512 0.98); one long walk among
 // little else is what those cut.  Beside answers, which then have a launch of their own: from 250 blocks and 1,800 stages on 0.61 to 1.0, below to 1.6.
-// With this choice the steps take 0.84 of the time of before on average, the worst 1.03.
+// With this choice the steps take 0.84 of the time of before on average, the worst 1.03.  Over 220 more, among them 130 of nine to 256 prompts at once, 0.68; what
+// takes longer are some of a hundred short prompts and more, for which two heads a wave had less to do before and behind its walks (14 heads in 2
+// groups, 256 prompts of 64 tokens 24.5 and 32 us, 100 of 100 21.8 and 27; 64 in 8, 64 of 32 14 and 15).  Rows of their own take 4 us more for every further
+// round of blocks (78 prompts of 2 to 207 tokens, 64 heads in 8 groups, one walk of 4,037 keys: in three parts 144 us, on shared rows 116).
 RowsPlan attention_rows_choice(int n_tiles, int nq, int nkv, int hd, int page_size, int max_tile_ctx, int mean_tile_walk, long long beside) {
   RowsPlan rows = attention_rows_plan(n_tiles, nq, nkv, hd, page_size, max_tile_ctx, mean_tile_walk, beside);
-  if (hd != 64 || !staged_prefill(page_size) || n_tiles < 1) return rows;
+  if (hd != 64 || !staged_prefill(page_size) || n_tiles < 1 || n_tiles > kRowsEntries) return rows;
   const int G = nq / nkv;
   RowsPlan shared = {0, 0, 1, true};
   const int sets_of_group = (G + 7) / 8;
@@ -641,13 +746,14 @@ RowsPlan attention_rows_choice(int n_tiles, int nq, int nkv, int hd, int page_si
   const float of_rest = (rest > 256.f ? 1.22f : rest > 0.f ? 0.85f : 0.f) * (rounds > 0.f ? fmaxf(0.f, 2.f * mean - longest) : mean);
   const float chain = (rounds > 0.f ? 1.2f : 0.85f) * longest, chip = fmaxf(0.65f / 256.f * stages + 4.8f / 512.f * blocks, 1.22f * rounds * mean + of_rest);
   if (rows.parts) {
-    float us = 12.f + fmaxf(1.95f * ceilf(longest / float(rows.parts)), 0.55f / 256.f * stages);
+    const float further = fmaxf(0.f, float(n_tiles) * float(rows.heads) / 8.f * float(rows.sets * rows.parts) / 512.f - 1.f);
+    float us = 12.f + fmaxf(1.95f * ceilf(longest / float(rows.parts)), 0.55f / 256.f * stages + 4.f * further);
     if (rows.parts > 1) us += 2.f + 5.3e-5f * float(n_tiles) * 32.f * float(nq) * float(rows.parts);
     return 1.05f * (7.f + fmaxf(chain, chip)) < us ? shared : rows;
   }
   if (beside > 0) return blocks >= 250.f && stages >= 1800.f && chain <= 8.f + 1.4f * chip ? shared : rows;
   if (blocks < 224.f) return blocks >= 150.f && stages >= 1000.f && chain <= 12.f + 1.5f * chip ? shared : rows;
-  return (G > 1 || stages >= 600.f) && chain <= 12.f + (G > 1 ? 3.f : 1.6f) * chip ? shared : rows;
+  return (G > 1 || (stages >= 600.f && (blocks <= 512.f || mean >= 2.f))) && chain <= 12.f + (G > 1 ? 3.f : 1.6f) * chip ? shared : rows;
 }
 
 int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q, int q_stride, const uint16_t* k_pool, const uint16_t* v_pool,
@@ -667,8 +773,9 @@ int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q
     }
     raised[shared][narrow] = true;
   }
-  const RowsShape shape = {plan.heads, plan.sets, n_tiles, plan.parts, tiles, q_start, q_len, ctx_len};
-  kernel<<<n_tiles * plan.sets * plan.parts * (shared ? 4 : 1), 256, lds, s>>>(q, q_stride, k_pool, v_pool, block_tables, max_blocks, shape, out, part_o, part_ml,
+  const RowsShape shape = {plan.heads, plan.sets, n_tiles, plan.parts, plan.direct, tiles, q_start, q_len, ctx_len};
+  // blocks of 64 rows of a sequence of t tiles: at most 32 t heads / 64, rounded up, which is t times (heads + 1) / 2 at most
+  kernel<<<n_tiles * plan.sets * plan.parts * (shared ? (plan.heads + 1) / 2 : 1), 256, lds, s>>>(q, q_stride, k_pool, v_pool, block_tables, max_blocks, shape, out, part_o, part_ml,
                                                                  nq, nkv, page_shift, num_pages, scale2);
   return check_launch("sp_attention (prefill)");
 }
