@@ -388,7 +388,7 @@ def cmd_demo(args) -> int:
     stats = engine.stats()
     replays = engine.model._graphs.replays if engine.model._graphs else 0
     summary = {"mode": "pressure" if args.pressure else "roomy", "rounds": rounds, "results": results, "stats": stats,
-               "graphs_recorded": len(engine.model._graphs.graphs) if engine.model._graphs else 0, "graph_replays": replays}
+               "graphs_recorded": engine.model._graphs.recorded if engine.model._graphs else 0, "graph_replays": replays}
     if args.json:
         print(json.dumps(summary, indent=2))
     else:

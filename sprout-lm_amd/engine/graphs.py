@@ -302,11 +302,20 @@ class DecodeGraphs:
     def _context_bucket(self, longest: int) -> int:
         return min(_bucket(longest, 256), -(-self.runner.max_positions // 256) * 256)
 
-    def _make_room(self, held: int = 0) -> None:
-        while self.graphs and held + sum(1 + (g.other is not None) for g in self.graphs.values()) >= self.max_graphs:
-            # the least recently used graph goes; a step launched ahead may still be running from it
+    @property
+    def recorded(self) -> int:
+        """Recorded decode steps that are kept."""
+        return sum(1 + (g.other is not None) for g in self.graphs.values())
+
+    def _make_room(self) -> None:
+        while self.recorded >= self.max_graphs and self.graphs:
+            # the least recently used graph goes, of a bucket with two that used longer ago; a step launched ahead may still be running from it
             torch.cuda.current_stream().synchronize()
-            self.graphs.pop(next(iter(self.graphs)))
+            oldest = next(iter(self.graphs))
+            if self.graphs[oldest].other is not None:
+                self.graphs[oldest].other = None
+            else:
+                self.graphs.pop(oldest)
 
     def portion_step(self, entries, record_at: int = 2):
         """Run a step that is not one token a request from a recorded graph, if its shape has been seen
@@ -373,18 +382,15 @@ class DecodeGraphs:
         key = (S, ctx_bucket)
         state, other = self.graphs.pop(key, None), None
         if state is not None:
-            if state.S != rows:           # the bucket's other step takes its place in front
-                state, other = state.other, state
-            else:
-                other = state.other
-            if other is not None:
-                other.other = None        # one names the other, not both each other: see __init__
+            state, other = (state, state.other) if state.S == rows else (state.other, state)      # the bucket's other step may take its place in front
         if state is None:
-            if other is not None and self.max_graphs < 2:
-                torch.cuda.current_stream().synchronize()      # see _make_room
-                other = None
-            self._make_room(other is not None)
+            if other is not None:
+                self.graphs[key] = other      # used last, before the one to come
+            self._make_room()
+            other = self.graphs.get(key)
             state = _DecodeGraph(runner, rows, ctx_bucket)
+        if other is not None:
+            other.other = None        # one names the other, not both each other: see __init__
         state.other = other
         self.graphs[key] = state          # most recently used last
         previous, sources = (None, None) if feed is None else (feed[0].sampled, feed[1])
