@@ -928,10 +928,21 @@ def pipe_plan(kind: int, T: int, N: int, K: int):
 
 def quad_plan(kind: int, T: int, N: int, K: int, hd: int = 0):
     """(block rows, block columns, splits of K, buffers of the activations) that the product on four waves a block would
-    take for T x N x K, or None where `pipe_plan`'s kernel or another has the product.  Runs nothing and needs no GPU."""
+    take for T x N x K, or None where `pipe_plan`'s kernel or another has the product.  Of gated products (PLAN_GATED) the best of the blocks whose
+    columns are whole sixty-fours: where `quad_odd_plan` has one, that runs.  Runs nothing and needs no GPU."""
     import ctypes
     plan = (ctypes.c_int * 4)()
     if library().sp_quad_plan(kind, T, N, K, hd, plan):
+        return None
+    return tuple(plan)
+
+
+def quad_odd_plan(T: int, N: int, K: int):
+    """(block rows, block columns, buffers of the activations) of a gated product of N gate and up rows that runs on blocks of 160 or 224 columns, or None
+    where it does not.  Runs nothing and needs no GPU."""
+    import ctypes
+    plan = (ctypes.c_int * 3)()
+    if library().sp_quad_odd_plan(T, N, K, plan):
         return None
     return tuple(plan)
 

@@ -1,7 +1,5 @@
 """Gated products on blocks of an odd number of tile columns a wave: every such shape, with token and row edges, few steps along K, and the
 activations, against float32 products of the same operands; and where the rule gives them a product."""
-import ctypes
-
 import pytest
 import torch
 
@@ -15,21 +13,17 @@ SIZES = [(193, 32800, 256, (256, 160)), (256, 33392, 256, (256, 160)), (511, 378
          (193, 41088, 320, (256, 192)), (700, 21552, 640, (256, 256))]
 
 
-def odd_plan(T, N, K):
-    plan = (ctypes.c_int * 3)()
-    return None if ops.library().sp_quad_odd_plan(T, N, K, plan) else tuple(plan[:2])
-
-
 def test_where_they_are_taken():
     try:
         ops.library()
     except Exception as e:      # no compiler here: nothing to ask
         pytest.skip(f"the kernel library cannot be built or loaded here: {e}")
     for T, N, K, shape in SIZES:
-        assert (odd_plan(T, N, K) or ops.quad_plan(ops.PLAN_GATED, T, N, K)[:2]) == shape, (T, N, K)
+        assert (ops.quad_odd_plan(T, N, K) or ops.quad_plan(ops.PLAN_GATED, T, N, K))[:2] == shape, (T, N, K)
+    assert ops.quad_odd_plan(640, 37888, 3584) == (320, 160, 2) and ops.quad_plan(ops.PLAN_GATED, 640, 37888, 3584)[1] % 64 == 0
     # 0.83, 0.91 and 0.81 of the time; 1.00, 1.00, 1.04 and 1.08 of it
-    assert odd_plan(320, 37888, 3584) and odd_plan(640, 37888, 3584) and odd_plan(264, 55296, 5120)
-    assert not any(odd_plan(*s) for s in ((264, 37888, 3584), (640, 9728, 896), (2048, 9728, 896), (2048, 37888, 3584)))
+    assert ops.quad_odd_plan(320, 37888, 3584) and ops.quad_odd_plan(640, 37888, 3584) and ops.quad_odd_plan(264, 55296, 5120)
+    assert not any(ops.quad_odd_plan(*s) for s in ((264, 37888, 3584), (640, 9728, 896), (2048, 9728, 896), (2048, 37888, 3584)))
 
 
 @pytest.mark.gpu
