@@ -1,17 +1,22 @@
-"""Prompt attention with two heads a wave over pages that hold more keys than the kernel fetches at a time, and as few as it takes,
-against the general kernel: walks that end within a run of 64 keys, in its first and in its last key, parts that begin within a page."""
+"""Prompt attention of heads of 64 over pages that hold more keys than the kernel fetches at a time, and as few as it takes,
+against the general kernel: walks that end within a run of 64 keys, in its first and in its last key, parts that begin within a page; on shared rows, on
+rows of their own and on those with walks in parts."""
 import pytest
 import torch
+
+from tests.attention_rows_helpers import OWN, PARTS, SHARED, form
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
 @pytest.mark.parametrize("page", [8, 64, 128, 256, 1024])
-@pytest.mark.parametrize("seqs", [[(4160, 2048)], [(4161, 2047)], [(16447, 1000), (300, 300)], [(33025, 513)]])
-def test_rows_attention_over_pages(page, seqs):
+@pytest.mark.parametrize("seqs,expected", [([(4160, 2048)], SHARED), ([(4161, 2047)], SHARED), ([(16447, 1000), (300, 300)], PARTS), ([(33025, 513)], PARTS),
+                                           ([(2305, 2048), (2111, 2047), (2240, 2001)], OWN)])
+def test_rows_attention_over_pages(page, seqs, expected):
     from sprout_lm_amd import ops
     nq, nkv = 14, 2
+    assert form(nq, nkv, seqs, page=page) == expected
     g = torch.Generator(device=DEV).manual_seed(page + seqs[0][0])
     rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
     pages = [-(-c // page) for c, _ in seqs]

@@ -101,3 +101,33 @@ def test_steps_that_repeat_bit_for_bit(nq, nkv, hd, page, hidden):
 
     first = step()
     assert all(torch.equal(step(), first) for _ in range(40))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("contexts", [[79, 256, 200], [400, 300, 512]])
+def test_keys_and_values_that_are_not_finite(contexts):
+    """As attention and product in launches of their own have it: a key whose score is minus infinity weighs nothing, an infinite or undefined value is in
+    every column of the rows that see it, and in no other sequence's."""
+    nq, nkv, hd, page, hidden = 14, 2, 64, 16, 896
+    inf = float("inf")
+    g = torch.Generator(device=DEV).manual_seed(contexts[0])
+    rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
+    T, pages = len(contexts), 32
+    q, k, v = rand(T, nq, hd), rand(T * pages, nkv, page, hd), rand(T * pages, nkv, hd, page)
+    q[..., 3] = q[..., 3].abs() + 0.1
+    k[0, :, 0, 3], k[2, 0, 5, 3], k[pages + 15, 1, 15, 3] = -inf, -inf, -inf
+    v[pages + 1, 0, 11, 2], v[pages + 12, 1, 12, 0] = inf, -inf         # the second sequence alone
+    v[2 * pages + 3, 1, 40, 8] = float("nan")                           # the third
+    q, k, v = q.view(T, -1).bfloat16(), k.bfloat16(), v.bfloat16()
+    w_o, before = (rand(hidden, nq * hd) * (nq * hd) ** -0.5).bfloat16(), rand(T, hidden)
+    tables = torch.arange(T * pages, device=DEV, dtype=torch.int32).view(T, pages)
+    batch = lambda: ops.AttentionBatch.build([1] * T, contexts, DEV)
+    folded, apart, out = before.clone(), before.clone(), torch.full_like(q, float("nan"))
+    assert project_waves(hd, nq, nkv, contexts, hidden) == (4 if max(contexts) <= 256 else 8)
+    assert ops.attention(q, nq * hd, k, v, tables, batch(), out, nq, nkv, hd, None, 0.125, project=(w_o, folded))
+    assert ops.attention(q, nq * hd, k, v, tables, batch(), out, nq, nkv, hd, None, 0.125) is False
+    ops.gemm(out, w_o, apart, accumulate=True)
+    assert apart[0].isfinite().all() and not apart[1].isfinite().any() and apart[2].isnan().all()
+    assert torch.equal(folded.isnan(), apart.isnan()) and torch.equal(folded[apart.isinf()], apart[apart.isinf()])
+    # outputs of attention off by a rounding of at most 2^-8 of their size on either side, weighed by rows of w_o of unit norm
+    assert (folded[0] - apart[0]).abs().max() <= 2 * 2.0 ** -8 * (out[0].float().abs() @ w_o.float().abs().T).max()

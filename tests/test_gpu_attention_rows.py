@@ -1,6 +1,8 @@
-"""Prompt attention with two heads a wave (heads of 64, groups that fill its eight slots) against the general kernel."""
+"""Prompt attention of heads of 64 against the general kernel, in each form that its launch takes; keys, values and queries that are not finite."""
 import pytest
 import torch
+
+from tests.attention_rows_helpers import OWN, PARTS, SHARED, form
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -13,20 +15,23 @@ def attention(kind, q, k, v, tables, batch, nq, nkv, **options):
     return out.double()
 
 
-# (heads, groups, tokens a page, [(context, queries)]): whole walks and 2 to 32 parts of the keys, a part of which lies beyond some
-# rows; groups of 6, 7, 8 and 12 heads (an odd head, a wave without one, two sets); queries in no whole tiles; walks that end
+# (heads, groups, tokens a page, [(context, queries)], form): whole walks and 14 to 32 parts of the keys, a part of which lies beyond some
+# rows; groups of 4 to 8 and of 12 heads (two sets); queries in no whole tiles; walks that end
 # in the first and in the last of a stage's steps; more page numbers than LDS holds
-CASES = [(64, 8, 8, [(1024, 1024)]), (48, 8, 32, [(700, 700), (331, 300), (33, 33), (9, 1)]), (24, 2, 64, [(2049, 2049)]),
-         (14, 2, 16, [(4129, 2048)]), (14, 2, 16, [(4224, 2017), (2100, 31)]), (14, 2, 16, [(33001, 250)]),
-         (7, 1, 8, [(16384, 1000), (200, 200)]), (64, 8, 8, [(33000, 2048)]), (56, 8, 16, [(4096, 4096 - 2048), (130, 130)]),
+CASES = [(64, 8, 8, [(1024, 1024)], OWN), (48, 8, 32, [(700, 700), (331, 300), (33, 33), (9, 1)], SHARED), (24, 2, 64, [(2049, 2049)], SHARED),
+         (14, 2, 16, [(4129, 2048)], SHARED), (14, 2, 16, [(4224, 2017), (2100, 31)], SHARED), (14, 2, 16, [(33001, 250)], PARTS),
+         (7, 1, 8, [(16384, 1000), (200, 200)], PARTS), (64, 8, 8, [(33000, 2048)], OWN), (56, 8, 16, [(4096, 4096 - 2048), (130, 130)], OWN),
          # a one-query sequence whose parts are no whole number of sixteen bytes, before the prompt's in the workspace
-         (7, 1, 16, [(700, 1), (16384, 1000)])]
+         (7, 1, 16, [(700, 1), (16384, 1000)], PARTS),
+         # whole walks with sizes like those that run on shared rows above
+         (48, 8, 32, [(1700, 1700), (1331, 1300), (33, 33), (9, 1)], OWN), (24, 2, 64, [(2049, 2049), (2081, 2017)], OWN), (32, 8, 16, [(2129, 2048), (2100, 1931)], OWN)]
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
 def test_rows_attention(case):
     from sprout_lm_amd import ops
-    nq, nkv, page, seqs = CASES[case]
+    nq, nkv, page, seqs, expected = CASES[case]
+    assert form(nq, nkv, seqs, page=page) == expected
     g = torch.Generator(device=DEV).manual_seed(case)
     rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
     pages = [-(-c // page) for c, _ in seqs]
@@ -48,11 +53,13 @@ def test_rows_attention(case):
     assert ((got - want).abs() <= 2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-6).all()
 
 
-def test_keys_and_values_that_are_not_finite():
+@pytest.mark.parametrize("nq,nkv,ctx,n,expected", [(14, 2, 4129, 2048, SHARED), (64, 8, 3340, 1100, OWN), (14, 2, 6000, 1097, PARTS)])
+def test_keys_and_values_that_are_not_finite(nq, nkv, ctx, n, expected):
     """As the general kernel has it: a key whose score is minus infinity weighs nothing, an infinite value is one for every row that
     sees it, NaN stays with the rows and dimensions it reaches.  All before the first query, so that every row sees them."""
     from sprout_lm_amd import ops
-    nq, nkv, page, ctx, n = 14, 2, 16, 4129, 2048
+    assert form(nq, nkv, [(ctx, n)]) == expected
+    page, G = 16, nq // nkv
     inf = float("inf")
     g = torch.Generator(device=DEV).manual_seed(5)
     rand = lambda *shape: torch.randn(*shape, device=DEV, generator=g)
@@ -69,7 +76,7 @@ def test_keys_and_values_that_are_not_finite():
     got, want = (x.view(n, nq, 64) for x in results)
     assert got[100, 3].isnan().all()      # (the general kernel's row of a query that is NaN has zeros)
     got[100, 3] = want[100, 3] = 0.0
-    assert torch.equal(got.isnan(), want.isnan()) and want.isinf().sum() == 7 * (n - 1) + 6
+    assert torch.equal(got.isnan(), want.isnan()) and want.isinf().sum() == G * n - 1
     assert torch.equal(got[want.isinf()], want[want.isinf()])
     good = want.isfinite()
     assert good.float().mean() > 0.95
