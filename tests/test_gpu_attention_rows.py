@@ -82,3 +82,33 @@ def test_keys_and_values_that_are_not_finite(nq, nkv, ctx, n, expected):
     assert good.float().mean() > 0.95
     # as above, of values of unit size
     assert ((got - want)[good].abs() <= 2.0 ** -8 * 4 + 2.0 ** -8 * want[good].abs()).all()
+
+
+@pytest.mark.parametrize("nq,nkv,ctx,n,expected", [(14, 2, 4129, 2048, SHARED), (64, 8, 3340, 1100, OWN), (14, 2, 6000, 1097, PARTS)])
+def test_a_key_with_most_of_the_weight(nq, nkv, ctx, n, expected):
+    """A key behind the first 32 whose weight against their maximum is between 2^8 and 2^12, and lies between two numbers that bfloat16 holds: the running
+    maximum has to follow it, so that it weighs 1."""
+    assert form(nq, nkv, [(ctx, n)]) == expected
+    page, first, at = 16, 32, 128 + 5
+    bits = torch.arange(0x4000, 0x4200, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)      # 2 to 32
+    scores = bits[(bits.double() > 5.6) & (bits.double() < 8.2)]
+    weights = scores.double().exp()
+    worst = ((weights.float().bfloat16().double() - weights) / weights).abs().argmax()
+    b, weight = scores[worst], weights[worst]
+    assert abs(float(weight.float().bfloat16()) - weight) > 0.0035 * weight
+    g = torch.Generator(device=DEV).manual_seed(3)
+    pages = -(-ctx // page)
+    k, v = (torch.zeros(pages, nkv, *shape, dtype=torch.bfloat16, device=DEV) for shape in ((page, 64), (64, page)))
+    k[..., 0] = -30.0
+    k[:first // page, ..., 0] = 0.0
+    k[at // page, :, at % page, 0] = b.to(DEV)
+    late = (1 + torch.rand(nkv, 64, device=DEV, generator=g)).bfloat16()
+    v[at // page, :, :, at % page] = late
+    q = torch.zeros(n, nq, 64, dtype=torch.bfloat16, device=DEV)
+    q[..., 0] = 8.0                                   # times 0.125: a key's first number is its score
+    tables = torch.arange(pages, device=DEV, dtype=torch.int32)[None].contiguous()
+    from sprout_lm_amd import ops
+    got = attention(0, q.view(n, -1), k, v, tables, ops.AttentionBatch.build([n], [ctx], DEV), nq, nkv).view(n, nkv, nq // nkv, 64)
+    want = late.double() * float(weight) / (float(weight) + first)
+    # the result is rounded to bfloat16 (2^-8 of it); the other keys' values are 0, their weights sum up in float32, or are e^-30
+    assert ((got - want[None, :, None]).abs() <= 2.0 ** -8 * want[None, :, None] * 1.001).all()
