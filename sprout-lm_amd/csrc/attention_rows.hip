@@ -13,11 +13,12 @@
 // tile's scores while the matrix cores sum the other tile's values and multiply its next keys (rows_half).  Whether a row has outgrown its
 // running maximum is seen from the sum of the weights that were taken against it: no maximum of the scores is formed (30 instructions
 // less a step) until that happens.
-// What bounds it is power: a step takes 1,070 cycles at 1.75 GHz with random numbers, with zeros as many at 2.24 GHz.  An even share of all
-// stages for every block instead of parts of each walk (one run of stages, cut anywhere) took as long: where CUs have one block
+// A step takes 1,070 cycles, at 1.75 GHz with random numbers and at 2.24 GHz with zeros: the clock is power's, the cycles are not.  810 of them are the
+// instructions; what the other 260 wait for has not been found (once in four steps there is a barrier, for which the loads of a stage have to have landed).
+// An even share of all stages for every block instead of parts of each walk (one run of stages, cut anywhere) took as long: where CUs have one block
 // instead of two the others run faster.
-// 14 heads of 64 in 2 groups, 2,048 queries over 32,768 keys, merge included: 309 -> 279 us on one machine (840 TFLOP/s), 640 over 8,192
-// 65 -> 52, 250 over 31,000 87 -> 61; 32 heads in 8 groups, 2,048 over 10,240 413 -> 181 (those took the kernels of attention_mfma.h).
+// 14 heads of 64 in 2 groups, 2,048 queries over 32,768 keys, merge included: 309 -> 279 us on one machine (233 GFLOP, 840 TFLOP/s), 283 -> 263 on another; on
+// that one 640 over 8,192 59 -> 48, 250 over 31,250 78 -> 55; 32 heads in 8 groups, 2,048 over 10,240 407 -> 176 (those took the kernels of attention_mfma.h).
 // (Stages of 64 keys in a ring of three with operands read where they are used: 366 us where 128 took 298; s_setprio around the matrix
 // instructions changed nothing.)
 //
@@ -184,7 +185,7 @@ __device__ __forceinline__ float rows_half(RowState& st, float scale2, const BET
   return sum[0] + sum[1];
 }
 
-// Each wave's sums and statistics of the block's 64 rows to LDS, once no wave reads its stages any more: four bytes of row r and dimension
+// Each wave's sums and statistics of the block's 64 rows to LDS, once no wave reads its stages any more: four numbers of row r from dimension
 // 4 n .. of wave w at ((w * 64 + r) * 16 + (n ^ r % 16)) * 16, so that rows lie on different banks.
 __device__ __forceinline__ void join_waves(const RowState& st, unsigned char* ring, float2* ml, int wave, int lane) {
   const int li = lane & 31, lk = lane >> 5;
@@ -785,8 +786,8 @@ int launch_attention_rows(hipStream_t s, const RowsPlan& plan, const uint16_t* q
 
 }  // namespace sprout
 
-// What sp_attention would do with a step's prompts on this kernel: plan = {heads of a set, sets, parts}.  Returns 1 where it does not take
-// them, else 0.  Runs nothing: for tests.
+// A step's prompts on rows of a wave's own, were there no blocks that share them (sp_attention_rows_choice says what runs; the workspace is for the larger of
+// both): plan = {heads of a set, sets, parts}.  Returns 1 where the other kernels are the faster ones, else 0.  Runs nothing: for tests.
 extern "C" int sp_attention_rows_plan(int hd, int page_size, int nq, int nkv, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long beside,
                                       int* plan) {
   if (nkv < 1 || nq < nkv || nq % nkv || page_size < 1 || n_tiles < 1 || max_tile_ctx < 1 || !plan) return 1;

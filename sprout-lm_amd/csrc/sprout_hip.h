@@ -144,9 +144,9 @@ int64_t sp_attention_workspace_floats(int dtype, int hd, int page_size, int nq, 
                                       int n_decode, int max_decode_ctx, int n_tiles, int max_tile_ctx);
 int64_t sp_attention_workspace_hinted(int dtype, int hd, int page_size, int nq, int nkv, int kernel_kind, int n_decode, int max_decode_ctx,
                                       int n_tiles, int max_tile_ctx, int mean_tile_walk, long long one_query_keys);
-// Whether heads of 64 of a step's prompts run as rows of all heads of a key/value head.  Runs nothing: for tests.
+// Whether heads of 64 of a step's prompts would run as rows of all heads of a key/value head, a wave's its own.  Runs nothing: for tests.
 int sp_attention_rows_plan(int hd, int page_size, int nq, int nkv, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long beside, int* plan);
-// ... and whether, in the end, a block's four waves share 64 of them.  Runs nothing: for tests.
+// ... and how they do run: so, on blocks whose four waves share 64 rows, or on other kernels.  Runs nothing: for tests.
 int sp_attention_rows_choice(int hd, int page_size, int nq, int nkv, int n_tiles, int max_tile_ctx, int mean_tile_walk, long long beside, int* plan);
 // On how many waves a block takes attention and output projection of one-query sequences of short contexts, 0: in launches of their own.  Runs nothing: for tests.
 int sp_attention_project_waves(int hd, int nq, int nkv, int n_decode, int max_decode_ctx, int hidden);
