@@ -117,8 +117,7 @@ def test_recorded_steps_at_real_layer_sizes_match_plain(tmp_path):
     print(f"recorded steps at real layer sizes: worst {worst:.2f} of the bound")
 
 
-@pytest.mark.parametrize("n,rows", [(40, 48), (50, 64)])
-def test_recorded_steps_of_many_sequences_at_real_layer_sizes(tmp_path, n, rows):
+def steps_at_real_layer_sizes(tmp_path, n, rows):
     """Between 17 and 64 sequences the decode kernels take the tokens in tiles along the grid (the q/k/v product
     with the norm folded in by 16, the accumulating products by 32) and the output head runs on the pipelined
     tiles: two layers with the sizes of Qwen2.5-0.5B, forty and fifty sequences at different positions (recorded steps of
@@ -144,6 +143,14 @@ def test_recorded_steps_of_many_sequences_at_real_layer_sizes(tmp_path, n, rows)
     worst = decode_through_graphs(runner, seqs, tokens, fed, steps, folder, f"{n} sequences")
     assert [(key, g.S) for key, g in runner._graphs.graphs.items()] == [((64, 256), rows)]
     print(f"recorded steps of {n} sequences at real layer sizes: worst {worst:.2f} of the bound")
+
+
+def test_recorded_steps_of_forty_sequences_at_real_layer_sizes(tmp_path):
+    steps_at_real_layer_sizes(tmp_path, 40, 48)
+
+
+def test_recorded_steps_of_fifty_sequences_at_real_layer_sizes(tmp_path):
+    steps_at_real_layer_sizes(tmp_path, 50, 64)
 
 
 def fed_step(runner, seqs, tokens, fed, takes, folder, dtype, label, recorded=True):
